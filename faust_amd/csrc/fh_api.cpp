@@ -119,6 +119,48 @@ DMatP make_dense(int dtype, int m, int n, const void* data, int ld, bool on_devi
   return M;
 }
 
+// The chain as op'd FP64 CSR factors in application order; false when it is
+// not one.  widest: the longest op'd row (1 << 30 when a factor does not know
+// its own), mean_max: the largest mean row length.
+static bool chain_csr_ops(const std::vector<DMatP>& f, char op, std::vector<ChainCsrOp>& ops, int* widest,
+                          double* mean_max) {
+  const int J = (int)f.size();
+  const char* e_ell = getenv("FH_CSR_ELL");
+  const bool ell_on = !(e_ell && e_ell[0] == '0');
+  int r = (op == 'N') ? f.back()->n : f.front()->m;
+  *widest = 0;
+  *mean_max = 0.0;
+  for (int i = 0; i < J; ++i) {
+    const DMat& S = (op == 'N') ? *f[J - 1 - i] : *f[i];
+    if (S.kind != K_CSR || S.dtype != FH_F64 || ((op == 'N') ? S.n : S.m) != r || (op != 'N' && !S.has_csc))
+      return false;
+    const bool tr = op != 'N';
+    const int wr = tr ? S.max_col : S.max_row;
+    *widest = std::max(*widest, wr < 0 ? (1 << 30) : wr);
+    const int rows = tr ? S.n : S.m;
+    *mean_max = std::max(*mean_max, (double)S.nnz / std::max(rows, 1));
+    const int ew = tr ? S.csr_tell_w : S.csr_ell_w;
+    ops.push_back({tr ? S.cp.as<int>() : S.rp.as<int>(), tr ? S.ri.as<int>() : S.ci.as<int>(),
+                   tr ? S.cv.as<double>() : S.v.as<double>(), rows, (int)S.nnz,
+                   ell_on && ew > 0 && ew % 8 == 0 && ew <= 32 ? 1 : 0});
+    r = rows;
+  }
+  return true;
+}
+
+size_t faust_ws_need_rm_f64(const std::vector<DMatP>& f, char op, int p, int* nbuf) {
+  std::vector<ChainCsrOp> ops;
+  int widest;
+  double mean;
+  if (f.empty() || p < RM_MIN_COLS || !chain_csr_ops(f, op, ops, &widest, &mean)) return 0;
+  const int in_rows = (op == 'N') ? f.back()->n : f.front()->m;
+  if (!csr_rm_fits(ops, in_rows, p)) return 0;
+  size_t r = (size_t)in_rows;  // the last factor's output is Y
+  for (size_t i = 0; i + 1 < ops.size(); ++i) r = std::max(r, (size_t)ops[i].rows);
+  *nbuf = std::min(2, (int)f.size());
+  return sizeof(double) * r * csr_rm_ld(p);
+}
+
 // Bytes of each of the (at most two) intermediates of an FP64 chain product;
 // *nbuf: how many of them the product uses.
 size_t faust_ws_need_f64(const std::vector<DMatP>& f, char op, int p, int* nbuf) {
@@ -131,7 +173,7 @@ size_t faust_ws_need_f64(const std::vector<DMatP>& f, char op, int p, int* nbuf)
 // Grow a Faust's own intermediates to `need` bytes (hipMalloc only when a
 // larger product than any before is requested) and return their addresses.
 ChainWs faust_ws_grow(DBuf* ws, size_t need, int nbuf, hipStream_t st, DBuf* ctl) {
-  ChainWs w{{nullptr, nullptr}, nullptr};
+  ChainWs w{{nullptr, nullptr}, nullptr, need};
   for (int b = 0; b < nbuf; ++b) {
     if (ws[b].bytes < need) {
       FH_HIP(hipStreamSynchronize(st));  // the old buffer may still be in use
@@ -154,9 +196,10 @@ ChainWs faust_ws_grow(DBuf* ws, size_t need, int nbuf, hipStream_t st, DBuf* ctl
 // ---------------------------------------------------------------- autotune
 // Execution forms of an FP64 CSR chain, all with the same bits: one launch
 // per factor, the staged one-launch chain (wc columns per workgroup), the
-// prefetched one-launch chain (wc columns, pf entries per row ahead).
+// prefetched one-launch chain (wc columns, pf entries per row ahead), one
+// launch per factor on row-major intermediates.
 struct ChainForm {
-  int kind;  // 0 per factor, 1 staged, 2 prefetched
+  int kind;  // 0 per factor, 1 staged, 2 prefetched, 3 row-major
   int wc, pf;
 };
 
@@ -245,33 +288,32 @@ void faust_multiply_f64(const std::vector<DMatP>& f, char op, const double* X, i
 
   // the chain as op'd CSR factors in application order, when it is one
   std::vector<ChainCsrOp> ops;
-  int r = in_rows0, widest = 0, nnz_max = 0;
+  int widest = 0;
   double mean_max = 0.0;
-  bool ok = true;
-  {
-    const char* e_ell = getenv("FH_CSR_ELL");
-    const bool ell_on = !(e_ell && e_ell[0] == '0');
-    for (int i = 0; i < J && ok; ++i) {
-      const DMat& S = (op == 'N') ? *f[J - 1 - i] : *f[i];
-      ok = S.kind == K_CSR && S.dtype == FH_F64 && ((op == 'N') ? S.n : S.m) == r && (op == 'N' || S.has_csc);
-      if (!ok) break;
-      const bool tr = op != 'N';
-      const int wr = tr ? S.max_col : S.max_row;
-      widest = std::max(widest, wr < 0 ? (1 << 30) : wr);
-      const int rows = tr ? S.n : S.m;
-      mean_max = std::max(mean_max, (double)S.nnz / std::max(rows, 1));
-      nnz_max = std::max(nnz_max, (int)S.nnz);
-      const int ew = tr ? S.csr_tell_w : S.csr_ell_w;
-      ops.push_back({tr ? S.cp.as<int>() : S.rp.as<int>(), tr ? S.ri.as<int>() : S.ci.as<int>(),
-                     tr ? S.cv.as<double>() : S.v.as<double>(), rows, (int)S.nnz,
-                     ell_on && ew > 0 && ew % 8 == 0 && ew <= 32 ? 1 : 0});
-      r = rows;
-    }
-  }
-  const int out_rows = r;
+  const bool ok = chain_csr_ops(f, op, ops, &widest, &mean_max);
+  int nnz_max = 0;
+  for (const auto& o : ops) nnz_max = std::max(nnz_max, o.nnz);
+  const int out_rows = ok ? ops.back().rows : 0;
   auto run = [&](const ChainForm& c, FaustTimers* tmr) {
     if (c.kind == 0) {
       per_factor(tmr);
+      return;
+    }
+    if (c.kind == 3) {
+      if (tmr) tmr->begin((size_t)J, st);
+      csr_rm_from_col(in_rows0, p, X, t1, st);
+      if (tmr) tmr->end((size_t)J, st);
+      const double* in = t1;
+      int in_rows = in_rows0;
+      for (int i = 0; i < J; ++i) {
+        const size_t slot = (op == 'N') ? (size_t)(J - 1 - i) : (size_t)i;
+        double* out = i == J - 1 ? Y : ((i & 1) ? t1 : t2);
+        if (tmr) tmr->begin(slot, st);
+        csr_rm_mul(ops[i], in_rows, p, in, out, i == J - 1, st);
+        if (tmr) tmr->end(slot, st);
+        in = out;
+        in_rows = ops[i].rows;
+      }
       return;
     }
     if (tmr) tmr->begin(0, st);
@@ -282,22 +324,29 @@ void faust_multiply_f64(const std::vector<DMatP>& f, char op, const double* X, i
     if (tmr) tmr->end(0, st);
   };
   auto done = [&](const ChainForm& c) {
-    if (launches) *launches = c.kind == 0 ? J : 1;
+    if (launches) *launches = c.kind == 0 ? J : c.kind == 3 ? J + 1 : 1;
   };
 
   if (ok) {
     // default form: prefetched (8 entries ahead unless the rows are long on
-    // average and some exceed 8), else the staged plan, else per factor
+    // average and some exceed 8), else row-major intermediates for blocks of
+    // columns, else the staged plan, else per factor
+    int rm_nbuf = 0;
+    const size_t rm_need = faust_ws_need_rm_f64(f, op, p, &rm_nbuf);
+    const bool rm_fits = rm_need > 0 && ws.cap >= rm_need && t1 && (rm_nbuf < 2 || t2);
+    const bool one_launch_off = getenv("FH_CHAIN_FUSED") || (getenv("FH_CHAIN_PF") && getenv("FH_CHAIN_PF")[0] == '0');
+    const bool rm_auto = rm_fits && mul_mode() == FH_MUL_AUTO && !one_launch_off;
     ChainForm def{0, 0, 0};
     const int pwc = csr_chain_pf_plan_f64(ops, in_rows0, p);
     const int swc = pwc > 0 ? 0 : csr_chain_plan_f64(ops, in_rows0, p);
     if (pwc > 0)
       def = {2, pwc, (widest <= 8 || mean_max <= 4.0) ? 8 : 16};
+    else if (rm_auto && (int64_t)nnz_max * p >= RM_TERMS_DEFAULT)
+      def = {3, 0, 0};
     else if (swc > 0)
       def = {1, swc, 0};
     ChainForm use = def;
-    const bool tunable = mul_mode() == FH_MUL_AUTO && autotune_on() && !getenv("FH_CHAIN_FUSED") &&
-                         !(getenv("FH_CHAIN_PF") && getenv("FH_CHAIN_PF")[0] == '0');
+    const bool tunable = mul_mode() == FH_MUL_AUTO && autotune_on() && !one_launch_off;
     if (tunable) {
       const std::string key = chain_sig(op, p, in_rows0, ops);
       bool known = false;
@@ -307,6 +356,7 @@ void faust_multiply_f64(const std::vector<DMatP>& f, char op, const double* X, i
         if (it != g_tune.end()) {
           use = it->second;
           known = true;
+          if (use.kind == 3 && !rm_fits) use = def;  // a caller whose workspace is too small for it
         }
       }
       if (!known && tune && !stream_capturing(st)) {
@@ -318,6 +368,7 @@ void faust_multiply_f64(const std::vector<DMatP>& f, char op, const double* X, i
           if (c.kind != def.kind || c.wc != def.wc || c.pf != def.pf) cand.push_back(c);
         };
         add({0, 0, 0});
+        if (rm_auto) add({3, 0, 0});
         const int fwc = csr_chain_fit_wc(ops, in_rows0, p);
         if (fwc > 0) add({1, fwc, 0});
         if (csr_chain_pf_fits(ops, in_rows0, p))
@@ -713,8 +764,10 @@ int fh_faust_multiply(fh_faust_t F, char op, const void* X, int p, void* Y, void
   hipStream_t st = (hipStream_t)stream;
   int nbuf = 0;
   if (F->f.front()->dtype == FH_F64) {
-    const size_t need = faust_ws_need_f64(F->f, op, p, &nbuf);
-    const ChainWs ws = faust_ws_grow(F->ws, need, nbuf, st);
+    size_t need = faust_ws_need_f64(F->f, op, p, &nbuf);
+    int rm_nbuf = 0;
+    need = std::max(need, faust_ws_need_rm_f64(F->f, op, p, &rm_nbuf));
+    const ChainWs ws = faust_ws_grow(F->ws, need, std::max(nbuf, rm_nbuf), st);
     faust_multiply_f64(F->f, op, (const double*)X, p, (double*)Y, st, ws, &F->timers, &F->last_launches);
   } else {
     const std::vector<DMatP> f = fp32_chain_factors(F->f, st);

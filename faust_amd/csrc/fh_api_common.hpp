@@ -109,8 +109,12 @@ DMatP make_dense(int dtype, int m, int n, const void* data, int ld, bool on_devi
 struct ChainWs {
   void* p[2];
   int* ctl;  // control block of the one-launch BSR chain (bsr_chain_ctl_bytes; zeroed when allocated), or null
+  size_t cap = 0;  // bytes of each non-null p[]
 };
 size_t faust_ws_need_f64(const std::vector<DMatP>& f, char op, int p, int* nbuf);
+// The same for the form with row-major intermediates (X's copy included);
+// 0 when the chain or its shape does not take it.
+size_t faust_ws_need_rm_f64(const std::vector<DMatP>& f, char op, int p, int* nbuf);
 ChainWs faust_ws_grow(DBuf* ws, size_t need, int nbuf, hipStream_t st, DBuf* ctl = nullptr);
 // Forgets the forms measured by the chain autotuners (FP64 and BSR / FP32 CSR).
 void autotune_clear();

@@ -189,6 +189,16 @@ void csr_chain_pf_run_f64(const std::vector<ChainCsrOp>& ops, int in_rows, int w
 // Columns per workgroup of the staged one-launch chain for this shape
 // (whatever the chain length), or 0 when it does not fit.
 int csr_chain_fit_wc(const std::vector<ChainCsrOp>& ops, int in_rows, int p);
+// The same chain with row-major intermediates, one launch per factor
+// (k_csr_rm_f64): csr_rm_from_col transposes X (column-major, ld = rows) into
+// rows of csr_rm_ld(p) values, csr_rm_mul applies one op'd factor to such rows
+// (out_col: Y column-major, ld = S.rows).  fits: the shapes it takes.
+constexpr int RM_MIN_COLS = 12;               // columns from which the form is measured
+constexpr int64_t RM_TERMS_DEFAULT = 1 << 20;  // entries x columns of a factor from which it is the unmeasured choice
+int csr_rm_ld(int p);
+bool csr_rm_fits(const std::vector<ChainCsrOp>& ops, int in_rows, int p);
+void csr_rm_from_col(int rows, int p, const double* X, double* R, hipStream_t st);
+void csr_rm_mul(const ChainCsrOp& S, int in_rows, int p, const double* X, double* Y, bool out_col, hipStream_t st);
 // C = alpha*op(A)*op(S) + beta*C, A dense col-major, S CSR.
 void dense_csr_f64(const double* A, int lda, char opA, int m, const DMat& S, char opS, double* C, int ldc,
                    double alpha, double beta, hipStream_t st);

@@ -14,6 +14,7 @@
 // GPU (two streams, two threads) race on it.  The intermediates are written
 // before they are read within a call, and the chain's counters are cleared by
 // the chain itself at its end, so nothing needs clearing between calls.
+#include <algorithm>
 #include <mutex>
 
 #include "fh_api_common.hpp"
@@ -79,7 +80,18 @@ extern "C" int fh_faust_multiply_noalloc(fh_faust_t F, char op, const void* X, i
       }
   int nbuf = 0;
   const bool act_f32 = F->act_dtype == FH_F32;
-  const size_t need = f64 ? faust_ws_need_f64(f, op, p, &nbuf) : faust_ws_need_mixed(f, op, p, &nbuf, act_f32);
+  size_t need = f64 ? faust_ws_need_f64(f, op, p, &nbuf) : faust_ws_need_mixed(f, op, p, &nbuf, act_f32);
+  if (f64) {
+    // room for the row-major form too where the array has it; without it the
+    // product runs in the forms that fit
+    int rm_nbuf = 0;
+    const size_t rm = std::max(need, faust_ws_need_rm_f64(f, op, p, &rm_nbuf));
+    rm_nbuf = std::max(rm_nbuf, nbuf);
+    if ((size_t)rm_nbuf * align256(rm) <= kScratchBytes) {
+      need = rm;
+      nbuf = rm_nbuf;
+    }
+  }
   const size_t slot = align256(need);
   // BSR chains also keep the one-launch chain's control block at the start of
   // the array (zero at load; every chain leaves its counters cleared)
@@ -91,7 +103,7 @@ extern "C" int fh_faust_multiply_noalloc(fh_faust_t F, char op, const void* X, i
                                 std::to_string(kScratchBytes) + "-byte scratch array");
   char* base = (nbuf > 0 || bsr) ? static_cast<char*>(scratch_address()) : nullptr;
   const ChainWs ws{{nbuf > 0 ? base + ctl_bytes : nullptr, nbuf > 1 ? base + ctl_bytes + slot : nullptr},
-                   bsr ? reinterpret_cast<int*>(base) : nullptr};
+                   bsr ? reinterpret_cast<int*>(base) : nullptr, need};
   if (f64)
     faust_multiply_f64(f, op, (const double*)X, p, (double*)Y, st, ws, nullptr, &F->last_launches, false);
   else

@@ -656,6 +656,152 @@ void csr_chain_pf_run_f64(const std::vector<ChainCsrOp>& ops, int in_rows, int w
   FH_LAUNCH_CHECK();
 }
 
+// ------------------------------------------------------ row-major chain
+// FP64 CSR chains on blocks of columns, one launch per factor with row-major
+// intermediates: X is transposed once (k_col2row_f64), every factor gathers
+// whole row segments, and the last one writes Y column-major through LDS.  A
+// workgroup computes 16 rows x a panel of 32 columns: the 16 lanes of a DPP
+// row share one row of S (two columns each), lane s loads the row's entry s,
+// and row_newbcast hands entry q to the 16 lanes, so an entry's gather is one
+// 256-byte read.  Column-major intermediates gather 8 bytes per lane from as
+// many cache lines, which is what bounds k_csr_spmm_f64 once X no longer
+// sits in L1.  Gathers go through a buffer resource whose range check drops
+// the lanes past the row's end or past column p: no branch, no traffic.
+// Workgroups are dealt to the 8 XCDs in turn, so each XCD takes a contiguous
+// run of the panel-major (panel, row block) list: with up to 8 panels an
+// XCD's L2 holds the one or two panels it gathers from.
+// Each output entry is the fma chain of k_csr_spmm_f64 (entries in row
+// order, from 0), so the bits are the same.
+// Measured, 6007 x 5003 and 5003^2 factors of 7 entries per row, 250 columns:
+// 9.7 us per factor (88 MB of gathers out of the L2s, 9 TB/s; 22 MB of
+// activations) and 6.4 us for the transpose, against 29 us per factor
+// column-major (52 us transposed, rows of up to 24 entries).  Two rows per
+// lane, with both rows' pointers and entries loaded together, gave 10.1 us.
+constexpr int RM_COLS = 32, RM_ROWS = 16;
+
+template <int Q>
+__device__ __forceinline__ unsigned rm_bcast(unsigned x) {
+  return (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x150 + Q, 0xf, 0xf, false);
+}
+
+// entries Q .. Q + 7 of the 16 held by the lanes: gathers, then the fma chain
+template <int Q>
+__device__ __forceinline__ void rm_batch8(const __amdgpu_buffer_rsrc_t rx, unsigned off, unsigned wlo, unsigned whi,
+                                          unsigned coff, int n, double& a0, double& a1) {
+  pfc_d2 x[8];
+  double w[8];
+#define FH_RM_GET(u)                                                                                             \
+  x[u] = __builtin_bit_cast(pfc_d2, __builtin_amdgcn_raw_buffer_load_b128(                                       \
+                                        rx, __builtin_elementwise_add_sat(rm_bcast<Q + u>(off), coff), 0, 0)); \
+  w[u] = __builtin_bit_cast(double, ((unsigned long long)rm_bcast<Q + u>(whi) << 32) | rm_bcast<Q + u>(wlo));
+  FH_RM_GET(0) FH_RM_GET(1) FH_RM_GET(2) FH_RM_GET(3) FH_RM_GET(4) FH_RM_GET(5) FH_RM_GET(6) FH_RM_GET(7)
+#undef FH_RM_GET
+  __builtin_amdgcn_sched_barrier(0);  // all gathers in flight before the first fma
+#pragma unroll
+  for (int u = 0; u < 8; ++u) {
+    const double f0 = fma(w[u], x[u].x, a0), f1 = fma(w[u], x[u].y, a1);
+    a0 = Q + u < n ? f0 : a0;
+    a1 = Q + u < n ? f1 : a1;
+  }
+}
+
+template <bool OUT_COL>
+__global__ __launch_bounds__(256) void k_csr_rm_f64(int rows, int p, const int* __restrict__ rp,
+                                                    const int* __restrict__ ci, const double* __restrict__ v,
+                                                    const double* __restrict__ X, unsigned xbytes, int ldr,
+                                                    double* __restrict__ Y, int ldy, int nrb, int npanels) {
+  __shared__ double tile[RM_ROWS][RM_COLS + 1];
+  const int t = threadIdx.x, s = t & 15;
+  const int total = nrb * npanels;
+  const int w0 = (blockIdx.x & 7) * (int)(gridDim.x >> 3) + (blockIdx.x >> 3);
+  if (w0 >= total) return;  // the whole workgroup
+  const int panel = w0 / nrb, rblk = w0 - panel * nrb;
+  const int c0 = panel * RM_COLS + 2 * s;
+  const unsigned coff = c0 < p ? (unsigned)c0 * 8u : 0xffffffffu;
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)X, 0, (int)xbytes, 0x00020000);
+  const int r = rblk * RM_ROWS + (t >> 4), rr = min(r, rows - 1);
+  const int e0 = rp[rr], len = r < rows ? rp[rr + 1] - e0 : 0;
+  double a0 = 0.0, a1 = 0.0;
+  for (int base = 0; __any(base < len); base += 16) {
+    const int n = len - base;  // entries left in this lane's row
+    const int e = s < n ? e0 + base + s : 0;
+    const int k = ci[e];
+    const unsigned long long wb = __builtin_bit_cast(unsigned long long, v[e]);
+    const unsigned off = s < n ? (unsigned)k * (unsigned)(ldr * 8) : 0xffffffffu;
+    rm_batch8<0>(rx, off, (unsigned)wb, (unsigned)(wb >> 32), coff, n, a0, a1);
+    if (__any(n > 8)) rm_batch8<8>(rx, off, (unsigned)wb, (unsigned)(wb >> 32), coff, n, a0, a1);
+  }
+  if (!OUT_COL) {
+    if (r < rows && c0 < p) *reinterpret_cast<pfc_d2*>(Y + (size_t)r * ldr + c0) = pfc_d2{a0, a1};
+    return;
+  }
+  tile[t >> 4][2 * s] = a0;
+  tile[t >> 4][2 * s + 1] = a1;
+  __syncthreads();
+  // lane -> row of the block, 16 columns at a time
+#pragma unroll
+  for (int q = 0; q < RM_COLS / 16; ++q) {
+    const int lr = t & 15, lc = (t >> 4) + 16 * q;
+    const int gr = rblk * RM_ROWS + lr, gc = panel * RM_COLS + lc;
+    if (gr < rows && gc < p) Y[(size_t)gc * ldy + gr] = tile[lr][lc];
+  }
+}
+
+// column-major (rows x p, ld ldx) -> row-major (rows x ldr), columns p .. ldr - 1 zero
+__global__ __launch_bounds__(256) void k_col2row_f64(int rows, int p, const double* __restrict__ X, int ldx,
+                                                     double* __restrict__ R, int ldr) {
+  __shared__ double tile[32][33];
+  const int t = threadIdx.x;
+  const int r0 = blockIdx.x * 32, c0 = blockIdx.y * 32;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int lc = (t >> 5) + 8 * q, lr = t & 31;
+    tile[lr][lc] = (r0 + lr < rows && c0 + lc < p) ? X[(size_t)(c0 + lc) * ldx + r0 + lr] : 0.0;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int lr = (t >> 4) + 16 * q, lc = 2 * (t & 15);
+    if (r0 + lr < rows && c0 + lc < ldr)
+      *reinterpret_cast<pfc_d2*>(R + (size_t)(r0 + lr) * ldr + c0 + lc) = pfc_d2{tile[lr][lc], tile[lr][lc + 1]};
+  }
+}
+
+int csr_rm_ld(int p) { return (p + 1) & ~1; }
+
+bool csr_rm_fits(const std::vector<ChainCsrOp>& ops, int in_rows, int p) {
+  if (ops.empty() || p < RM_MIN_COLS || in_rows < 1) return false;
+  size_t r = (size_t)in_rows;
+  for (const auto& o : ops) {
+    if (o.rows < 1) return false;
+    r = std::max(r, (size_t)o.rows);
+  }
+  // buffer offsets are 32-bit and the all-ones offset is out of range; launches are below 2^31 workgroups
+  return r * csr_rm_ld(p) * sizeof(double) < 0xffffff00u &&
+         (r / RM_ROWS + 1) * ((size_t)p / RM_COLS + 1) < (size_t)1 << 28;
+}
+
+void csr_rm_from_col(int rows, int p, const double* X, double* R, hipStream_t st) {
+  const int ldr = csr_rm_ld(p);
+  const dim3 grid((unsigned)((rows + 31) / 32), (unsigned)((ldr + 31) / 32));
+  hipLaunchKernelGGL(k_col2row_f64, grid, dim3(256), 0, st, rows, p, X, rows, R, ldr);
+  FH_LAUNCH_CHECK();
+}
+
+void csr_rm_mul(const ChainCsrOp& S, int in_rows, int p, const double* X, double* Y, bool out_col, hipStream_t st) {
+  const int ldr = csr_rm_ld(p);
+  const int nrb = (S.rows + RM_ROWS - 1) / RM_ROWS, npanels = (p + RM_COLS - 1) / RM_COLS;
+  const dim3 grid((unsigned)((nrb * npanels + 7) / 8 * 8));
+  const unsigned xbytes = (unsigned)((size_t)in_rows * ldr * sizeof(double));
+  if (out_col)
+    hipLaunchKernelGGL(k_csr_rm_f64<true>, grid, dim3(256), 0, st, S.rows, p, S.rp, S.ci, S.v, X, xbytes, ldr, Y,
+                       S.rows, nrb, npanels);
+  else
+    hipLaunchKernelGGL(k_csr_rm_f64<false>, grid, dim3(256), 0, st, S.rows, p, S.rp, S.ci, S.v, X, xbytes, ldr, Y,
+                       S.rows, nrb, npanels);
+  FH_LAUNCH_CHECK();
+}
+
 // C(i,j) = alpha * sum_{k in col j of op(S)} op(A)(i,k) * op(S)(k,j) + beta*C(i,j)
 // (cp, ri, cv) is the column-compressed form of op(S): CSC of S for op N,
 // CSR of S for op T.
