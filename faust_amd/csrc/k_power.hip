@@ -28,6 +28,8 @@
 // operators: with those in the loop, the compiler waited for every load in
 // flight at the start of each operator, the prefetched set included
 // (hierarchy 24.3 -> 23.6 s).
+#include <algorithm>
+#include <climits>
 #include <cstdlib>
 #include <map>
 #include <mutex>
@@ -48,6 +50,7 @@ struct PwOp {
   const double* v;  // sparse values or dense data (ld = rows of A)
   int lda;
   int rpo;      // sparse only: offset of the row pointers' copy in dynamic LDS, or -1
+  int width;    // sparse only: the longest row, -1 when unknown
   int64_t nnz;  // sparse only
 };
 
@@ -414,6 +417,319 @@ __global__ __launch_bounds__(PW_THREADS) void k_power_iteration(const PwJob* __r
 }
 
 // ---------------------------------------------------------------------------
+// LDS form: chains whose operators all fit one workgroup's LDS (at most 1024
+// rows each), one workgroup per chain like the persistent form, and the same
+// bits.  That form waits on global loads, on scalar loads of the operator
+// descriptors and on barriers of 16 waves whatever the chain; here every
+// entry is staged once, a workgroup has only as many waves as the longest
+// vector needs (one for up to 64, where no barrier is left), and a round's
+// two sums (the Rayleigh quotient and the next round's squared norm) share one
+// reduction, whose last six levels are lane permutes in registers.
+//
+// Staged layout: a sparse operator's entry q of row r at [q][r] (values, then
+// the columns of all operators behind them), so the 64 rows of a wave read
+// consecutive words; rows shorter than the operator's width are padded with
+// value -0 and the column of a slot that always holds +0, and adding -0
+// changes no bit of an fma chain.  A dense operator's row r, column q is at
+// [q][r] and needs no columns.  Rows of up to four entries are read into
+// registers while the operator before is computed.
+// Measured on the hierarchy of the Hadamard matrix of order 64 (10 iterations
+// per PALM4MSA, 300 launches of one or two chains of 2 to 10 operators): 339
+// -> 97 us per launch, 168 -> 99 ms in all.  Norms of chains of random
+// factors, us per call: 5 factors of 64^2 with 2 entries per row 374 -> 132,
+// 2 of 64^2 with 32 entries 1920 -> 454, a dense 64^2 one 1037 -> 199.
+constexpr int PL_MAX_OPS = 36;             // operators per chain (both chains' descriptors are kernel arguments)
+constexpr int PL_ROWS = 1024;              // longest vector
+constexpr int PL_LDS_BYTES = 152 * 1024;   // dynamic LDS (operators and the three vectors)
+
+struct PlOp {
+  const int* rp;    // sparse: row pointers, columns; dense: unused
+  const int* ci;
+  const double* v;  // sparse values or dense data
+  int kind, trans;  // as PwOp
+  int rows, cols;
+  int width;        // staged entries per row (sparse: the widest row, rounded up to 2)
+  int lda;
+};
+struct PlJob {
+  PlOp ops[PL_MAX_OPS];
+  int nops, n;
+  int ld;    // vector slots: the longest vector + 1, the last one always +0
+  int nval;  // staged values of all operators
+};
+struct PlArgs {
+  PlJob job[2];
+};
+
+__device__ __forceinline__ double pl_bits(unsigned lo, unsigned hi) {
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+// x of lane l + H in lane l (the lanes that the halving tree still uses)
+template <int H>
+__device__ __forceinline__ double pl_down(double x) {
+  const unsigned long long u = __builtin_bit_cast(unsigned long long, x);
+  const unsigned lo = (unsigned)u, hi = (unsigned)(u >> 32);
+  if constexpr (H == 32) {
+    return pl_bits(__builtin_amdgcn_permlane32_swap(lo, lo, false, false)[1],
+                   __builtin_amdgcn_permlane32_swap(hi, hi, false, false)[1]);
+  } else if constexpr (H == 16) {
+    return pl_bits(__builtin_amdgcn_permlane16_swap(lo, lo, false, false)[1],
+                   __builtin_amdgcn_permlane16_swap(hi, hi, false, false)[1]);
+  } else {  // row_shl:H
+    return pl_bits((unsigned)__builtin_amdgcn_update_dpp(0, (int)lo, 0x100 + H, 0xf, 0xf, true),
+                   (unsigned)__builtin_amdgcn_update_dpp(0, (int)hi, 0x100 + H, 0xf, 0xf, true));
+  }
+}
+// lane 0: the halving tree over the wave's 64 values; the same on every lane after
+__device__ __forceinline__ double pl_tree(double v) {
+  v = v + pl_down<32>(v);
+  v = v + pl_down<16>(v);
+  v = v + pl_down<8>(v);
+  v = v + pl_down<4>(v);
+  v = v + pl_down<2>(v);
+  v = v + pl_down<1>(v);
+  v = 0.0 + v;  // the chunk's sum added to the total
+  const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+  return pl_bits(__builtin_amdgcn_readfirstlane((unsigned)u), __builtin_amdgcn_readfirstlane((unsigned)(u >> 32)));
+}
+
+// canonical <x, y> and <y, y> over n <= 1024 values, and whether any y is not
+// 0; xt, yt: this thread's values (0 past n), which are also in LDS (x, y).
+template <int NT>
+__device__ __forceinline__ void pl_sums(const double* x, const double* y, int n, double xt, double yt, double* red,
+                                        int* flag, double& sxy, double& syy, int& any) {
+  const int t = threadIdx.x, l = t & 63;
+  double a = 0.0, b = 0.0;
+  int nz = 0;
+  if (NT <= 256) {  // one value per lane of the canonical 256
+    a = fma(xt, yt, 0.0);
+    b = fma(yt, yt, 0.0);
+    nz = yt != 0.0;
+  } else {
+    __syncthreads();  // y complete
+    if (t < RED_LANES)
+#pragma unroll
+      for (int m = 0; m < PL_ROWS / RED_LANES; ++m) {
+        const int i = t + m * RED_LANES;
+        if (i < n) {
+          const double u = x[i], w = y[i];
+          a = fma(u, w, a);
+          b = fma(w, w, b);
+          nz |= w != 0.0;
+        }
+      }
+  }
+  if (NT == 64) {
+    any = __any(nz);
+    sxy = pl_tree(a + 0.0);
+    syy = pl_tree(b + 0.0);
+    return;
+  }
+  constexpr int NW = NT < RED_LANES ? NT / 64 : RED_LANES / 64;
+  const int wnz = __any(nz);
+  if (t < 64 * NW) {
+    red[t] = a;
+    red[RED_LANES + t] = b;
+    if (l == 0) flag[t >> 6] = wnz;
+  }
+  __syncthreads();
+  // lane l of every wave: levels 128 and 64 of the tree (lanes past NT hold 0)
+  if (NW == 2) {
+    a = (red[l] + 0.0) + (red[l + 64] + 0.0);
+    b = (red[RED_LANES + l] + 0.0) + (red[RED_LANES + l + 64] + 0.0);
+    any = flag[0] | flag[1];
+  } else {
+    a = (red[l] + red[l + 128]) + (red[l + 64] + red[l + 192]);
+    b = (red[RED_LANES + l] + red[RED_LANES + l + 128]) + (red[RED_LANES + l + 64] + red[RED_LANES + l + 192]);
+    any = flag[0] | flag[1] | flag[2] | flag[3];
+  }
+  sxy = pl_tree(a);
+  syy = pl_tree(b);
+}
+
+struct PlPre {
+  double v[4];
+  int c[4];
+};
+
+template <int NT>
+__global__ __launch_bounds__(NT) void k_power_lds(PlArgs args, const double* __restrict__ x0, int maxit, double thr,
+                                                  double* __restrict__ out) {
+  extern __shared__ double lds[];  // values, three vectors, columns
+  __shared__ double red[2 * RED_LANES];
+  __shared__ int flag[4];
+  __shared__ int4 desc[PL_MAX_OPS];  // per operator: rows, width (0: dense), first value, first column (dense: columns)
+  const PlJob& job = args.job[blockIdx.x];
+  const int t = threadIdx.x, nops = job.nops, n = job.n, ld = job.ld;
+  double* const val = lds;
+  double* vec = lds + job.nval;
+  int* const col = reinterpret_cast<int*>(vec + 3 * ld);
+  double *xn = vec, *b0 = vec + ld, *b1 = vec + 2 * ld;
+  {
+    int vo = 0, co = 0;
+    for (int s = 0; s < nops; ++s) {
+      const PlOp o = job.ops[s];
+      const bool sp = o.kind == 1;
+      if (t == 0) desc[s] = make_int4(o.rows, sp ? o.width : 0, vo, sp ? co : o.cols);
+      if (t < o.rows) {
+        if (sp) {
+          const int p0 = o.rp[t], len = o.rp[t + 1] - p0;
+          for (int q = 0; q < o.width; ++q) {
+            const bool on = q < len;
+            const int p = on ? p0 + q : 0;
+            const double w = o.v[p];
+            const int c = o.ci[p];
+            val[vo + q * o.rows + t] = on ? w : -0.0;
+            col[co + q * o.rows + t] = on ? c : ld - 1;
+          }
+        } else {
+          const double* a = o.trans ? o.v + (size_t)t * o.lda : o.v + t;
+          const size_t st = o.trans ? 1 : (size_t)o.lda;
+#pragma unroll 8
+          for (int q = 0; q < o.cols; ++q) val[vo + q * o.rows + t] = a[q * st];
+        }
+      }
+      vo += o.rows * (sp ? o.width : o.cols);
+      co += sp ? o.rows * o.width : 0;
+    }
+  }
+  if (t < 3) vec[t * ld + ld - 1] = 0.0;
+  double xt = t < n ? x0[t] : 0.0;
+  if (t < n) b0[t] = xt;
+  __syncthreads();
+  // entries of row t of operator s, when its rows have at most four
+  auto fetch = [&](const int4 d, PlPre& f) {
+    const int r = min(t, d.x - 1), w = d.y;
+    if (w == 0 || w > 4) return;
+    const double* v = val + d.z + r;
+    const int* c = col + d.w + r;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      f.v[q] = v[q * d.x];
+      f.c[q] = c[q * d.x];
+    }
+    if (w > 2)
+#pragma unroll
+      for (int q = 2; q < 4; ++q) {
+        f.v[q] = v[q * d.x];
+        f.c[q] = c[q * d.x];
+      }
+  };
+  auto row = [&](const int4 d, const PlPre& f, const double* cur) {
+    const int w = d.y;
+    double acc = 0.0;
+    if (w == 0) {
+      const double* v = val + d.z + t;
+      const int cols = d.w;
+      int q = 0;
+      for (; q + 8 <= cols; q += 8) {
+        double m[8], x[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          m[u] = v[(q + u) * d.x];
+          x[u] = cur[q + u];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) acc = fma(m[u], x[u], acc);
+      }
+      for (; q < cols; ++q) acc = fma(v[q * d.x], cur[q], acc);
+      return acc;
+    }
+    if (w <= 4) {
+      const double y0 = cur[f.c[0]], y1 = cur[f.c[1]];
+      if (w > 2) {
+        const double y2 = cur[f.c[2]], y3 = cur[f.c[3]];
+        acc = fma(f.v[1], y1, fma(f.v[0], y0, acc));
+        return fma(f.v[3], y3, fma(f.v[2], y2, acc));
+      }
+      return fma(f.v[1], y1, fma(f.v[0], y0, acc));
+    }
+    const double* v = val + d.z + t;
+    const int* c = col + d.w + t;
+    int q = 0;
+    for (; q + 8 <= w; q += 8) {
+      int k[8];
+      double m[8], x[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        k[u] = c[(q + u) * d.x];
+        m[u] = v[(q + u) * d.x];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) x[u] = cur[k[u]];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) acc = fma(m[u], x[u], acc);
+    }
+    for (; q < w; q += 2) {  // widths are even
+      const int k0 = c[q * d.x], k1 = c[(q + 1) * d.x];
+      const double m0 = v[q * d.x], m1 = v[(q + 1) * d.x];
+      const double x0v = cur[k0], x1v = cur[k1];
+      acc = fma(m1, x1v, fma(m0, x0v, acc));
+    }
+    return acc;
+  };
+  // lane s of every wave keeps operator s's descriptor
+  const int4 dl = desc[min(t & 63, nops - 1)];
+  auto get = [&](int s) {
+    return make_int4(__builtin_amdgcn_readlane(dl.x, s), __builtin_amdgcn_readlane(dl.y, s),
+                     __builtin_amdgcn_readlane(dl.z, s), __builtin_amdgcn_readlane(dl.w, s));
+  };
+  double lambda = 0.0, lambda_old = 1.0, sxy = 0.0, syy;
+  int it = 0, status = 0, any = 1;
+  pl_sums<NT>(b0, b0, n, xt, xt, red, flag, sxy, syy, any);
+  double yt = xt;  // the current vector's value, unnormalised
+  const double athr = fabs(thr);
+  PlPre f0, f1;
+  while ((fabs(lambda_old - lambda) > athr || fabs(lambda) <= athr) && it < maxit) {
+    it++;
+    lambda_old = lambda;
+    const double nrm = sqrt(syy);
+    if (nrm == 0.0) {
+      status = 1;
+      break;
+    }
+    int4 d = get(nops - 1);
+    fetch(d, f0);
+    const double inv = 1 / nrm;
+    xt = yt * inv;  // yt is +0 past n, inv finite or not: the lanes past n are not stored
+    if (t < n) xn[t] = xt;
+    __syncthreads();
+    const double* cur = xn;
+    double* nxt = b0;
+    for (int s = nops - 1; s >= 0; --s) {
+      const int4 dn = get(max(s - 1, 0));
+      if (s > 0) fetch(dn, f1);
+      yt = 0.0;
+      if (t < d.x) {
+        yt = row(d, f0, cur);
+        nxt[t] = yt;
+      }
+      if (s > 0) __syncthreads();
+      cur = nxt;
+      nxt = nxt == b0 ? b1 : b0;
+      d = dn;
+      f0 = f1;
+    }
+    if (t >= n) {
+      yt = 0.0;
+      xt = 0.0;
+    }
+    pl_sums<NT>(xn, cur, n, xt, yt, red, flag, sxy, syy, any);
+    if (!any) {
+      status = 2;
+      break;
+    }
+    lambda = sxy;
+  }
+  if (t == 0) {
+    double* o = out + 3 * blockIdx.x;
+    o[0] = (status == 2) ? 0.0 : lambda;
+    o[1] = (it < maxit) ? (double)it : -1.0;
+    o[2] = (double)status;
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Wide form: one launch per operator per round, for chains whose operators are
 // too large for a single CU to stream every round.  Each row is still one fma
 // chain on one lane (k ascending), so the result is bit-identical to the
@@ -706,7 +1022,9 @@ static std::vector<PwOp> pw_ops(const std::vector<ChainOp>& ops) {
       FH_CHECK(M.dtype == FH_F64, "power_iteration: FP64 dense or CSR factors only");
       o.kind = 1;
       o.trans = 0;
+      o.lda = 0;
       o.nnz = M.nnz;
+      o.width = tr ? M.max_col : M.max_row;
       if (tr) {
         FH_CHECK(M.has_csc, "power_iteration: CSC twin missing");
         o.rp = M.cp.as<int>();
@@ -726,6 +1044,7 @@ static std::vector<PwOp> pw_ops(const std::vector<ChainOp>& ops) {
       o.rp = o.ci = reinterpret_cast<const int*>(o.v);
       o.lda = M.m;
       o.nnz = 0;
+      o.width = -1;
     }
   }
   return h;
@@ -838,13 +1157,106 @@ static void power_iteration_persistent(const std::vector<std::vector<PwOp>>& hs_
   }
 }
 
+// the LDS form's job for a chain, when it fits: every operator dense or of
+// known width, at most PL_ROWS rows and columns, all entries in PL_LDS_BYTES;
+// lds receives the bytes
+static bool pl_job(const std::vector<PwOp>& h, int n, PlJob& j, size_t* lds) {
+  if (getenv("FH_POWER_WIDE")) return false;  // one of the other forms is asked for
+  if (h.empty() || h.size() > (size_t)PL_MAX_OPS || n < 1 || n > PL_ROWS) return false;
+  int longest = n;
+  size_t nval = 0, ncol = 0;
+  for (size_t s = 0; s < h.size(); ++s) {
+    const PwOp& o = h[s];
+    if (o.rows < 1 || o.cols < 1 || o.rows > PL_ROWS || o.cols > PL_ROWS || (o.kind == 1 && o.width < 0)) return false;
+    longest = std::max({longest, o.rows, o.cols});
+    const int w = o.kind == 1 ? std::max(2, (o.width + 1) & ~1) : o.cols;
+    nval += (size_t)o.rows * w;
+    if (o.kind == 1) ncol += (size_t)o.rows * w;
+    j.ops[s] = PlOp{o.rp, o.ci, o.v, o.kind, o.trans, o.rows, o.cols, w, o.lda};
+  }
+  j.nops = (int)h.size();
+  j.n = n;
+  j.ld = longest + 1;
+  *lds = sizeof(double) * (nval + 3 * (size_t)j.ld) + sizeof(int) * ncol;
+  j.nval = (int)std::min<size_t>(nval, INT_MAX);
+  return *lds <= PL_LDS_BYTES;
+}
+
+// start vector on the device: power_x0(PL_ROWS), whose first n values are
+// power_x0(n) for every n (one random sequence), uploaded once per device
+static const double* pl_x0() {
+  constexpr int kMaxDevices = 64;
+  static std::mutex mu;
+  static double* dx[kMaxDevices] = {};
+  int dev = 0;
+  FH_HIP(hipGetDevice(&dev));
+  FH_CHECK(dev >= 0 && dev < kMaxDevices, "power_iteration: device index out of range");
+  const std::vector<double>& x = power_x0(PL_ROWS);
+  std::lock_guard<std::mutex> lk(mu);
+  if (!dx[dev]) {
+    double* p = static_cast<double*>(dev_alloc(sizeof(double) * PL_ROWS));  // held to process end
+    FH_HIP(hipMemcpy(p, x.data(), sizeof(double) * PL_ROWS, hipMemcpyHostToDevice));
+    dx[dev] = p;
+  }
+  return dx[dev];
+}
+
+template <int NT>
+static void pl_go(const PlArgs& a, int jobs, size_t lds, int maxit, double thr, double* out, hipStream_t st) {
+  static const hipError_t attr = hipFuncSetAttribute((const void*)k_power_lds<NT>,
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, PL_LDS_BYTES);
+  FH_HIP(attr);
+  hipLaunchKernelGGL(k_power_lds<NT>, dim3(jobs), dim3(NT), lds, st, a, pl_x0(), maxit, thr, out);
+  FH_LAUNCH_CHECK();
+}
+
+// one or two chains in the LDS form; false (and nothing done) when one does not fit it
+static bool power_iteration_lds(const std::vector<std::vector<PwOp>>& hs, const std::vector<int>& ns, int maxit,
+                                double thr, double* lam, int* flags, hipStream_t st) {
+  const int J = (int)hs.size();
+  PlArgs a;
+  size_t lds = 0;
+  int longest = 1;
+  for (int k = 0; k < J; ++k) {
+    size_t b = 0;
+    if (!pl_job(hs[k], ns[k], a.job[k], &b)) return false;
+    lds = std::max(lds, b);
+    longest = std::max(longest, a.job[k].ld - 1);
+  }
+  DBuf dout(sizeof(double) * 3 * J);
+  double* out = dout.as<double>();
+  if (longest <= 64)
+    pl_go<64>(a, J, lds, maxit, thr, out, st);
+  else if (longest <= 128)
+    pl_go<128>(a, J, lds, maxit, thr, out, st);
+  else if (longest <= 256)
+    pl_go<256>(a, J, lds, maxit, thr, out, st);
+  else if (longest <= 512)
+    pl_go<512>(a, J, lds, maxit, thr, out, st);
+  else
+    pl_go<1024>(a, J, lds, maxit, thr, out, st);
+  double res[6];
+  FH_HIP(hipMemcpyAsync(res, out, sizeof(double) * 3 * J, hipMemcpyDeviceToHost, st));
+  FH_HIP(hipStreamSynchronize(st));
+  for (int k = 0; k < J; ++k) {
+    if (res[3 * k + 2] == 1.0) throw Error(FH_ERR_NUMERIC, "Can't normalize a zero-norm vector.");
+    lam[k] = res[3 * k];
+    flags[k] = (int)res[3 * k + 1];
+  }
+  return true;
+}
+
 double power_iteration_f64(const std::vector<ChainOp>& ops, int n, int maxit, double thr, int* flag,
                            hipStream_t st) {
   FH_CHECK(maxit > 0, "power_iteration: nbr_iter_max <= 0");
   std::vector<PwOp> h = pw_ops(ops);
-  if (!pw_persistent(h, n)) return power_iteration_wide(h, n, power_x0(n), maxit, thr, flag, st);
   double lam;
   int fl;
+  if (power_iteration_lds({h}, {n}, maxit, thr, &lam, &fl, st)) {
+    if (flag) *flag = fl;
+    return lam;
+  }
+  if (!pw_persistent(h, n)) return power_iteration_wide(h, n, power_x0(n), maxit, thr, flag, st);
   power_iteration_persistent({h}, {n}, maxit, thr, &lam, &fl, st);
   if (flag) *flag = fl;
   return lam;
@@ -854,13 +1266,19 @@ void power_iteration_pair_f64(const std::vector<ChainOp>& ops1, int n1, const st
                               int maxit, double thr, double* lam1, double* lam2, int* flag, hipStream_t st) {
   FH_CHECK(maxit > 0, "power_iteration: nbr_iter_max <= 0");
   std::vector<PwOp> h1 = pw_ops(ops1), h2 = pw_ops(ops2);
+  double lam[2];
+  int fl[2];
+  if (power_iteration_lds({h1, h2}, {n1, n2}, maxit, thr, lam, fl, st)) {
+    *lam1 = lam[0];
+    *lam2 = lam[1];
+    if (flag) *flag = fl[1];
+    return;
+  }
   if (!pw_persistent(h1, n1) || !pw_persistent(h2, n2)) {
     *lam1 = power_iteration_f64(ops1, n1, maxit, thr, flag, st);
     *lam2 = power_iteration_f64(ops2, n2, maxit, thr, flag, st);
     return;
   }
-  double lam[2];
-  int fl[2];
   power_iteration_persistent({h1, h2}, {n1, n2}, maxit, thr, lam, fl, st);
   *lam1 = lam[0];
   *lam2 = lam[1];

@@ -238,6 +238,9 @@ void dense_to_csr_f64(const double* D, int m, int n, DMat& out, hipStream_t st) 
   chunk_offsets(hc, nchc, n, offc, cp);
   const int64_t nnz = rp[m];
   out.nnz = nnz;
+  out.max_row = out.max_col = 0;
+  for (int i = 0; i < m; ++i) out.max_row = std::max(out.max_row, rp[i + 1] - rp[i]);
+  for (int j = 0; j < n; ++j) out.max_col = std::max(out.max_col, cp[j + 1] - cp[j]);
   out.rp.alloc(sizeof(int) * (m + 1));
   out.cp.alloc(sizeof(int) * (n + 1));
   FH_HIP(hipMemcpyAsync(out.rp.p, rp.data(), sizeof(int) * (m + 1), hipMemcpyHostToDevice, st));
