@@ -435,21 +435,24 @@ DMatP faust_get_product_f64(const std::vector<DMatP>& f, hipStream_t st) {
   return mat;
 }
 
-static bool chain_is_zero(const std::vector<DMatP>& f, hipStream_t st) {
+// count: dense factors whose entries have not been counted are counted now
+// (a wait); without it only the known counts are looked at, and a chain with
+// an all-zero factor gives norm 0 by its first round's product
+static bool chain_is_zero(const std::vector<DMatP>& f, bool count, hipStream_t st) {
   for (auto& x : f)
-    if (nnz_of(*x, st) == 0) return true;
+    if ((count || x->nnz >= 0) && nnz_of(*x, st) == 0) return true;
   return false;
 }
 
 // the power-iteration chain of F^H F (or F F^H, the smaller side); false when
 // the norm is known without it (*known: 1 for an empty Faust, 0 for a zero one)
 static bool spectral_chain(const std::vector<DMatP>& f, std::vector<ChainOp>& ops, int& n, double* known,
-                           hipStream_t st) {
+                           bool count, hipStream_t st) {
   if (f.empty()) {
     *known = 1.0;
     return false;
   }
-  if (chain_is_zero(f, st)) {
+  if (chain_is_zero(f, count, st)) {
     *known = 0.0;
     return false;
   }
@@ -467,11 +470,12 @@ static bool spectral_chain(const std::vector<DMatP>& f, std::vector<ChainOp>& op
 }
 
 // Transform::spectralNorm (faust_Transform.hpp:684-709)
-double faust_spectral_norm_f64(const std::vector<DMatP>& f, int maxit, double thr, int* flag, hipStream_t st) {
+double faust_spectral_norm_f64(const std::vector<DMatP>& f, int maxit, double thr, int* flag, hipStream_t st,
+                               bool count) {
   std::vector<ChainOp> ops;
   int n = 0;
   double known;
-  if (!spectral_chain(f, ops, n, &known, st)) return known;
+  if (!spectral_chain(f, ops, n, &known, count, st)) return known;
   double lam = power_iteration_f64(ops, n, maxit, thr, flag, st);
   return std::fabs(std::sqrt(lam));
 }
@@ -484,7 +488,7 @@ void faust_spectral_norm_pair_f64(const std::vector<DMatP>& f1, const std::vecto
   std::vector<ChainOp> o1, o2;
   int m1 = 0, m2 = 0;
   double k1, k2;
-  const bool p1 = spectral_chain(f1, o1, m1, &k1, st), p2 = spectral_chain(f2, o2, m2, &k2, st);
+  const bool p1 = spectral_chain(f1, o1, m1, &k1, false, st), p2 = spectral_chain(f2, o2, m2, &k2, false, st);
   if (p1 && p2) {
     double l1, l2;
     power_iteration_pair_f64(o1, m1, o2, m2, maxit, thr, &l1, &l2, flag, st);
@@ -855,12 +859,10 @@ int fh_norm_frob(int dtype, const void* M, int64_t n, double* out, void* stream)
   FH_API_BEGIN
   FH_CHECK(dtype == FH_F64 && out, "fh_norm_frob: FP64 only");
   hipStream_t st = (hipStream_t)stream;
-  DBuf s(sizeof(double));
-  reduce_dot_f64((const double*)M, (const double*)M, n, s.as<double>(), st);
-  double h;
-  FH_HIP(hipMemcpyAsync(&h, s.p, sizeof(double), hipMemcpyDeviceToHost, st));
+  double* s = mail() + MAIL_SUM;
+  reduce_dot_f64((const double*)M, (const double*)M, n, s, st);
   FH_HIP(hipStreamSynchronize(st));
-  *out = std::sqrt(h);
+  *out = std::sqrt(*s);
   FH_API_END
 }
 
@@ -868,10 +870,10 @@ int fh_dot(int dtype, const void* x, const void* y, int64_t n, double* out, void
   FH_API_BEGIN
   FH_CHECK(dtype == FH_F64 && out, "fh_dot: FP64 only");
   hipStream_t st = (hipStream_t)stream;
-  DBuf s(sizeof(double));
-  reduce_dot_f64((const double*)x, (const double*)y, n, s.as<double>(), st);
-  FH_HIP(hipMemcpyAsync(out, s.p, sizeof(double), hipMemcpyDeviceToHost, st));
+  double* s = mail() + MAIL_SUM;
+  reduce_dot_f64((const double*)x, (const double*)y, n, s, st);
   FH_HIP(hipStreamSynchronize(st));
+  *out = *s;
   FH_API_END
 }
 

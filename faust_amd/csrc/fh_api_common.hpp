@@ -128,7 +128,8 @@ void autotune_put_mode(const std::string& key, int mode);
 void faust_multiply_f64(const std::vector<DMatP>& f, char op, const double* X, int p, double* Y, hipStream_t st,
                         const ChainWs& ws, FaustTimers* tm = nullptr, int* launches = nullptr, bool tune = true);
 DMatP faust_get_product_f64(const std::vector<DMatP>& f, hipStream_t st);
-double faust_spectral_norm_f64(const std::vector<DMatP>& f, int maxit, double thr, int* flag, hipStream_t st);
+double faust_spectral_norm_f64(const std::vector<DMatP>& f, int maxit, double thr, int* flag, hipStream_t st,
+                               bool count = true);
 void faust_spectral_norm_pair_f64(const std::vector<DMatP>& f1, const std::vector<DMatP>& f2, int maxit, double thr,
                                   int* flag, double* n1, double* n2, hipStream_t st);
 // FP32 / BF16 paths (k_mixed.hip, k_bsr.hip)

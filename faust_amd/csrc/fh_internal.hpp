@@ -86,6 +86,15 @@ struct DBuf {
   template <class T> T* as() const { return static_cast<T*>(p); }
 };
 
+// This thread's page of pinned host memory, written by kernels: a scalar that
+// the host decides on is stored there by the kernel that computes it, and read
+// after the stream is synchronized, with no copy in between.  Slots are used
+// by one call at a time, except that the squared norm of a deferred
+// normalisation (MAIL_NORM) stays until the caller has looked at it.
+double* mail();
+enum { MAIL_NORM = 0, MAIL_CSR = 1 /* nnz, widest row, widest column */, MAIL_SUM = 4 /* two sums */,
+       MAIL_POWER = 8 /* three per chain, two chains */, MAIL_COUNT = 14 };
+
 inline size_t dtype_size(int dt) { return dt == FH_F64 ? 8 : dt == FH_F32 ? 4 : 2; }
 
 // ------------------------------------------------------------ matrices
@@ -206,11 +215,12 @@ void dense_csr_f64(const double* A, int lda, char opA, int m, const DMat& S, cha
 void gemm_f64(char opA, char opB, int m, int n, int k, double alpha, const double* A, int lda, const double* B,
               int ldb, double beta, double* C, int ldc, hipStream_t st);
 
-// canonical reductions; result written to a device double
-void reduce_dot_f64(const double* x, const double* y, int64_t n, double* out, hipStream_t st);
-void reduce_sum_f64(const double* x, int64_t n, double* out, hipStream_t st);
+// canonical reductions; result written to a double that the device can write
+// (device memory or a mail slot), and to out2 too when given
+void reduce_dot_f64(const double* x, const double* y, int64_t n, double* out, hipStream_t st, double* out2 = nullptr);
+void reduce_sum_f64(const double* x, int64_t n, double* out, hipStream_t st, double* out2 = nullptr);
 void diag_dot_f64(const double* A, const double* S, int m, int n, double* diag, hipStream_t st);
-// dense -> CSR (drops exact zeros), nnz returned on host (synchronizes)
+// dense -> CSR and CSC (drops exact zeros; synchronizes once, for the sizes)
 void dense_to_csr_f64(const double* D, int m, int n, DMat& out, hipStream_t st);
 void csr_to_dense_f64(const DMat& S, double* D, hipStream_t st);
 int64_t count_nnz_f64(const double* D, int64_t n, hipStream_t st);
@@ -223,10 +233,14 @@ void sub_f64(double* y, const double* x, int64_t n, hipStream_t st);  // y = y -
 void fill_f64(double* x, int64_t n, double v, hipStream_t st);
 void eye_f64(double* x, int m, int n, hipStream_t st);
 // projectors on dense col-major M (k per row/col/global); exact partial_sort tie semantics
+// defer_norm: the check that the normalised matrix is not zero is left to
+// check_norm(), called after the stream has been synchronized
 void prox_f64(int name, double* M, int m, int n, int64_t k, bool normalized, bool pos, const double* supp,
-              hipStream_t st);
+              hipStream_t st, bool defer_norm = false);
+void check_norm();
 // normcol / normlin: every column / row scaled to 2-norm s (faust_prox.hpp:205-255)
-void prox_real_f64(int name, double* M, int m, int n, double s, bool normalized, bool pos, hipStream_t st);
+void prox_real_f64(int name, double* M, int m, int n, double s, bool normalized, bool pos, hipStream_t st,
+                   bool defer_norm = false);
 
 // power iteration over a chain of (factor, op) applied last to first.
 struct ChainOp {

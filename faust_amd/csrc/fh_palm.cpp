@@ -123,13 +123,6 @@ static Chain packed(const Chain& c, hipStream_t st) {
 }
 
 // ------------------------------------------------------------ PALM pieces
-static double read_scalar(const DBuf& b, hipStream_t st) {
-  double h;
-  FH_HIP(hipMemcpyAsync(&h, b.p, sizeof(double), hipMemcpyDeviceToHost, st));
-  FH_HIP(hipStreamSynchronize(st));
-  return h;
-}
-
 static double fro_norm(const DMat& M, hipStream_t st) {
   DMatP D;
   const DMat* p = &M;
@@ -137,9 +130,10 @@ static double fro_norm(const DMat& M, hipStream_t st) {
     D = dense_of(M, st);
     p = D.get();
   }
-  DBuf s(sizeof(double));
-  reduce_dot_f64(p->d.as<double>(), p->d.as<double>(), (int64_t)p->m * p->n, s.as<double>(), st);
-  return std::sqrt(read_scalar(s, st));
+  double* s = mail() + MAIL_SUM;
+  reduce_dot_f64(p->d.as<double>(), p->d.as<double>(), (int64_t)p->m * p->n, s, st);
+  FH_HIP(hipStreamSynchronize(st));
+  return std::sqrt(*s);
 }
 
 // multiply_order_opt_all_ends, MatGeneric version (faust_prod_opt.hpp:49-86)
@@ -217,9 +211,9 @@ static void grad2(const Chain& pL, const Chain& pR, const DMat& A, double lambda
     facts = {L, tmp.get()};
     fl = {'T', 'N'};
   }
-  DMat g;
-  mul_all_ends(facts, g, lambda / c, 0.0, fl, st);
-  sub_f64(D.d.as<double>(), g.d.as<double>(), (int64_t)D.m * D.n, st);
+  // D - g with g = (lambda/c) acc: the product's epilogue gives
+  // fma(1, D, -(lambda/c) acc), the same rounding of the same terms
+  mul_all_ends(facts, D, -(lambda / c), 1.0, fl, st);
 }
 
 // compute_n_apply_grad1 (faust_palm4msa2020.hpp:304-361), taken by palm4msa2
@@ -282,12 +276,14 @@ static void update_lambda(const Chain& S, const std::vector<Chain>& pL, const st
   } else
     Smat = faust_get_product_f64(S, st);
   const int m = A.m, nc = A.n;
-  DBuf diag(sizeof(double) * std::max(nc, 1)), tr(sizeof(double)), ss(sizeof(double));
+  DBuf diag(sizeof(double) * std::max(nc, 1));
+  double* sums = mail() + MAIL_SUM;
   diag_dot_f64(A.d.as<double>(), Smat->d.as<double>(), m, nc, diag.as<double>(), st);
-  reduce_sum_f64(diag.as<double>(), nc, tr.as<double>(), st);
-  reduce_dot_f64(Smat->d.as<double>(), Smat->d.as<double>(), (int64_t)m * nc, ss.as<double>(), st);
-  const double htr = read_scalar(tr, st);
-  const double nS = std::sqrt(read_scalar(ss, st));
+  reduce_sum_f64(diag.as<double>(), nc, sums, st);
+  reduce_dot_f64(Smat->d.as<double>(), Smat->d.as<double>(), (int64_t)m * nc, sums + 1, st);
+  FH_HIP(hipStreamSynchronize(st));
+  const double htr = sums[0];
+  const double nS = std::sqrt(sums[1]);
   if (nS == 0.0) throw Error(FH_ERR_NUMERIC, "Error in update_lambda: S Frobenius norm is zero, can't compute lambda.");
   if (std::isnan(htr) || std::isnan(nS))
     throw Error(FH_ERR_NUMERIC, "Error in update_lambda: S (the Faust) contains nan elements");
@@ -299,10 +295,11 @@ static double calc_rel_err(const Chain& S, const DMat& A, double lambda, hipStre
   const int64_t N = (int64_t)A.m * A.n;
   scale_f64(P->d.as<double>(), N, nullptr, lambda, 0, st);
   sub_f64(P->d.as<double>(), A.d.as<double>(), N, st);
-  DBuf s1(sizeof(double)), s2(sizeof(double));
-  reduce_dot_f64(P->d.as<double>(), P->d.as<double>(), N, s1.as<double>(), st);
-  reduce_dot_f64(A.d.as<double>(), A.d.as<double>(), N, s2.as<double>(), st);
-  return std::sqrt(read_scalar(s1, st)) / std::sqrt(read_scalar(s2, st));
+  double* sums = mail() + MAIL_SUM;
+  reduce_dot_f64(P->d.as<double>(), P->d.as<double>(), N, sums, st);
+  reduce_dot_f64(A.d.as<double>(), A.d.as<double>(), N, sums + 1, st);
+  FH_HIP(hipStreamSynchronize(st));
+  return std::sqrt(sums[0]) / std::sqrt(sums[1]);
 }
 
 static int64_t sparse_size(int64_t nnz, int64_t nrows) { return nnz * (8 + 4) + (nrows + 1) * 4; }
@@ -314,11 +311,12 @@ struct DevCons {
 };
 
 // ConstraintInt / ConstraintMat / ConstraintFPP::project on a dense device matrix
-static void apply_cons(const fh_constraint& c, const double* dsupp, double* M, hipStream_t st) {
+static void apply_cons(const fh_constraint& c, const double* dsupp, double* M, hipStream_t st,
+                       bool defer_norm = false) {
   if (c.name == FH_PROX_NORMCOL || c.name == FH_PROX_NORMLIN)
-    prox_real_f64(c.name, M, c.nrows, c.ncols, c.s, c.normalized != 0, c.pos != 0, st);
+    prox_real_f64(c.name, M, c.nrows, c.ncols, c.s, c.normalized != 0, c.pos != 0, st, defer_norm);
   else
-    prox_f64(c.name, M, c.nrows, c.ncols, c.k, c.normalized != 0, c.pos != 0, dsupp, st);
+    prox_f64(c.name, M, c.nrows, c.ncols, c.k, c.normalized != 0, c.pos != 0, dsupp, st, defer_norm);
 }
 
 // ConstraintInt/ConstraintMat/ConstraintFPP::project_gen (faust_prox_gen.hpp:1-25,118-210)
@@ -332,17 +330,23 @@ static DMatP project_gen(const fh_constraint& c, const double* dsupp, DMatP D, i
     case FH_PROX_SPLIN: out_dense = sparse_size(c.k * n, m) > dense_size(m, n); break;
     default: break;
   }
-  apply_cons(c, dsupp, D->d.as<double>(), st);
+  // the check for a zero projection waits for the conversion's own wait
+  apply_cons(c, dsupp, D->d.as<double>(), st, true);
   D->nnz = -1;
   if (factor_format == 2) {
     // supp, normcol, normlin: the format follows the real nonzero count
     if (c.name == FH_PROX_SUPP || c.name == FH_PROX_NORMCOL || c.name == FH_PROX_NORMLIN)
       out_dense = sparse_size(nnz_of(*D, st), m) > dense_size(m, n);
-    if (out_dense) return D;
-    return to_sparse(*D, st);
+  } else {
+    out_dense = factor_format != 1;
   }
-  if (factor_format == 1) return to_sparse(*D, st);
-  return D;
+  DMatP out = D;
+  if (out_dense)
+    FH_HIP(hipStreamSynchronize(st));
+  else
+    out = to_sparse(*D, st);
+  check_norm();
+  return out;
 }
 
 struct Palm {
@@ -424,9 +428,9 @@ static void palm4msa2(Palm& P, Chain& S, double& lambda, hipStream_t st) {
         if (!pR[f_id].empty() && !pL[f_id].empty())
           faust_spectral_norm_pair_f64(pR[f_id], pL[f_id], p.norm2_max_iter, p.norm2_threshold, &flag, &nR, &nL, st);
         else if (!pR[f_id].empty())
-          nR = faust_spectral_norm_f64(pR[f_id], p.norm2_max_iter, p.norm2_threshold, &flag, st);
+          nR = faust_spectral_norm_f64(pR[f_id], p.norm2_max_iter, p.norm2_threshold, &flag, st, false);
         else if (!pL[f_id].empty())
-          nL = faust_spectral_norm_f64(pL[f_id], p.norm2_max_iter, p.norm2_threshold, &flag, st);
+          nL = faust_spectral_norm_f64(pL[f_id], p.norm2_max_iter, p.norm2_threshold, &flag, st, false);
         if (std::isnan(nL) || std::isnan(nR))
           throw Error(FH_ERR_NUMERIC, "2-norm computation error: R or L 2-norm is NaN.");
         if ((nR == 0 && (it > 0 || !p.is_update_way_R2L)) || (nL == 0 && (it > 0 || p.is_update_way_R2L)))
@@ -545,10 +549,12 @@ static double specnorm16(const DF& A, int maxit, double thr, hipStream_t st) {
 
 // trace(X^T Y): diagonal fma chains (k ascending), canonical sum
 static double trace_xty(const DMat& X, const DMat& Y, hipStream_t st) {
-  DBuf dg(sizeof(double) * std::max(X.n, 1)), s(sizeof(double));
+  DBuf dg(sizeof(double) * std::max(X.n, 1));
+  double* s = mail() + MAIL_SUM;
   diag_dot_f64(X.d.as<double>(), Y.d.as<double>(), X.m, X.n, dg.as<double>(), st);
-  reduce_sum_f64(dg.as<double>(), X.n, s.as<double>(), st);
-  return read_scalar(s, st);
+  reduce_sum_f64(dg.as<double>(), X.n, s, st);
+  FH_HIP(hipStreamSynchronize(st));
+  return *s;
 }
 
 struct Palm16 {

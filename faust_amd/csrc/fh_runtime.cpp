@@ -81,6 +81,42 @@ void pool_trim() {
   g_free.clear();
 }
 
+// Pages of pinned host memory, one per thread that asked, taken from and given
+// back to a list (so there are as many as threads at work at once); they are
+// not returned to the driver, whose teardown may precede the threads'.
+namespace {
+std::mutex g_mail_mu;
+std::vector<double*> g_mail_free;
+
+struct MailPage {
+  double* p = nullptr;
+  ~MailPage() {
+    if (!p) return;
+    std::lock_guard<std::mutex> lk(g_mail_mu);
+    g_mail_free.push_back(p);
+  }
+};
+}  // namespace
+
+double* mail() {
+  static thread_local MailPage page;
+  if (!page.p) {
+    {
+      std::lock_guard<std::mutex> lk(g_mail_mu);
+      if (!g_mail_free.empty()) {
+        page.p = g_mail_free.back();
+        g_mail_free.pop_back();
+      }
+    }
+    if (!page.p) {
+      void* q = nullptr;
+      FH_HIP(hipHostMalloc(&q, 4096, hipHostMallocPortable | hipHostMallocMapped));
+      page.p = static_cast<double*>(q);
+    }
+  }
+  return page.p;
+}
+
 }  // namespace fh
 
 extern "C" {

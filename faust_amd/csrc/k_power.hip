@@ -1223,8 +1223,7 @@ static bool power_iteration_lds(const std::vector<std::vector<PwOp>>& hs, const 
     lds = std::max(lds, b);
     longest = std::max(longest, a.job[k].ld - 1);
   }
-  DBuf dout(sizeof(double) * 3 * J);
-  double* out = dout.as<double>();
+  double* out = mail() + MAIL_POWER;
   if (longest <= 64)
     pl_go<64>(a, J, lds, maxit, thr, out, st);
   else if (longest <= 128)
@@ -1235,9 +1234,8 @@ static bool power_iteration_lds(const std::vector<std::vector<PwOp>>& hs, const 
     pl_go<512>(a, J, lds, maxit, thr, out, st);
   else
     pl_go<1024>(a, J, lds, maxit, thr, out, st);
-  double res[6];
-  FH_HIP(hipMemcpyAsync(res, out, sizeof(double) * 3 * J, hipMemcpyDeviceToHost, st));
   FH_HIP(hipStreamSynchronize(st));
+  const double* res = out;
   for (int k = 0; k < J; ++k) {
     if (res[3 * k + 2] == 1.0) throw Error(FH_ERR_NUMERIC, "Can't normalize a zero-norm vector.");
     lam[k] = res[3 * k];

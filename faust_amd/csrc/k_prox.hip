@@ -11,6 +11,7 @@
 // canonical Frobenius normalisation (faust_prox.hpp:72-200;
 // MatDense::normalize, faust_MatDense.hpp:1226-1250).
 #include <algorithm>
+#include <climits>
 
 #include "fh_internal.hpp"
 #include "heap_select.hpp"
@@ -98,19 +99,23 @@ __device__ bool wg_select_threshold(KeyAt key_at, int len, int k, unsigned* hist
   return prefix != 0;  // tied zeros: every choice gives the same output
 }
 
-// One 64-lane workgroup per line.  along_rows: line i is row i (splin);
-// otherwise line j is column j (spcol).  Dynamic LDS holds the line values and
+// One 64-lane workgroup per line: the first ncol_lines are columns (spcol), the
+// rest rows (splin), written to outc and outr; a line is staged before it is
+// written, so an output may be M itself (when only one kind is selected).
+// Dynamic LDS holds the line values and
 // the heap when they fit (lds_ok), else per-line global scratch is used.  The
 // radix threshold decides the support unless ties straddle the k boundary;
 // only those lines run the heap selection on one lane.
-__global__ __launch_bounds__(64) void k_prox_lines(const double* __restrict__ M, int m, int n, int along_rows, int k,
-                                                   double* __restrict__ out, int lds_ok, double* __restrict__ gvals,
+__global__ __launch_bounds__(64) void k_prox_lines(const double* M, int m, int n, int ncol_lines, int k, double* outc,
+                                                   double* outr, int lds_ok, double* __restrict__ gvals,
                                                    int* __restrict__ gidx, double* __restrict__ gabs) {
   extern __shared__ double smem[];
   __shared__ unsigned hist[256];
   __shared__ int sh[3];
-  const int line = blockIdx.x;
+  const bool along_rows = (int)blockIdx.x >= ncol_lines;
+  const int line = along_rows ? blockIdx.x - ncol_lines : blockIdx.x;
   const int len = along_rows ? n : m;
+  double* out = along_rows ? outr : outc;
   double* vals;
   double* habs;
   int* hidx;
@@ -119,9 +124,9 @@ __global__ __launch_bounds__(64) void k_prox_lines(const double* __restrict__ M,
     habs = smem + len;
     hidx = reinterpret_cast<int*>(smem + len + k);
   } else {
-    vals = gvals + (size_t)line * len;
-    habs = gabs + (size_t)line * k;
-    hidx = gidx + (size_t)line * k;
+    vals = gvals + (size_t)blockIdx.x * max(m, n);
+    habs = gabs + (size_t)blockIdx.x * k;
+    hidx = gidx + (size_t)blockIdx.x * k;
   }
   const int lane = threadIdx.x;
   for (int t = lane; t < len; t += 64) vals[t] = along_rows ? M[(size_t)t * m + line] : M[(size_t)line * m + t];
@@ -154,39 +159,139 @@ struct SpSel {
   int ambiguous;
 };
 
+// The k-th largest magnitude of N entries in one workgroup: a radix select with
+// 11-bit digits (the exponent first) over the entries in global memory, 16
+// loads in flight per thread, until at most SP_LIST candidates share the
+// digits found; those are then gathered in LDS and ranked against each other.
+// Ties that straddle k (see wg_select_threshold) are settled by the exact heap
+// selection on one lane, and the k entries it keeps are saved before the
+// caller overwrites M.  8-bit digits over all of M until the bin was exact
+// took 45 us for 256 x 256 entries.
+constexpr int SP_BITS = 11, SP_BINS = 1 << SP_BITS, SP_LIST = 512, SP_LOADS = 16;
 __global__ __launch_bounds__(1024) void k_sp_threshold(const double* __restrict__ M, int N, int k,
-                                                       SpSel* __restrict__ sel) {
-  __shared__ unsigned hist[256];
-  __shared__ int sh[3];
-  unsigned long long T;
-  const bool amb = wg_select_threshold([M](int i) { return mag_key(M[i]); }, N, k, hist, sh, &T);
-  if (threadIdx.x == 0) {
-    sel->T = T;
-    sel->ambiguous = amb ? 1 : 0;
+                                                       SpSel* __restrict__ sel, int* __restrict__ hidx,
+                                                       double* __restrict__ habs, double* __restrict__ hval) {
+  __shared__ unsigned hist[SP_BINS];
+  __shared__ unsigned wtot[16];
+  __shared__ int sh[3], nlist, amb;
+  __shared__ unsigned long long list[SP_LIST];
+  __shared__ unsigned long long thr;
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  unsigned long long prefix = 0, mask = 1ull << 63;  // magnitudes have no sign bit
+  int kk = k;
+  // runs f(key) for every entry
+  auto each = [&](auto&& f) {
+    for (int64_t i0 = t; i0 < N; i0 += 1024 * SP_LOADS) {
+      unsigned long long x[SP_LOADS];
+#pragma unroll
+      for (int u = 0; u < SP_LOADS; ++u) x[u] = mag_key(M[min(i0 + 1024 * u, (int64_t)N - 1)]);
+#pragma unroll
+      for (int u = 0; u < SP_LOADS; ++u)
+        if (i0 + 1024 * u < N) f(x[u]);
+    }
+  };
+  bool done = false;
+  for (int shift = 63 - SP_BITS; !done; shift = max(shift - SP_BITS, 0)) {
+    const int bits = mask == 1ull << 63 ? SP_BITS : min(SP_BITS, __builtin_ctzll(mask));
+    for (int b = t; b < SP_BINS; b += 1024) hist[b] = 0u;
+    if (t == 0) nlist = 0;
+    __syncthreads();
+    // two (digit, count) pairs per thread ahead of the LDS atomics
+    unsigned d0 = SP_BINS, c0 = 0, d1 = SP_BINS, c1 = 0;
+    const unsigned dmask = (1u << bits) - 1;
+    each([&](unsigned long long x) {
+      if ((x & mask) != prefix) return;
+      const unsigned d = (unsigned)(x >> shift) & dmask;
+      if (d == d0) {
+        ++c0;
+      } else if (d == d1) {
+        ++c1;
+      } else {
+        if (c1) atomicAdd(&hist[d1], c1);
+        d1 = d0;
+        c1 = c0;
+        d0 = d;
+        c0 = 1;
+      }
+    });
+    if (c0) atomicAdd(&hist[d0], c0);
+    if (c1) atomicAdd(&hist[d1], c1);
+    __syncthreads();
+    // thread t owns the bins SP_BINS - 1 - 2t and the one below; inclusive scan from the top
+    const int hi = SP_BINS - 1 - 2 * t;
+    const unsigned h0 = hist[hi], h1 = hist[hi - 1];
+    unsigned incl = h0 + h1;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const unsigned o = __shfl_up(incl, d, 64);
+      if (lane >= d) incl += o;
+    }
+    if (lane == 63) wtot[w] = incl;
+    __syncthreads();
+    for (int q = 0; q < w; ++q) incl += wtot[q];
+    const int before = (int)(incl - h0 - h1);
+    if (before < kk && kk <= (int)incl) {
+      const bool first = before + (int)h0 >= kk;
+      sh[0] = first ? hi : hi - 1;
+      sh[1] = kk - before - (first ? 0 : (int)h0);
+      sh[2] = first ? (int)h0 : (int)h1;
+    }
+    __syncthreads();
+    const int cnt = sh[2];
+    kk = sh[1];
+    prefix |= (unsigned long long)sh[0] << shift;
+    mask |= (unsigned long long)dmask << shift;
+    if (cnt == kk || shift == 0) {  // every candidate is taken, or all are equal
+      if (t == 0) {
+        thr = prefix;
+        amb = cnt != kk && prefix != 0;
+      }
+      done = true;
+    } else if (cnt <= SP_LIST) {
+      each([&](unsigned long long x) {
+        if ((x & mask) == prefix) list[atomicAdd(&nlist, 1)] = x;
+      });
+      __syncthreads();
+      if (t < cnt) {  // x is the threshold when fewer than kk are larger and at least kk are as large
+        const unsigned long long x = list[t];
+        int gt = 0, ge = 0;
+        for (int q = 0; q < cnt; ++q) {
+          gt += list[q] > x;
+          ge += list[q] >= x;
+        }
+        if (gt < kk && kk <= ge) {  // the same values from every thread that gets here
+          thr = x;
+          amb = ge != kk && x != 0;
+        }
+      }
+      done = true;
+    }
+    __syncthreads();
   }
+  if (t == 0) {
+    sel->T = thr;
+    sel->ambiguous = amb;
+    if (amb) heap_select<double>(N, k, [M](int i) { return fabs(M[i]); }, hidx, habs);
+  }
+  if (!amb) return;
+  __threadfence_block();
+  __syncthreads();
+  for (int q = t; q < k; q += 1024) hval[q] = M[hidx[q]];
 }
 
-// exact heap selection on one lane, only when the threshold left ties open
-__global__ __launch_bounds__(64) void k_prox_global_select(const double* __restrict__ M, int64_t N, int k,
-                                                           const SpSel* __restrict__ sel, int* __restrict__ hidx,
-                                                           double* __restrict__ habs) {
-  if (!sel->ambiguous) return;
-  if (threadIdx.x == 0) heap_select<double>((int)N, k, [M](int i) { return fabs(M[i]); }, hidx, habs);
-}
-
-__global__ void k_sp_apply(const double* __restrict__ M, int64_t N, const SpSel* __restrict__ sel,
-                           double* __restrict__ out) {
+// in place; the ambiguous case clears everything and k_scatter_sel puts the saved entries back
+__global__ void k_sp_apply(double* __restrict__ M, int64_t N, const SpSel* __restrict__ sel) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= N) return;
   const double x = M[i];
-  out[i] = (!sel->ambiguous && mag_key(x) >= sel->T) ? x : 0.0;
+  M[i] = (!sel->ambiguous && mag_key(x) >= sel->T) ? x : 0.0;
 }
 
-__global__ void k_scatter_sel(const double* __restrict__ M, const int* __restrict__ idx, int k,
-                              const SpSel* __restrict__ sel, double* __restrict__ out) {
+__global__ void k_scatter_sel(double* __restrict__ M, const int* __restrict__ idx, const double* __restrict__ val,
+                              int k, const SpSel* __restrict__ sel) {
   if (!sel->ambiguous) return;
   int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q < k) out[idx[q]] = M[idx[q]];
+  if (q < k) M[idx[q]] = val[q];
 }
 
 __global__ void k_pos(double* __restrict__ M, int64_t n) {
@@ -194,8 +299,8 @@ __global__ void k_pos(double* __restrict__ M, int64_t n) {
   if (i < n && (float)M[i] < 0.0f) M[i] = 0.0;
 }
 
-__global__ void k_union(const double* __restrict__ Mc, const double* __restrict__ Ml, double* __restrict__ out,
-                        int64_t n) {
+// Mc and Ml may be out
+__global__ void k_union(const double* Mc, const double* Ml, double* out, int64_t n) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) {
     double c = Mc[i];
@@ -251,40 +356,47 @@ __global__ __launch_bounds__(256) void k_line_norm_scale(double* __restrict__ M,
 
 static inline dim3 g1(int64_t n) { return dim3((unsigned)((n + 255) / 256)); }
 
-// top-k per line into `out` (dense, same shape as M)
-static void prox_lines(const double* M, int m, int n, bool along_rows, int k, double* out, hipStream_t st) {
-  const int nlines = along_rows ? m : n;
-  const int len = along_rows ? n : m;
+// top-k per column into outc and per row into outr (dense, same shape as M;
+// null: not selected; M itself when the other is null)
+static void prox_lines(const double* M, int m, int n, int k, double* outc, double* outr, hipStream_t st) {
+  const int ncl = outc ? n : 0, nlines = ncl + (outr ? m : 0);
+  const int len = outc && outr ? std::max(m, n) : outc ? m : n;
   if (nlines == 0) return;
   size_t lds = sizeof(double) * ((size_t)len + k) + sizeof(int) * (size_t)k;
   const size_t LDS_MAX = 60 * 1024;
   if (lds <= LDS_MAX) {
-    hipLaunchKernelGGL(k_prox_lines, dim3(nlines), dim3(64), lds, st, M, m, n, along_rows ? 1 : 0, k, out, 1,
+    hipLaunchKernelGGL(k_prox_lines, dim3(nlines), dim3(64), lds, st, M, m, n, ncl, k, outc, outr, 1,
                        (double*)nullptr, (int*)nullptr, (double*)nullptr);
   } else {
-    DBuf gv(sizeof(double) * (size_t)nlines * len), gi(sizeof(int) * (size_t)nlines * k),
+    DBuf gv(sizeof(double) * (size_t)nlines * std::max(m, n)), gi(sizeof(int) * (size_t)nlines * k),
         ga(sizeof(double) * (size_t)nlines * k);
-    hipLaunchKernelGGL(k_prox_lines, dim3(nlines), dim3(64), 0, st, M, m, n, along_rows ? 1 : 0, k, out, 0,
-                       gv.as<double>(), gi.as<int>(), ga.as<double>());
+    hipLaunchKernelGGL(k_prox_lines, dim3(nlines), dim3(64), 0, st, M, m, n, ncl, k, outc, outr, 0, gv.as<double>(),
+                       gi.as<int>(), ga.as<double>());
     FH_LAUNCH_CHECK();
     return;
   }
   FH_LAUNCH_CHECK();
 }
 
-static void normalize_inplace(double* M, int64_t N, hipStream_t st) {
+void check_norm() {
+  if (mail()[MAIL_NORM] == 0.0) throw Error(FH_ERR_NUMERIC, "the norm is zero, can't normalize.");
+}
+
+static void normalize_inplace(double* M, int64_t N, hipStream_t st, bool defer_norm) {
+  double* sq = mail() + MAIL_NORM;
   DBuf s(sizeof(double));
-  reduce_dot_f64(M, M, N, s.as<double>(), st);
-  double h = 0;
-  FH_HIP(hipMemcpyAsync(&h, s.p, sizeof(double), hipMemcpyDeviceToHost, st));
-  FH_HIP(hipStreamSynchronize(st));
-  if (h == 0.0) throw Error(FH_ERR_NUMERIC, "the norm is zero, can't normalize.");
+  reduce_dot_f64(M, M, N, s.as<double>(), st, sq);
+  if (!defer_norm) {
+    FH_HIP(hipStreamSynchronize(st));
+    check_norm();
+  }
   scale_f64(M, N, s.as<double>(), 0.0, 1, st);
 }
 
 void prox_f64(int name, double* M, int m, int n, int64_t k, bool normalized, bool pos, const double* supp,
-              hipStream_t st) {
+              hipStream_t st, bool defer_norm) {
   const int64_t N = (int64_t)m * n;
+  if (defer_norm) mail()[MAIL_NORM] = 1.0;  // nothing to check unless a norm is taken
   if (N == 0) return;
   auto zero_all = [&]() { FH_HIP(hipMemsetAsync(M, 0, sizeof(double) * N, st)); };
   switch (name) {
@@ -294,18 +406,15 @@ void prox_f64(int name, double* M, int m, int n, int64_t k, bool normalized, boo
         zero_all();
       else if (k < N) {
         FH_CHECK(N < (int64_t)1 << 31, "prox_sp: matrix too large");
-        DBuf hi(sizeof(int) * k), ha(sizeof(double) * k), out(sizeof(double) * N), sel(sizeof(SpSel));
-        hipLaunchKernelGGL(k_sp_threshold, dim3(1), dim3(1024), 0, st, M, (int)N, (int)k, sel.as<SpSel>());
+        DBuf hi(sizeof(int) * k), ha(sizeof(double) * k), hv(sizeof(double) * k), sel(sizeof(SpSel));
+        hipLaunchKernelGGL(k_sp_threshold, dim3(1), dim3(1024), 0, st, M, (int)N, (int)k, sel.as<SpSel>(),
+                           hi.as<int>(), ha.as<double>(), hv.as<double>());
         FH_LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_prox_global_select, dim3(1), dim3(64), 0, st, M, N, (int)k, sel.as<SpSel>(),
-                           hi.as<int>(), ha.as<double>());
+        hipLaunchKernelGGL(k_sp_apply, g1(N), dim3(256), 0, st, M, N, sel.as<SpSel>());
         FH_LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_sp_apply, g1(N), dim3(256), 0, st, M, N, sel.as<SpSel>(), out.as<double>());
+        hipLaunchKernelGGL(k_scatter_sel, g1(k), dim3(256), 0, st, M, hi.as<int>(), hv.as<double>(), (int)k,
+                           sel.as<SpSel>());
         FH_LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_scatter_sel, g1(k), dim3(256), 0, st, M, hi.as<int>(), (int)k, sel.as<SpSel>(),
-                           out.as<double>());
-        FH_LAUNCH_CHECK();
-        FH_HIP(hipMemcpyAsync(M, out.p, sizeof(double) * N, hipMemcpyDeviceToDevice, st));
       }
       break;
     }
@@ -315,27 +424,23 @@ void prox_f64(int name, double* M, int m, int n, int64_t k, bool normalized, boo
       if (pos) hipLaunchKernelGGL(k_pos, g1(N), dim3(256), 0, st, M, N);
       if (k <= 0)
         zero_all();
-      else if (k < (rows ? n : m)) {
-        DBuf out(sizeof(double) * N);
-        prox_lines(M, m, n, rows, (int)k, out.as<double>(), st);
-        FH_HIP(hipMemcpyAsync(M, out.p, sizeof(double) * N, hipMemcpyDeviceToDevice, st));
-      }
+      else if (k < (rows ? n : m))
+        prox_lines(M, m, n, (int)k, rows ? nullptr : M, rows ? M : nullptr, st);
       break;
     }
     case FH_PROX_SPLINCOL: {
       // faust_prox.hpp:180-200: both selections run on the input (pos only
       // affects the matrix that is then overwritten)
-      DBuf mc(sizeof(double) * N), ml(sizeof(double) * N);
-      FH_HIP(hipMemcpyAsync(mc.p, M, sizeof(double) * N, hipMemcpyDeviceToDevice, st));
-      FH_HIP(hipMemcpyAsync(ml.p, M, sizeof(double) * N, hipMemcpyDeviceToDevice, st));
       if (k <= 0) {
-        FH_HIP(hipMemsetAsync(mc.p, 0, sizeof(double) * N, st));
-        FH_HIP(hipMemsetAsync(ml.p, 0, sizeof(double) * N, st));
-      } else {
-        if (k < m) prox_lines(M, m, n, false, (int)k, mc.as<double>(), st);
-        if (k < n) prox_lines(M, m, n, true, (int)k, ml.as<double>(), st);
+        zero_all();
+        break;
       }
-      hipLaunchKernelGGL(k_union, g1(N), dim3(256), 0, st, mc.as<double>(), ml.as<double>(), M, N);
+      // a selection that keeps whole lines is M itself
+      DBuf mc(k < m ? sizeof(double) * N : 0), ml(k < n ? sizeof(double) * N : 0);
+      prox_lines(M, m, n, (int)std::min<int64_t>(k, INT_MAX), mc.as<double>(), ml.as<double>(), st);
+      const double* pc = k < m ? mc.as<double>() : M;
+      const double* pl = k < n ? ml.as<double>() : M;
+      hipLaunchKernelGGL(k_union, g1(N), dim3(256), 0, st, pc, pl, M, N);
       FH_LAUNCH_CHECK();
       break;
     }
@@ -349,11 +454,13 @@ void prox_f64(int name, double* M, int m, int n, int64_t k, bool normalized, boo
     default:
       throw Error(FH_ERR_ARG, "prox: unknown constraint");
   }
-  if (normalized) normalize_inplace(M, N, st);
+  if (normalized) normalize_inplace(M, N, st, defer_norm);
 }
 
-void prox_real_f64(int name, double* M, int m, int n, double s, bool normalized, bool pos, hipStream_t st) {
+void prox_real_f64(int name, double* M, int m, int n, double s, bool normalized, bool pos, hipStream_t st,
+                   bool defer_norm) {
   const int64_t N = (int64_t)m * n;
+  if (defer_norm) mail()[MAIL_NORM] = 1.0;
   FH_CHECK(name == FH_PROX_NORMCOL || name == FH_PROX_NORMLIN, "prox: unknown real-parameter constraint");
   if (N == 0) return;
   if (pos) {
@@ -368,7 +475,7 @@ void prox_real_f64(int name, double* M, int m, int n, double s, bool normalized,
     hipLaunchKernelGGL(k_line_norm_scale, dim3(rows ? m : n), dim3(256), 0, st, M, m, n, rows ? 1 : 0, s);
   }
   FH_LAUNCH_CHECK();
-  if (normalized) normalize_inplace(M, N, st);
+  if (normalized) normalize_inplace(M, N, st, defer_norm);
 }
 
 }  // namespace fh
