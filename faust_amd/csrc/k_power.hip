@@ -735,28 +735,116 @@ __global__ __launch_bounds__(NT) void k_power_lds(PlArgs args, const double* __r
 // chain on one lane (k ascending), so the result is bit-identical to the
 // persistent kernel; the row data is staged through LDS by all 256 threads of
 // the workgroup in contiguous chunks, and the first R lanes (one per row) run
-// the chains.  A device state carries lambda, the round count and a done flag: the
-// host enqueues rounds ahead and launches after convergence return at once.
+// the chains.  A round's boundary (the zero test, the Rayleigh quotient, the
+// loop test and the normalisation) runs at the start of its first operator's
+// launch, in every workgroup alike and while that operator's first entries are
+// on their way; workgroup 0 stores what the next round needs.  A device state
+// carries lambda, the round count and a done flag (two copies: a round reads
+// one and writes the other, so no workgroup reads what another one writes);
+// the host enqueues rounds ahead and launches after convergence return at once.
 struct PwState {
   double lambda, lambda_old;
   int it, status, done, pad;
 };
 
 constexpr int PW_WIDE_THREADS = 256;
-constexpr int PW_CH = 2048;  // entries per LDS chunk
+constexpr int PW_CH = 2048;  // entries per LDS chunk of a sparse operator
+
+// A round boundary: xa = the chain's output (first round: the start vector,
+// mode 0), xn_in = the vector it was applied to, xn_out = its successor.
+// Used when first; res (host memory) receives lambda, flag, status, done.
+struct PwBound {
+  int first, mode, n, maxit;
+  double thr;
+  const double* xa;
+  const double* xn_in;
+  double* xn_out;
+  const PwState* in;
+  PwState* out;
+  double* res;
+};
+
+__device__ __forceinline__ void pw_post(const PwState& st, int maxit, double* res) {
+  res[0] = st.status == 2 ? 0.0 : st.lambda;
+  res[1] = st.it < maxit ? (double)st.it : -1.0;
+  res[2] = (double)st.status;
+  res[3] = 1.0;
+}
+
+// The boundary in a workgroup of 256 threads; lead: this one stores the
+// results.  Writes the normalised vector to xs (LDS) and returns true, or
+// returns false when the iteration is over.  red: 512 doubles, flag: 4 ints of LDS.
+__device__ __forceinline__ bool pw_bound(const PwBound& b, bool lead, double* xs, double* red, int* flag) {
+  const int t = threadIdx.x, l = t & 63;
+  PwState st = *b.in;
+  if (!st.done) {
+    double sxy = 0.0, syy = 0.0;
+    int nz = 0;
+    for (int i = t; i < b.n; i += RED_LANES) {
+      const double y = b.xa[i], x = b.mode ? b.xn_in[i] : 0.0;
+      xs[i] = y;
+      sxy = fma(x, y, sxy);
+      syy = fma(y, y, syy);
+      nz |= y != 0.0;
+    }
+    const int any_w = __any(nz);
+    red[t] = sxy;
+    red[RED_LANES + t] = syy;
+    if (l == 0) flag[t >> 6] = any_w;
+    __syncthreads();
+    sxy = pl_tree((red[l] + red[l + 128]) + (red[l + 64] + red[l + 192]));
+    syy = pl_tree((red[RED_LANES + l] + red[RED_LANES + l + 128]) + (red[RED_LANES + l + 64] + red[RED_LANES + l + 192]));
+    const int any = flag[0] | flag[1] | flag[2] | flag[3];
+    if (b.mode && !any) {
+      st.status = 2;
+      st.done = 1;
+    } else {
+      const double lambda = b.mode ? sxy : st.lambda;
+      const double athr = fabs(b.thr);
+      st.lambda = lambda;
+      if (!((fabs(st.lambda_old - lambda) > athr || fabs(lambda) <= athr) && st.it < b.maxit)) {
+        st.done = 1;
+      } else {
+        st.it++;
+        st.lambda_old = lambda;
+        const double nrm = sqrt(syy);
+        if (nrm == 0.0) {
+          st.status = 1;
+          st.done = 1;
+        } else {
+          const double inv = 1 / nrm;
+          for (int i = t; i < b.n; i += RED_LANES) {
+            const double x = xs[i] * inv;
+            xs[i] = x;
+            if (lead) b.xn_out[i] = x;
+          }
+        }
+      }
+    }
+    if (lead && t == 0 && st.done) pw_post(st, b.maxit, b.res);
+  }
+  if (lead && t == 0) *b.out = st;
+  return !st.done;
+}
 
 // sparse rows (row pointers rp, indices ci, values v): rows r0..r0+R-1 per workgroup
 __global__ __launch_bounds__(PW_WIDE_THREADS) void k_pw_csr(const int* __restrict__ rp, const int* __restrict__ ci,
                                                             const double* __restrict__ v, int rows, int cols, int R,
                                                             const double* __restrict__ cur, double* __restrict__ nxt,
-                                                            const PwState* __restrict__ s) {
+                                                            const PwState* __restrict__ s, PwBound bound) {
   __shared__ double xs[PW_VMAX];
   __shared__ double sv[PW_CH];
   __shared__ int sci[PW_CH];
-  if (s->done) return;
+  __shared__ double red[2 * RED_LANES];
+  __shared__ int flag[4];
   const int t = threadIdx.x;
+  if (bound.first) {
+    if (!pw_bound(bound, blockIdx.x == 0, xs, red, flag)) return;
+  } else {
+    if (s->done) return;
+    for (int i = t; i < cols; i += PW_WIDE_THREADS) xs[i] = cur[i];
+  }
   const int r0 = blockIdx.x * R, r1 = min(rows, r0 + R), nr = r1 - r0;
-  for (int i = t; i < cols; i += PW_WIDE_THREADS) xs[i] = cur[i];
   const int p0 = rp[r0], p1 = rp[r1];
   int p = 0, pe = 0;
   if (t < nr) {
@@ -780,38 +868,110 @@ __global__ __launch_bounds__(PW_WIDE_THREADS) void k_pw_csr(const int* __restric
   if (t < nr) nxt[r0 + t] = acc;
 }
 
-// dense op(A) rows (A column-major, leading dimension lda); trans: op(A) = A^T
-__global__ __launch_bounds__(PW_WIDE_THREADS) void k_pw_dense(const double* __restrict__ A, int lda, int trans,
-                                                              int rows, int cols, int R,
-                                                              const double* __restrict__ cur,
+// dense op(A) rows (A column-major, leading dimension lda); TRANS: op(A) = A^T.
+// A workgroup computes four rows.  Its entries come in chunks of 1024 columns,
+// 16 loads per thread issued together; they go to LDS in four parts of 256
+// columns, each followed by a barrier, and the first wave runs the four chains
+// over one part while the others store the next as it arrives.  Workgroups
+// are dealt to the XCDs in turn, so each XCD takes a contiguous run of rows:
+// the four workgroups that share the 128-byte lines of a column find them in
+// one L2.  The floor is the chain: 1024 dependent fma, 2.7 us; its lanes read
+// pairs of columns 16 ahead, since waiting for each 16 took as long again.
+// Measured per launch in chains of 20 operators of order 1024 (8 MiB each):
+// 23 us with loads of one entry at a time, 14.2 with the parts above, 10.2
+// with the lanes reading ahead; order 256 (PALM4MSA's step sizes): 5.4 us and
+// a boundary launch of 3.8 us per round -> 4.9 us and none.
+constexpr int PD_ROWS = 4, PD_PARTS = 4, PD_PCOLS = 256, PD_COLS = PD_PARTS * PD_PCOLS, PD_LD = PD_PCOLS + 2;
+constexpr int PD_LOADS = PD_ROWS * PD_PCOLS / PW_WIDE_THREADS;  // per thread and part
+template <bool TRANS>
+__global__ __launch_bounds__(PW_WIDE_THREADS) void k_pw_dense(const double* __restrict__ A, int lda, int rows,
+                                                              int cols, const double* __restrict__ cur,
                                                               double* __restrict__ nxt,
-                                                              const PwState* __restrict__ s) {
-  __shared__ double xs[PW_VMAX];
-  __shared__ double tile[PW_CH];  // R rows x C columns, row stride C + 1 (odd: no bank conflicts)
-  if (s->done) return;
+                                                              const PwState* __restrict__ s, PwBound bound) {
+  __shared__ __align__(16) double xs[PW_VMAX];
+  __shared__ __align__(16) double tile[PD_PARTS][PD_ROWS * PD_LD];  // [row][column]
+  __shared__ double red[2 * RED_LANES];
+  __shared__ int flag[4];
   const int t = threadIdx.x;
-  const int r0 = blockIdx.x * R, nr = min(rows, r0 + R) - r0;
-  const int C = PW_CH / R - 2;
-  for (int i = t; i < cols; i += PW_WIDE_THREADS) xs[i] = cur[i];
-  double acc = 0.0;
-  for (int c0 = 0; c0 < cols; c0 += C) {
-    const int nc = min(C, cols - c0);
-    __syncthreads();
-    if (trans) {  // row i of A^T = column r0+i of A: contiguous in c
-      for (int q = t; q < nr * nc; q += PW_WIDE_THREADS) {
-        const int i = q / nc, c = q - i * nc;
-        tile[i * (C + 1) + c] = A[(size_t)(r0 + i) * lda + c0 + c];
-      }
-    } else {  // row i of A: element (i, c) at (c0+c)*lda + r0 + i
-      for (int q = t; q < nr * nc; q += PW_WIDE_THREADS) {
-        const int c = q / nr, i = q - c * nr;
-        tile[i * (C + 1) + c] = A[(size_t)(c0 + c) * lda + r0 + i];
-      }
+  const int rb = (blockIdx.x & 7) * (int)(gridDim.x >> 3) + (blockIdx.x >> 3);
+  const int r0 = rb * PD_ROWS, nr = min(rows - r0, PD_ROWS);
+  if (nr <= 0) return;  // the grid is a multiple of 8
+  double x[PD_PARTS][PD_LOADS];
+  // entry u of this thread in a part: its row and column there
+  auto at = [&](int u, int& i, int& c) {
+    const int e = t + PW_WIDE_THREADS * u;
+    i = TRANS ? e / PD_PCOLS : e % PD_ROWS;
+    c = TRANS ? e % PD_PCOLS : e / PD_ROWS;
+  };
+  auto fetch = [&](int c0, double (&v)[PD_LOADS]) {
+#pragma unroll
+    for (int u = 0; u < PD_LOADS; ++u) {
+      int i, c;
+      at(u, i, c);
+      const int r = min(r0 + i, rows - 1), k = min(c0 + c, cols - 1);  // entries past the end are not used
+      v[u] = TRANS ? A[(size_t)r * lda + k] : A[(size_t)k * lda + r];
     }
-    __syncthreads();
-    if (t < nr) {
-      const double* row = tile + t * (C + 1);
-      for (int c = 0; c < nc; ++c) acc = fma(row[c], xs[c0 + c], acc);
+  };
+#pragma unroll
+  for (int j = 0; j < PD_PARTS; ++j) fetch(j * PD_PCOLS, x[j]);
+  if (bound.first) {
+    if (!pw_bound(bound, rb == 0, xs, red, flag)) return;
+  } else {
+    if (s->done) return;
+    for (int i = t; i < cols; i += PW_WIDE_THREADS) xs[i] = cur[i];
+  }
+  double acc = 0.0;
+  for (int c0 = 0; c0 < cols; c0 += PD_COLS) {
+#pragma unroll
+    for (int j = 0; j < PD_PARTS; ++j) {
+      const int p0 = c0 + j * PD_PCOLS;
+      if (p0 < cols) {  // the same for the whole workgroup
+        // this part of the tile was last read before the previous part's barrier
+#pragma unroll
+        for (int u = 0; u < PD_LOADS; ++u) {
+          int i, c;
+          at(u, i, c);
+          tile[j][i * PD_LD + c] = x[j][u];
+        }
+        if (p0 + PD_COLS < cols) fetch(p0 + PD_COLS, x[j]);
+        __syncthreads();
+        if (t < PD_ROWS) {
+          const int nc = min(PD_PCOLS, cols - p0);
+          const pw_d2* m = reinterpret_cast<const pw_d2*>(tile[j] + t * PD_LD);
+          const pw_d2* xc = reinterpret_cast<const pw_d2*>(xs + p0);
+          // 16 columns at a time, the next 16 on their way from LDS meanwhile
+          // (reads past the part stay inside the arrays and are not used)
+          pw_d2 a[2][8], y[2][8];
+          auto load = [&](int c, pw_d2 (&la)[8], pw_d2 (&ly)[8]) {
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+              la[u] = m[min(c, PD_PCOLS - 16) / 2 + u];
+              ly[u] = xc[min(c, PD_PCOLS - 16) / 2 + u];
+            }
+          };
+          auto mac = [&](const pw_d2 (&la)[8], const pw_d2 (&ly)[8]) {
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+              acc = fma(la[u].x, ly[u].x, acc);
+              acc = fma(la[u].y, ly[u].y, acc);
+            }
+          };
+          load(0, a[0], y[0]);
+          int c = 0;
+          for (; c + 32 <= nc; c += 32) {
+            load(c + 16, a[1], y[1]);
+            __builtin_amdgcn_sched_barrier(0);
+            mac(a[0], y[0]);
+            __builtin_amdgcn_sched_barrier(0);
+            load(c + 32, a[0], y[0]);
+            __builtin_amdgcn_sched_barrier(0);
+            mac(a[1], y[1]);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          const double* ms = tile[j] + t * PD_LD;
+          for (; c < nc; ++c) acc = fma(ms[c], xs[p0 + c], acc);
+        }
+      }
     }
   }
   if (t < nr) nxt[r0 + t] = acc;
@@ -849,56 +1009,47 @@ __global__ __launch_bounds__(PW_WIDE_THREADS) void k_pw_dense_g(const double* __
   nxt[r] = acc;
 }
 
-// One round boundary.  mode 1: finish the previous round (xa = chain output):
-// zero test and lambda = <xn, xa>.  Then the loop test of the persistent
-// kernel, and if it continues: it++, normalise xa into xn.
-__global__ __launch_bounds__(PW_THREADS) void k_pw_step(int n, double* __restrict__ xa, double* __restrict__ xn,
-                                                         PwState* __restrict__ s, int maxit, double thr, int mode) {
+// A boundary of its own: in front of an operator that reads x from global
+// memory, and after the last round (which only evaluates the loop test).
+__global__ __launch_bounds__(PW_THREADS) void k_pw_step(PwBound b) {
   __shared__ double red[RED_LANES];
   __shared__ double tot;
   const int t = threadIdx.x;
-  const PwState st = *s;
-  __syncthreads();
-  if (st.done) return;
-  double lambda = st.lambda, lambda_old = st.lambda_old;
-  int it = st.it;
-  if (mode == 1) {
+  PwState st = *b.in;
+  if (st.done) {
+    if (t == 0) *b.out = st;
+    return;
+  }
+  if (b.mode == 1) {
     int nz = 0;
-    for (int i = t; i < n; i += PW_THREADS) nz |= (xa[i] != 0.0);
+    for (int i = t; i < b.n; i += PW_THREADS) nz |= (b.xa[i] != 0.0);
     if (!__syncthreads_or(nz)) {
-      if (t == 0) {
-        s->status = 2;
-        s->done = 1;
+      st.status = 2;
+      st.done = 1;
+    } else {
+      st.lambda = pw_dot(b.xn_in, b.xa, b.n, red, &tot);
+    }
+  }
+  if (!st.done) {
+    const double athr = fabs(b.thr);
+    if (!((fabs(st.lambda_old - st.lambda) > athr || fabs(st.lambda) <= athr) && st.it < b.maxit)) {
+      st.done = 1;
+    } else {
+      st.it++;
+      st.lambda_old = st.lambda;
+      const double nrm = sqrt(pw_dot(b.xa, b.xa, b.n, red, &tot));
+      if (nrm == 0.0) {
+        st.status = 1;
+        st.done = 1;
+      } else {
+        const double inv = 1 / nrm;
+        for (int i = t; i < b.n; i += PW_THREADS) b.xn_out[i] = b.xa[i] * inv;
       }
-      return;
     }
-    lambda = pw_dot(xn, xa, n, red, &tot);
   }
-  const double athr = fabs(thr);
-  if (!((fabs(lambda_old - lambda) > athr || fabs(lambda) <= athr) && it < maxit)) {
-    if (t == 0) {
-      s->lambda = lambda;
-      s->done = 1;
-    }
-    return;
-  }
-  it++;
-  lambda_old = lambda;
-  const double nrm = sqrt(pw_dot(xa, xa, n, red, &tot));
-  if (nrm == 0.0) {
-    if (t == 0) {
-      s->it = it;
-      s->status = 1;
-      s->done = 1;
-    }
-    return;
-  }
-  const double inv = 1 / nrm;
-  for (int i = t; i < n; i += PW_THREADS) xn[i] = xa[i] * inv;
   if (t == 0) {
-    s->lambda = lambda;
-    s->lambda_old = lambda_old;
-    s->it = it;
+    if (st.done) pw_post(st, b.maxit, b.res);
+    *b.out = st;
   }
 }
 
@@ -926,21 +1077,44 @@ const std::vector<double>& power_x0(int n) {
   return cache.emplace(n, std::move(x)).first->second;
 }
 
-// Per-round time estimates (seconds): the persistent kernel streams every
-// operator through one CU (~100 GB/s); the wide form pays a launch per
-// operator but spreads the rows over the chip, leaving each row's fma chain
-// (about 4 ns per term) as its floor.  FH_POWER_WIDE=0/1 forces a form.
+// start vector on the device: power_x0(PL_ROWS), whose first n values are
+// power_x0(n) for every n (one random sequence), uploaded once per device
+static const double* pl_x0() {
+  constexpr int kMaxDevices = 64;
+  static std::mutex mu;
+  static double* dx[kMaxDevices] = {};
+  int dev = 0;
+  FH_HIP(hipGetDevice(&dev));
+  FH_CHECK(dev >= 0 && dev < kMaxDevices, "power_iteration: device index out of range");
+  const std::vector<double>& x = power_x0(PL_ROWS);
+  std::lock_guard<std::mutex> lk(mu);
+  if (!dx[dev]) {
+    double* p = static_cast<double*>(dev_alloc(sizeof(double) * PL_ROWS));  // held to process end
+    FH_HIP(hipMemcpy(p, x.data(), sizeof(double) * PL_ROWS, hipMemcpyHostToDevice));
+    dx[dev] = p;
+  }
+  return dx[dev];
+}
+
+// Per-round time estimates (seconds).  The persistent kernel streams every
+// operator through one CU (~100 GB/s), and an entry of a row it does not load
+// ahead (dense, or more than PW_PF) is a dependent load (~90 ns: 10.7 us per
+// operator of a dense 128 x 100 chain, 4.5 us with 32 entries per row); the
+// wide form pays a launch per operator but spreads the rows over the chip,
+// leaving each row's fma chain (about 4 ns per term) as its floor.
+// FH_POWER_WIDE=0/1 forces a form.
 static bool use_wide_form(const std::vector<PwOp>& h) {
   if (const char* e = getenv("FH_POWER_WIDE")) {
     if (e[0] == '0') return false;
     if (e[0] == '1') return true;
   }
-  double single = 3e-6, wide = 4e-6;
+  double single = 3e-6, wide = 1e-6;
   for (const PwOp& o : h) {
     const double entries = o.kind == 1 ? (double)o.nnz : (double)o.rows * o.cols;
     const double bytes = entries * (o.kind == 1 ? 12.0 : 8.0);
-    single += bytes / 100e9 + 0.4e-6;
-    wide += 3e-6 + (entries / std::max(o.rows, 1)) * 4e-9 + bytes / 1.5e12;
+    const double row = o.kind == 1 ? (o.width >= 0 ? o.width : entries / std::max(o.rows, 1)) : o.cols;
+    single += std::max(bytes / 100e9, row > PW_PF ? row * 90e-9 : 0.0) + 0.4e-6;
+    wide += 4e-6 + row * 4e-9 + bytes / 3e12;
   }
   return wide < single;
 }
@@ -949,63 +1123,84 @@ static double power_iteration_wide(const std::vector<PwOp>& h, int n, const std:
                                    double thr, int* flag, hipStream_t st) {
   int vmax = n;
   for (const PwOp& o : h) vmax = std::max(vmax, std::max(o.rows, o.cols));
-  DBuf xa(sizeof(double) * n), xn(sizeof(double) * n), b0(sizeof(double) * vmax), b1(sizeof(double) * vmax),
-      ds(sizeof(PwState));
+  // the chain's output and the normalised vector alternate between two halves:
+  // a boundary reads the previous round's while its launch writes this one's
+  DBuf xa(sizeof(double) * 2 * n), xn(sizeof(double) * 2 * n), b0(sizeof(double) * vmax), b1(sizeof(double) * vmax),
+      ds(sizeof(PwState) * 2);
   PwState* dst = ds.as<PwState>();
-  FH_HIP(hipMemcpyAsync(xa.p, x0.data(), sizeof(double) * n, hipMemcpyHostToDevice, st));
+  double* res = mail() + MAIL_POWER;
+  res[3] = 0.0;  // set by the boundary that ends the iteration
+  const double* start = xa.as<double>();
+  if (n <= PL_ROWS)
+    start = pl_x0();
+  else
+    FH_HIP(hipMemcpyAsync(xa.p, x0.data(), sizeof(double) * n, hipMemcpyHostToDevice, st));
   hipLaunchKernelGGL(k_pw_init, dim3(1), dim3(64), 0, st, dst);
   FH_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_pw_step, dim3(1), dim3(PW_THREADS), 0, st, n, xa.as<double>(), xn.as<double>(), dst, maxit,
-                     thr, 0);
-  FH_LAUNCH_CHECK();
   const int nops = (int)h.size();
-  PwState hs{};
+  const bool fused = h.back().cols <= PW_VMAX;  // the boundary runs in the first operator's launch
   int next_check = 4;
-  for (int round = 1; round <= maxit; ++round) {
-    const double* cur = xn.as<double>();
+  PwBound b{};
+  b.n = n;
+  b.maxit = maxit;
+  b.thr = thr;
+  b.res = res;
+  for (int round = 1; round <= maxit + 1; ++round) {
+    b.mode = round > 1;
+    b.xa = round > 1 ? xa.as<double>() + (size_t)((round - 1) & 1) * n : start;
+    double* const xa_out = xa.as<double>() + (size_t)(round & 1) * n;
+    b.xn_in = xn.as<double>() + (size_t)((round - 1) & 1) * n;
+    b.xn_out = xn.as<double>() + (size_t)(round & 1) * n;
+    b.in = dst + ((round - 1) & 1);
+    b.out = dst + (round & 1);
+    const bool last = round > maxit;  // every round ran: the loop test alone
+    b.first = 0;
+    if (!fused || last) {
+      hipLaunchKernelGGL(k_pw_step, dim3(1), dim3(PW_THREADS), 0, st, b);
+      FH_LAUNCH_CHECK();
+      if (last) break;
+    }
+    const double* cur = b.xn_out;
     for (int s = nops - 1; s >= 0; --s) {
       const PwOp& o = h[s];
-      double* out = (s == 0) ? xa.as<double>() : (((nops - 1 - s) & 1) ? b1.as<double>() : b0.as<double>());
-      int R = 1;
-      while (R < 8 && (o.rows + 2 * R - 1) / (2 * R) >= 256) R *= 2;
-      const dim3 grid((o.rows + R - 1) / R);
+      b.first = fused && s == nops - 1;
+      double* out = (s == 0) ? xa_out : (((nops - 1 - s) & 1) ? b1.as<double>() : b0.as<double>());
       if (o.cols > PW_VMAX) {  // x does not fit LDS: read it from global memory
         const dim3 gg((o.rows + PW_WIDE_THREADS - 1) / PW_WIDE_THREADS);
         if (o.kind == 1)
           hipLaunchKernelGGL(k_pw_csr_g, gg, dim3(PW_WIDE_THREADS), 0, st, o.rp, o.ci, o.v, o.rows, cur, out,
-                             (const PwState*)dst);
+                             (const PwState*)b.out);
         else
           hipLaunchKernelGGL(k_pw_dense_g, gg, dim3(PW_WIDE_THREADS), 0, st, o.v, o.lda, o.trans, o.rows, o.cols,
-                             cur, out, (const PwState*)dst);
-      } else if (o.kind == 1)
-        hipLaunchKernelGGL(k_pw_csr, grid, dim3(PW_WIDE_THREADS), 0, st, o.rp, o.ci, o.v, o.rows, o.cols, R, cur,
-                           out, (const PwState*)dst);
-      else
-        hipLaunchKernelGGL(k_pw_dense, grid, dim3(PW_WIDE_THREADS), 0, st, o.v, o.lda, o.trans, o.rows, o.cols, R,
-                           cur, out, (const PwState*)dst);
+                             cur, out, (const PwState*)b.out);
+      } else if (o.kind == 1) {
+        int R = 1;
+        while (R < 8 && (o.rows + 2 * R - 1) / (2 * R) >= 256) R *= 2;
+        hipLaunchKernelGGL(k_pw_csr, dim3((o.rows + R - 1) / R), dim3(PW_WIDE_THREADS), 0, st, o.rp, o.ci, o.v,
+                           o.rows, o.cols, R, cur, out, (const PwState*)b.out, b);
+      } else {
+        const int nb = (o.rows + PD_ROWS - 1) / PD_ROWS;
+        const dim3 grid((unsigned)((nb + 7) / 8 * 8));
+        if (o.trans)
+          hipLaunchKernelGGL(k_pw_dense<true>, grid, dim3(PW_WIDE_THREADS), 0, st, o.v, o.lda, o.rows, o.cols, cur,
+                             out, (const PwState*)b.out, b);
+        else
+          hipLaunchKernelGGL(k_pw_dense<false>, grid, dim3(PW_WIDE_THREADS), 0, st, o.v, o.lda, o.rows, o.cols, cur,
+                             out, (const PwState*)b.out, b);
+      }
       FH_LAUNCH_CHECK();
       cur = out;
     }
-    hipLaunchKernelGGL(k_pw_step, dim3(1), dim3(PW_THREADS), 0, st, n, xa.as<double>(), xn.as<double>(), dst,
-                       maxit, thr, 1);
-    FH_LAUNCH_CHECK();
-    if (round == next_check || round == maxit) {
-      FH_HIP(hipMemcpyAsync(&hs, dst, sizeof(PwState), hipMemcpyDeviceToHost, st));
+    if (round == next_check) {
       FH_HIP(hipStreamSynchronize(st));
-      if (hs.done) break;
+      if (res[3] != 0.0) break;
       next_check += 8;
     }
   }
-  if (!hs.done) {  // every round ran: one more step evaluates the loop test
-    hipLaunchKernelGGL(k_pw_step, dim3(1), dim3(PW_THREADS), 0, st, n, xa.as<double>(), xn.as<double>(), dst,
-                       maxit, thr, 1);
-    FH_LAUNCH_CHECK();
-    FH_HIP(hipMemcpyAsync(&hs, dst, sizeof(PwState), hipMemcpyDeviceToHost, st));
-    FH_HIP(hipStreamSynchronize(st));
-  }
-  if (hs.status == 1) throw Error(FH_ERR_NUMERIC, "Can't normalize a zero-norm vector.");
-  if (flag) *flag = (hs.it < maxit) ? hs.it : -1;
-  return hs.status == 2 ? 0.0 : hs.lambda;
+  FH_HIP(hipStreamSynchronize(st));
+  if (res[2] == 1.0) throw Error(FH_ERR_NUMERIC, "Can't normalize a zero-norm vector.");
+  if (flag) *flag = (int)res[1];
+  return res[0];
 }
 
 static std::vector<PwOp> pw_ops(const std::vector<ChainOp>& ops) {
@@ -1180,25 +1375,6 @@ static bool pl_job(const std::vector<PwOp>& h, int n, PlJob& j, size_t* lds) {
   *lds = sizeof(double) * (nval + 3 * (size_t)j.ld) + sizeof(int) * ncol;
   j.nval = (int)std::min<size_t>(nval, INT_MAX);
   return *lds <= PL_LDS_BYTES;
-}
-
-// start vector on the device: power_x0(PL_ROWS), whose first n values are
-// power_x0(n) for every n (one random sequence), uploaded once per device
-static const double* pl_x0() {
-  constexpr int kMaxDevices = 64;
-  static std::mutex mu;
-  static double* dx[kMaxDevices] = {};
-  int dev = 0;
-  FH_HIP(hipGetDevice(&dev));
-  FH_CHECK(dev >= 0 && dev < kMaxDevices, "power_iteration: device index out of range");
-  const std::vector<double>& x = power_x0(PL_ROWS);
-  std::lock_guard<std::mutex> lk(mu);
-  if (!dx[dev]) {
-    double* p = static_cast<double*>(dev_alloc(sizeof(double) * PL_ROWS));  // held to process end
-    FH_HIP(hipMemcpy(p, x.data(), sizeof(double) * PL_ROWS, hipMemcpyHostToDevice));
-    dx[dev] = p;
-  }
-  return dx[dev];
 }
 
 template <int NT>

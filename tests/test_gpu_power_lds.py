@@ -46,3 +46,15 @@ def test_power_lds_zero_product(gpu):
     b[20:, :] = 1.0
     facs = [sp.csr_matrix(a), sp.csr_matrix(b)]
     assert faust_amd.Faust(facs).norm(2) == oracle.spectral_norm(facs)[0] == 0.0
+
+
+@pytest.mark.parametrize("m,n", [(1, 5), (255, 257), (37, 1536), (1030, 1023), (1100, 2048), (2100, 260)])
+def test_power_wide_dense_bits(gpu, monkeypatch, m, n):
+    # k_pw_dense's parts and row groups, the boundary inside the first operator's launch and (2100) before it
+    monkeypatch.setenv("FH_POWER_WIDE", "1")
+    rng = np.random.default_rng(m)
+    facs = [np.asfortranarray(rng.standard_normal((m, n))), _uneven(n, n, 4, rng)]
+    for fs in (facs, facs[:1], facs[::-1] if m == n else facs[1:]):
+        F = faust_amd.Faust(fs)
+        for maxit in (1, 4, 5, 100):
+            assert F.norm(2, max_num_its=maxit) == oracle.spectral_norm(fs, maxit)[0]
