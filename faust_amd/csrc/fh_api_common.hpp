@@ -149,6 +149,8 @@ void bsr_chain_launch(const std::vector<DMatP>& f, char op, const void* X, int p
 int faust_multiply_mixed(const std::vector<DMatP>& f, char op, const void* X, int p, void* Y, hipStream_t st,
                           const ChainWs& ws, FaustTimers* tm = nullptr, bool act_f32 = false, bool tune = true);
 // Y = alpha op(B) X + beta Y, B an FP32 BSR factor, X / Y FP32 column-major
+// (in_tiled / out_tiled: X / Y in the tiles of a chain's intermediates instead)
 void bsr_mul_f32(const DMat& B, char op, const float* X, int ldx, int p, float* Y, int ldy, float alpha, float beta,
-                 hipStream_t st);
+                 hipStream_t st, bool in_tiled = false, bool out_tiled = false);
+size_t faust_ws_need_f32_tiled(const std::vector<DMatP>& f, char op, int p, int* nbuf);
 }  // namespace fh

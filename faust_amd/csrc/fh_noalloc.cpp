@@ -92,6 +92,11 @@ extern "C" int fh_faust_multiply_noalloc(fh_faust_t F, char op, const void* X, i
       nbuf = rm_nbuf;
     }
   }
+  if (act_f32) {
+    int tbuf = 0;
+    const size_t tiled = std::max(need, faust_ws_need_f32_tiled(f, op, p, &tbuf));
+    if ((size_t)nbuf * align256(tiled) <= kScratchBytes) need = tiled;
+  }
   const size_t slot = align256(need);
   // BSR chains also keep the one-launch chain's control block at the start of
   // the array (zero at load; every chain leaves its counters cleared)

@@ -549,9 +549,9 @@ static void bsr_mul(const DMat& B, char op, const void* X, int ldx, int p, void*
 // the arithmetic of MatBSR<float>::multiply (faust_MatBSR.hpp:828-836) on
 // v_mfma_f32_32x32x2_f32: a wave owns one block row x one 32-column tile and
 // runs 16 K-steps per block; in step s lane (h, r) feeds A = B(r, 16h + s)
-// and B = X(16h + s, tile column r), so the blocks (stored that way, 16
-// consecutive floats per lane) and the X column segments are 4 float4 loads
-// per lane.  Blocks in row order (b ascending, then step by step), FP32
+// and B = X(16h + s, tile column r): 16 consecutive floats of a block row and
+// of an X column, four float4 loads each (the blocks are stored with float4 u
+// of lane l at u*64 + l, so theirs are contiguous).  Blocks in row order (b ascending, then step by step), FP32
 // accumulation.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 __global__ __launch_bounds__(256) void k_bsr_f32(int nbr, int p, const int* __restrict__ brp,
@@ -569,12 +569,12 @@ __global__ __launch_bounds__(256) void k_bsr_f32(int nbr, int p, const int* __re
   const int b0 = brp[br], b1 = brp[br + 1];
   for (int b = b0; b < b1; ++b) {
     const int bc = bci[b];
-    const f32x4* ap = reinterpret_cast<const f32x4*>(blk + (size_t)b * 1024 + lane * 16);
+    const f32x4* ap = reinterpret_cast<const f32x4*>(blk + (size_t)b * 1024) + lane;
     const f32x4* xp = reinterpret_cast<const f32x4*>(X + (size_t)j * ldx + bc * 32 + h * 16);
     f32x4 a[4], x[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      a[q] = ap[q];
+      a[q] = ap[64 * q];
       x[q] = xp[q];
     }
 #pragma unroll
@@ -604,7 +604,20 @@ __global__ __launch_bounds__(256) void k_bsr_f32(int nbr, int p, const int* __re
 // MFMA sequence of every output tile is k_bsr_f32's (blocks ascending, 16
 // K-steps each), so the bits are the same.  Consecutive workgroups walk the
 // column groups first (one group per XCD pair, as in k_bsr_shared).
+//
+// IN_TILED / OUT_TILED: X / Y is an intermediate of a chain, kept in 32 x 32
+// tiles in operand order (float4 u of lane l, rows 16 (l / 32) + 4u .. + 3 of
+// column l % 32, at u*64 + l; tile of block row b, panel g at b*G + g), so a
+// wave's operand is four contiguous 1 KiB loads and its output four stores of
+// two 512-byte runs.  Column-major, each of those loads touches 32 cache lines
+// a whole column apart (a power of two for most orders, so few L2 channels)
+// and comes back to them four times.  8192^2, 4 blocks per row, 512 columns:
+// 19.3 -> 17.4 us per launch (rows of 1 to 12 blocks, the transpose: 24 -> 21
+// us with partial rounds loaded as whole ones, not block by block).  A launch
+// reads 50 MB through the fabric (each XCD its 128 columns of X and half the
+// blocks) and has 6.8 us of MFMA, which starts when the loads land.
 constexpr int BF32_CH = 4;  // blocks staged per round
+template <bool IN_TILED, bool OUT_TILED>
 __global__ __launch_bounds__(256) void k_bsr_f32s(int nbr, int p, const int* __restrict__ brp,
                                                   const int* __restrict__ bci, const float* __restrict__ blk,
                                                   const float* __restrict__ X, int ldx, float* __restrict__ Y, int ldy,
@@ -614,6 +627,7 @@ __global__ __launch_bounds__(256) void k_bsr_f32s(int nbr, int p, const int* __r
   const int g = blockIdx.x % ngroups, br = blockIdx.x / ngroups;
   if (br >= nbr) return;
   const int h = lane >> 5, r = lane & 31;
+  const int G = (p + 31) >> 5, panel = min(g * 4 + wave, G - 1);  // waves past the last panel repeat it
   const int jc = g * 128 + wave * 32 + r;
   const bool jok = jc < p;
   const int j = jok ? jc : 0;  // columns past p read column 0; their outputs are not stored
@@ -621,55 +635,46 @@ __global__ __launch_bounds__(256) void k_bsr_f32s(int nbr, int p, const int* __r
   const int b0 = brp[br], b1 = brp[br + 1];
   for (int c0 = b0; c0 < b1; c0 += BF32_CH) {
     const int nb = min(BF32_CH, b1 - c0);
+    // the staging loads and this wave's X operands of the round's blocks are
+    // issued together, before any LDS write or MFMA (a partial round loads its
+    // last block again in place of the missing ones)
+    f32x4 stg[BF32_CH], x[BF32_CH][4];
+    int bc[BF32_CH];
+#pragma unroll
+    for (int q = 0; q < BF32_CH; ++q) {
+      const int b = c0 + min(q, nb - 1);
+      bc[q] = bci[b];
+      stg[q] = reinterpret_cast<const f32x4*>(blk + (size_t)b * 1024)[t];
+    }
+#pragma unroll
+    for (int q = 0; q < BF32_CH; ++q) {
+      const f32x4* xp = IN_TILED ? reinterpret_cast<const f32x4*>(X) + ((size_t)bc[q] * G + panel) * 256 + lane
+                                 : reinterpret_cast<const f32x4*>(X + (size_t)j * ldx + bc[q] * 32 + h * 16);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) x[q][u] = xp[IN_TILED ? 64 * u : u];
+    }
+    __builtin_amdgcn_sched_barrier(0);
     if (c0 > b0) lds_barrier();  // the previous round's blocks are consumed
-    if (nb == BF32_CH) {
-      // a full round: the staging loads and this wave's X column segments of
-      // all its blocks are issued together, before any LDS write or MFMA
-      f32x4 stg[BF32_CH], x[BF32_CH][4];
 #pragma unroll
-      for (int q = 0; q < BF32_CH; ++q) stg[q] = reinterpret_cast<const f32x4*>(blk + (size_t)(c0 + q) * 1024)[t];
+    for (int q = 0; q < BF32_CH; ++q) sa[q * 256 + t] = stg[q];
+    lds_barrier();
 #pragma unroll
-      for (int q = 0; q < BF32_CH; ++q) {
-        const f32x4* xp = reinterpret_cast<const f32x4*>(X + (size_t)j * ldx + bci[c0 + q] * 32 + h * 16);
+    for (int q = 0; q < BF32_CH; ++q) {
+      if (q >= nb) break;
+      f32x4 a[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) x[q][u] = xp[u];
-      }
-      __builtin_amdgcn_sched_barrier(0);
+      for (int u = 0; u < 4; ++u) a[u] = sa[q * 256 + u * 64 + lane];
 #pragma unroll
-      for (int q = 0; q < BF32_CH; ++q) sa[q * 256 + t] = stg[q];
-      lds_barrier();
-#pragma unroll
-      for (int q = 0; q < BF32_CH; ++q) {
-        f32x4 a[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) a[u] = sa[q * 256 + lane * 4 + u];
-#pragma unroll
-        for (int s4 = 0; s4 < 16; ++s4)
-          acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s4 >> 2][s4 & 3], x[q][s4 >> 2][s4 & 3], acc, 0, 0, 0);
-      }
-    } else {
-      // the row's last, partial round: one block at a time
-      for (int q = 0; q < nb; ++q) {
-        if (q > 0) __syncthreads();
-        sa[t] = reinterpret_cast<const f32x4*>(blk + (size_t)(c0 + q) * 1024)[t];
-        const f32x4* xp = reinterpret_cast<const f32x4*>(X + (size_t)j * ldx + bci[c0 + q] * 32 + h * 16);
-        f32x4 x[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) x[u] = xp[u];
-        __syncthreads();
-        f32x4 a[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) a[u] = sa[lane * 4 + u];
-#pragma unroll
-        for (int s4 = 0; s4 < 16; ++s4)
-          acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s4 >> 2][s4 & 3], x[s4 >> 2][s4 & 3], acc, 0, 0, 0);
-      }
+      for (int s4 = 0; s4 < 16; ++s4)
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s4 >> 2][s4 & 3], x[q][s4 >> 2][s4 & 3], acc, 0, 0, 0);
     }
   }
   if (!jok) return;
 #pragma unroll
   for (int gg = 0; gg < 4; ++gg) {
-    f32x4* yq = reinterpret_cast<f32x4*>(Y + (size_t)j * ldy + br * 32 + 8 * gg + 4 * h);
+    f32x4* yq = OUT_TILED ? reinterpret_cast<f32x4*>(Y) + ((size_t)br * G + panel) * 256 +
+                                (2 * (gg & 1) + h) * 64 + (gg >> 1) * 32 + r
+                          : reinterpret_cast<f32x4*>(Y + (size_t)j * ldy + br * 32 + 8 * gg + 4 * h);
     f32x4 v = {alpha * acc[4 * gg], alpha * acc[4 * gg + 1], alpha * acc[4 * gg + 2], alpha * acc[4 * gg + 3]};
     if (beta != 0.0f) {
       const f32x4 old = *yq;
@@ -682,28 +687,36 @@ __global__ __launch_bounds__(256) void k_bsr_f32s(int nbr, int p, const int* __r
   }
 }
 
+static bool bsr_f32_per_wave() {
+  const char* e = getenv("FH_BSR_F32_KERNEL");
+  return e && e[0] == '0';
+}
+
 void bsr_mul_f32(const DMat& B, char op, const float* X, int ldx, int p, float* Y, int ldy, float alpha, float beta,
-                 hipStream_t st) {
+                 hipStream_t st, bool in_tiled, bool out_tiled) {
   FH_CHECK(B.kind == K_BSR && B.dtype == FH_F32 && B.f32dat.p, "FP32 activations need an FP32 BSR factor");
   const bool tr = op != 'N';
   const int rows = tr ? B.n : B.m;
   const int nbr = rows / 32;
-  FH_CHECK(ldx % 4 == 0 && ldy % 4 == 0 && ((uintptr_t)X & 15) == 0 && ((uintptr_t)Y & 15) == 0,
+  FH_CHECK((in_tiled || ldx % 4 == 0) && (out_tiled || ldy % 4 == 0) && ((uintptr_t)X & 15) == 0 &&
+               ((uintptr_t)Y & 15) == 0,
            "FP32 BSR path: X and Y must be 16-byte aligned with leading dimensions that are multiples of 4");
   if (nbr == 0 || p == 0) return;
   const int* brp = (tr ? B.tbrp : B.brp).as<int>();
   const int* bci = (tr ? B.tbci : B.bci).as<int>();
   const float* blk = (tr ? B.tf32dat : B.f32dat).as<float>();
   // FH_BSR_F32_KERNEL=0: one wave per (block row, tile), blocks from global memory
-  const char* e = getenv("FH_BSR_F32_KERNEL");
-  if (e && e[0] == '0') {
+  if (bsr_f32_per_wave()) {
+    FH_CHECK(!in_tiled && !out_tiled, "FP32 BSR path: the per-wave kernel takes column-major operands");
     const int ntiles = (p + 31) / 32;
     const dim3 grid((unsigned)(ntiles * ((nbr + 3) / 4)));
     hipLaunchKernelGGL(k_bsr_f32, grid, dim3(256), 0, st, nbr, p, brp, bci, blk, X, ldx, Y, ldy, alpha, beta, ntiles);
   } else {
     const int ngroups = (p + 127) / 128;
-    hipLaunchKernelGGL(k_bsr_f32s, dim3((unsigned)(ngroups * nbr)), dim3(256), 0, st, nbr, p, brp, bci, blk, X, ldx,
-                       Y, ldy, alpha, beta, ngroups);
+    auto kern = in_tiled ? (out_tiled ? k_bsr_f32s<true, true> : k_bsr_f32s<true, false>)
+                         : (out_tiled ? k_bsr_f32s<false, true> : k_bsr_f32s<false, false>);
+    hipLaunchKernelGGL(kern, dim3((unsigned)(ngroups * nbr)), dim3(256), 0, st, nbr, p, brp, bci, blk, X, ldx, Y, ldy,
+                       alpha, beta, ngroups);
   }
   FH_LAUNCH_CHECK();
 }
@@ -1129,6 +1142,20 @@ static bool chain_verified(int sync, int* ctl, hipStream_t st) {
   return true;
 }
 
+// Bytes of each tiled intermediate of an FP32 BSR chain with FP32 activations
+// (p padded to whole 32-column panels); 0 where the chain keeps column-major
+// ones: a single factor, the per-wave kernel, or so few columns that the
+// padding costs more than the layout gives.
+constexpr int BF32_TILED_MIN = 17;
+size_t faust_ws_need_f32_tiled(const std::vector<DMatP>& f, char op, int p, int* nbuf) {
+  const int J = (int)f.size();
+  if (J < 2 || p < BF32_TILED_MIN || bsr_f32_per_wave()) return 0;
+  int maxr = 0;  // the last factor's output is Y
+  for (int i = 0; i + 1 < J; ++i) maxr = std::max(maxr, op == 'N' ? f[J - 1 - i]->m : f[i]->n);
+  *nbuf = std::min(2, J - 1);
+  return sizeof(float) * (size_t)maxr * (((size_t)p + 31) / 32 * 32);
+}
+
 // Bytes of each intermediate of a BSR or FP32 CSR chain product (*nbuf of
 // them): BSR intermediates are tiled, p padded to whole 32-column groups;
 // FP32 CSR ones are row-major with ld = p rounded up to 4.
@@ -1165,8 +1192,11 @@ static int multiply_mixed_run(const std::vector<DMatP>& f, char op, const void* 
   const int ldr = bsr ? 0 : (p + 3) & ~3;
   int in_rows = (op == 'N') ? f.back()->n : f.front()->m;
   if (act_f32) {
-    // FP32 BSR factors with FP32 activations: one k_bsr_f32 launch per factor,
-    // column-major FP32 intermediates
+    // FP32 BSR factors with FP32 activations: one launch per factor, FP32
+    // intermediates, tiled where the workspace has room for whole panels
+    int tbuf = 0;
+    const size_t tneed = faust_ws_need_f32_tiled(f, op, p, &tbuf);
+    const bool tiled = tneed > 0 && ws.cap >= tneed;
     const float* in = static_cast<const float*>(X);
     for (int i = 0; i < J; ++i) {
       const DMat& S = (op == 'N') ? *f[J - 1 - i] : *f[i];
@@ -1175,7 +1205,7 @@ static int multiply_mixed_run(const std::vector<DMatP>& f, char op, const void* 
       float* out = (i == J - 1) ? static_cast<float*>(Y) : static_cast<float*>(ws.p[i & 1]);
       const size_t slot = (op == 'N') ? (size_t)(J - 1 - i) : (size_t)i;
       if (tm) tm->begin(slot, st);
-      bsr_mul_f32(S, op, in, in_rows, p, out, out_rows, 1.0f, 0.0f, st);
+      bsr_mul_f32(S, op, in, in_rows, p, out, out_rows, 1.0f, 0.0f, st, tiled && i > 0, tiled && i < J - 1);
       if (tm) tm->end(slot, st);
       in = out;
       in_rows = out_rows;
@@ -1355,7 +1385,7 @@ void bsr_to_host(const DMat& M, void* bdata, int32_t* browptr, int32_t* bcolinds
       for (int l = 0; l < 64; ++l)
         for (int q = 0; q < 16; ++q) {
           const int r = l & 31, c = (l >> 5) * 16 + q;
-          static_cast<float*>(bdata)[b * 1024 + (size_t)c * 32 + r] = f[b * 1024 + l * 16 + q];
+          static_cast<float*>(bdata)[b * 1024 + (size_t)c * 32 + r] = f[b * 1024 + ((q >> 2) * 64 + l) * 4 + (q & 3)];
         }
     return;
   }
@@ -1451,8 +1481,9 @@ DMatP make_bsr(int dtype, int m, int n, int bnnz, const int32_t* browptr, const 
       for (int l = 0; l < 64; ++l)
         for (int q = 0; q < 16; ++q) {
           const int r = l & 31, c = (l >> 5) * 16 + q;
-          f32[(size_t)b * 1024 + l * 16 + q] = src[(size_t)b * 1024 + (size_t)c * 32 + r];          // B(r, c)
-          tf32[(size_t)tslot_of[b] * 1024 + l * 16 + q] = src[(size_t)b * 1024 + (size_t)r * 32 + c];  // B(c, r)
+          const size_t o = ((q >> 2) * 64 + l) * 4 + (q & 3);
+          f32[(size_t)b * 1024 + o] = src[(size_t)b * 1024 + (size_t)c * 32 + r];          // B(r, c)
+          tf32[(size_t)tslot_of[b] * 1024 + o] = src[(size_t)b * 1024 + (size_t)r * 32 + c];  // B(c, r)
         }
   }
   up(M->brp, browptr, sizeof(int) * (nbr + 1));
