@@ -155,10 +155,10 @@ size_t faust_ws_need_rm_f64(const std::vector<DMatP>& f, char op, int p, int* nb
   if (f.empty() || p < RM_MIN_COLS || !chain_csr_ops(f, op, ops, &widest, &mean)) return 0;
   const int in_rows = (op == 'N') ? f.back()->n : f.front()->m;
   if (!csr_rm_fits(ops, in_rows, p)) return 0;
-  size_t r = (size_t)in_rows;  // the last factor's output is Y
-  for (size_t i = 0; i + 1 < ops.size(); ++i) r = std::max(r, (size_t)ops[i].rows);
+  int r = in_rows;  // the last factor's output is Y
+  for (size_t i = 0; i + 1 < ops.size(); ++i) r = std::max(r, ops[i].rows);
   *nbuf = std::min(2, (int)f.size());
-  return sizeof(double) * r * csr_rm_ld(p);
+  return sizeof(double) * csr_rm_size(r, p);
 }
 
 // Bytes of each of the (at most two) intermediates of an FP64 chain product;
@@ -778,7 +778,10 @@ int fh_faust_multiply(fh_faust_t F, char op, const void* X, int p, void* Y, void
     const bool act_f32 = F->act_dtype == FH_F32;
     size_t need = faust_ws_need_mixed(f, op, p, &nbuf, act_f32);
     int tbuf = 0;
-    if (act_f32) need = std::max(need, faust_ws_need_f32_tiled(f, op, p, &tbuf));
+    if (act_f32)
+      need = std::max(need, faust_ws_need_f32_tiled(f, op, p, &tbuf));
+    else if (f.front()->kind == K_CSR)
+      need = std::max(need, faust_ws_need_f32_panels(f, op, p, &tbuf));
     const ChainWs ws =
         faust_ws_grow(F->ws, need, nbuf, st, (f.front()->kind == K_BSR && !act_f32) ? &F->ctl : nullptr);
     F->last_launches = faust_multiply_mixed(f, op, X, p, Y, st, ws, &F->timers, act_f32);

@@ -152,5 +152,6 @@ int faust_multiply_mixed(const std::vector<DMatP>& f, char op, const void* X, in
 // (in_tiled / out_tiled: X / Y in the tiles of a chain's intermediates instead)
 void bsr_mul_f32(const DMat& B, char op, const float* X, int ldx, int p, float* Y, int ldy, float alpha, float beta,
                  hipStream_t st, bool in_tiled = false, bool out_tiled = false);
+size_t faust_ws_need_f32_panels(const std::vector<DMatP>& f, char op, int p, int* nbuf);
 size_t faust_ws_need_f32_tiled(const std::vector<DMatP>& f, char op, int p, int* nbuf);
 }  // namespace fh

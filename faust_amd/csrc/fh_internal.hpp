@@ -200,11 +200,12 @@ void csr_chain_pf_run_f64(const std::vector<ChainCsrOp>& ops, int in_rows, int w
 int csr_chain_fit_wc(const std::vector<ChainCsrOp>& ops, int in_rows, int p);
 // The same chain with row-major intermediates, one launch per factor
 // (k_csr_rm_f64): csr_rm_from_col transposes X (column-major, ld = rows) into
-// rows of csr_rm_ld(p) values, csr_rm_mul applies one op'd factor to such rows
+// panels of rows of csr_rm_ld(p) values (csr_rm_size in all), csr_rm_mul applies one op'd factor to such rows
 // (out_col: Y column-major, ld = S.rows).  fits: the shapes it takes.
 constexpr int RM_MIN_COLS = 12;               // columns from which the form is measured
 constexpr int64_t RM_TERMS_DEFAULT = 1 << 20;  // entries x columns of a factor from which it is the unmeasured choice
 int csr_rm_ld(int p);
+size_t csr_rm_size(int rows, int p);
 bool csr_rm_fits(const std::vector<ChainCsrOp>& ops, int in_rows, int p);
 void csr_rm_from_col(int rows, int p, const double* X, double* R, hipStream_t st);
 void csr_rm_mul(const ChainCsrOp& S, int in_rows, int p, const double* X, double* Y, bool out_col, hipStream_t st);

@@ -92,10 +92,12 @@ extern "C" int fh_faust_multiply_noalloc(fh_faust_t F, char op, const void* X, i
       nbuf = rm_nbuf;
     }
   }
-  if (act_f32) {
+  if (!f64 && (act_f32 || f.front()->kind == K_CSR)) {
+    // likewise for the padded layouts of FP32 intermediates
     int tbuf = 0;
-    const size_t tiled = std::max(need, faust_ws_need_f32_tiled(f, op, p, &tbuf));
-    if ((size_t)nbuf * align256(tiled) <= kScratchBytes) need = tiled;
+    const size_t padded = std::max(need, act_f32 ? faust_ws_need_f32_tiled(f, op, p, &tbuf)
+                                                 : faust_ws_need_f32_panels(f, op, p, &tbuf));
+    if ((size_t)nbuf * align256(padded) <= kScratchBytes) need = padded;
   }
   const size_t slot = align256(need);
   // BSR chains also keep the one-launch chain's control block at the start of

@@ -722,132 +722,128 @@ void bsr_mul_f32(const DMat& B, char op, const float* X, int ldx, int p, float* 
 }
 
 // ---------------------------------------------------------------- FP32 CSR
-// A row's batch of NB (<= 16) index/value pairs reaches its 8 lanes with two
-// loads per lane: lane s of the row's group loads entries s and 8 + s (entry
-// indices clamped to the row's last entry), and ds_swizzle hands entry q to
-// every lane of the group from lane q % 8.  All 8 lanes of a group must be
-// active (a group is one row).
-template <int Q, int NB>
-struct CsrBcast {
-  static __device__ __forceinline__ void go(int ia, int ib, float fa, float fb, int* cc, float* ww) {
-    constexpr int PAT = 0x18 | ((Q & 7) << 5);  // lane (l & ~7) | (Q % 8) within each 32
-    cc[Q] = __builtin_amdgcn_ds_swizzle(Q < 8 ? ia : ib, PAT);
-    ww[Q] = __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(Q < 8 ? fa : fb), PAT));
-    CsrBcast<Q + 1, NB>::go(ia, ib, fa, fb, cc, ww);
+// Row-major gather SpMM: Y[r, c] = alpha * sum_e v[e] * X[ci[e], c] + beta*Y.
+// A workgroup computes 32 rows x a panel of 32 columns, 8 lanes (one float4
+// each) per row.  Lane s of a row loads its entries s and 8 + s of a batch of
+// 16 and hands them to the row's other lanes through DPP row broadcasts (one
+// per half of the 16 lanes).  Gathers go through a buffer resource
+// whose range check returns zeros, without traffic, for the lanes past column
+// p and for the entries past the row's end, whose weight is -0: adding -0 x 0
+// leaves every fma chain as it is, so no term is selected.
+// ELL: ci / v are the ELL view (NB slots per row, column -1 in unused slots;
+// rp unused), so a row's entries load without the row pointer first.
+// OUT_COL: write Y column-major (ld = ldy) through an LDS transpose.
+// Workgroups are dealt to the XCDs in turn; XCD x takes a contiguous run of
+// the panel-major (panel, row block) list, so with up to 8 panels its L2
+// holds the one or two panels it gathers from.
+// Rows of X are ldx apart, panels xpanel (Y: ldy, ypanel).  Chains keep their
+// intermediates panel by panel: in whole rows of 256 columns, the 128 bytes of
+// each row that a panel's XCD gathers lie on a quarter of its L2 channels.
+// 16384^2, 12 entries per row, 256 columns: 12.8 us per launch (201 MB out of
+// the L2s, 46 MB through the fabric), 14.3 us in whole rows, 14.5 us with
+// ds_swizzle broadcasts and selected terms; the last one 16.9 -> 12.9 us.
+template <int Q>
+__device__ __forceinline__ unsigned csr_bcast8(unsigned x) {
+  // lane Q to lanes 0-7 of a DPP row, lane 8 + Q to lanes 8-15
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)x, 0x150 + Q, 0xf, 0x3, false);
+  return (unsigned)__builtin_amdgcn_update_dpp(lo, (int)x, 0x158 + Q, 0xf, 0xc, false);
+}
+template <int Q, int N>
+struct CsrGather {  // entries Q .. N - 1 of the 8 held by the lanes
+  static __device__ __forceinline__ void go(const __amdgpu_buffer_rsrc_t rx, unsigned off, unsigned w, unsigned coff,
+                                            f32x4* x, float* ww) {
+    x[Q] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                         rx, __builtin_elementwise_add_sat(csr_bcast8<Q>(off), coff), 0, 0));
+    ww[Q] = __uint_as_float(csr_bcast8<Q>(w));
+    CsrGather<Q + 1, N>::go(rx, off, w, coff, x, ww);
   }
 };
-template <int NB>
-struct CsrBcast<NB, NB> {
-  static __device__ __forceinline__ void go(int, int, float, float, int*, float*) {}
+template <int N>
+struct CsrGather<N, N> {
+  static __device__ __forceinline__ void go(const __amdgpu_buffer_rsrc_t, unsigned, unsigned, unsigned, f32x4*,
+                                            float*) {}
 };
+
+// NB entries (at most 16) of a row from the lanes' two entries each
 template <int NB>
-__device__ __forceinline__ void csr_batch_idx(const int* __restrict__ ci, const float* __restrict__ v, int base,
-                                              int nb, int s, int (&cc)[NB], float (&ww)[NB]) {
-  static_assert(NB <= 16, "two entries per lane");
-  const int ea = base + min(s, nb - 1);
-  const int ia = ci[ea];
-  const float fa = v[ea];
-  int ib = ia;
-  float fb = fa;
-  if (NB > 8) {
-    const int eb = base + min(8 + s, nb - 1);
-    ib = ci[eb];
-    fb = v[eb];
-  }
-  CsrBcast<0, NB>::go(ia, ib, fa, fb, cc, ww);
+__device__ __forceinline__ void csr_terms(const __amdgpu_buffer_rsrc_t rx, const unsigned (&off)[2],
+                                          const unsigned (&w)[2], unsigned coff, f32x4& acc) {
+  f32x4 x[NB];
+  float ww[NB];
+  CsrGather<0, (NB < 8 ? NB : 8)>::go(rx, off[0], w[0], coff, x, ww);
+  if constexpr (NB > 8) CsrGather<0, NB - 8>::go(rx, off[1], w[1], coff, x + 8, ww + 8);
+  __builtin_amdgcn_sched_barrier(0);  // all gathers in flight before the first FMA
+#pragma unroll
+  for (int q = 0; q < NB; ++q)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[c] = fmaf(ww[q], x[q][c], acc[c]);
 }
 
-// Row-major gather SpMM: Y[r, c] = alpha * sum_e v[e] * X[ci[e], c] + beta*Y.
-// OUT_COL: write Y column-major (ld = ldy) through an LDS transpose.
-// ELL: ci / v are the ELL view (NB slots per row, column -1 in unused
-// slots; rp unused), so a row's pairs load without the row pointer first;
-// the terms and their order are those of the CSR form.
 template <bool OUT_COL, int NB, bool ELL = false>
 __global__ __launch_bounds__(256) void k_csr_rm_f32(int rows, int p, const int* __restrict__ rp,
                                                     const int* __restrict__ ci, const float* __restrict__ v,
-                                                    const float* __restrict__ X, int ldx, float* __restrict__ Y,
-                                                    int ldy, float alpha, float beta, int npanels) {
+                                                    const float* __restrict__ X, unsigned xbytes, int ldx,
+                                                    size_t xpanel, float* __restrict__ Y, int ldy, size_t ypanel,
+                                                    float alpha, float beta, int nrb, int npanels) {
   __shared__ float tile[32][33];
-  const int t = threadIdx.x;
-  const int panel = blockIdx.x % npanels, rblk = blockIdx.x / npanels;
-  const int r = rblk * 32 + (t >> 3);
-  const int c0 = panel * 32 + (t & 7) * 4;
-  const int cg = c0 < p ? c0 : 0;  // lanes past p gather column 0 and store nothing
-  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (ELL && r < rows) {
-    int cc[NB];
-    float ww[NB];
-    csr_batch_idx<NB>(ci, v, r * NB, NB, t & 7, cc, ww);
-    float4 xx[NB];
+  const int t = threadIdx.x, s = t & 7;
+  const int w0 = (blockIdx.x & 7) * (int)(gridDim.x >> 3) + (blockIdx.x >> 3);
+  if (w0 >= nrb * npanels) return;  // the whole workgroup
+  const int panel = w0 / nrb, rblk = w0 - panel * nrb;
+  const int r = rblk * 32 + (t >> 3), rr = min(r, rows - 1);
+  const int c0 = panel * 32 + s * 4;
+  const unsigned coff = c0 < p ? 16u * s : 0xffffffffu;
+  const __amdgpu_buffer_rsrc_t rx =
+      __builtin_amdgcn_make_buffer_rsrc((void*)(X + panel * xpanel), 0, (int)xbytes, 0x00020000);
+  f32x4 acc = {};
+  // entries e and e + 8 of the batch for this lane (n: entries left in the row)
+  auto entries = [&](int e, int n, unsigned (&off)[2], unsigned (&w)[2]) {
 #pragma unroll
-    for (int q = 0; q < NB; ++q) xx[q] = *reinterpret_cast<const float4*>(X + (size_t)max(cc[q], 0) * ldx + cg);
-    __builtin_amdgcn_sched_barrier(0);  // all gathers in flight before the first FMA
-#pragma unroll
-    for (int q = 0; q < NB; ++q) {
-      const bool on = cc[q] >= 0;  // unused slots are not accumulated
-      acc.x = on ? fmaf(ww[q], xx[q].x, acc.x) : acc.x;
-      acc.y = on ? fmaf(ww[q], xx[q].y, acc.y) : acc.y;
-      acc.z = on ? fmaf(ww[q], xx[q].z, acc.z) : acc.z;
-      acc.w = on ? fmaf(ww[q], xx[q].w, acc.w) : acc.w;
+    for (int h = 0; h < (NB > 8 ? 2 : 1); ++h) {
+      const bool on = s + 8 * h < n;
+      const int q = on ? e + s + 8 * h : 0;
+      const int k = ci[q];
+      const float f = v[q];
+      const bool use = on && k >= 0;
+      off[h] = use ? (unsigned)k * (unsigned)(ldx * 4) : 0xffffffffu;
+      w[h] = use ? __float_as_uint(f) : 0x80000000u;
     }
-  }
-  if (!ELL && r < rows) {  // the same for the row's 8 lanes, as the broadcast needs
-    const int e0 = rp[r], e1 = rp[r + 1];
-    // batches of up to NB nonzeros (NB: the widest row rounded up to 4, at
-    // most 16): the index/value pairs, then all row gathers, then the FMAs,
-    // so NB gathers are in flight per thread.  The loads are unconditional
-    // (indices clamped to the row's last entry; the extra terms are not
-    // accumulated): a conditional load would become a branch that waits for
-    // the loads before it.
-    for (int base = e0; base < e1; base += NB) {
-      const int nb = min(NB, e1 - base);
-      int cc[NB];
-      float ww[NB];
-      csr_batch_idx<NB>(ci, v, base, nb, t & 7, cc, ww);
-      float4 xx[NB];
-#pragma unroll
-      for (int q = 0; q < NB; ++q) xx[q] = *reinterpret_cast<const float4*>(X + (size_t)cc[q] * ldx + cg);
-      __builtin_amdgcn_sched_barrier(0);  // all gathers in flight before the first FMA
-#pragma unroll
-      for (int q = 0; q < NB; ++q) {
-        const bool on = q < nb;  // terms past the row end are not accumulated
-        acc.x = on ? fmaf(ww[q], xx[q].x, acc.x) : acc.x;
-        acc.y = on ? fmaf(ww[q], xx[q].y, acc.y) : acc.y;
-        acc.z = on ? fmaf(ww[q], xx[q].z, acc.z) : acc.z;
-        acc.w = on ? fmaf(ww[q], xx[q].w, acc.w) : acc.w;
-      }
+  };
+  unsigned off[2], w[2];
+  if (ELL) {
+    entries(rr * NB, r < rows ? NB : 0, off, w);
+    csr_terms<NB>(rx, off, w, coff, acc);
+  } else {
+    const int e0 = rp[rr], len = r < rows ? rp[rr + 1] - e0 : 0;
+    for (int base = 0; __any(base < len); base += NB) {
+      entries(e0 + base, min(len - base, NB), off, w);
+      csr_terms<NB>(rx, off, w, coff, acc);
     }
   }
   if (!OUT_COL) {
     if (r < rows && c0 < p) {
-      float4* y = reinterpret_cast<float4*>(Y + (size_t)r * ldy + c0);
-      float4 o = make_float4(alpha * acc.x, alpha * acc.y, alpha * acc.z, alpha * acc.w);
+      f32x4* y = reinterpret_cast<f32x4*>(Y + panel * ypanel + (size_t)r * ldy + 4 * s);
+      f32x4 o = {alpha * acc[0], alpha * acc[1], alpha * acc[2], alpha * acc[3]};
       if (beta != 0.0f) {
-        const float4 old = *y;
-        o.x = fmaf(beta, old.x, o.x);
-        o.y = fmaf(beta, old.y, o.y);
-        o.z = fmaf(beta, old.z, o.z);
-        o.w = fmaf(beta, old.w, o.w);
+        const f32x4 old = *y;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) o[c] = fmaf(beta, old[c], o[c]);
       }
       *y = o;
     }
     return;
   }
-  const int lr = t >> 3, lc = (t & 7) * 4;
-  tile[lr][lc + 0] = acc.x;
-  tile[lr][lc + 1] = acc.y;
-  tile[lr][lc + 2] = acc.z;
-  tile[lr][lc + 3] = acc.w;
+  const int lr = t >> 3, lc = s * 4;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) tile[lr][lc + c] = acc[c];
   __syncthreads();
-  // thread -> column (t >> 3), 4 consecutive rows (t & 7) * 4
-  const int cc = t >> 3, rr = (t & 7) * 4;
-  const int gc = panel * 32 + cc;
-  if (gc >= p) return;
+  // lane -> row of the block, 8 columns at a time
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    const int gr = rblk * 32 + rr + q;
-    if (gr < rows) {
-      float o = alpha * tile[rr + q][cc];
+    const int row = t & 31, cc = (t >> 5) + 8 * q;
+    const int gr = rblk * 32 + row, gc = panel * 32 + cc;
+    if (gr < rows && gc < p) {
+      float o = alpha * tile[row][cc];
       float* y = Y + (size_t)gc * ldy + gr;
       if (beta != 0.0f) o = fmaf(beta, *y, o);
       *y = o;
@@ -861,13 +857,15 @@ __global__ __launch_bounds__(256) void k_csr_rm_f32(int rows, int p, const int* 
 template <bool OUT_COL>
 __global__ __launch_bounds__(256) void k_csr_rm2_f32(int rows, int p, const int* __restrict__ rp,
                                                      const int* __restrict__ ci, const float* __restrict__ v,
-                                                     const float* __restrict__ X, int ldx, float* __restrict__ Y,
-                                                     int ldy, float alpha, float beta, int npanels) {
+                                                     const float* __restrict__ X, int ldx, size_t xpanel,
+                                                     float* __restrict__ Y, int ldy, size_t ypanel, float alpha,
+                                                     float beta, int npanels) {
   __shared__ float tile[64][33];
   constexpr int NB = 8;
   const int t = threadIdx.x;
   const int panel = blockIdx.x % npanels, rblk = blockIdx.x / npanels;
   const int c0 = panel * 32 + (t & 7) * 4;
+  X += panel * xpanel + (t & 7) * 4;
   int r[2], e0[2], e1[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
@@ -895,7 +893,7 @@ __global__ __launch_bounds__(256) void k_csr_rm2_f32(int rows, int p, const int*
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int q = 0; q < NB; ++q)
-        xx[i][q] = cc[i][q] >= 0 ? *reinterpret_cast<const float4*>(X + (size_t)cc[i][q] * ldx + c0)
+        xx[i][q] = cc[i][q] >= 0 ? *reinterpret_cast<const float4*>(X + (size_t)cc[i][q] * ldx)
                                  : make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -911,7 +909,7 @@ __global__ __launch_bounds__(256) void k_csr_rm2_f32(int rows, int p, const int*
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       if (r[i] < rows && c0 < p) {
-        float4* y = reinterpret_cast<float4*>(Y + (size_t)r[i] * ldy + c0);
+        float4* y = reinterpret_cast<float4*>(Y + panel * ypanel + (size_t)r[i] * ldy + (t & 7) * 4);
         float4 o = make_float4(alpha * acc[i].x, alpha * acc[i].y, alpha * acc[i].z, alpha * acc[i].w);
         if (beta != 0.0f) {
           const float4 old = *y;
@@ -960,51 +958,74 @@ static int csr_rows_per_thread() {
   return (e && e[0] == '2') ? 2 : 1;
 }
 
-// column-major (rows x p, ld) -> row-major (rows x ldr), zero-padding columns p..ldr
+// column-major (rows x p, ld) -> rows ldr apart of panels of 32 columns
+// `panel` apart, p padded to a multiple of 4 with zeros: tiles of 64 rows x 32 columns, 256-byte reads (a lane per row, eight
+// in flight) and 128-byte writes; with four scalar loads per thread at a
+// 16-byte stride, 16384 x 256 took 11.6 us, now 6.4
 __global__ __launch_bounds__(256) void k_col2row_f32(int rows, int p, const float* __restrict__ X, int ldx,
-                                                     float* __restrict__ R, int ldr) {
-  __shared__ float tile[32][33];
+                                                     float* __restrict__ R, int ldr, size_t panel) {
+  __shared__ float tile[64][33];
   const int t = threadIdx.x;
-  const int r0 = blockIdx.x * 32, c0 = blockIdx.y * 32;
-  // read: thread -> column c0 + (t >> 3), rows r0 + (t & 7)*4 .. +3
-  const int cc = t >> 3, rr = (t & 7) * 4;
+  const int r0 = blockIdx.x * 64, c0 = blockIdx.y * 32;
+  const int row = min(r0 + (t & 63), rows - 1);
+  float x[8];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int gr = r0 + rr + q, gc = c0 + cc;
-    tile[rr + q][cc] = (gr < rows && gc < p) ? X[(size_t)gc * ldx + gr] : 0.0f;
-  }
+  for (int q = 0; q < 8; ++q) x[q] = X[(size_t)min(c0 + (t >> 6) + 4 * q, p - 1) * ldx + row];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) tile[t & 63][(t >> 6) + 4 * q] = c0 + (t >> 6) + 4 * q < p ? x[q] : 0.0f;
   __syncthreads();
-  const int lr = t >> 3, lc = (t & 7) * 4;
-  const int gr = r0 + lr;
-  if (gr >= rows) return;
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int gc = c0 + lc + q;
-    if (gc < ldr) R[(size_t)gr * ldr + gc] = tile[lr][lc + q];
+  for (int q = 0; q < 2; ++q) {
+    const int lr = (t >> 3) + 32 * q, lc = (t & 7) * 4;
+    if (r0 + lr < rows && c0 + lc < ((p + 3) & ~3))
+      *reinterpret_cast<f32x4*>(R + blockIdx.y * panel + (size_t)(r0 + lr) * ldr + lc) =
+          f32x4{tile[lr][lc], tile[lr][lc + 1], tile[lr][lc + 2], tile[lr][lc + 3]};
   }
 }
 
-static void csr_f32_mul_rm(const DMat& S, char op, const float* X, int ldx, int p, float* Y, int ldy, bool out_col,
+// rows of a row-major operand of p columns: ld values apart, panels of 32
+// columns `panel` values apart
+struct RowLay {
+  int ld;
+  size_t panel;
+};
+static RowLay csr_lay(int rows, int p, bool panels) {
+  if (!panels || p <= 32) return {(p + 3) & ~3, 32};
+  return {32, (size_t)rows * 32};
+}
+
+// values of such an operand, panel by panel
+static size_t csr_panel_size(int rows, int p) {
+  return (size_t)rows * (p <= 32 ? (p + 3) & ~3 : (p + 31) / 32 * 32);
+}
+
+static void csr_f32_mul_rm(const DMat& S, char op, const float* X, RowLay xl, int p, float* Y, RowLay yl, bool out_col,
                            float alpha, float beta, hipStream_t st) {
   const bool tr = op != 'N';
-  const int rows = tr ? S.n : S.m;
+  const int rows = tr ? S.n : S.m, xrows = tr ? S.m : S.n;
   if (rows == 0 || p == 0) return;
   const int* rp = tr ? S.cp.as<int>() : S.rp.as<int>();
   const int* ci = tr ? S.ri.as<int>() : S.ci.as<int>();
   const float* v = tr ? S.cv.as<float>() : S.v.as<float>();
   const int npanels = (p + 31) / 32;
-  if (csr_rows_per_thread() == 2) {
+  const int ldx = xl.ld, ldy = yl.ld;
+  // a panel's buffer offsets are 32-bit (the all-ones offset is out of range);
+  // beyond 4 GiB, two rows per thread with 64-bit addresses
+  const size_t xb = sizeof(float) * (size_t)xrows * ldx;
+  if (csr_rows_per_thread() == 2 || xb >= 0xffffff00u) {
     const dim3 grid2((unsigned)(npanels * ((rows + 63) / 64)));
     if (out_col)
-      hipLaunchKernelGGL(k_csr_rm2_f32<true>, grid2, dim3(256), 0, st, rows, p, rp, ci, v, X, ldx, Y, ldy, alpha,
-                         beta, npanels);
+      hipLaunchKernelGGL(k_csr_rm2_f32<true>, grid2, dim3(256), 0, st, rows, p, rp, ci, v, X, ldx, xl.panel, Y, ldy,
+                         yl.panel, alpha, beta, npanels);
     else
-      hipLaunchKernelGGL(k_csr_rm2_f32<false>, grid2, dim3(256), 0, st, rows, p, rp, ci, v, X, ldx, Y, ldy, alpha,
-                         beta, npanels);
+      hipLaunchKernelGGL(k_csr_rm2_f32<false>, grid2, dim3(256), 0, st, rows, p, rp, ci, v, X, ldx, xl.panel, Y, ldy,
+                         yl.panel, alpha, beta, npanels);
     FH_LAUNCH_CHECK();
     return;
   }
-  dim3 grid((unsigned)(npanels * ((rows + 31) / 32)));
+  const int nrb = (rows + 31) / 32;
+  const unsigned xbytes = (unsigned)xb;
+  const dim3 grid((unsigned)(((size_t)npanels * nrb + 7) / 8 * 8));
   const int ew = tr ? S.csr_tell_w : S.csr_ell_w;
   const char* e_ell = getenv("FH_CSR_ELL");
   if (ew > 0 && !(e_ell && e_ell[0] == '0')) {
@@ -1012,8 +1033,8 @@ static void csr_f32_mul_rm(const DMat& S, char op, const float* X, int ldx, int 
     const int* eci = tr ? S.csr_tell_ci.as<int>() : S.csr_ell_ci.as<int>();
     const float* ev = tr ? S.csr_tell_v.as<float>() : S.csr_ell_v.as<float>();
 #define FH_CSR_ELL_GO(OC, NB)                                                                                       \
-  hipLaunchKernelGGL((k_csr_rm_f32<OC, NB, true>), grid, dim3(256), 0, st, rows, p, nullptr, eci, ev, X, ldx, Y, ldy, \
-                     alpha, beta, npanels)
+  hipLaunchKernelGGL((k_csr_rm_f32<OC, NB, true>), grid, dim3(256), 0, st, rows, p, nullptr, eci, ev, X, xbytes, ldx, \
+                     xl.panel, Y, ldy, yl.panel, alpha, beta, nrb, npanels)
     switch (ew * 2 + (out_col ? 1 : 0)) {
       case 8: FH_CSR_ELL_GO(false, 4); break;
       case 9: FH_CSR_ELL_GO(true, 4); break;
@@ -1032,8 +1053,8 @@ static void csr_f32_mul_rm(const DMat& S, char op, const float* X, int ldx, int 
   const int widest = tr ? S.max_col : S.max_row;
   const int nb = (widest < 0 || widest > 12) ? 16 : std::max(4, (widest + 3) / 4 * 4);
 #define FH_CSR_GO(OC, NB)                                                                                  \
-  hipLaunchKernelGGL((k_csr_rm_f32<OC, NB>), grid, dim3(256), 0, st, rows, p, rp, ci, v, X, ldx, Y, ldy, alpha, \
-                     beta, npanels)
+  hipLaunchKernelGGL((k_csr_rm_f32<OC, NB>), grid, dim3(256), 0, st, rows, p, rp, ci, v, X, xbytes, ldx, \
+                     xl.panel, Y, ldy, yl.panel, alpha, beta, nrb, npanels)
   switch (nb * 2 + (out_col ? 1 : 0)) {
     case 8: FH_CSR_GO(false, 4); break;
     case 9: FH_CSR_GO(true, 4); break;
@@ -1048,10 +1069,10 @@ static void csr_f32_mul_rm(const DMat& S, char op, const float* X, int ldx, int 
   FH_LAUNCH_CHECK();
 }
 
-static void col2row(int rows, int p, const float* X, int ldx, float* R, int ldr, hipStream_t st) {
+static void col2row(int rows, int p, const float* X, int ldx, float* R, RowLay l, hipStream_t st) {
   if (rows == 0 || p == 0) return;
-  dim3 grid((rows + 31) / 32, (ldr + 31) / 32);
-  hipLaunchKernelGGL(k_col2row_f32, grid, dim3(256), 0, st, rows, p, X, ldx, R, ldr);
+  dim3 grid((rows + 63) / 64, (p + 31) / 32);
+  hipLaunchKernelGGL(k_col2row_f32, grid, dim3(256), 0, st, rows, p, X, ldx, R, l.ld, l.panel);
   FH_LAUNCH_CHECK();
 }
 
@@ -1107,10 +1128,10 @@ void mixed_mul_dense(const DMat& S, char op, const void* X, int ldx, int ncols, 
   }
   FH_CHECK(S.kind == K_CSR && S.dtype == FH_F32, "FP32/BF16 products: BSR or FP32 CSR factors only");
   const int in_rows = op == 'N' ? S.n : S.m;
-  const int ldr = (ncols + 3) & ~3;
-  DBuf R(sizeof(float) * std::max<size_t>((size_t)in_rows * ldr, 1));
-  col2row(in_rows, ncols, (const float*)X, ldx, R.as<float>(), ldr, st);
-  csr_f32_mul_rm(S, op, R.as<float>(), ldr, ncols, (float*)Y, ldy, true, a, b, st);
+  const RowLay l = csr_lay(in_rows, ncols, true);
+  DBuf R(sizeof(float) * std::max<size_t>(csr_panel_size(in_rows, ncols), 1));
+  col2row(in_rows, ncols, (const float*)X, ldx, R.as<float>(), l, st);
+  csr_f32_mul_rm(S, op, R.as<float>(), l, ncols, (float*)Y, RowLay{ldy, 0}, true, a, b, st);
   FH_HIP(hipStreamSynchronize(st));  // R returns to the pool
 }
 
@@ -1156,6 +1177,15 @@ size_t faust_ws_need_f32_tiled(const std::vector<DMatP>& f, char op, int p, int*
   return sizeof(float) * (size_t)maxr * (((size_t)p + 31) / 32 * 32);
 }
 
+// Bytes of each panel-by-panel intermediate of an FP32 CSR chain (X's copy
+// included; p padded to whole panels beyond one).
+size_t faust_ws_need_f32_panels(const std::vector<DMatP>& f, char op, int p, int* nbuf) {
+  int maxr = (op == 'N') ? f.back()->n : f.front()->m;
+  for (auto& x : f) maxr = std::max(maxr, op == 'N' ? x->m : x->n);
+  *nbuf = std::min(2, (int)f.size());
+  return sizeof(float) * csr_panel_size(maxr, p);
+}
+
 // Bytes of each intermediate of a BSR or FP32 CSR chain product (*nbuf of
 // them): BSR intermediates are tiled, p padded to whole 32-column groups;
 // FP32 CSR ones are row-major with ld = p rounded up to 4.
@@ -1189,7 +1219,6 @@ static int multiply_mixed_run(const std::vector<DMatP>& f, char op, const void* 
                               const ChainWs& ws, FaustTimers* tm, bool act_f32) {
   const int J = (int)f.size();
   const bool bsr = f[0]->kind == K_BSR;
-  const int ldr = bsr ? 0 : (p + 3) & ~3;
   int in_rows = (op == 'N') ? f.back()->n : f.front()->m;
   if (act_f32) {
     // FP32 BSR factors with FP32 activations: one launch per factor, FP32
@@ -1239,9 +1268,12 @@ static int multiply_mixed_run(const std::vector<DMatP>& f, char op, const void* 
     }
     return J;
   }
-  // FP32 CSR: transpose the input once, chain in row-major, last factor writes column-major
+  // FP32 CSR: transpose the input once, chain in row-major (panel by panel
+  // where the workspace has room for whole panels), last factor writes column-major
+  int pbuf = 0;
+  const bool panels = ws.cap >= faust_ws_need_f32_panels(f, op, p, &pbuf);
   if (tm) tm->begin(J, st);
-  col2row(in_rows, p, (const float*)X, in_rows, static_cast<float*>(ws.p[0]), ldr, st);
+  col2row(in_rows, p, (const float*)X, in_rows, static_cast<float*>(ws.p[0]), csr_lay(in_rows, p, panels), st);
   if (tm) tm->end(J, st);
   const float* in = static_cast<const float*>(ws.p[0]);
   for (int i = 0; i < J; ++i) {
@@ -1252,7 +1284,8 @@ static int multiply_mixed_run(const std::vector<DMatP>& f, char op, const void* 
     float* out = last ? (float*)Y : static_cast<float*>(ws.p[(i + 1) & 1]);
     const size_t slot = (op == 'N') ? (size_t)(J - 1 - i) : (size_t)i;
     if (tm) tm->begin(slot, st);
-    csr_f32_mul_rm(S, op, in, ldr, p, out, last ? out_rows : ldr, last, 1.0f, 0.0f, st);
+    csr_f32_mul_rm(S, op, in, csr_lay(in_rows, p, panels), p, out,
+                   last ? RowLay{out_rows, 0} : csr_lay(out_rows, p, panels), last, 1.0f, 0.0f, st);
     if (tm) tm->end(slot, st);
     in = out;
     in_rows = out_rows;

@@ -659,24 +659,30 @@ void csr_chain_pf_run_f64(const std::vector<ChainCsrOp>& ops, int in_rows, int w
 // ------------------------------------------------------ row-major chain
 // FP64 CSR chains on blocks of columns, one launch per factor with row-major
 // intermediates: X is transposed once (k_col2row_f64), every factor gathers
-// whole row segments, and the last one writes Y column-major through LDS.  A
+// whole row segments, and the last one writes Y column-major through LDS.
+// Intermediates are kept panel by panel (32 columns, rows of 32 values one
+// after the other): with whole rows of a power of two of columns, the one
+// segment of each row that a panel's XCD gathers would lie on a few of its L2
+// channels.  A
 // workgroup computes 16 rows x a panel of 32 columns: the 16 lanes of a DPP
 // row share one row of S (two columns each), lane s loads the row's entry s,
 // and row_newbcast hands entry q to the 16 lanes, so an entry's gather is one
 // 256-byte read.  Column-major intermediates gather 8 bytes per lane from as
 // many cache lines, which is what bounds k_csr_spmm_f64 once X no longer
-// sits in L1.  Gathers go through a buffer resource whose range check drops
-// the lanes past the row's end or past column p: no branch, no traffic.
+// sits in L1.  Gathers go through a buffer resource whose range check returns
+// zeros, without traffic, for the lanes past column p and for the entries past
+// the row's end, whose weight is -0: adding -0 x 0 leaves the chain as it is.
 // Workgroups are dealt to the 8 XCDs in turn, so each XCD takes a contiguous
 // run of the panel-major (panel, row block) list: with up to 8 panels an
 // XCD's L2 holds the one or two panels it gathers from.
 // Each output entry is the fma chain of k_csr_spmm_f64 (entries in row
 // order, from 0), so the bits are the same.
 // Measured, 6007 x 5003 and 5003^2 factors of 7 entries per row, 250 columns:
-// 9.7 us per factor (88 MB of gathers out of the L2s, 9 TB/s; 22 MB of
+// 8.7 us per factor (88 MB of gathers out of the L2s, 10 TB/s; 22 MB of
 // activations) and 6.4 us for the transpose, against 29 us per factor
-// column-major (52 us transposed, rows of up to 24 entries).  Two rows per
-// lane, with both rows' pointers and entries loaded together, gave 10.1 us.
+// column-major (52 us transposed, rows of up to 24 entries).  In whole rows of
+// 250 values 9.8 us; two rows per lane, with both rows' pointers and entries
+// loaded together, 10.1 us against those.
 constexpr int RM_COLS = 32, RM_ROWS = 16;
 
 template <int Q>
@@ -687,7 +693,7 @@ __device__ __forceinline__ unsigned rm_bcast(unsigned x) {
 // entries Q .. Q + 7 of the 16 held by the lanes: gathers, then the fma chain
 template <int Q>
 __device__ __forceinline__ void rm_batch8(const __amdgpu_buffer_rsrc_t rx, unsigned off, unsigned wlo, unsigned whi,
-                                          unsigned coff, int n, double& a0, double& a1) {
+                                          unsigned coff, double& a0, double& a1) {
   pfc_d2 x[8];
   double w[8];
 #define FH_RM_GET(u)                                                                                             \
@@ -699,9 +705,8 @@ __device__ __forceinline__ void rm_batch8(const __amdgpu_buffer_rsrc_t rx, unsig
   __builtin_amdgcn_sched_barrier(0);  // all gathers in flight before the first fma
 #pragma unroll
   for (int u = 0; u < 8; ++u) {
-    const double f0 = fma(w[u], x[u].x, a0), f1 = fma(w[u], x[u].y, a1);
-    a0 = Q + u < n ? f0 : a0;
-    a1 = Q + u < n ? f1 : a1;
+    a0 = fma(w[u], x[u].x, a0);
+    a1 = fma(w[u], x[u].y, a1);
   }
 }
 
@@ -717,8 +722,9 @@ __global__ __launch_bounds__(256) void k_csr_rm_f64(int rows, int p, const int* 
   if (w0 >= total) return;  // the whole workgroup
   const int panel = w0 / nrb, rblk = w0 - panel * nrb;
   const int c0 = panel * RM_COLS + 2 * s;
-  const unsigned coff = c0 < p ? (unsigned)c0 * 8u : 0xffffffffu;
-  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)X, 0, (int)xbytes, 0x00020000);
+  const unsigned coff = c0 < p ? 16u * s : 0xffffffffu;
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(X + (size_t)panel * (xbytes / sizeof(double))), 0, (int)xbytes, 0x00020000);
   const int r = rblk * RM_ROWS + (t >> 4), rr = min(r, rows - 1);
   const int e0 = rp[rr], len = r < rows ? rp[rr + 1] - e0 : 0;
   double a0 = 0.0, a1 = 0.0;
@@ -726,13 +732,15 @@ __global__ __launch_bounds__(256) void k_csr_rm_f64(int rows, int p, const int* 
     const int n = len - base;  // entries left in this lane's row
     const int e = s < n ? e0 + base + s : 0;
     const int k = ci[e];
-    const unsigned long long wb = __builtin_bit_cast(unsigned long long, v[e]);
+    const double ve = v[e];
+    const unsigned long long wb = __builtin_bit_cast(unsigned long long, s < n ? ve : -0.0);
     const unsigned off = s < n ? (unsigned)k * (unsigned)(ldr * 8) : 0xffffffffu;
-    rm_batch8<0>(rx, off, (unsigned)wb, (unsigned)(wb >> 32), coff, n, a0, a1);
-    if (__any(n > 8)) rm_batch8<8>(rx, off, (unsigned)wb, (unsigned)(wb >> 32), coff, n, a0, a1);
+    rm_batch8<0>(rx, off, (unsigned)wb, (unsigned)(wb >> 32), coff, a0, a1);
+    if (__any(n > 8)) rm_batch8<8>(rx, off, (unsigned)wb, (unsigned)(wb >> 32), coff, a0, a1);
   }
   if (!OUT_COL) {
-    if (r < rows && c0 < p) *reinterpret_cast<pfc_d2*>(Y + (size_t)r * ldr + c0) = pfc_d2{a0, a1};
+    if (r < rows && c0 < p)
+      *reinterpret_cast<pfc_d2*>(Y + ((size_t)panel * rows + r) * ldr + 2 * s) = pfc_d2{a0, a1};
     return;
   }
   tile[t >> 4][2 * s] = a0;
@@ -747,7 +755,7 @@ __global__ __launch_bounds__(256) void k_csr_rm_f64(int rows, int p, const int* 
   }
 }
 
-// column-major (rows x p, ld ldx) -> row-major (rows x ldr), columns p .. ldr - 1 zero
+// column-major (rows x p, ld ldx) -> panels of rows of ldr values, columns past p zero
 __global__ __launch_bounds__(256) void k_col2row_f64(int rows, int p, const double* __restrict__ X, int ldx,
                                                      double* __restrict__ R, int ldr) {
   __shared__ double tile[32][33];
@@ -762,12 +770,15 @@ __global__ __launch_bounds__(256) void k_col2row_f64(int rows, int p, const doub
 #pragma unroll
   for (int q = 0; q < 2; ++q) {
     const int lr = (t >> 4) + 16 * q, lc = 2 * (t & 15);
-    if (r0 + lr < rows && c0 + lc < ldr)
-      *reinterpret_cast<pfc_d2*>(R + (size_t)(r0 + lr) * ldr + c0 + lc) = pfc_d2{tile[lr][lc], tile[lr][lc + 1]};
+    if (r0 + lr < rows && lc < ldr)
+      *reinterpret_cast<pfc_d2*>(R + ((size_t)blockIdx.y * rows + r0 + lr) * ldr + lc) =
+          pfc_d2{tile[lr][lc], tile[lr][lc + 1]};
   }
 }
 
-int csr_rm_ld(int p) { return (p + 1) & ~1; }
+int csr_rm_ld(int p) { return p < RM_COLS ? (p + 1) & ~1 : RM_COLS; }
+
+size_t csr_rm_size(int rows, int p) { return (size_t)rows * csr_rm_ld(p) * ((p + RM_COLS - 1) / RM_COLS); }
 
 bool csr_rm_fits(const std::vector<ChainCsrOp>& ops, int in_rows, int p) {
   if (ops.empty() || p < RM_MIN_COLS || in_rows < 1) return false;
@@ -776,14 +787,14 @@ bool csr_rm_fits(const std::vector<ChainCsrOp>& ops, int in_rows, int p) {
     if (o.rows < 1) return false;
     r = std::max(r, (size_t)o.rows);
   }
-  // buffer offsets are 32-bit and the all-ones offset is out of range; launches are below 2^31 workgroups
-  return r * csr_rm_ld(p) * sizeof(double) < 0xffffff00u &&
+  // a panel's buffer offsets are 32-bit and the all-ones offset is out of range; launches are below 2^31 workgroups
+  return r * RM_COLS * sizeof(double) < 0xffffff00u &&
          (r / RM_ROWS + 1) * ((size_t)p / RM_COLS + 1) < (size_t)1 << 28;
 }
 
 void csr_rm_from_col(int rows, int p, const double* X, double* R, hipStream_t st) {
   const int ldr = csr_rm_ld(p);
-  const dim3 grid((unsigned)((rows + 31) / 32), (unsigned)((ldr + 31) / 32));
+  const dim3 grid((unsigned)((rows + 31) / 32), (unsigned)((p + RM_COLS - 1) / RM_COLS));
   hipLaunchKernelGGL(k_col2row_f64, grid, dim3(256), 0, st, rows, p, X, rows, R, ldr);
   FH_LAUNCH_CHECK();
 }

@@ -73,3 +73,29 @@ def test_row_major_chain_noalloc_and_graph(gpu, monkeypatch):
         torch.cuda.synchronize()
         assert torch.equal(Y, F.matmul_device(X))
         assert np.array_equal(Y.cpu().numpy().T, oracle.chain_multiply(facs, np.asfortranarray(X.cpu().numpy().T), "N"))
+
+
+@pytest.mark.parametrize("p", [1, 4, 31, 32, 33, 63, 256, 257])
+@pytest.mark.parametrize("ell", ["1", "0"])
+def test_fp32_panels(gpu, monkeypatch, p, ell):
+    # FP32 CSR chains panel by panel: rows of 0 to 40 entries (CSR form) or up to 12 (ELL form); the same
+    # bits from the two-rows-per-thread kernel, and close to FP64
+    monkeypatch.setenv("FH_CSR_ELL", ell)
+    rng = np.random.default_rng(p)
+    dims = (333, 260, 129)
+    facs = [_ragged(dims[i], dims[i + 1], rng) if ell == "0" else faust_amd.rand_csr(dims[i], dims[i + 1], 12, rng)
+            for i in range(2)]
+    F = faust_amd.Faust(facs, dtype=np.float32)
+    for G, op, n in ((F, "N", dims[-1]), (F.T, "T", dims[0])):
+        X = np.asfortranarray(rng.standard_normal((n, p)).astype(np.float32))
+        monkeypatch.delenv("FH_CSR_RPT", raising=False)
+        Y = G @ X
+        monkeypatch.setenv("FH_CSR_RPT", "2")
+        assert np.array_equal(Y, G @ X)
+        f32 = [f.astype(np.float32).astype(np.float64) for f in facs]
+        want = oracle.chain_multiply(f32, X.astype(np.float64), op)
+        # two factors of at most 40 terms, each rounding below 2^-24 of the term sizes
+        bound = np.abs(X.astype(np.float64))
+        for f in (reversed(f32) if op == "N" else f32):
+            bound = np.abs(f if op == "N" else f.T) @ bound
+        assert np.all(np.abs(Y - want) <= 2.0 ** -24 * 2 * 41 * bound)
