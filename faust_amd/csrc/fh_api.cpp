@@ -74,20 +74,22 @@ DMatP make_csr_from_host(int dtype, int m, int n, int nnz, const int32_t* rp, co
   M->max_col = 0;
   for (int j = 0; j < n; ++j) M->max_col = std::max(M->max_col, cp[j + 1] - cp[j]);
   if (dtype == FH_F32 || dtype == FH_F64) {
-    // ELL views for the gather kernels (rows of S, rows of S^T): the widest
-    // row rounded up to the kernel's batch, at most 16 slots for FP32 (in 4s)
-    // and 32 for FP64 (in 8s)
-    const int quant = dtype == FH_F32 ? 4 : 8, wmax = dtype == FH_F32 ? 16 : 32;
+    // ELL views for the gather kernels (rows of S, rows of S^T).  FP32: the
+    // widest row rounded up to 4, at most 16 slots, a row's slots together (its
+    // lanes load them).  FP64: rounded up to 2, 4 or a multiple of 8, at most
+    // 32, pair of slots by pair (a lane per row, so a wave's loads are contiguous)
+    const bool by_pair = dtype == FH_F64;
     auto ell = [&](int nr, const int* ptr, const int* idx, const char* val, int widest, int& w, DBuf& dc, DBuf& dv) {
       w = 0;
-      if (nr == 0 || widest > wmax) return;
-      w = std::max(quant, (widest + quant - 1) / quant * quant);
+      if (nr == 0 || widest > (by_pair ? 32 : 16)) return;
+      w = by_pair ? (widest <= 2 ? 2 : widest <= 4 ? 4 : (widest + 7) / 8 * 8) : std::max(4, (widest + 3) / 4 * 4);
       std::vector<int> hc((size_t)nr * w, -1);
       std::vector<char> hv((size_t)nr * w * esz, 0);
       for (int r = 0; r < nr; ++r)
         for (int e = ptr[r]; e < ptr[r + 1]; ++e) {
-          hc[(size_t)r * w + (e - ptr[r])] = idx[e];
-          std::memcpy(hv.data() + ((size_t)r * w + (e - ptr[r])) * esz, val + (size_t)e * esz, esz);
+          const size_t q = e - ptr[r], at = by_pair ? (q / 2 * nr + r) * 2 + q % 2 : (size_t)r * w + q;
+          hc[at] = idx[e];
+          std::memcpy(hv.data() + at * esz, val + (size_t)e * esz, esz);
         }
       dc.alloc(sizeof(int) * hc.size());
       dv.alloc(hv.size());
@@ -142,7 +144,9 @@ static bool chain_csr_ops(const std::vector<DMatP>& f, char op, std::vector<Chai
     const int ew = tr ? S.csr_tell_w : S.csr_ell_w;
     ops.push_back({tr ? S.cp.as<int>() : S.rp.as<int>(), tr ? S.ri.as<int>() : S.ci.as<int>(),
                    tr ? S.cv.as<double>() : S.v.as<double>(), rows, (int)S.nnz,
-                   ell_on && ew > 0 && ew % 8 == 0 && ew <= 32 ? 1 : 0});
+                   ell_on && ew > 0 && ew <= 32 ? ew : 0,
+                   tr ? S.csr_tell_ci.as<int>() : S.csr_ell_ci.as<int>(),
+                   tr ? S.csr_tell_v.as<double>() : S.csr_ell_v.as<double>()});
     r = rows;
   }
   return true;
@@ -335,7 +339,9 @@ void faust_multiply_f64(const std::vector<DMatP>& f, char op, const double* X, i
     const size_t rm_need = faust_ws_need_rm_f64(f, op, p, &rm_nbuf);
     const bool rm_fits = rm_need > 0 && ws.cap >= rm_need && t1 && (rm_nbuf < 2 || t2);
     const bool one_launch_off = getenv("FH_CHAIN_FUSED") || (getenv("FH_CHAIN_PF") && getenv("FH_CHAIN_PF")[0] == '0');
-    const bool rm_auto = rm_fits && mul_mode() == FH_MUL_AUTO && !one_launch_off;
+    // (chains that fit the one-launch form keep to that and to one launch per factor)
+    const bool rm_auto =
+        rm_fits && mul_mode() == FH_MUL_AUTO && !one_launch_off && !csr_chain_pf_fits(ops, in_rows0, p);
     ChainForm def{0, 0, 0};
     const int pwc = csr_chain_pf_plan_f64(ops, in_rows0, p);
     const int swc = pwc > 0 ? 0 : csr_chain_plan_f64(ops, in_rows0, p);

@@ -137,10 +137,11 @@ struct DMat {
   // loading the slot first; tebdat likewise for the transpose
   DBuf ebdat, tebdat;
   // CSR uploaded from the host (FP32 / FP64): ELL view of the rows (and of
-  // the transpose's rows) for the gather kernels, csr_ell_w slots per row
-  // (the widest row rounded up to 4 for FP32, at most 16; to 8 for FP64, at
-  // most 32; 0: none), slot q of row r at r * w + q, unused slots with
-  // column -1 and value 0
+  // the transpose's rows) for the gather kernels, csr_ell_w slots per row (0:
+  // none), unused slots with column -1 and value 0.  FP32: the widest row
+  // rounded up to 4, at most 16, slot q of row r at r * w + q; FP64: rounded up
+  // to 2, 4 or a multiple of 8, at most 32, slots 2q and 2q + 1 of row r at
+  // (q * rows + r) * 2
   int csr_ell_w = 0, csr_tell_w = 0;
   DBuf csr_ell_ci, csr_ell_v, csr_tell_ci, csr_tell_v;
   bool is_identity = false;
@@ -180,7 +181,9 @@ struct ChainCsrOp {
   const double* v;
   int rows;
   int nnz;
-  int ell;
+  int ell;            // slots per row of the ELL view, 0: none
+  const int* eci;     // ELL view: columns (-1: unused slot) and values
+  const double* ev;
 };
 int csr_chain_plan_f64(const std::vector<ChainCsrOp>& ops, int in_rows, int p);
 void csr_chain_run_f64(const std::vector<ChainCsrOp>& ops, int in_rows, int wc, const double* X, int ldx, int p,

@@ -579,13 +579,10 @@ __global__ void k_bfly_leaf_csr(const double* v, int n, int logs, const int* col
   ri[2 * (size_t)r + 1] = rb + s;
   cv_col[2 * (size_t)r] = w0;
   cv_col[2 * (size_t)r + 1] = w1;
-  for (int q = 0; q < 8; ++q) {
-    const size_t e = (size_t)r * 8 + q;
-    ell_ci[e] = q == 0 ? c0 : q == 1 ? c1 : -1;
-    ell_v[e] = q == 0 ? v0 : q == 1 ? v1 : 0.0;
-    tell_ci[e] = q == 0 ? rb : q == 1 ? rb + s : -1;
-    tell_v[e] = q == 0 ? w0 : q == 1 ? w1 : 0.0;
-  }
+  reinterpret_cast<int2*>(ell_ci)[r] = {c0, c1};  // two slots: one pair per row
+  reinterpret_cast<double2*>(ell_v)[r] = {v0, v1};
+  reinterpret_cast<int2*>(tell_ci)[r] = {rb, rb + s};
+  reinterpret_cast<double2*>(tell_v)[r] = {w0, w1};
   if (r == 0) {
     rp[n] = 2 * n;
     cp[n] = 2 * n;
@@ -595,7 +592,7 @@ __global__ void k_bfly_leaf_csr(const double* v, int n, int logs, const int* col
 void bfly_leaf_csr(const double* v, int n, int logs, const int* colmap, const int* colinv, DMat& M, hipStream_t st) {
   FH_CHECK(n >= 4 && (n & (n - 1)) == 0 && logs >= 0 && (2 << logs) <= n, "butterfly: bad leaf node");
   FH_CHECK((colmap == nullptr) == (colinv == nullptr), "butterfly: leaf relabelling needs both maps");
-  const size_t nz = 2 * (size_t)n, ne = 8 * (size_t)n;
+  const size_t nz = 2 * (size_t)n;
   M.kind = K_CSR;
   M.dtype = FH_F64;
   M.m = M.n = n;
@@ -608,11 +605,11 @@ void bfly_leaf_csr(const double* v, int n, int logs, const int* colmap, const in
   M.cv.alloc(sizeof(double) * nz);
   M.has_csc = true;
   M.max_row = M.max_col = 2;
-  M.csr_ell_w = M.csr_tell_w = 8;  // the FP64 gather kernels' slot quantum
-  M.csr_ell_ci.alloc(sizeof(int) * ne);
-  M.csr_ell_v.alloc(sizeof(double) * ne);
-  M.csr_tell_ci.alloc(sizeof(int) * ne);
-  M.csr_tell_v.alloc(sizeof(double) * ne);
+  M.csr_ell_w = M.csr_tell_w = 2;
+  M.csr_ell_ci.alloc(sizeof(int) * nz);
+  M.csr_ell_v.alloc(sizeof(double) * nz);
+  M.csr_tell_ci.alloc(sizeof(int) * nz);
+  M.csr_tell_v.alloc(sizeof(double) * nz);
   hipLaunchKernelGGL(k_bfly_leaf_csr, dim3((n + 255) / 256), dim3(256), 0, st, v, n, logs, colmap, colinv,
                      M.rp.as<int>(), M.ci.as<int>(), M.v.as<double>(), M.cp.as<int>(), M.ri.as<int>(),
                      M.cv.as<double>(), M.csr_ell_ci.as<int>(), M.csr_ell_v.as<double>(), M.csr_tell_ci.as<int>(),

@@ -8,7 +8,10 @@
 // inside each column, so the k order is the same as the oracle's.  CSR
 // factors uploaded from the host with rows of at most 32 entries (and their
 // transposes) are also kept as ELL views, read without the row pointer; the
-// terms and their order are unchanged.
+// terms and their order are unchanged.  Bound by the latency of index -> gather
+// -> chain and, until the slots lay pair by pair, by the loads of the slots:
+// 1024 x 1024 with up to 22 entries per row, 64 columns 5.0 -> 4.2 us; rows of
+// two entries (8192 x 8, in two slots instead of eight) 6.3 -> 4.8 us.
 #include <algorithm>
 #include <cstdlib>
 
@@ -18,7 +21,10 @@ namespace fh {
 
 // Y(i,j) = alpha * sum_p v[p] * X(ci[p], j) + beta * Y(i,j)
 // transX: X(k,j) is read as X[j + k*ldx] (op(X) = X^T).
-// EW > 0: ci / v are the matrix's ELL view with EW slots per row.
+// EW > 0: ci / v are the matrix's ELL view with EW slots per row, pair of
+// slots by pair (a wave's 64 rows load contiguous bytes; with all of a row's
+// slots together each of its loads touched 32 lines that the next ones came
+// back to).
 template <bool TRANSX, int EW = 0>
 __global__ __launch_bounds__(256) void k_csr_spmm_f64(int nrows, int ncols, const int* __restrict__ rp,
                                                        const int* __restrict__ ci, const double* __restrict__ v,
@@ -28,29 +34,34 @@ __global__ __launch_bounds__(256) void k_csr_spmm_f64(int nrows, int ncols, cons
   const int j = blockIdx.y * 4 + (threadIdx.x >> 6);
   if (i >= nrows || j >= ncols) return;
   double acc = 0.0;
-  if (EW > 0) {
-    // ELL view (EW slots per row, column -1 in unused slots; rp unused): the
-    // same batches of 8 terms in the same order, without the row pointer
-    const int* ec = ci + (size_t)i * EW;
-    const double* ev = v + (size_t)i * EW;
+  if constexpr (EW > 0) {
+    // ELL view (column -1 in unused slots; rp unused): batches of up to 8
+    // terms, without the row pointer
+    constexpr int NB = EW < 8 ? EW : 8;
+    const int2* ec = reinterpret_cast<const int2*>(ci) + i;
+    const double2* ev = reinterpret_cast<const double2*>(v) + i;
     const double* xj = X + (size_t)j * ldx;
 #pragma unroll
-    for (int base = 0; base < EW; base += 8) {
-      int cc[8];
-      double ww[8], xx[8];
+    for (int base = 0; base < EW; base += NB) {
+      int cc[NB];
+      double ww[NB], xx[NB];
 #pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        cc[q] = ec[base + q];
-        ww[q] = ev[base + q];
+      for (int q = 0; q < NB; q += 2) {
+        const int2 c2 = ec[(size_t)((base + q) / 2) * nrows];
+        const double2 w2 = ev[(size_t)((base + q) / 2) * nrows];
+        cc[q] = c2.x;
+        cc[q + 1] = c2.y;
+        ww[q] = w2.x;
+        ww[q + 1] = w2.y;
       }
 #pragma unroll
-      for (int q = 0; q < 8; ++q) {
+      for (int q = 0; q < NB; ++q) {
         const int c = max(cc[q], 0);
         xx[q] = TRANSX ? X[(size_t)c * ldx + j] : xj[c];
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int q = 0; q < 8; ++q) {
+      for (int q = 0; q < NB; ++q) {
         const double f = fma(ww[q], xx[q], acc);
         acc = cc[q] >= 0 ? f : acc;
       }
@@ -102,13 +113,17 @@ void csr_spmm_f64_x(const DMat& S, char op, const double* X, int ldx, int transX
   dim3 grid((rows + 63) / 64, (ncols + 3) / 4);
   const int ew = (S.dtype == FH_F64) ? (tr ? S.csr_tell_w : S.csr_ell_w) : 0;
   const char* e_ell = getenv("FH_CSR_ELL");
-  if (ew > 0 && ew % 8 == 0 && ew <= 32 && !(e_ell && e_ell[0] == '0')) {
-    // ELL view: every row's slots at i * ew, no row pointer in the chain
+  if (ew > 0 && ew <= 32 && !(e_ell && e_ell[0] == '0')) {
+    // ELL view: no row pointer in the chain
     const int* eci = tr ? S.csr_tell_ci.as<int>() : S.csr_ell_ci.as<int>();
     const double* ev = tr ? S.csr_tell_v.as<double>() : S.csr_ell_v.as<double>();
 #define FH_ELL64(T, W) \
   hipLaunchKernelGGL((k_csr_spmm_f64<T, W>), grid, dim3(256), 0, st, rows, ncols, nullptr, eci, ev, X, ldx, Y, ldy, alpha, beta)
     switch (ew * 2 + (transX ? 1 : 0)) {
+      case 4: FH_ELL64(false, 2); break;
+      case 5: FH_ELL64(true, 2); break;
+      case 8: FH_ELL64(false, 4); break;
+      case 9: FH_ELL64(true, 4); break;
       case 16: FH_ELL64(false, 8); break;
       case 17: FH_ELL64(true, 8); break;
       case 32: FH_ELL64(false, 16); break;
@@ -398,17 +413,24 @@ void csr_chain_run_f64(const std::vector<ChainCsrOp>& ops, int in_rows, int wc, 
 // FP64 CSR chains whose factors and input have at most 1024 rows, in one
 // launch of 1024 threads per workgroup: thread t owns row t of every factor,
 // a workgroup WC columns of X.  Every factor's row pointers are copied into
-// LDS at the start; a thread loads the first PF entries (values, columns) of
+// LDS at the start (chains whose rows all fit PF slots of their ELL views read
+// those instead, coalesced and without row pointers); a thread loads the first PF entries (values, columns) of
 // its row of factor f + 2 while it computes factor f (two register sets,
 // loads through buffer resources that return zeros past the factor's
 // entries), and the barriers between factors order only the LDS activations,
 // so those loads stay in flight across them.  Rows longer than PF read the
 // rest of their entries in batches of 8.  Each output entry is the fma chain of
 // k_csr_spmm_f64 (k ascending from 0; the last factor applies alpha / beta),
-// so the bits are those of the factor-by-factor path.
+// so the bits are those of the factor-by-factor path.  Bound by the LDS gathers
+// of 1024 rows from one workgroup (8 per entry and wave, random banks) and the
+// factor-to-factor barriers.  1024 x 1024, 5 factors of 8 entries per row: one
+// column 12.3 -> 9.9 us, 64 columns 12.6 -> 10.2 (ELL slots, and the entries of
+// a row in batches whose LDS reads are in flight together, against one entry
+// after the other behind row pointers).
 constexpr int PFC_THREADS = 1024;
 constexpr int PFC_RP_INTS = 16 * 1024;  // LDS ints for the row pointers of the whole chain
 
+typedef unsigned int pfc_u2 __attribute__((ext_vector_type(2)));
 typedef unsigned int pfc_u4 __attribute__((ext_vector_type(4)));
 typedef double pfc_d2 __attribute__((ext_vector_type(2)));
 typedef const __attribute__((address_space(1))) double* pfc_gd;
@@ -428,10 +450,30 @@ __device__ __forceinline__ void pfc_lds_barrier() {
 }
 
 // loads the first PF entries of row r of factor S (rows past the factor get
-// n = 0 and read entries that are not used)
-template <int PF>
+// n = 0 and read entries that are not used).  ELL: the row's slots (S.ell of
+// them, at most PF), without a row pointer; unused ones get column 0 and
+// n counts the row's entries, which come first
+template <int PF, bool ELL>
 __device__ __forceinline__ void pfc_fetch(const ChainCsrOp& S, const int* rpl, int rpo, int r, PfcRow<PF>& f) {
   const int rr = min(r, S.rows - 1);
+  if (ELL) {
+    const int w = S.ell, n = S.rows * w;  // slots past w are out of range: zeros, no traffic
+    f.p = 0;
+    f.n = r < S.rows ? w : 0;
+    const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc((void*)S.ev, 0, n * 8, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc((void*)S.eci, 0, n * 4, 0x00020000);
+#pragma unroll
+    for (int k = 0; k < PF; k += 2) {
+      const pfc_u2 c = __builtin_amdgcn_raw_buffer_load_b64(rc, ((k / 2) * S.rows + rr) * 8, 0, 0);
+      const pfc_d2 v =
+          __builtin_bit_cast(pfc_d2, __builtin_amdgcn_raw_buffer_load_b128(rv, ((k / 2) * S.rows + rr) * 16, 0, 0));
+      f.c[k] = (int)c.x;
+      f.c[k + 1] = (int)c.y;
+      f.v[k] = v.x;
+      f.v[k + 1] = v.y;
+    }
+    return;
+  }
   const int p0 = rpl[rpo + rr], p1 = rpl[rpo + rr + 1];
   f.p = p0;
   f.n = r < S.rows ? p1 - p0 : 0;
@@ -461,17 +503,31 @@ __device__ __forceinline__ void pfc_settle(const PfcRow<PF>& f) {
 }
 
 // one factor: row t of S from cur (R x WC in LDS) into acc, entries from f
-template <int PF, int WC>
+template <int PF, int WC, bool ELL>
 __device__ __forceinline__ void pfc_row(const ChainCsrOp& S, const PfcRow<PF>& f, const double* cur, int R,
                                         double (&acc)[WC]) {
 #pragma unroll
   for (int c = 0; c < WC; ++c) acc[c] = 0.0;
+  // eight entries at a time without branches between them, so that their LDS
+  // reads are in flight together: past the row's end the columns are those of
+  // a later row (or 0), valid ones, and the terms are not kept
 #pragma unroll
-  for (int k = 0; k < PF; ++k)
-    if (k < f.n) {
+  for (int k0 = 0; k0 < PF; k0 += 8)
+    if (k0 == 0 || __any(k0 < f.n)) {
+      double x[8][WC];
 #pragma unroll
-      for (int c = 0; c < WC; ++c) acc[c] = fma(f.v[k], cur[c * R + f.c[k]], acc[c]);
+      for (int k = 0; k < 8; ++k)
+#pragma unroll
+        for (int c = 0; c < WC; ++c) x[k][c] = cur[c * R + (ELL ? max(f.c[k0 + k], 0) : f.c[k0 + k])];
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+#pragma unroll
+        for (int c = 0; c < WC; ++c) {
+          const double a = fma(f.v[k0 + k], x[k][c], acc[c]);
+          acc[c] = k0 + k < f.n && (!ELL || f.c[k0 + k] >= 0) ? a : acc[c];
+        }
     }
+  if (ELL) return;  // at most PF slots
   if (f.n > PF) {
     // the rest of the row in batches of 8: loads issued together (indices
     // clamped inside the row), then the fma chain in k order
@@ -497,7 +553,7 @@ __device__ __forceinline__ void pfc_row(const ChainCsrOp& S, const PfcRow<PF>& f
   }
 }
 
-template <int PF, int WC>
+template <int PF, int WC, bool ELL>
 __device__ __forceinline__ void pfc_factor(const ChainArgsF64& a, const int* rpl, const int* rpo, int f,
                                            const double* cur, double* nxt, PfcRow<PF>& fr, int c0, int p,
                                            double* __restrict__ Y, int ldy, double alpha, double beta) {
@@ -506,10 +562,10 @@ __device__ __forceinline__ void pfc_factor(const ChainArgsF64& a, const int* rpl
   f = __builtin_amdgcn_readfirstlane(f);
   const ChainCsrOp S = a.f[f];
   double acc[WC];
-  if (t < S.rows) pfc_row<PF, WC>(S, fr, cur, a.R, acc);
+  if (t < S.rows) pfc_row<PF, WC, ELL>(S, fr, cur, a.R, acc);
   // entries of the factor after next into the registers just consumed
   const int f2 = min(f + 2, a.J - 1);
-  pfc_fetch<PF>(a.f[f2], rpl, rpo[f2], t, fr);
+  pfc_fetch<PF, ELL>(a.f[f2], rpl, ELL ? 0 : rpo[f2], t, fr);
   if (t < S.rows) {
     if (f < a.J - 1) {
 #pragma unroll
@@ -527,7 +583,7 @@ __device__ __forceinline__ void pfc_factor(const ChainArgsF64& a, const int* rpl
   pfc_lds_barrier();
 }
 
-template <int PF, int WC>
+template <int PF, int WC, bool ELL>
 __global__ __launch_bounds__(PFC_THREADS) void k_chain_pf_f64(ChainArgsF64 a, const double* __restrict__ X, int ldx,
                                                               int p, double* __restrict__ Y, int ldy, double alpha,
                                                               double beta) {
@@ -539,29 +595,53 @@ __global__ __launch_bounds__(PFC_THREADS) void k_chain_pf_f64(ChainArgsF64 a, co
   double* cur = lds;
   double* nxt = lds + (size_t)R * WC;
   int* rpl = reinterpret_cast<int*>(lds + (size_t)2 * R * WC);
-  int off = 0;
-  for (int f = 0; f < a.J; ++f) {
-    const ChainCsrOp S = a.f[f];
-    if (t == 0) rpo[f] = off;
-    for (int i = t; i <= S.rows; i += PFC_THREADS) rpl[off + i] = S.rp[i];
-    off += S.rows + 1;
+  PfcRow<PF> fa, fb;  // entries of the factors applied 1st, 3rd, ... and 2nd, 4th, ...
+  if (ELL) {
+    pfc_fetch<PF, ELL>(a.f[0], rpl, 0, t, fa);
+    pfc_fetch<PF, ELL>(a.f[min(1, a.J - 1)], rpl, 0, t, fb);
+  } else {
+    // four factors' row pointers in flight at a time (rows <= PFC_THREADS)
+    int off = 0;
+    for (int f0 = 0; f0 < a.J; f0 += 4) {
+      int q[4], q1[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const ChainCsrOp S = a.f[min(f0 + u, a.J - 1)];
+        const int tt = min(t, S.rows - 1);
+        q[u] = S.rp[tt];
+        q1[u] = S.rp[tt + 1];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (f0 + u < a.J) {
+          const int rows = a.f[f0 + u].rows;
+          if (t < rows) rpl[off + t] = q[u];
+          if (t == rows - 1) rpl[off + rows] = q1[u];
+          if (t == 0) rpo[f0 + u] = off;
+          off += rows + 1;
+        }
+    }
   }
   const int n0 = a.in_rows;
   for (int i = t; i < n0 * WC; i += PFC_THREADS) {
     const int c = i / n0, r = i - c * n0;
     cur[(size_t)c * R + r] = (c0 + c < p) ? X[(size_t)(c0 + c) * ldx + r] : 0.0;
   }
-  __syncthreads();
-  PfcRow<PF> fa, fb;  // entries of the factors applied 1st, 3rd, ... and 2nd, 4th, ...
-  pfc_fetch<PF>(a.f[0], rpl, rpo[0], t, fa);
-  pfc_fetch<PF>(a.f[min(1, a.J - 1)], rpl, rpo[min(1, a.J - 1)], t, fb);
+  if (ELL)
+    pfc_lds_barrier();
+  else
+    __syncthreads();
+  if (!ELL) {
+    pfc_fetch<PF, ELL>(a.f[0], rpl, rpo[0], t, fa);
+    pfc_fetch<PF, ELL>(a.f[min(1, a.J - 1)], rpl, rpo[min(1, a.J - 1)], t, fb);
+  }
   for (int f = 0; f < a.J; f += 2) {
-    pfc_factor<PF, WC>(a, rpl, rpo, f, cur, nxt, fa, c0, p, Y, ldy, alpha, beta);
+    pfc_factor<PF, WC, ELL>(a, rpl, rpo, f, cur, nxt, fa, c0, p, Y, ldy, alpha, beta);
     double* sw = cur;
     cur = nxt;
     nxt = sw;
     if (f + 1 == a.J) break;
-    pfc_factor<PF, WC>(a, rpl, rpo, f + 1, cur, nxt, fb, c0, p, Y, ldy, alpha, beta);
+    pfc_factor<PF, WC, ELL>(a, rpl, rpo, f + 1, cur, nxt, fb, c0, p, Y, ldy, alpha, beta);
     sw = cur;
     cur = nxt;
     nxt = sw;
@@ -616,17 +696,17 @@ int csr_chain_fit_wc(const std::vector<ChainCsrOp>& ops, int in_rows, int p) {
   return (wc == 0 || (p + wc - 1) / wc > 1024) ? 0 : wc;
 }
 
-template <int PF, int WC>
+template <int PF, int WC, bool ELL>
 static void pfc_go(const ChainArgsF64& a, size_t lds, const double* X, int ldx, int p, double* Y, int ldy,
                    double alpha, double beta, hipStream_t st) {
   static bool attr = false;
   if (!attr) {
-    FH_HIP(hipFuncSetAttribute((const void*)k_chain_pf_f64<PF, WC>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    FH_HIP(hipFuncSetAttribute((const void*)k_chain_pf_f64<PF, WC, ELL>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)(sizeof(double) * 2 * PFC_THREADS * 4 + sizeof(int) * PFC_RP_INTS)));
     attr = true;
   }
   const dim3 grid((unsigned)((p + WC - 1) / WC));
-  hipLaunchKernelGGL((k_chain_pf_f64<PF, WC>), grid, dim3(PFC_THREADS), lds, st, a, X, ldx, p, Y, ldy, alpha, beta);
+  hipLaunchKernelGGL((k_chain_pf_f64<PF, WC, ELL>), grid, dim3(PFC_THREADS), lds, st, a, X, ldx, p, Y, ldy, alpha, beta);
 }
 
 void csr_chain_pf_run_f64(const std::vector<ChainCsrOp>& ops, int in_rows, int wc, int pf, const double* X, int ldx,
@@ -645,8 +725,18 @@ void csr_chain_pf_run_f64(const std::vector<ChainCsrOp>& ops, int in_rows, int w
     rp_ints += (size_t)ops[i].rows + 1;
   }
   FH_CHECK(a.R <= PFC_THREADS && rp_ints <= (size_t)PFC_RP_INTS, "prefetched chain: shape out of range");
-  const size_t lds = sizeof(double) * 2 * (size_t)a.R * wc + sizeof(int) * rp_ints;
-#define FH_PFC(PF, WC) pfc_go<PF, WC>(a, lds, X, ldx, p, Y, ldy, alpha, beta, st)
+  int widest = 0;
+  bool all_ell = true;
+  for (const ChainCsrOp& o : ops) {
+    all_ell = all_ell && o.ell > 0;
+    widest = std::max(widest, o.ell);
+  }
+  // rows of at most pf slots everywhere: no row pointers at all
+  const bool ell = all_ell && widest <= pf;
+  const size_t lds = sizeof(double) * 2 * (size_t)a.R * wc + (ell ? 0 : sizeof(int) * rp_ints);
+#define FH_PFC(PF, WC)                                                             \
+  (ell ? pfc_go<PF, WC, true>(a, lds, X, ldx, p, Y, ldy, alpha, beta, st)          \
+       : pfc_go<PF, WC, false>(a, lds, X, ldx, p, Y, ldy, alpha, beta, st))
   if (pf == 8) {
     if (wc == 1) FH_PFC(8, 1); else if (wc == 2) FH_PFC(8, 2); else FH_PFC(8, 4);
   } else {
