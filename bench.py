@@ -12,7 +12,7 @@ per step, from the library's per-factor event timers, is subtracted).  `cpu_base
 oracle (CPU FP64 restatement of the reference) timed on this host on a
 bounded sample of the same workload.  `palm` times, on 512 targets, the
 tuned batched PALM4MSA (FP32 + FP64 frozen-support refinement, HIP graphs,
-autotuned tiles) until every target has reached, FP64-verified, the error
+matrix-core tiles) until every target has reached, FP64-verified, the error
 its FP64 PALM4MSA reaches in 220 iterations, against the plain FP64 GPU form
 and the batched FP64 form.  `butterfly` times the butterfly factorization
 (fact.butterfly, host matrix in, Faust out) at orders 1024 / 4096 / 16384 on
@@ -174,7 +174,7 @@ def palm_batched_vs_plain(cpu=True, plain_all=False):
     PALM4MSA reaches in 220 iterations, taken from the batched FP64 run (the
     plain FP64 form's own error is checked against it on every target the
     plain form runs).  Tuned form: FP32 iterations on the batched grouped-GEMM
-    engine (one HIP graph per iteration, autotuned tiles; at most 400), then
+    engine (one HIP graph per iteration, matrix-core tiles; at most 400), then
     FP64 frozen-support sweeps, with an FP64 error check every 10 iterations;
     its time runs until every target has reached its error (set-up
     included).  The FP32 iterations end 0.15 % above the FP64 error at 220

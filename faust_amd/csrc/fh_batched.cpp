@@ -4,14 +4,11 @@
 // updates with packed partial products, as palm4msa2 with the
 // ParamsPalm4MSA defaults: faust_palm4msa2020.hpp:47-300), captures it into
 // a HIP graph on a private stream, and replays the graph for every
-// iteration.  Tile sizes of the grouped GEMM are picked per target size by a
-// timing autotuner at set-up.  The mixed-precision scheme runs the main
-// iterations in FP32, then refinement sweeps in FP64 with every factor
+// iteration.  The mixed-precision scheme runs the main iterations in FP32, then refinement sweeps in FP64 with every factor
 // projected on its frozen FP32 support (prox supp), and verifies the final
 // relative error in FP64.
 #include <algorithm>
 #include <chrono>
-#include <map>
 #include <numeric>
 #include <type_traits>
 
@@ -46,7 +43,7 @@ struct Batch {
   std::vector<Stage> stages;
   DBuf tiles32, tiles64, tilesM;
   int nt32 = 0, nt64 = 0, ntM = 0;
-  std::vector<int> tile_of;  // per target: 32 or 64 (VALU), BGEMM_MFMA (FP32 MFMA, 64 x 64)
+  std::vector<int> tile_of;  // per target: 32 or 64 (VALU), BGEMM_MFMA (64 x 64)
   int prox_mode = 0;
   int maxit = 100;
   double thr = 1e-6;
@@ -107,17 +104,39 @@ static void batch_alloc(Batch<T>& B, const BatchSpec& sp, bool masks) {
   FH_HIP(hipMemcpy(B.powv.p, hv.data(), sizeof(double) * hv.size(), hipMemcpyHostToDevice));
 }
 
+// GEMM tiles.  The kernels give XCD x the x-th eighth of a list in order, so
+// the lists are laid out for that: rows of tiles (which share op(A)'s rows),
+// the largest targets first, each to the XCD with the least work so far; the
+// shorter eighths are filled up with tiles of no job.  (In the targets' order
+// an XCD that got the large ones worked nearly twice as long as the average.)
 template <class T>
 static void build_tiles(Batch<T>& B) {
-  std::vector<int3> t32, t64, tm;
-  for (int b = 0; b < B.sp.nt; ++b) {
-    const int code = B.tile_of[b], n = B.sp.n[b];
+  std::vector<int> ord(B.sp.nt);
+  std::iota(ord.begin(), ord.end(), 0);
+  std::stable_sort(ord.begin(), ord.end(), [&](int a, int b) { return B.sp.n[a] > B.sp.n[b]; });
+  auto deal = [&](int code) {
     const int tile = code == 32 ? 32 : 64;
-    const int nt = (n + tile - 1) / tile;
-    std::vector<int3>& l = code == 32 ? t32 : (code == 64 ? t64 : tm);
-    for (int i = 0; i < nt; ++i)
-      for (int j = 0; j < nt; ++j) l.push_back(make_int3(b, i, j));
-  }
+    std::vector<int3> x[8];
+    int64_t work[8] = {};
+    for (int b : ord) {
+      if (B.tile_of[b] != code) continue;
+      const int n = B.sp.n[b], nt = (n + tile - 1) / tile;
+      for (int i = 0; i < nt; ++i) {
+        const int to = (int)(std::min_element(work, work + 8) - work);
+        for (int j = 0; j < nt; ++j) x[to].push_back(make_int3(b, i, j));
+        work[to] += (int64_t)nt * n;
+      }
+    }
+    size_t most = 0;
+    for (const auto& l : x) most = std::max(most, l.size());
+    std::vector<int3> all;
+    for (auto& l : x) {
+      l.resize(most, make_int3(-1, 0, 0));
+      all.insert(all.end(), l.begin(), l.end());
+    }
+    return all;
+  };
+  const std::vector<int3> t32 = deal(32), t64 = deal(64), tm = deal(BGEMM_MFMA);
   auto up = [](DBuf& d, int& cnt, const std::vector<int3>& v) {
     cnt = (int)v.size();
     d.alloc(sizeof(int3) * std::max<size_t>(v.size(), 1));
@@ -158,8 +177,10 @@ static void add_gemm(Batch<T>& B, std::function<BGemmJob<T>(int)> mk) {
                             side, side == 0 ? g.transA : g.transB, g.alpha_mode, g.beta_mode, g.target};
         // transposed dense operands do not occur next to a factor in the schedule
         FH_CHECK((side == 0 ? g.transB : g.transA) == 0, "batched PALM: transposed dense operand of a sparse product");
-        // about 8 K output entries per workgroup (the staged factor serves all of them)
-        const int n = B.sp.n[b], nc = std::max(1, std::min(n, 8192 / n));
+        // about 2 K output entries per workgroup: 48 targets of 64 .. 512 make 1400
+        // workgroups (of 8 K entries they made 350, 1.4 waves per SIMD waiting
+        // for their gathers: 105 us a product against 38)
+        const int n = B.sp.n[b], nc = std::max(1, std::min(n, 2048 / n));
         for (int j0 = 0; j0 < n; j0 += nc) tl.push_back(make_int3(b, j0, std::min(nc, n - j0)));
       }
       typename Batch<T>::Stage s;
@@ -427,66 +448,15 @@ static void run_iteration(Batch<T>& B, hipStream_t st) {
   for (auto& s : B.stages) run_stage(B, s, st);
 }
 
-// Autotuner: for every distinct target size, time one full-size GEMM stage
-// with 32- and 64-wide VALU tiles and (FP32) the 64 x 64 MFMA tile, and keep
-// the fastest.
+// GEMM tiles: the 64 x 64 one on the matrix cores for every target;
+// FH_BGEMM_TILE=32 / 64 asks for the VALU tiles (65: the matrix cores).
 template <class T>
-static void autotune(Batch<T>& B, hipStream_t st) {
-  std::map<int, std::vector<int>> by_n;
-  for (int b = 0; b < B.sp.nt; ++b) by_n[B.sp.n[b]].push_back(b);
-  B.tile_of.assign(B.sp.nt, 64);
-  // FH_BGEMM_TILE=32 / 64 / 65 (MFMA, FP32 only) fixes the choice
-  if (const char* e = getenv("FH_BGEMM_TILE")) {
-    const int code = atoi(e);
-    if (code == 32 || code == 64 || (code == BGEMM_MFMA && std::is_same<T, float>::value)) {
-      B.tile_of.assign(B.sp.nt, code);
-      return;
-    }
-  }
-  // a GEMM stage over the members of one size class
-  const typename Batch<T>::Stage* g = nullptr;
-  for (auto& s : B.stages)
-    if (s.kind == 0) { g = &s; break; }
-  if (!g) return;
-  hipEvent_t e0, e1;
-  FH_HIP(hipEventCreate(&e0));
-  FH_HIP(hipEventCreate(&e1));
-  BScal sc{B.lam.template as<double>(), B.nR.template as<double>(), B.nL.template as<double>()};
-  for (auto& kv : by_n) {
-    float best = 1e30f;
-    int best_tile = 64;
-    std::vector<int> cands{32, 64};
-    if (std::is_same<T, float>::value) cands.push_back(BGEMM_MFMA);
-    for (int code : cands) {
-      const int tile = code == 32 ? 32 : 64;
-      std::vector<int3> tl;
-      for (int b : kv.second) {
-        const int nt = (kv.first + tile - 1) / tile;
-        for (int i = 0; i < nt; ++i)
-          for (int j = 0; j < nt; ++j) tl.push_back(make_int3(b, i, j));
-      }
-      DBuf dt(sizeof(int3) * tl.size());
-      FH_HIP(hipMemcpy(dt.p, tl.data(), sizeof(int3) * tl.size(), hipMemcpyHostToDevice));
-      // the fastest of 3 timed launches, so that one slow launch does not decide the tile
-      float ms = 1e30f;
-      for (int rep = 0; rep < 3; ++rep) {
-        FH_HIP(hipEventRecord(e0, st));
-        launch_bgemm<T>(g->jobs.template as<BGemmJob<T>>(), dt.as<int3>(), (int)tl.size(), code, sc, st);
-        FH_HIP(hipEventRecord(e1, st));
-        FH_HIP(hipEventSynchronize(e1));
-        float t = 0.f;
-        FH_HIP(hipEventElapsedTime(&t, e0, e1));
-        ms = std::min(ms, t);
-      }
-      if (ms < best) {
-        best = ms;
-        best_tile = code;
-      }
-    }
-    for (int b : kv.second) B.tile_of[b] = best_tile;
-  }
-  FH_HIP(hipEventDestroy(e0));
-  FH_HIP(hipEventDestroy(e1));
+static void pick_tiles(Batch<T>& B) {
+  int code = BGEMM_MFMA;
+  if (const char* e = getenv("FH_BGEMM_TILE"))
+    if (const int c = atoi(e); c == 32 || c == 64) code = c;
+  B.tile_of.assign(B.sp.nt, code);
+  build_tiles(B);
 }
 
 template <class T>
@@ -533,7 +503,7 @@ struct Verifier {
     BatchSpec vs = s;
     vs.nf = 1;
     batch_alloc(V, vs, false);
-    V.tile_of.assign(s.nt, 64);
+    V.tile_of.assign(s.nt, BGEMM_MFMA);
     build_tiles(V);
     // V slots (nf = 1): 0 A, 1 running product, 2 factor cast to FP64, 3 GEMM output
     for (int b = 0; b < s.nt; ++b) {
@@ -585,7 +555,7 @@ struct Verifier {
     launch_bcast(cast_jobs[sp.nf - 1].as<BCastJob>(), sp.nt, f32, st);
     for (int f = sp.nf - 2; f >= 0; --f) {
       launch_bcast(cast_jobs[f].as<BCastJob>(), sp.nt, f32, st);
-      launch_bgemm<double>(gemm_jobs[0].as<BGemmJob<double>>(), V.tiles64.as<int3>(), V.nt64, 64, sc, st);
+      launch_bgemm<double>(gemm_jobs[0].as<BGemmJob<double>>(), V.tilesM.as<int3>(), V.ntM, BGEMM_MFMA, sc, st);
       launch_bcast(copy_jobs.as<BCastJob>(), sp.nt, false, st);
     }
     launch_brelerr<double>(lam_jobs.as<BLamJob<double>>(), sp.nt, B.lam.template as<double>(), out.as<double>(), st);
@@ -660,31 +630,29 @@ void load_batch(Batch<T>& B, const std::vector<const double*>& Ad, const double*
                 const double* lambda_init, hipStream_t st) {
   const int nf = B.sp.nf;
   std::vector<double> lam(B.sp.nt, 1.0);
+  // the targets (already FP64 on the device in Ad) and palm4msa2's default
+  // left-to-right factors, S_0 = 0 (as the arena is) and the others identity,
+  // by one launch; given factors from the host
+  std::vector<BLoadJob> h;
   for (int b = 0; b < B.sp.nt; ++b) {
     const int n = B.sp.n[b];
     const int64_t len = (int64_t)n * n;
-    // A (already FP64 on the device in Ad)
-    if constexpr (std::is_same<T, float>::value) {
-      std::vector<double> h(len);
-      FH_HIP(hipMemcpy(h.data(), Ad[b], sizeof(double) * len, hipMemcpyDeviceToHost));
-      std::vector<float> hf(h.begin(), h.end());
-      FH_HIP(hipMemcpy(B.mat(b, B.sA()), hf.data(), sizeof(float) * len, hipMemcpyHostToDevice));
-    } else {
-      FH_HIP(hipMemcpy(B.mat(b, B.sA()), Ad[b], sizeof(double) * len, hipMemcpyDeviceToDevice));
-    }
+    h.push_back({B.mat(b, B.sA()), Ad[b], len, n});
     for (int f = 0; f < nf; ++f) {
-      std::vector<T> h(len, T(0));
       const double* src = init ? init[(size_t)b * nf + f] : nullptr;
       if (src) {
-        for (int64_t i = 0; i < len; ++i) h[i] = (T)src[i];
+        std::vector<T> hs(src, src + len);
+        FH_HIP(hipMemcpy(B.mat(b, B.sS(f)), hs.data(), sizeof(T) * len, hipMemcpyHostToDevice));
       } else if (f > 0) {
-        // palm4msa2 default init, left-to-right: S_0 = 0, the others identity
-        for (int i = 0; i < n; ++i) h[(int64_t)i * n + i] = T(1);
+        h.push_back({B.mat(b, B.sS(f)), nullptr, len, n});
       }
-      FH_HIP(hipMemcpy(B.mat(b, B.sS(f)), h.data(), sizeof(T) * len, hipMemcpyHostToDevice));
     }
     if (lambda_init) lam[b] = lambda_init[b];
   }
+  DBuf jobs(sizeof(BLoadJob) * h.size());
+  FH_HIP(hipMemcpy(jobs.p, h.data(), sizeof(BLoadJob) * h.size(), hipMemcpyHostToDevice));
+  launch_bload<T>(jobs.as<BLoadJob>(), (int)h.size(), st);
+  FH_HIP(hipStreamSynchronize(st));  // jobs is freed on return
   FH_HIP(hipMemcpy(B.lam.p, lam.data(), sizeof(double) * B.sp.nt, hipMemcpyHostToDevice));
 }
 
@@ -744,14 +712,9 @@ extern "C" int fh_palm4msa_batched(int ntargets, int nfacts, const int* n, const
       B.sparse = sparse;
       if (sparse) sparse_alloc(B, kv);
     }
-    B.tile_of.assign(ntargets, 64);
-    build_tiles(B);
+    pick_tiles(B);
     build_schedule(B, kv);
     if (B.sparse) sparse_build_all(B, st);
-    if (p->autotune) {
-      autotune(B, st);
-      build_tiles(B);
-    }
     r->ms[0] = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     Verifier ver;
     Progress pr;
@@ -779,10 +742,7 @@ extern "C" int fh_palm4msa_batched(int ntargets, int nfacts, const int* n, const
       }
       FH_HIP(hipMemcpyAsync(D.lam.p, B.lam.p, sizeof(double) * ntargets, hipMemcpyDeviceToDevice, st));
       FH_HIP(hipMemcpyAsync(D.powv.p, B.powv.p, B.powv.bytes, hipMemcpyDeviceToDevice, st));
-      D.tile_of = B.tile_of;  // the FP32 MFMA tile has no FP64 form: its targets take 64-wide VALU tiles
-      for (int& t : D.tile_of)
-        if (t == BGEMM_MFMA) t = 64;
-      build_tiles(D);
+      pick_tiles(D);
       build_schedule(D, {});
       FH_HIP(hipStreamSynchronize(st));
       const double setup_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t1).count();
@@ -832,13 +792,8 @@ extern "C" int fh_palm4msa_batched(int ntargets, int nfacts, const int* n, const
         for (int f = 0; f < nfacts; ++f)
           FH_HIP(hipMemcpy(B.mat(b, B.sMASK(f)), supp[(size_t)b * nfacts + f], sizeof(double) * n[b] * n[b],
                            hipMemcpyHostToDevice));
-    B.tile_of.assign(ntargets, 64);
-    build_tiles(B);
+    pick_tiles(B);
     build_schedule(B, kv);
-    if (p->autotune) {
-      autotune(B, st);
-      build_tiles(B);
-    }
     r->ms[0] = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     Verifier ver;
     Progress pr;

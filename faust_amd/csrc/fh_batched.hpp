@@ -6,7 +6,7 @@
 namespace fh {
 
 constexpr int BATCH_NMAX = 2048;  // largest target edge (power-iteration vectors live in LDS)
-constexpr int BGEMM_MFMA = 65;    // tile code of the FP32 MFMA grouped GEMM (64 x 64 tiles)
+constexpr int BGEMM_MFMA = 65;    // tile code of the grouped GEMM on the matrix cores (64 x 64 tiles)
 
 // C_out = alpha_b * op(A) op(B) + beta * C_in on n x n column-major blocks;
 // alpha mode 0 -> 1, 1 -> lambda_b, 2 -> -lambda_b / c_b with
@@ -114,6 +114,16 @@ struct BLamJob {
   int64_t len;
   int target;
 };
+
+// dst (the batch's type) = src (FP64), or the n x n identity for a null src
+struct BLoadJob {
+  void* dst;
+  const double* src;
+  int64_t len;
+  int n;
+};
+template <class T>
+void launch_bload(const BLoadJob* jobs, int njobs, hipStream_t st);
 
 template <class T>
 void launch_bgemm(const BGemmJob<T>* jobs, const int3* tiles, int ntiles, int tile, const BScal& sc, hipStream_t st);

@@ -59,6 +59,7 @@ __global__ __launch_bounds__(256) void k_bgemm(const BGemmJob<T>* __restrict__ j
   const int tix = xcd_tile(per);
   if (tix >= ntiles) return;
   const int3 tl = tiles[tix];
+  if (tl.x < 0) return;
   const BGemmJob<T> J = jobs[tl.x];
   const int t = threadIdx.x, tx = t & 15, ty = t >> 4;
   const int i0 = tl.y * TILE, j0 = tl.z * TILE;
@@ -115,85 +116,122 @@ __global__ __launch_bounds__(256) void k_bgemm(const BGemmJob<T>* __restrict__ j
   }
 }
 
-// FP32 on the matrix cores: v_mfma_f32_32x32x2_f32, workgroup tile 64 x 64
-// (four waves of 32 x 32), K staged through LDS 32 at a time.  Operand
-// lanes: A lane l holds op(A)[row l % 32][k + l / 32], B lane l holds
-// op(B)[k + l / 32][col l % 32]; the accumulator holds rows
-// 8*(r/4) + 4*(l/32) + r%4 of column l % 32 (r = 0..15).
+// On the matrix cores, workgroup tile 64 x 64 (four waves of 32 x 32), K in
+// slabs of KS through double-buffered LDS: the next slab's values are loaded
+// into registers while the current one multiplies, indices clamped instead of
+// guarded (rows and columns past the matrix are not stored; k past its end is
+// zeroed on the way into LDS).  FP32: v_mfma_f32_32x32x2_f32, A lane l holds
+// op(A)[row l % 32][k + l / 32], B lane l op(B)[k + l / 32][col l % 32]; the
+// accumulator holds rows 8*(r/4) + 4*(l/32) + r%4 of column l % 32 (r = 0..15).
+// FP64: v_mfma_f64_16x16x4_f64, whose four terms are four fmas in ascending k,
+// so an entry is the same fma chain as on the vector units; op(B)'s values go
+// in as the first operand, which leaves register r of lane l with row l % 16,
+// column l / 16 + 4 r.  The same bits as the VALU tiles, and faster at every
+// size of 32 .. 512, so no target's tile is chosen by timing any more (the
+// timing took 16 ms of a call).  Bound by the slabs' loads: 48 targets of
+// 64 .. 512, 3 GFLOP: FP32 165 us in two launches (VALU and matrix cores) -> 99, FP64 330 -> 150.
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef double f64x4 __attribute__((ext_vector_type(4)));
 
-__global__ __launch_bounds__(256) void k_bgemm_mfma_f32(const BGemmJob<float>* __restrict__ jobs,
-                                                        const int3* __restrict__ tiles, BScal sc, int ntiles,
-                                                        int per) {
-  constexpr int TILE = 64, KS = 32;
-  __shared__ float As[KS][TILE + 4];
-  __shared__ float Bs[KS][TILE + 4];
+template <class T>
+__global__ __launch_bounds__(256) void k_bgemm_mfma(const BGemmJob<T>* __restrict__ jobs,
+                                                    const int3* __restrict__ tiles, BScal sc, int ntiles, int per) {
+  constexpr bool F32 = sizeof(T) == 4;
+  constexpr int TILE = 64, KS = F32 ? 32 : 16, NE = TILE * KS / 256;
+  __shared__ T As[2][KS][TILE + 1];
+  __shared__ T Bs[2][KS][TILE + 1];
   const int tix = xcd_tile(per);
   if (tix >= ntiles) return;
   const int3 tl = tiles[tix];
-  const BGemmJob<float> J = jobs[tl.x];
+  if (tl.x < 0) return;
+  const BGemmJob<T> J = jobs[tl.x];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int wr = wave & 1, wc = wave >> 1;
+  const int wr = (wave & 1) * 32, wc = (wave >> 1) * 32;
   const int i0 = tl.y * TILE, j0 = tl.z * TILE;
-  f32x16 acc = {};
-  const bool inside = i0 + TILE <= J.m && j0 + TILE <= J.n;
+  typedef const __attribute__((address_space(1))) T* GT;
+  const GT A = (GT)J.A, B = (GT)J.B;
+  // element q of this thread: (row ii + ir q, k ka + kr q) of the slab
+  const int iiA = J.transA ? t / KS : t % TILE, kaA = J.transA ? t % KS : t / TILE;
+  const int irA = J.transA ? 256 / KS : 0, krA = J.transA ? 0 : 256 / TILE;
+  const int iiB = J.transB ? t % TILE : t / KS, kaB = J.transB ? t / TILE : t % KS;
+  const int irB = J.transB ? 0 : 256 / KS, krB = J.transB ? 256 / TILE : 0;
+  T av[NE], bv[NE];
+  auto load = [&](int k0) {
+#pragma unroll
+    for (int q = 0; q < NE; ++q) {
+      const int gi = min(i0 + iiA + irA * q, J.m - 1), ka = min(k0 + kaA + krA * q, J.k - 1);
+      av[q] = A[J.transA ? (size_t)gi * J.k + ka : (size_t)ka * J.m + gi];
+      const int gj = min(j0 + iiB + irB * q, J.n - 1), kb = min(k0 + kaB + krB * q, J.k - 1);
+      bv[q] = B[J.transB ? (size_t)kb * J.n + gj : (size_t)gj * J.k + kb];
+    }
+  };
+  auto store = [&](int buf, int k0) {
+#pragma unroll
+    for (int q = 0; q < NE; ++q) {
+      const int ka = kaA + krA * q, kb = kaB + krB * q;
+      As[buf][ka][iiA + irA * q] = k0 + ka < J.k ? av[q] : T(0);
+      Bs[buf][kb][iiB + irB * q] = k0 + kb < J.k ? bv[q] : T(0);
+    }
+  };
+  f32x16 acc32 = {};
+  f64x4 acc64[2][2] = {};
+  load(0);
+  store(0, 0);
+  __syncthreads();
+  int buf = 0;
   for (int k0 = 0; k0 < J.k; k0 += KS) {
-    if (inside && k0 + KS <= J.k) {
-      // whole tile inside: 8 + 8 unconditional loads per thread, all in flight
-      float av[TILE * KS / 256], bv[TILE * KS / 256];
+    const bool more = k0 + KS < J.k;
+    if (more) load(k0 + KS);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (F32) {
 #pragma unroll
-      for (int q = 0; q < TILE * KS / 256; ++q) {
-        const int e = t + 256 * q;
-        const int ii = J.transA ? e / KS : e % TILE, ka = J.transA ? e % KS : e / TILE;
-        av[q] = J.transA ? J.A[(size_t)(i0 + ii) * J.k + k0 + ka] : J.A[(size_t)(k0 + ka) * J.m + i0 + ii];
-        const int jj = J.transB ? e % TILE : e / KS, kb = J.transB ? e / TILE : e % KS;
-        bv[q] = J.transB ? J.B[(size_t)(k0 + kb) * J.n + j0 + jj] : J.B[(size_t)(j0 + jj) * J.k + k0 + kb];
-      }
-#pragma unroll
-      for (int q = 0; q < TILE * KS / 256; ++q) {
-        const int e = t + 256 * q;
-        const int ii = J.transA ? e / KS : e % TILE, ka = J.transA ? e % KS : e / TILE;
-        As[ka][ii] = av[q];
-        const int jj = J.transB ? e % TILE : e / KS, kb = J.transB ? e / TILE : e % KS;
-        Bs[kb][jj] = bv[q];
+      for (int kk = 0; kk < KS; kk += 2) {
+        const float a = As[buf][kk + (lane >> 5)][wr + (lane & 31)];
+        const float b = Bs[buf][kk + (lane >> 5)][wc + (lane & 31)];
+        acc32 = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc32, 0, 0, 0);
       }
     } else {
-      for (int e = t; e < TILE * KS; e += 256) {
-        int ii, kk;
-        if (!J.transA) { ii = e % TILE; kk = e / TILE; } else { kk = e % KS; ii = e / KS; }
-        const int gi = i0 + ii, gk = k0 + kk;
-        As[kk][ii] = (gi < J.m && gk < J.k) ? (J.transA ? J.A[(size_t)gi * J.k + gk] : J.A[(size_t)gk * J.m + gi])
-                                            : 0.0f;
-      }
-      for (int e = t; e < TILE * KS; e += 256) {
-        int jj, kk;
-        if (J.transB) { jj = e % TILE; kk = e / TILE; } else { kk = e % KS; jj = e / KS; }
-        const int gj = j0 + jj, gk = k0 + kk;
-        Bs[kk][jj] = (gj < J.n && gk < J.k) ? (J.transB ? J.B[(size_t)gk * J.n + gj] : J.B[(size_t)gj * J.k + gk])
-                                            : 0.0f;
-      }
-    }
-    __syncthreads();
 #pragma unroll
-    for (int kk = 0; kk < KS; kk += 2) {
-      const float a = As[kk + (lane >> 5)][wr * 32 + (lane & 31)];
-      const float b = Bs[kk + (lane >> 5)][wc * 32 + (lane & 31)];
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc, 0, 0, 0);
+      for (int kk = 0; kk < KS; kk += 4) {
+        double a[2], b[2];
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+          a[x] = As[buf][kk + (lane >> 4)][wr + 16 * x + (lane & 15)];
+          b[x] = Bs[buf][kk + (lane >> 4)][wc + 16 * x + (lane & 15)];
+        }
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+          for (int y = 0; y < 2; ++y)
+            acc64[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[y], a[x], acc64[x][y], 0, 0, 0);
+      }
     }
+    __builtin_amdgcn_sched_barrier(0);
+    if (more) store(buf ^ 1, k0 + KS);  // the other buffer was last read before the previous barrier
     __syncthreads();
+    buf ^= 1;
   }
-  const float alpha = job_alpha<float>(J.alpha_mode, J.target, sc);
-  const float beta = J.beta_mode == 0 ? 0.0f : (J.beta_mode == 1 ? -1.0f : 1.0f);
-  const int gj = j0 + wc * 32 + (lane & 31);
-  if (gj >= J.n) return;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int gi = i0 + wr * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-    if (gi >= J.m) continue;
+  const T alpha = job_alpha<T>(J.alpha_mode, J.target, sc);
+  const T beta = J.beta_mode == 0 ? T(0) : (J.beta_mode == 1 ? T(-1) : T(1));
+  auto out = [&](int gi, int gj, T acc) {
+    if (gi >= J.m || gj >= J.n) return;
     const size_t o = (size_t)gj * J.m + gi;
-    float v = alpha * acc[r];
-    if (J.beta_mode) v = fmaf(beta, J.Cin[o], v);
+    T v = alpha * acc;
+    if (J.beta_mode) v = fma(beta, J.Cin[o], v);
     J.Cout[o] = v;
+  };
+  if constexpr (F32) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      out(i0 + wr + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3), j0 + wc + (lane & 31), acc32[r]);
+  } else {
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int y = 0; y < 2; ++y)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          out(i0 + wr + 16 * x + (lane & 15), j0 + wc + 16 * y + (lane >> 4) + 4 * r, acc64[x][y][r]);
   }
 }
 
@@ -203,19 +241,6 @@ __global__ __launch_bounds__(256) void k_bgemm_mfma_f32(const BGemmJob<float>* _
 // sqrt(lambda) goes to out[target].  warm: start from (and store) the last
 // normalised vector of this job slot.
 
-__device__ double block_sum_d(double v, double* red) {
-  const int t = threadIdx.x;
-  red[t] = v;
-  __syncthreads();
-  for (int s = blockDim.x / 2; s >= 1; s >>= 1) {
-    if (t < s) red[t] = red[t] + red[t + s];
-    __syncthreads();
-  }
-  const double r = red[0];
-  __syncthreads();
-  return r;
-}
-
 __device__ __forceinline__ double wave_sum_d(double v) {
   for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
@@ -223,10 +248,17 @@ __device__ __forceinline__ double wave_sum_d(double v) {
 
 // The step size stays FP64 whatever the factor precision: vectors and sums
 // are double, matrix entries are widened on load.
+//
+// 1024 threads; bound by the 2 n^2 entries a round reads from L2 through one
+// CU and, before, by chains of four waves: a wave summed one column after the
+// other behind six dependent shuffles, and 256 threads walked the rows.  Four
+// columns per wave at a time and a thread per row (two rows past 1024).  The
+// sums over a whole vector keep the order of 256 threads: thread t < 256 takes
+// entries t, t + 256, ...  48 targets of 64 .. 512 in FP64: 840 -> 170 us.
 template <class T>
-__global__ __launch_bounds__(256) void k_bpower(const BPowJob<T>* __restrict__ jobs, int maxit, double thr,
-                                                int warm) {
-  __shared__ double x[BATCH_NMAX], y[BATCH_NMAX];
+__global__ __launch_bounds__(1024) void k_bpower(const BPowJob<T>* __restrict__ jobs, int maxit, double thr,
+                                                 int warm) {
+  __shared__ double x[BATCH_NMAX], y[BATCH_NMAX], z[BATCH_NMAX];
   __shared__ double red[256];
   const BPowJob<T> J = jobs[blockIdx.x];
   const int n = J.n, t = threadIdx.x, lane = t & 63, wave = t >> 6;
@@ -234,7 +266,27 @@ __global__ __launch_bounds__(256) void k_bpower(const BPowJob<T>* __restrict__ j
     if (t == 0) J.out[J.target] = 1.0;
     return;
   }
-  for (int i = t; i < n; i += 256) x[i] = J.vec[i];
+  typedef const __attribute__((address_space(1))) T* GT;
+  const GT P = (GT)J.P;
+  // sum over threads t < 256 by halves, to every thread
+  auto block_sum = [&](double v) {
+    if (t < 256) red[t] = v;
+    __syncthreads();
+    for (int s = 128; s >= 64; s >>= 1) {
+      if (t < s) red[t] = red[t] + red[t + s];
+      __syncthreads();
+    }
+    if (t < 64) {
+      double r = red[t];
+      for (int s = 32; s >= 1; s >>= 1) r = r + __shfl_down(r, s, 64);  // lane 0: the halves in the same order
+      if (t == 0) red[0] = r;
+    }
+    __syncthreads();
+    const double r = red[0];
+    __syncthreads();
+    return r;
+  };
+  for (int i = t; i < n; i += 1024) x[i] = J.vec[i];
   __syncthreads();
   double lambda_old = 1.0, lambda = 0.0;
   int it = 0;
@@ -243,68 +295,91 @@ __global__ __launch_bounds__(256) void k_bpower(const BPowJob<T>* __restrict__ j
     ++it;
     lambda_old = lambda;
     double ss = 0.0;
-    for (int i = t; i < n; i += 256) ss = fma(x[i], x[i], ss);
-    const double nrm = sqrt(block_sum_d(ss, red));
+    if (t < 256)
+      for (int i = t; i < n; i += 256) ss = fma(x[i], x[i], ss);
+    const double nrm = sqrt(block_sum(ss));
     if (nrm == 0.0) {
       zero = true;
       break;
     }
     const double inv = 1.0 / nrm;
-    for (int i = t; i < n; i += 256) x[i] = x[i] * inv;
+    for (int i = t; i < n; i += 1024) x[i] = x[i] * inv;
     __syncthreads();
-    // y = P^T x: one wave per column of P (contiguous), lanes split k
-    for (int i = wave; i < n; i += 4) {
-      const T* col = J.P + (size_t)i * n;
-      double a = 0.0;
-      for (int k = lane; k < n; k += 64) a = fma((double)col[k], x[k], a);
-      a = wave_sum_d(a);
-      if (lane == 0) y[i] = a;
+    // y = P^T x: four columns of P (contiguous) per wave at a time, lanes split k
+    for (int i0 = wave * 4; i0 < n; i0 += 64) {
+      double a[4] = {0.0, 0.0, 0.0, 0.0};
+      for (int k0 = lane; k0 < n; k0 += 128) {
+        T c[2][4];
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) c[u][q] = P[(size_t)min(i0 + q, n - 1) * n + min(k0 + 64 * u, n - 1)];
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+          if (k0 + 64 * u < n) {
+            const double xk = x[k0 + 64 * u];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) a[q] = fma((double)c[u][q], xk, a[q]);
+          }
+      }
+#pragma unroll
+      for (int o = 32; o >= 1; o >>= 1)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) a[q] += __shfl_xor(a[q], o, 64);
+      if (lane == 0)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (i0 + q < n) y[i0 + q] = a[q];
     }
     __syncthreads();
     // z = P y (threads over rows: coalesced), lambda = <x, z>
-    double dot = 0.0;
-    double z[BATCH_NMAX / 256];
     int nz = 0;
-#pragma unroll
-    for (int q = 0; q < BATCH_NMAX / 256; ++q) {
-      const int i = t + 256 * q;
+    for (int i = t; i < n; i += 1024) {
       double a = 0.0;
-      if (i < n) {
-        for (int k = 0; k < n; ++k) a = fma((double)J.P[(size_t)k * n + i], y[k], a);
-        dot = fma(x[i], a, dot);
-        nz |= (a != 0.0);
+      for (int k0 = 0; k0 < n; k0 += 16) {
+        T c[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) c[u] = P[(size_t)min(k0 + u, n - 1) * n + i];
+#pragma unroll
+        for (int u = 0; u < 16; ++u)
+          if (k0 + u < n) a = fma((double)c[u], y[k0 + u], a);
       }
-      z[q] = a;
+      nz |= (a != 0.0);
+      z[i] = a;
     }
-    lambda = block_sum_d(dot, red);
+    __syncthreads();
+    double dot = 0.0;
+    if (t < 256)
+      for (int i = t; i < n; i += 256) dot = fma(x[i], z[i], dot);
+    lambda = block_sum(dot);
     if (!__syncthreads_or(nz)) {
       lambda = 0.0;
       zero = true;
       break;
     }
-#pragma unroll
-    for (int q = 0; q < BATCH_NMAX / 256; ++q)
-      if (t + 256 * q < n) x[t + 256 * q] = z[q];
+    for (int i = t; i < n; i += 1024) x[i] = z[i];
     __syncthreads();
   }
   if (warm && !zero)
-    for (int i = t; i < n; i += 256) J.vec[i] = x[i];
+    for (int i = t; i < n; i += 1024) J.vec[i] = x[i];
   if (t == 0) J.out[J.target] = sqrt(fabs(lambda));
 }
 
 // ---------------------------------------------------------------- sparse factors
-// Compressed rows and columns of a dense n x n factor (one 256-thread
+// Compressed rows and columns of a dense n x n factor (one 1024-thread
 // workgroup per job), entries of a row in column order and of a column in row
 // order whatever the thread timing.  Entries beyond cap are not written (the
 // caller sizes cap to the projection's nonzero count).
+constexpr int BSP_NT = 1024;
+
 __device__ void block_excl_scan_int(int* a, int n, int* part) {
-  // a[0..n) -> exclusive prefix sums; part: 256 ints of LDS scratch
+  // a[0..n) -> exclusive prefix sums (by the first 256 threads); part: 256 ints of LDS scratch
   const int t = threadIdx.x;
   const int per = (n + 255) / 256;
   const int lo = min(t * per, n), hi = min(lo + per, n);
   int s = 0;
   for (int i = lo; i < hi; ++i) s += a[i];
-  part[t] = s;
+  if (t < 256) part[t] = s;
   __syncthreads();
   if (t == 0) {
     int run = 0;
@@ -315,7 +390,7 @@ __device__ void block_excl_scan_int(int* a, int n, int* part) {
     }
   }
   __syncthreads();
-  int run = part[t];
+  int run = t < 256 ? part[t] : 0;
   for (int i = lo; i < hi; ++i) {
     const int v = a[i];
     a[i] = run;
@@ -328,25 +403,33 @@ __device__ void block_excl_scan_int(int* a, int n, int* part) {
 // sorted in LDS by column-major position gives the compressed columns in
 // order (entry q of the sorted list is entry q of the columns), sorted again
 // by row-major position the compressed rows; the pointers are lower bounds
-// in the sorted lists.  The result equals the dense scan's.
+// in the sorted lists.  The result equals the dense scan's.  Bound by the
+// steps of the sort (LDS latency): 2048 entries 126 us with 256 threads and a
+// barrier per step -> 37.
 constexpr int BSP_SORT = 8192;
 
-__device__ void bitonic_sort_lds(int* a, int P) {  // P a power of two, 256 threads
+// P a power of two, BSP_NT threads.  Pair q of a step with stride j is
+// (i, i + j), i = q with a zero bit put in at j's place; a wave's 64 pairs of a
+// step with j <= 64 lie in its own 128 entries, so those steps (56 of 66 at
+// P = 2048) need no barrier.
+__device__ void bitonic_sort_lds(int* a, int P) {
   for (int k = 2; k <= P; k <<= 1)
     for (int j = k >> 1; j > 0; j >>= 1) {
-      for (int i = threadIdx.x; i < P; i += 256) {
-        const int l = i ^ j;
-        if (l > i) {
-          const bool up = (i & k) == 0;
-          const int x = a[i], y = a[l];
-          if ((x > y) == up) {
-            a[i] = y;
-            a[l] = x;
-          }
-        }
+      for (int q = threadIdx.x; q < P / 2; q += BSP_NT) {
+        const int i = ((q & ~(j - 1)) << 1) | (q & (j - 1));
+        const bool up = (i & k) == 0;
+        const int x = a[i], y = a[i + j];
+        a[i] = up ? min(x, y) : max(x, y);
+        a[i + j] = up ? max(x, y) : min(x, y);
       }
-      __syncthreads();
+      if (j > 64 || (j == 1 && k >= 128)) {
+        __syncthreads();
+      } else {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+      }
     }
+  __syncthreads();
 }
 
 __device__ __forceinline__ int lower_bound_lds(const int* a, int cnt, int key) {
@@ -367,26 +450,26 @@ __device__ void bsparse_from_list(const BSpBuildJob<T>& J, int nk, int* keys) {
   const BSpFac<T> F = J.F;
   int P = 1;
   while (P < nk) P <<= 1;
-  for (int q = t; q < P; q += 256) keys[q] = q < nk ? F.klist[q] : INT_MAX;
+  for (int q = t; q < P; q += BSP_NT) keys[q] = q < nk ? F.klist[q] : INT_MAX;
   __syncthreads();
   bitonic_sort_lds(keys, P);
   // compressed columns: positions j * n + i ascending
-  for (int j = t; j <= n; j += 256) F.cp[j] = lower_bound_lds(keys, nk, j * n);
-  for (int q = t; q < nk; q += 256) {
+  for (int j = t; j <= n; j += BSP_NT) F.cp[j] = lower_bound_lds(keys, nk, j * n);
+  for (int q = t; q < nk; q += BSP_NT) {
     const int idx = keys[q], j = idx / n;
     F.ri[q] = idx - j * n;
     F.cv[q] = J.M[idx];
   }
   __syncthreads();
   // compressed rows: positions i * n + j ascending
-  for (int q = t; q < nk; q += 256) {
+  for (int q = t; q < nk; q += BSP_NT) {
     const int idx = keys[q], j = idx / n, i = idx - j * n;
     keys[q] = i * n + j;
   }
   __syncthreads();
   bitonic_sort_lds(keys, P);
-  for (int i = t; i <= n; i += 256) F.rp[i] = lower_bound_lds(keys, nk, i * n);
-  for (int q = t; q < nk; q += 256) {
+  for (int i = t; i <= n; i += BSP_NT) F.rp[i] = lower_bound_lds(keys, nk, i * n);
+  for (int q = t; q < nk; q += BSP_NT) {
     const int key = keys[q], i = key / n, j = key - i * n;
     F.ci[q] = j;
     F.v[q] = J.M[(size_t)j * n + i];
@@ -394,7 +477,7 @@ __device__ void bsparse_from_list(const BSpBuildJob<T>& J, int nk, int* keys) {
 }
 
 template <class T>
-__global__ __launch_bounds__(256) void k_bsparse(const BSpBuildJob<T>* __restrict__ jobs) {
+__global__ __launch_bounds__(BSP_NT) void k_bsparse(const BSpBuildJob<T>* __restrict__ jobs) {
   __shared__ int cc[BATCH_NMAX + 1], rc[BATCH_NMAX + 1];
   __shared__ int part[256];
   __shared__ int keys[BSP_SORT];
@@ -410,13 +493,13 @@ __global__ __launch_bounds__(256) void k_bsparse(const BSpBuildJob<T>* __restric
   }
   // global (not flat) loads, so that their waits do not also wait for the LDS atomics
   const __attribute__((address_space(1))) T* M = (const __attribute__((address_space(1))) T*)J.M;
-  for (int i = t; i <= n; i += 256) cc[i] = 0;
+  for (int i = t; i <= n; i += BSP_NT) cc[i] = 0;
   __syncthreads();
-  // counts: thread t walks rows t, t + 256, ... column by column (the 256
+  // counts: thread t walks rows t, t + 1024, ... column by column (the 1024
   // rows of one column step are one coalesced read); row counts in a
   // register, column counts by LDS atomics (integer sums)
   constexpr int UB = 16;  // columns loaded together before they are tested
-  for (int i0 = 0; i0 < n; i0 += 256) {
+  for (int i0 = 0; i0 < n; i0 += BSP_NT) {
     const int i = i0 + t;
     int c = 0;
     if (i < n)
@@ -439,7 +522,7 @@ __global__ __launch_bounds__(256) void k_bsparse(const BSpBuildJob<T>* __restric
   block_excl_scan_int(rc, n + 1, part);
   // pointers clamped to cap, so that a factor with more entries than room
   // (which a sp projection does not produce) is cut, never read past its arrays
-  for (int i = t; i <= n; i += 256) {
+  for (int i = t; i <= n; i += BSP_NT) {
     F.cp[i] = min(cc[i], F.cap);
     F.rp[i] = min(rc[i], F.cap);
   }
@@ -447,7 +530,7 @@ __global__ __launch_bounds__(256) void k_bsparse(const BSpBuildJob<T>* __restric
   // fill: a row's entries in column order from the thread's own walk; a
   // column's entries at slots claimed by LDS atomics (cc becomes the running
   // end of each column), put in row order below
-  for (int i0 = 0; i0 < n; i0 += 256) {
+  for (int i0 = 0; i0 < n; i0 += BSP_NT) {
     const int i = i0 + t;
     if (i >= n) continue;
     int q = rc[i];
@@ -476,7 +559,7 @@ __global__ __launch_bounds__(256) void k_bsparse(const BSpBuildJob<T>* __restric
   }
   __syncthreads();
   // each column's entries by row (insertion sort: a sp factor has a few per column)
-  for (int j = t; j < n; j += 256) {
+  for (int j = t; j < n; j += BSP_NT) {
     const int a = min(F.cp[j], F.cap), e = min(cc[j], F.cap);
     for (int p = a + 1; p < e; ++p) {
       const int r = F.ri[p];
@@ -550,7 +633,11 @@ __device__ __forceinline__ BSpFac<T> bsp_load(const __attribute__((address_space
 // Rows t and t + 256 (n <= 512) of one factor in one orientation: their
 // first BSP_REG entries, loaded once per job and kept in registers over all
 // the rounds; the rest of a longer row, entries [s, e) of the factor's
-// arrays, is read from memory.  A row with fewer entries is padded with
+// arrays, is copied into LDS while there is room (at o), else read from
+// memory in every round, eight at a time either way.  (One at a time from
+// memory a row of 65 entries took most of a round: 512 x 512 learned factors,
+// two of them, 91 us a launch of few rounds -> 70, 263 -> 201 us in the mean of
+// 20 iterations.)  A row with fewer entries is padded with
 // (-0) x in[BSP_PAD], where the slot BSP_PAD of every vector holds +0:
 // -0 x +0 = -0 and acc + (-0) == acc for every acc, so the padding leaves
 // each sum bit-identical.
@@ -558,15 +645,23 @@ constexpr int BSP_REG = 4;
 constexpr int BSP_PAD = 512;
 template <class T>
 struct BspRows {
-  int s[2], e[2];
+  int s[2], e[2], o[2];  // o: place in LDS, -1: not there
   int k[2][BSP_REG];
   T v[2][BSP_REG];
   const __attribute__((address_space(1))) int* ix;
   const __attribute__((address_space(1))) T* vv;
 };
 
+constexpr int BSP_OV = 4096;  // entries
 template <class T>
-__device__ __forceinline__ void bsp_rows_load(BspRows<T>& R, const BSpFac<T>& F, bool trans, int n) {
+struct BspOv {
+  T* v;
+  int* k;
+  int* used;
+};
+
+template <class T>
+__device__ __forceinline__ void bsp_rows_load(BspRows<T>& R, const BSpFac<T>& F, bool trans, int n, BspOv<T> ov) {
   typedef const __attribute__((address_space(1))) int* GI;
   typedef const __attribute__((address_space(1))) T* GV;
   const GI p0 = (GI)(trans ? F.cp : F.rp);
@@ -597,11 +692,24 @@ __device__ __forceinline__ void bsp_rows_load(BspRows<T>& R, const BSpFac<T>& F,
       }
     R.s[r] = a[r] + BSP_REG;
     R.e[r] = max(b[r], a[r] + BSP_REG);
+    R.o[r] = -1;
+    const int cnt = R.e[r] - R.s[r];
+    if (cnt > 0) {
+      const int at = atomicAdd(ov.used, cnt);
+      if (at + cnt <= BSP_OV) {
+        R.o[r] = at;
+        for (int q = 0; q < cnt; ++q) {
+          ov.k[at + q] = R.ix[R.s[r] + q];
+          ov.v[at + q] = R.vv[R.s[r] + q];
+        }
+      }
+    }
   }
 }
 
 template <class T>
-__device__ __forceinline__ void bsp_rows_apply(const BspRows<T>& R, const double* in, double* out, int n) {
+__device__ __forceinline__ void bsp_rows_apply(const BspRows<T>& R, const double* in, double* out, int n,
+                                               BspOv<T> ov) {
 #pragma unroll
   for (int r = 0; r < 2; ++r) {
     const int i = threadIdx.x + 256 * r;
@@ -617,11 +725,38 @@ __device__ __forceinline__ void bsp_rows_apply(const BspRows<T>& R, const double
         acc = fma((double)vu, in[R.k[r][u]], acc);
       }
       if (R.e[r] > R.s[r]) {
-        // the rest of a long row; its start is made opaque so that its
-        // addresses are formed here rather than kept over the rounds
-        int q = R.s[r];
+        // the rest of a long row, eight entries at a time: loads together
+        // (indices clamped inside the row), then the fma chain in order.  Its
+        // start is made opaque so that its addresses are formed here rather
+        // than kept over the rounds
+        const int cnt = R.e[r] - R.s[r];
+        int q = R.o[r] >= 0 ? R.o[r] : R.s[r];
         asm volatile("" : "+v"(q));
-        for (; q < R.e[r]; ++q) acc = fma((double)R.vv[q], in[R.ix[q]], acc);
+        for (int b = 0; b < cnt; b += 8) {
+          int k[8];
+          T v[8];
+          if (R.o[r] >= 0) {
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+              k[u] = ov.k[q + min(b + u, cnt - 1)];
+              v[u] = ov.v[q + min(b + u, cnt - 1)];
+            }
+          } else {
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+              k[u] = R.ix[q + min(b + u, cnt - 1)];
+              v[u] = R.vv[q + min(b + u, cnt - 1)];
+            }
+          }
+          double xv[8];
+#pragma unroll
+          for (int u = 0; u < 8; ++u) xv[u] = in[k[u]];
+#pragma unroll
+          for (int u = 0; u < 8; ++u) {
+            const double f = fma((double)v[u], xv[u], acc);
+            acc = b + u < cnt ? f : acc;
+          }
+        }
       }
       out[i] = acc;
     }
@@ -659,7 +794,7 @@ __device__ __forceinline__ void block_sum_w2(double& a, double& b, double* red) 
 // read from memory each round.
 template <class T, int MC>
 __device__ __forceinline__ void bpower_sp_job(const BPowSpJob<T>& J, int maxit, double thr, int warm, double* x,
-                                              double* u, double* w, double* red) {
+                                              double* u, double* w, double* red, BspOv<T> ov) {
   const int n = J.n, t = threadIdx.x, m = MC > 0 ? MC : J.m;
   const __attribute__((address_space(4))) BSpFac<T>* fac = (const __attribute__((address_space(4))) BSpFac<T>*)J.fac;
   BspRows<T> cols[MC > 0 ? MC : 1], rows[MC > 0 ? MC : 1];
@@ -667,8 +802,8 @@ __device__ __forceinline__ void bpower_sp_job(const BPowSpJob<T>& J, int maxit, 
 #pragma unroll
     for (int c = 0; c < (MC > 0 ? MC : 1); ++c) {
       const BSpFac<T> F = bsp_load(fac + c);
-      bsp_rows_load(cols[c], F, true, n);
-      bsp_rows_load(rows[c], F, false, n);
+      bsp_rows_load(cols[c], F, true, n, ov);
+      bsp_rows_load(rows[c], F, false, n, ov);
     }
   }
   for (int i = t; i < n; i += 256) x[i] = J.vec[i];
@@ -705,13 +840,13 @@ __device__ __forceinline__ void bpower_sp_job(const BPowSpJob<T>& J, int maxit, 
       // y = P^T x = F_{m-1}^T ... F_0^T x, then z = P y = F_0 ... F_{m-1} y
 #pragma unroll
       for (int c = 0; c < (MC > 0 ? MC : 1); ++c) {
-        bsp_rows_apply(cols[c], cur, nxt, n);
+        bsp_rows_apply(cols[c], cur, nxt, n, ov);
         cur = nxt;
         nxt = (nxt == u) ? w : u;
       }
 #pragma unroll
       for (int c = (MC > 0 ? MC : 1) - 1; c >= 0; --c) {
-        bsp_rows_apply(rows[c], cur, nxt, n);
+        bsp_rows_apply(rows[c], cur, nxt, n, ov);
         cur = nxt;
         nxt = (nxt == u) ? w : u;
       }
@@ -761,14 +896,14 @@ __global__ __launch_bounds__(256) void k_bpower_sp(const BPowSpJob<T>* __restric
     if (threadIdx.x == 0) J.out[J.target] = 1.0;
     return;
   }
-  bpower_sp_job<T, 0>(J, maxit, thr, warm, lds, lds + nmax, lds + 2 * nmax, red);
+  bpower_sp_job<T, 0>(J, maxit, thr, warm, lds, lds + nmax, lds + 2 * nmax, red, BspOv<T>{});
 }
 
 // Jobs of MC factors (or none) of edge n <= 512: rows in registers, vectors
 // at fixed LDS offsets (so that every gather is one LDS read at a constant
 // offset from the entry's index).
 template <class T, int MC>
-__global__ __launch_bounds__(256, 4) void k_bpower_sp_reg(const BPowSpJob<T>* __restrict__ jobs, int maxit, double thr,
+__global__ __launch_bounds__(256, 2) void k_bpower_sp_reg(const BPowSpJob<T>* __restrict__ jobs, int maxit, double thr,
                                                        int warm) {
   __shared__ double x[BSP_PAD + 2], u[BSP_PAD + 2], w[BSP_PAD + 2];
   __shared__ double red[8];
@@ -777,8 +912,14 @@ __global__ __launch_bounds__(256, 4) void k_bpower_sp_reg(const BPowSpJob<T>* __
     if (threadIdx.x == 0) J.out[J.target] = 1.0;
     return;
   }
-  if (threadIdx.x == 0) x[BSP_PAD] = u[BSP_PAD] = w[BSP_PAD] = 0.0;
-  bpower_sp_job<T, MC>(J, maxit, thr, warm, x, u, w, red);
+  __shared__ T ov_v[BSP_OV];
+  __shared__ int ov_k[BSP_OV], ov_used;
+  if (threadIdx.x == 0) {
+    x[BSP_PAD] = u[BSP_PAD] = w[BSP_PAD] = 0.0;
+    ov_used = 0;
+  }
+  __syncthreads();
+  bpower_sp_job<T, MC>(J, maxit, thr, warm, x, u, w, red, BspOv<T>{ov_v, ov_k, &ov_used});
 }
 
 // Batched sparse x dense products (BSpmmJob): a workgroup computes the
@@ -788,8 +929,12 @@ __global__ __launch_bounds__(256, 4) void k_bpower_sp_reg(const BPowSpJob<T>* __
 // left each column of X is staged too and gathered from LDS, with S on the
 // right the lanes read the combined columns of X directly (coalesced).  Each
 // output entry is one fma chain over the entries in their stored order, FP32
-// (T) accumulation like the dense GEMM it replaces.  Factors with more
-// entries than the LDS room read them from global memory instead.
+// (T) accumulation like the dense GEMM it replaces.  Lists with more
+// entries than the LDS room are read from global memory instead.  With S on
+// the right only the entries of the tile's columns are staged.  Bound by the
+// latency of the gathers and of long rows and columns; a row's entries go four
+// at a time with their LDS reads in flight together.  48 targets of 64 .. 512:
+// 62 .. 105 us -> 33 .. 45.
 constexpr int SPMM_LDS_BYTES = 16 * 1024;
 constexpr int SPMM_XCOLS = 2048;  // entries of X staged per column block (S on the left)
 constexpr int SPMM_CB = 4;        // columns per block with S on the right
@@ -855,6 +1000,49 @@ __device__ __forceinline__ void bspmm_body(const SpmmCtx<T>& C) {
     // staging when they fit 8 slots: one row (n <= 256, up to 8 columns) or
     // two rows of up to 4 columns (n <= 512 with blocks of 4 columns)
     const bool pre = C.beta_mode && (n <= 256 || (n <= 512 && cb <= 4));
+    // row i's sums over the staged columns: four entries at a time, their list
+    // reads and then their gathers in flight together (indices clamped inside
+    // the row, terms past its end not kept), in stored order
+    auto row = [&](int i, int m, T* acc) {
+      const int qe = C.s_p[i + 1];
+      for (int q0 = C.s_p[i]; q0 < qe; q0 += 4) {
+        int k[4];
+        T v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int q = min(q0 + u, qe - 1);
+          k[u] = ix[q];
+          v[u] = vv[q];
+        }
+        if (m > 4) {
+          T x[4][8];
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int c = 0; c < 8; ++c) x[u][c] = C.s_x[min(c, m - 1) * n + k[u]];
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+              const T f = fma(v[u], x[u][c], acc[c]);
+              acc[c] = q0 + u < qe ? f : acc[c];
+            }
+        } else {
+          T x[4][4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) x[u][c] = C.s_x[min(c, m - 1) * n + k[u]];
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+              const T f = fma(v[u], x[u][c], acc[c]);
+              acc[c] = q0 + u < qe ? f : acc[c];
+            }
+        }
+      }
+    };
     for (int jb = 0; jb < nc; jb += cb) {
       const int m = min(cb, nc - jb);
       T old[8];
@@ -897,13 +1085,7 @@ __device__ __forceinline__ void bspmm_body(const SpmmCtx<T>& C) {
           T acc[8];
 #pragma unroll
           for (int c = 0; c < 8; ++c) acc[c] = T(0);
-          for (int q = C.s_p[i], qe = C.s_p[i + 1]; q < qe; ++q) {
-            const int k = ix[q];
-            const T v = vv[q];
-#pragma unroll
-            for (int c = 0; c < 8; ++c)
-              if (c < m) acc[c] = fma(v, C.s_x[c * n + k], acc[c]);
-          }
+          row(i, m, acc);
           out_pre(i, j0 + jb, m, acc, old + 4 * r);
         }
         __syncthreads();  // s_x is rewritten for the next block
@@ -913,13 +1095,7 @@ __device__ __forceinline__ void bspmm_body(const SpmmCtx<T>& C) {
         T acc[8];
 #pragma unroll
         for (int c = 0; c < 8; ++c) acc[c] = T(0);
-        for (int q = C.s_p[i], qe = C.s_p[i + 1]; q < qe; ++q) {
-          const int k = ix[q];
-          const T v = vv[q];
-#pragma unroll
-          for (int c = 0; c < 8; ++c)
-            if (c < m) acc[c] = fma(v, C.s_x[c * n + k], acc[c]);
-        }
+        row(i, m, acc);
         out8(i, j0 + jb, m, acc);
       }
       __syncthreads();  // s_x is rewritten for the next block
@@ -934,7 +1110,7 @@ __device__ __forceinline__ void bspmm_body(const SpmmCtx<T>& C) {
         int qa[SPMM_CB], qe[SPMM_CB];
 #pragma unroll
         for (int c = 0; c < SPMM_CB; ++c) {
-          const int j = min(j0 + jb + c, j0 + nc - 1);
+          const int j = min(jb + c, nc - 1);  // s_p holds the tile's columns
           qa[c] = C.s_p[j];
           qe[c] = C.s_p[j + 1];
 #pragma unroll
@@ -998,13 +1174,15 @@ __global__ __launch_bounds__(256, 4) void k_bspmm(const BSpmmJob<T>* __restrict_
   const int* p0 = rows_of_S ? J.S.rp : J.S.cp;
   const int* ix = rows_of_S ? J.S.ci : J.S.ri;
   const T* vv = rows_of_S ? J.S.v : J.S.cv;
-  const int nnz = p0[n];
+  // S on the left: every row; S on the right: the columns of this tile
+  const int first = J.side == 0 ? 0 : tl.y, cnt = J.side == 0 ? n : tl.z;
+  const int base = p0[first], nnz = p0[first + cnt] - base;
   const bool lds = nnz <= ENT;
-  for (int i = t; i <= n; i += 256) s_p[i] = p0[i];
+  for (int i = t; i <= cnt; i += 256) s_p[i] = p0[first + i] - (lds ? base : 0);
   if (lds)
     for (int q = t; q < nnz; q += 256) {
-      s_ix[q] = ix[q];
-      s_v[q] = vv[q];
+      s_ix[q] = ix[base + q];
+      s_v[q] = vv[base + q];
     }
   __syncthreads();
   SpmmCtx<T> C;
@@ -1033,6 +1211,14 @@ __global__ __launch_bounds__(256, 4) void k_bspmm(const BSpmmJob<T>* __restrict_
 // (radix select on the magnitude bits; among entries equal to the k-th
 // largest the lowest indices are kept), then divide by the Frobenius norm.
 // SUPP: multiply by the 0/1 mask, then normalise.
+//
+// Bound by the instructions of one CU over the target's entries (and, before,
+// by LDS atomics of 64 lanes on a few bins: every pass of the radix select
+// binned every entry).  Now one pass finds a lower bound of the k-th largest
+// key, one lists the few entries above it, the digits are taken from that list
+// only, and one writes.  512 x 512, k = 2048: 230 us -> 91; the masked form in
+// FP64 290 -> 209.  The general passes stay for ties' ranks, for k past
+// 4096 and where the list does not fit.
 
 template <class T> struct KeyOf;
 template <> struct KeyOf<float> {
@@ -1047,6 +1233,8 @@ template <> struct KeyOf<double> {
 };
 
 constexpr int BSEL_BITS = 11;  // radix-select digit width (bins in LDS: 2048)
+constexpr int BSEL_TOP = 4;  // largest keys per thread for the candidates' bound: k up to 4096
+constexpr int BSEL_CAND_BYTES = 128 * 1024;  // LDS for the candidates' keys
 
 template <class T, int MODE>  // MODE 0: SP, 1: SUPP
 __global__ __launch_bounds__(1024) void k_bprox(const BProxJob<T>* __restrict__ jobs) {
@@ -1060,16 +1248,45 @@ __global__ __launch_bounds__(1024) void k_bprox(const BProxJob<T>* __restrict__ 
   __shared__ long long s_kk;
   __shared__ unsigned s_eq;
   // the kept entries of the untied path, so that the normalisation scales
-  // them alone instead of every entry
-  constexpr int KEEP_LIST = 8192;
-  __shared__ int kept[KEEP_LIST];
-  __shared__ int s_nkept;
+  // them alone instead of every entry; before that, the candidates' keys
+  constexpr int KEEP_LIST = 8192, CAND = MODE == 0 ? BSEL_CAND_BYTES / (int)sizeof(K) : KEEP_LIST * 4 / (int)sizeof(K);
+  __shared__ K cand[CAND];
+  int* kept = reinterpret_cast<int*>(cand);
+  __shared__ int s_nkept, s_ncand;
+  __shared__ K s_lo, s_hi;
+  // loads of a thread in flight in the passes over the target: with eight, a
+  // pass over 512 x 512 took 32 rounds of memory latency
+  constexpr int UL = 128 / (int)sizeof(K);
   const BProxJob<T> J = jobs[blockIdx.x];
   const int t = threadIdx.x;
   const int64_t len = J.len;
   // global (not flat) accesses: their waits do not wait for the LDS atomics
   typedef __attribute__((address_space(1))) T* GT;
   GT M = (GT)J.M;
+  // f(constant: whole chunk, i0) for the entries in chunks of UL * 1024 from i0
+  auto chunks = [&](auto f) {
+    int64_t i0 = 0;
+    for (; i0 + UL * 1024 <= len; i0 += UL * 1024) f(std::integral_constant<bool, true>{}, i0);
+    if (i0 < len) f(std::integral_constant<bool, false>{}, i0);
+  };
+  // this thread's entry u of a chunk (len < 2^23); the last one's index is clamped
+  auto entry = [&](auto full, int64_t i0, int u) -> T {
+    if constexpr (decltype(full)::value)
+      return (M + i0 + u * 1024)[t];
+    else
+      return M[min((int)i0 + u * 1024 + t, (int)len - 1)];
+  };
+  // room for c items of this lane in a list of n: the lane's first place
+  auto places = [&](int c, int* n) {
+    int incl = c;
+    for (int off = 1; off < 64; off <<= 1) {
+      const int o = __shfl_up(incl, off);
+      if ((t & 63) >= off) incl += o;
+    }
+    int at = 0;
+    if ((t & 63) == 63 && incl > 0) at = atomicAdd(n, incl);
+    return __builtin_amdgcn_readlane(at, 63) + incl - c;
+  };
   // ss: this thread's sum of squares over i = t, t + 1024, ... of the
   // projected entries (fma in that order, as the separate pass below)
   T ss = T(0);
@@ -1077,35 +1294,150 @@ __global__ __launch_bounds__(1024) void k_bprox(const BProxJob<T>* __restrict__ 
   if (t == 0) s_nkept = -1;  // no list
   __syncthreads();
   if (MODE == 1) {
-    for (int64_t i = t; i < len; i += 1024) M[i] = M[i] * J.mask[i];
+    const __attribute__((address_space(1))) T* mask = (const __attribute__((address_space(1))) T*)J.mask;
+    for (int64_t i0 = 0; i0 < len; i0 += 16 * 1024) {
+      T xv[16], mv[16];
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        const int64_t i = min(i0 + u * 1024 + t, len - 1);
+        xv[u] = M[i];
+        mv[u] = mask[i];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        const int64_t i = i0 + u * 1024 + t;
+        if (i < len) {
+          const T y = xv[u] * mv[u];
+          M[i] = y;
+          ss = fma(y, y, ss);
+        }
+      }
+    }
+    have_ss = true;
   } else if (J.k < len) {
     if (J.k <= 0) {
       for (int64_t i = t; i < len; i += 1024) M[i] = T(0);
     } else {
       K prefix = 0, mask = 0;
       long long kk = J.k;  // rank still to find among keys matching prefix
-      // digits of up to BSEL_BITS bits from the top: 3 passes for FP32 keys,
-      // 6 for FP64
-      for (int hi = KO::BITS; hi > 0; hi -= BSEL_BITS) {
+      // Candidates: when each of the 1024 threads has G entries, 1024 G >= k, the
+      // least of the threads' G-th largest keys has at least k entries at or
+      // above it, so the k-th largest key is among those.  Thread t takes entry
+      // (t + 37 m) mod 1024 of the m-th 1024 entries, so that it meets many rows
+      // and columns and rows of small entries do not make a small bound (with
+      // threads along rows the list overflowed).  The list holds some 1024 times
+      // 7 (G = 1) to 13 (G = 4) entries whatever the size.
+      const int G = (int)min((long long)BSEL_TOP + 1, (kk + 1023) / 1024);
+      const bool grouped = G <= BSEL_TOP && len >= 1024 * (int64_t)G;
+      if (t == 0) {
+        s_lo = grouped ? ~(K)0 : 0;
+        s_hi = 0;
+        s_ncand = 0;
+      }
+      __syncthreads();
+      if (grouped) {
+        const int blocks = (int)(len >> 10);  // whole ones, at least G
+        K lo = 0, hi = 0;
+        auto walk = [&](auto gc) {  // a compile-time G: the thread's largest keys stay in registers
+          constexpr int GC = decltype(gc)::value;
+          K top[GC];  // descending
+#pragma unroll
+          for (int g = 0; g < GC; ++g) top[g] = 0;
+          auto take = [&](K x) {
+#pragma unroll
+            for (int g = 0; g < GC; ++g) {
+              const K y = min(top[g], x);
+              top[g] = max(top[g], x);
+              x = y;
+            }
+          };
+          for (int m = 0; m < blocks; m += UL) {
+            K kv[UL];
+#pragma unroll
+            for (int u = 0; u < UL; ++u) {
+              const int mm = min(m + u, blocks - 1);
+              kv[u] = KO::key(M[((int64_t)mm << 10) + ((t + 37 * mm) & 1023)]);
+            }
+#pragma unroll
+            for (int u = 0; u < UL; ++u)
+              if (m + u < blocks) take(kv[u]);
+          }
+          const int64_t e = ((int64_t)blocks << 10) + t;
+          if (e < len) take(KO::key(M[e]));
+          lo = top[GC - 1];
+          hi = top[0];
+        };
+        if (G == 1) walk(std::integral_constant<int, 1>{});
+        else if (G == 2) walk(std::integral_constant<int, 2>{});
+        else if (G == 3) walk(std::integral_constant<int, 3>{});
+        else walk(std::integral_constant<int, 4>{});
+        for (int off = 32; off > 0; off >>= 1) {
+          lo = min(lo, (K)__shfl_xor(lo, off));
+          hi = max(hi, (K)__shfl_xor(hi, off));
+        }
+        if ((t & 63) == 0) {
+          atomicMin(&s_lo, lo);
+          atomicMax(&s_hi, hi);
+        }
+        __syncthreads();
+      }
+      const K lo = s_lo;
+      if (grouped) {
+        chunks([&](auto full, int64_t i0) {
+          K kv[UL];
+#pragma unroll
+          for (int u = 0; u < UL; ++u) kv[u] = KO::key(entry(full, i0, u));
+          int c = 0;
+#pragma unroll
+          for (int u = 0; u < UL; ++u) {
+            if (!decltype(full)::value && (int)i0 + u * 1024 + t >= (int)len) kv[u] = 0;
+            // lo == 0 makes every entry a candidate, also the ones past the end: the list is then not used
+            c += kv[u] >= lo;
+          }
+          int at = places(c, &s_ncand);
+#pragma unroll
+          for (int u = 0; u < UL; ++u)
+            if (kv[u] >= lo) {
+              if (at < CAND) cand[at] = kv[u] - lo;
+              ++at;
+            }
+        });
+        __syncthreads();
+      }
+      const int nc = s_ncand;
+      const bool listed_c = grouped && lo > 0 && nc <= CAND;  // else every entry is binned, by all of its bits
+      const K range = s_hi - lo;
+      const int bits =
+          !listed_c ? KO::BITS : (range == 0 ? 1 : 64 - __clzll((long long)(unsigned long long)range));
+      // digits of up to BSEL_BITS bits from the top
+      for (int hi = bits; hi > 0; hi -= BSEL_BITS) {
         const int shift = hi > BSEL_BITS ? hi - BSEL_BITS : 0;
         const int nb = 1 << (hi - shift);
         const K dmask = (K)(nb - 1);
         for (int b = t; b < nb; b += 1024) hist[b] = 0;
         __syncthreads();
-        // eight entries per thread loaded before they are binned, so that the
-        // loads are in flight together
-        int64_t i0 = t;
-        for (; i0 + 7 * 1024 < len; i0 += 8 * 1024) {
-          K kv[8];
+        if (listed_c) {
+          for (int q = t; q < nc; q += 1024) {
+            const K key = cand[q];
+            if ((key & mask) == prefix) atomicAdd(&hist[(key >> shift) & dmask], 1u);
+          }
+        } else {
+          // eight entries per thread loaded before they are binned, so that the
+          // loads are in flight together
+          int64_t i0 = t;
+          for (; i0 + 7 * 1024 < len; i0 += 8 * 1024) {
+            K kv[8];
 #pragma unroll
-          for (int u = 0; u < 8; ++u) kv[u] = KO::key(M[i0 + u * 1024]);
+            for (int u = 0; u < 8; ++u) kv[u] = KO::key(M[i0 + u * 1024]);
 #pragma unroll
-          for (int u = 0; u < 8; ++u)
-            if ((kv[u] & mask) == prefix) atomicAdd(&hist[(kv[u] >> shift) & dmask], 1u);
-        }
-        for (int64_t i = i0; i < len; i += 1024) {
-          const K key = KO::key(M[i]);
-          if ((key & mask) == prefix) atomicAdd(&hist[(key >> shift) & dmask], 1u);
+            for (int u = 0; u < 8; ++u)
+              if ((kv[u] & mask) == prefix) atomicAdd(&hist[(kv[u] >> shift) & dmask], 1u);
+          }
+          for (int64_t i = i0; i < len; i += 1024) {
+            const K key = KO::key(M[i]);
+            if ((key & mask) == prefix) atomicAdd(&hist[(key >> shift) & dmask], 1u);
+          }
         }
         __syncthreads();
         // the bin holding the kk-th largest key: thread t owns bins
@@ -1151,33 +1483,40 @@ __global__ __launch_bounds__(1024) void k_bprox(const BProxJob<T>* __restrict__ 
         mask |= (dmask << shift);
         __syncthreads();
       }
+      if (listed_c) prefix += lo;
       // keys > prefix are kept; kk entries equal to prefix are kept, lowest index first
       if ((long long)s_eq == kk) {
         // every entry equal to the k-th largest key is kept: no ranking, and
         // the sum of squares is taken on the way
         if (t == 0) s_nkept = 0;
         __syncthreads();
-        auto one = [&](int64_t i, T x) {
-          const bool keep = KO::key(x) >= prefix;
-          if (!keep) M[i] = T(0);
-          const T y = keep ? x : T(0);
-          ss = fma(y, y, ss);
-          if (keep) {
-            const int slot = atomicAdd(&s_nkept, 1);
-            if (slot < KEEP_LIST) kept[slot] = (int)i;
+        // UL loads in flight, then the entries in order (the order of the
+        // sum of squares is that of the separate pass); a wave asks for its
+        // places in the list once per UL entries
+        chunks([&](auto full, int64_t i0) {
+          T xv[UL];
+          int c = 0;
+#pragma unroll
+          for (int u = 0; u < UL; ++u) xv[u] = entry(full, i0, u);
+          unsigned keep = 0;
+#pragma unroll
+          for (int u = 0; u < UL; ++u) {
+            const bool in = decltype(full)::value || (int)i0 + u * 1024 + t < (int)len;
+            const bool k = in && KO::key(xv[u]) >= prefix;
+            const T y = k ? xv[u] : T(0);
+            ss = fma(y, y, ss);
+            if (in) (M + i0 + u * 1024)[t] = y;
+            keep |= (unsigned)k << u;
           }
-        };
-        // eight loads in flight, then the entries in order (the order of the
-        // sum of squares is unchanged)
-        int64_t i0 = t;
-        for (; i0 + 7 * 1024 < len; i0 += 8 * 1024) {
-          T xv[8];
-#pragma unroll
-          for (int u = 0; u < 8; ++u) xv[u] = M[i0 + u * 1024];
-#pragma unroll
-          for (int u = 0; u < 8; ++u) one(i0 + u * 1024, xv[u]);
-        }
-        for (int64_t i = i0; i < len; i += 1024) one(i, M[i]);
+          c = __popc(keep);
+          int at = places(c, &s_nkept);
+          while (keep) {
+            const int u = __ffs(keep) - 1;
+            keep &= keep - 1;
+            if (at < KEEP_LIST) kept[at] = (int)i0 + u * 1024 + t;
+            ++at;
+          }
+        });
         have_ss = true;
       } else {
         const int64_t chunk = (len + 1023) / 1024;
@@ -1224,7 +1563,17 @@ __global__ __launch_bounds__(1024) void k_bprox(const BProxJob<T>* __restrict__ 
       // only the kept entries are nonzero (0 * inv = 0 for the others)
       for (int q = t; q < nk; q += 1024) M[kept[q]] = M[kept[q]] * inv;
     } else {
-      for (int64_t i = t; i < len; i += 1024) M[i] = M[i] * inv;
+      for (int64_t i0 = 0; i0 < len; i0 += 16 * 1024) {
+        T xv[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) xv[u] = M[min(i0 + u * 1024 + t, len - 1)];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+          const int64_t i = i0 + u * 1024 + t;
+          if (i < len) M[i] = xv[u] * inv;
+        }
+      }
     }
   }
   // the kept entries for the compressed form built next
@@ -1356,13 +1705,9 @@ void launch_bgemm(const BGemmJob<T>* jobs, const int3* tiles, int ntiles, int ti
   const int per = xcd_per(ntiles);
   const unsigned grid = per > 0 ? 8u * per : (unsigned)ntiles;
   if (tile == BGEMM_MFMA) {
-    if constexpr (std::is_same<T, float>::value) {
-      hipLaunchKernelGGL(k_bgemm_mfma_f32, dim3(grid), dim3(256), 0, st, jobs, tiles, sc, ntiles, per);
-      FH_LAUNCH_CHECK();
-      return;
-    } else {
-      throw Error(FH_ERR_ARG, "batched GEMM: the MFMA tile is FP32 only");
-    }
+    hipLaunchKernelGGL(k_bgemm_mfma<T>, dim3(grid), dim3(256), 0, st, jobs, tiles, sc, ntiles, per);
+    FH_LAUNCH_CHECK();
+    return;
   }
   if (tile == 32)
     hipLaunchKernelGGL((k_bgemm<T, 32>), dim3(grid), dim3(256), 0, st, jobs, tiles, sc, ntiles, per);
@@ -1374,7 +1719,7 @@ void launch_bgemm(const BGemmJob<T>* jobs, const int3* tiles, int ntiles, int ti
 template <class T>
 void launch_bpower(const BPowJob<T>* jobs, int njobs, int maxit, double thr, int warm, hipStream_t st) {
   if (njobs == 0) return;
-  hipLaunchKernelGGL(k_bpower<T>, dim3(njobs), dim3(256), 0, st, jobs, maxit, thr, warm);
+  hipLaunchKernelGGL(k_bpower<T>, dim3(njobs), dim3(1024), 0, st, jobs, maxit, thr, warm);
   FH_LAUNCH_CHECK();
 }
 
@@ -1390,7 +1735,7 @@ void launch_bspmm(const BSpmmJob<T>* jobs, const int3* tiles, int ntiles, const 
 template <class T>
 void launch_bsparse(const BSpBuildJob<T>* jobs, int njobs, hipStream_t st) {
   if (njobs == 0) return;
-  hipLaunchKernelGGL(k_bsparse<T>, dim3(njobs), dim3(256), 0, st, jobs);
+  hipLaunchKernelGGL(k_bsparse<T>, dim3(njobs), dim3(BSP_NT), 0, st, jobs);
   FH_LAUNCH_CHECK();
 }
 
@@ -1434,6 +1779,22 @@ void launch_brelerr(const BLamJob<T>* jobs, int njobs, const double* lambda, dou
   FH_LAUNCH_CHECK();
 }
 
+// An FP64 matrix (src) in the batch's type, or the identity (src null, edge n), per job.
+template <class T>
+__global__ __launch_bounds__(256) void k_bload(const BLoadJob* __restrict__ jobs) {
+  const BLoadJob J = jobs[blockIdx.y];
+  T* dst = static_cast<T*>(J.dst);
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < J.len; i += (int64_t)gridDim.x * 256)
+    dst[i] = J.src ? (T)J.src[i] : (i % (J.n + 1) == 0 ? T(1) : T(0));
+}
+
+template <class T>
+void launch_bload(const BLoadJob* jobs, int njobs, hipStream_t st) {
+  if (njobs == 0) return;
+  hipLaunchKernelGGL(k_bload<T>, dim3(64, (unsigned)njobs), dim3(256), 0, st, jobs);
+  FH_LAUNCH_CHECK();
+}
+
 template <class S>
 __global__ __launch_bounds__(256) void k_bcast(const BCastJob* __restrict__ jobs) {
   const BCastJob J = jobs[blockIdx.y];
@@ -1468,6 +1829,7 @@ void launch_bcopy(T* dst, const T* src, int64_t n, hipStream_t st) {
   template void launch_bpower_sp<T>(const BPowSpJob<T>*, int, int, int, int, double, int, hipStream_t);    \
   template void launch_blambda<T>(const BLamJob<T>*, int, double*, hipStream_t);                            \
   template void launch_brelerr<T>(const BLamJob<T>*, int, const double*, double*, hipStream_t);             \
+  template void launch_bload<T>(const BLoadJob*, int, hipStream_t);                                         \
   template void launch_bcopy<T>(T*, const T*, int64_t, hipStream_t);
 FH_INST(float)
 FH_INST(double)

@@ -312,7 +312,7 @@ typedef struct {
   int norm2_max_iter;  /* default 100 */
   double norm2_threshold; /* default 1e-6 */
   int use_graph;       /* capture one iteration in a HIP graph */
-  int autotune;        /* time 32/64 GEMM tiles per target size at set-up */
+  int autotune;        /* accepted; one GEMM tile is the quickest at every size, so nothing is timed */
   int check_every;     /* > 0: FP64 relative-error check every check_every iterations */
   double target_err;   /* stop when every target's FP64 relative error <= target_err */
   const double *target_errs; /* per-target thresholds (ntargets of them) in place of target_err, or NULL */
