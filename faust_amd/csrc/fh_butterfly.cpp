@@ -26,6 +26,8 @@ namespace {
 struct BNode {
   int a = 0, b = 0;  // supports [a, b)
   DBuf v;            // n x 2^(b-a) values, row-major (the root: the matrix itself)
+  const double* given = nullptr;  // the root when the caller's matrix already lies like that, else null
+  const double* values() const { return given ? given : (const double*)v.p; }
 };
 using BNodeP = std::shared_ptr<BNode>;
 
@@ -45,9 +47,9 @@ struct Bfly {
     Y->b = nd->b;
     X->v.alloc((sizeof(double) * (size_t)n) << (c - nd->a));
     Y->v.alloc((sizeof(double) * (size_t)n) << (nd->b - c));
-    FH_CHECK(nd->v.p != nullptr, "butterfly: node without values");
+    FH_CHECK(nd->values() != nullptr, "butterfly: node without values");
     BflyStep s;
-    s.in = (const double*)nd->v.p;
+    s.in = nd->values();
     s.in_logB = nd->b - nd->a;
     s.in_logs = L - nd->b;
     s.n = n;
@@ -206,8 +208,14 @@ fh_faust_s* butterfly_run(const double* A, size_t lda, int row_major, int n, int
   B.root = std::make_shared<BNode>();
   B.root->a = 0;
   B.root->b = B.L;
-  B.root->v.alloc(sizeof(double) * (size_t)n * n);
-  bfly_root(A, lda, row_major, n, (const int*)pinv_dev.p, (double*)B.root->v.p, st);
+  if (row_major && lda == (size_t)n && !perm) {
+    // read in place: only the first split reads the root, on the caller's
+    // stream, and this call waits for it (the copy of 128 MiB took 50 us)
+    B.root->given = A;
+  } else {
+    B.root->v.alloc(sizeof(double) * (size_t)n * n);
+    bfly_root(A, lda, row_major, n, (const int*)pinv_dev.p, (double*)B.root->v.p, st);
+  }
   std::vector<BNodeP> nodes = dir == FH_BUTTERFLY_BBTREE ? bfly_balanced(B) : bfly_directional(B, dir == FH_BUTTERFLY_RIGHT);
   FH_CHECK((int)nodes.size() == B.L, "butterfly: wrong number of factors");
   for (int k = 0; k < B.L; ++k)

@@ -493,6 +493,203 @@ __global__ __launch_bounds__(BF_THREADS) void k_bfly_gram_mfma(BflyStep s) {
   for (int j = tid; j < d; j += BF_THREADS) bf_put_col(s, tr, t, j, M[j * ld + jb] * vs * kc);
 }
 
+// Blocks with a side of 4 and one of at most 16: a block per lane, everything
+// in registers, with the sums of k_bfly_gram (its one active thread per
+// 256-thread workgroup, its barriers and its trace loop over LDS took 35 us for
+// 4096 4 x 4 blocks; bound here by the chain of squarings, 5 us).  G and its
+// powers are symmetric bit for bit, so entries (p, q), p <= q are kept.
+template <int LOGD>
+__global__ __launch_bounds__(64) void k_bfly_gram4(BflyStep s) {
+  constexpr int D = 1 << LOGD;
+  const int t = blockIdx.x * 64 + threadIdx.x;
+  if (t >= s.n) return;
+  const bool tr = s.logBx < s.logBy;
+  double W[D][4];
+#pragma unroll
+  for (int i = 0; i < D; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) W[i][j] = bf_w0(s, tr, t, j, i);
+  double M[4][4];
+#pragma unroll
+  for (int p = 0; p < 4; ++p)
+#pragma unroll
+    for (int q = p; q < 4; ++q) {
+      double g = 0.0;
+#pragma unroll
+      for (int i = 0; i < D; ++i) g = fma(W[i][p], W[i][q], g);
+      M[p][q] = M[q][p] = g;
+    }
+  const double tau = ((M[0][0] + M[1][1]) + M[2][2]) + M[3][3];
+  if (tau > 0.0) {
+    double scale = 1.0 / tau;
+    for (int k = 0; k < BF_MAX_SQ; ++k) {
+      const double sc2 = scale * scale;
+      double N[4][4];
+#pragma unroll
+      for (int p = 0; p < 4; ++p)
+#pragma unroll
+        for (int q = p; q < 4; ++q) {
+          double g = 0.0;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) g = fma(M[r][p], M[r][q], g);
+          N[p][q] = N[q][p] = g * sc2;
+        }
+#pragma unroll
+      for (int p = 0; p < 4; ++p)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) M[p][q] = N[p][q];
+      const double tr2 = ((M[0][0] + M[1][1]) + M[2][2]) + M[3][3];
+      scale = 1.0 / tr2;
+      if (tr2 >= 1.0 - 16.0 * DBL_EPSILON) break;
+    }
+  }
+  // column jb of M in constant-index form (jb differs from lane to lane)
+  double best = M[0][0], c[4] = {M[0][0], M[1][0], M[2][0], M[3][0]};
+#pragma unroll
+  for (int j = 1; j < 4; ++j) {
+    const bool up = M[j][j] > best;
+    best = up ? M[j][j] : best;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) c[i] = up ? M[i][j] : c[i];
+  }
+  double vn = 0.0;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) vn = fma(c[j], c[j], vn);
+  const double vs = vn > 0.0 ? 1.0 / sqrt(vn) : 0.0;
+  double w[D], q2[D];
+#pragma unroll
+  for (int i = 0; i < D; ++i) {
+    w[i] = 0.0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w[i] = fma(W[i][j], c[j] * vs, w[i]);
+    q2[i] = w[i] * w[i];
+  }
+#pragma unroll
+  for (int o = D / 2; o >= 1; o >>= 1)  // the halves in the order of a wave sum
+#pragma unroll
+    for (int i = 0; i < o; ++i) q2[i] = q2[i] + q2[i + o];
+  const double lam = q2[0];
+  double kl = 0.0, kc = 0.0;
+  if (lam > 0.0 && vn > 0.0) {
+    const double sigma = sqrt(lam), rs = sqrt(sigma);
+    kl = 1.0 / rs;
+    kc = rs;
+  }
+#pragma unroll
+  for (int i = 0; i < D; ++i) bf_put_len(s, tr, t, i, w[i] * kl);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) bf_put_col(s, tr, t, j, c[j] * vs * kc);
+}
+
+// Blocks with a side of 16 and one of 16 .. 256 on FP64 MFMA: the whole block in
+// LDS, read once and along the node's rows whichever way it lies, and the 16 x 16
+// part in one wave without workgroup barriers (in k_bfly_gram_mfma three waves
+// waited for it at three barriers a square, and the block was read three
+// times).  The sums are those of k_bfly_gram_mfma.  4096 blocks: 16 x 256
+// (128 MiB) 119 -> 56 us, 16 x 16 49 -> 17 us; bound by reading the root, then
+// by the chain of squares.
+__device__ __forceinline__ void bf_wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+template <int CTRL>
+__device__ __forceinline__ double bf_row_add(double v) {  // v + the value CTRL (row_ror) brings
+  const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+  return v + __builtin_bit_cast(double, (unsigned long long)(unsigned)hi << 32 | (unsigned)lo);
+}
+// sum over the 16 lanes of a row, as the xor butterfly of 8, 4, 2, 1 (after each
+// step the values repeat with its period, so a rotation brings the same one)
+__device__ __forceinline__ double bf_row_sum(double v) {
+  v = bf_row_add<0x128>(v);
+  v = bf_row_add<0x124>(v);
+  v = bf_row_add<0x122>(v);
+  return bf_row_add<0x121>(v);
+}
+
+template <int LOGD>
+__global__ __launch_bounds__(LOGD <= 6 ? 64 : BF_THREADS) void k_bfly_gram16(BflyStep s) {
+  constexpr int D = 1 << LOGD, NT = LOGD <= 6 ? 64 : BF_THREADS, LD = 17, PER = D * 16 / NT;
+  __shared__ double W[D * LD], M[16 * LD], v[16];
+  __shared__ double red[NT / 64], s_vn;
+  const int t = bf_block_index(blockIdx.x, gridDim.x), tid = threadIdx.x;
+  const int lane = tid & 63, li = lane & 15, lk = lane >> 4;
+  const bool tr = s.logBx < s.logBy;
+  {
+    double x[PER];
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const int e = tid + k * NT;
+      const int i = tr ? e & (D - 1) : e >> 4, j = tr ? e >> LOGD : e & 15;
+      x[k] = bf_w0(s, tr, t, j, i);
+    }
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const int e = tid + k * NT;
+      const int i = tr ? e & (D - 1) : e >> 4, j = tr ? e >> LOGD : e & 15;
+      W[i * LD + j] = x[k];
+    }
+  }
+  __syncthreads();
+  if (tid < 64) {
+    bf_d4 acc = {0.0, 0.0, 0.0, 0.0};
+    for (int i0 = 0; i0 < D; i0 += 4) {
+      const double w = W[(i0 + lk) * LD + li];
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(w, w, acc, 0, 0, 0);
+    }
+    bf_store_tile(M, LD, 0, 0, li, lk, acc, 1.0);
+    bf_wave_fence();
+    const double tau = bf_row_sum(M[li * LD + li]);
+    if (tau > 0.0) {
+      double scale = 1.0 / tau;  // M holds the current matrix / scale
+      for (int k = 0; k < BF_MAX_SQ; ++k) {
+        const double sc2 = scale * scale;
+        double m[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) m[q] = M[(4 * q + lk) * LD + li];
+        acc = bf_d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(m[q], m[q], acc, 0, 0, 0);
+        bf_wave_fence();
+        bf_store_tile(M, LD, 0, 0, li, lk, acc, sc2);
+        bf_wave_fence();
+        const double tr2 = bf_row_sum(M[li * LD + li]);
+        scale = 1.0 / tr2;
+        if (tr2 >= 1.0 - 16.0 * DBL_EPSILON) break;  // tr(M^2) = 1: M is rank one
+      }
+    }
+    // v: the column of largest diagonal entry, normalised
+    int jb = 0;
+    for (int j = 1; j < 16; ++j)
+      if (M[j * LD + j] > M[jb * LD + jb]) jb = j;
+    double vn = 0.0;
+    for (int j = 0; j < 16; ++j) vn = fma(M[j * LD + jb], M[j * LD + jb], vn);
+    const double vs = vn > 0.0 ? 1.0 / sqrt(vn) : 0.0;
+    if (tid < 16) v[tid] = M[tid * LD + jb] * vs;
+    if (tid == 0) s_vn = vn;
+  }
+  __syncthreads();
+  // w = W0 v, sigma = |w|
+  double w = 0.0;
+  if (tid < D)
+    for (int j = 0; j < 16; ++j) w = fma(W[tid * LD + j], v[j], w);
+  const double part = wave_sum(w * w);
+  if (lane == 0) red[tid >> 6] = part;
+  __syncthreads();
+  double lam = 0.0;
+  for (int q = 0; q < NT / 64; ++q) lam += red[q];
+  double kl = 0.0, kc = 0.0;
+  if (lam > 0.0 && s_vn > 0.0) {
+    const double sigma = sqrt(lam), rs = sqrt(sigma);
+    kl = 1.0 / rs;
+    kc = rs;
+  }
+  if (tid < D) bf_put_len(s, tr, t, tid, w * kl);
+  if (tid < 16) bf_put_col(s, tr, t, tid, v[tid] * kc);
+}
+
 // The root node (the whole matrix, row-major: value (r, c) at r n + c) from
 // the caller's matrix with its columns permuted: root(r, c) = A(r, pinv[c])
 // (pinv == nullptr: no permutation).  Column-major A goes through 32 x 32
@@ -681,8 +878,24 @@ void bfly_split(const BflyStep& s, hipStream_t st) {
   } else {
     FH_CHECK(bfly_block_fits(s.logBx, s.logBy), "butterfly: block too large for one workgroup's LDS");
     const size_t lds = bfly_block_lds_bytes(s.logBx, s.logBy);
-    const int logd = std::min(s.logBx, s.logBy);
-    if (bfly_use_mfma(logd)) {
+    const int logd = std::min(s.logBx, s.logBy), logD = std::max(s.logBx, s.logBy);
+    if (logd == 2 && logD <= 4) {
+      const dim3 grid((s.n + 63) / 64);
+      if (logD == 2)
+        hipLaunchKernelGGL(k_bfly_gram4<2>, grid, dim3(64), 0, st, s);
+      else if (logD == 3)
+        hipLaunchKernelGGL(k_bfly_gram4<3>, grid, dim3(64), 0, st, s);
+      else
+        hipLaunchKernelGGL(k_bfly_gram4<4>, grid, dim3(64), 0, st, s);
+    } else if (bfly_use_mfma(logd) && logd == 4 && logD <= 8) {
+      switch (logD) {
+        case 4: hipLaunchKernelGGL(k_bfly_gram16<4>, dim3(s.n), dim3(64), 0, st, s); break;
+        case 5: hipLaunchKernelGGL(k_bfly_gram16<5>, dim3(s.n), dim3(64), 0, st, s); break;
+        case 6: hipLaunchKernelGGL(k_bfly_gram16<6>, dim3(s.n), dim3(64), 0, st, s); break;
+        case 7: hipLaunchKernelGGL(k_bfly_gram16<7>, dim3(s.n), dim3(BF_THREADS), 0, st, s); break;
+        default: hipLaunchKernelGGL(k_bfly_gram16<8>, dim3(s.n), dim3(BF_THREADS), 0, st, s); break;
+      }
+    } else if (bfly_use_mfma(logd)) {
       // upper 16 x 16 tiles per wave: 1 (d <= 32), 3 (d = 64), 9 (d = 128)
       if (logd <= 5)
         hipLaunchKernelGGL(k_bfly_gram_mfma<1>, dim3(s.n), dim3(BF_THREADS), lds, st, s);

@@ -300,3 +300,25 @@ def test_bbtree_order_32768(gpu):
     X = rng.standard_normal((n, 4))
     Y, R = F @ X, B @ X
     assert np.linalg.norm(Y - R) <= 1e-12 * np.linalg.norm(R)
+
+
+@pytest.mark.parametrize("n", [16, 32, 64, 128, 256, 512, 1024, 2048, 4096])
+@pytest.mark.parametrize("scale", [1.0, 1e-70, 1e70])  # the first square holds entries of scale^4: 1e-308 .. 1e308
+def test_small_side_blocks(gpu, n, scale):
+    """Blocks with a side of 4 (a block per lane) and 16 (in LDS): each of bbtree's splits of these orders, against
+    the oracle up to 1024 and, with zero rows and columns, without NaN; the same bits for the matrix read in place
+    (row-major on the GPU) and copied (column-major)."""
+    torch = pytest.importorskip("torch")
+    rng = np.random.default_rng(n)
+    M = rng.standard_normal((n, n)) * scale
+    F = fact.butterfly(M, type="bbtree")
+    if n <= 1024 and scale == 1.0:
+        _compare(F, ob.butterfly(M, ob.BALANCED))
+    Md = torch.from_numpy(M).cuda()
+    G = fact.butterfly(Md, type="bbtree")
+    assert np.array_equal(Md.cpu().numpy(), M)
+    for a, b in zip(_host(F), _host(G)):
+        assert np.array_equal(_dense(a), _dense(b))
+    M[: n // 2] = 0.0
+    M[:, n // 4: n // 2] = 0.0
+    assert all(np.isfinite(_dense(f)).all() for f in _host(fact.butterfly(M, type="bbtree")))
