@@ -1158,7 +1158,7 @@ __device__ __forceinline__ void bspmm_body(const SpmmCtx<T>& C) {
 }
 
 template <class T>
-__global__ __launch_bounds__(256, 4) void k_bspmm(const BSpmmJob<T>* __restrict__ jobs, const int3* __restrict__ tiles,
+__global__ __launch_bounds__(256, sizeof(T) == 4 ? 4 : 3) void k_bspmm(const BSpmmJob<T>* __restrict__ jobs, const int3* __restrict__ tiles,
                                                   BScal sc, int ntiles, int per) {
   constexpr int ENT = SPMM_LDS_BYTES / (sizeof(int) + sizeof(T));
   __shared__ int s_p[BATCH_NMAX + 1];
