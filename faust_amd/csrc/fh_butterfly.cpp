@@ -143,15 +143,6 @@ std::vector<BNodeP> bfly_directional(Bfly& B, bool right) {
   return facs;
 }
 
-// CSR of a leaf [i, i+1) (2 entries per row), built on the device; with
-// colmap / colinv (device) its columns are relabelled by colmap and sorted
-// within each row
-DMatP leaf_csr(const BNode& nd, int n, int L, const int* colmap, const int* colinv, hipStream_t st) {
-  auto M = std::make_shared<DMat>();
-  bfly_leaf_csr((const double*)nd.v.p, n, L - nd.b, colmap, colinv, *M, st);
-  return M;
-}
-
 DMatP leaf_dense(const BNode& nd, int n, int L, hipStream_t st) {
   auto M = std::make_shared<DMat>();
   M->kind = K_DENSE;
@@ -221,18 +212,23 @@ fh_faust_s* butterfly_run(const double* A, size_t lda, int row_major, int n, int
   for (int k = 0; k < B.L; ++k)
     FH_CHECK(nodes[k]->a == k && nodes[k]->b == k + 1, "butterfly: factor out of order");
   auto r = std::make_unique<fh_faust_s>();
+  // CSR leaves (2 entries per row) built on the device, all by one launch
+  std::vector<BflyLeaf> leaves;
   for (int k = 0; k < B.L; ++k) {
-    const bool last = k == B.L - 1;
-    if (last && perm && mul_perm) {
+    const bool relabel = k == B.L - 1 && perm && mul_perm;
+    if (relabel || dir == FH_BUTTERFLY_BBTREE) {
       // (F P)[:, c] = F[:, perm[c]]: column j of the last factor moves to pinv[j]
-      r->f.push_back(leaf_csr(*nodes[k], n, B.L, (const int*)pinv_dev.p, (const int*)perm_dev.p, st));
-    } else if (dir == FH_BUTTERFLY_BBTREE) {
-      r->f.push_back(leaf_csr(*nodes[k], n, B.L, nullptr, nullptr, st));
+      // (its columns are relabelled and sorted within each row)
+      r->f.push_back(std::make_shared<DMat>());
+      leaves.push_back({nodes[k]->values(), B.L - nodes[k]->b, relabel ? (const int*)pinv_dev.p : nullptr,
+                        relabel ? (const int*)perm_dev.p : nullptr, r->f.back().get()});
     } else {
       r->f.push_back(leaf_dense(*nodes[k], n, B.L, st));
+      nodes[k].reset();
     }
-    nodes[k].reset();
   }
+  bfly_leaves_csr(leaves, n, st);
+  nodes.clear();
   if (perm && !mul_perm) {
     // P as a factor of its own: row perm[i] holds a 1 at column i
     std::vector<int32_t> rp(n + 1), ci(n);
