@@ -1089,9 +1089,14 @@ static const double* pl_x0() {
   const std::vector<double>& x = power_x0(PL_ROWS);
   std::lock_guard<std::mutex> lk(mu);
   if (!dx[dev]) {
-    double* p = static_cast<double*>(dev_alloc(sizeof(double) * PL_ROWS));  // held to process end
-    FH_HIP(hipMemcpy(p, x.data(), sizeof(double) * PL_ROWS, hipMemcpyHostToDevice));
-    dx[dev] = p;
+    // held to process end, and not a block of the pool: work queued on the
+    // caller's stream may still use one, and this copy does not wait for it
+    void* p = nullptr;
+    FH_HIP(hipMalloc(&p, sizeof(double) * PL_ROWS));
+    const hipError_t e = hipMemcpy(p, x.data(), sizeof(double) * PL_ROWS, hipMemcpyHostToDevice);
+    if (e != hipSuccess) (void)hipFree(p);
+    FH_HIP(e);
+    dx[dev] = static_cast<double*>(p);
   }
   return dx[dev];
 }
