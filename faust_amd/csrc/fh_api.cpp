@@ -152,19 +152,6 @@ static bool chain_csr_ops(const std::vector<DMatP>& f, char op, std::vector<Chai
   return true;
 }
 
-size_t faust_ws_need_rm_f64(const std::vector<DMatP>& f, char op, int p, int* nbuf) {
-  std::vector<ChainCsrOp> ops;
-  int widest;
-  double mean;
-  if (f.empty() || p < RM_MIN_COLS || !chain_csr_ops(f, op, ops, &widest, &mean)) return 0;
-  const int in_rows = (op == 'N') ? f.back()->n : f.front()->m;
-  if (!csr_rm_fits(ops, in_rows, p)) return 0;
-  int r = in_rows;  // the last factor's output is Y
-  for (size_t i = 0; i + 1 < ops.size(); ++i) r = std::max(r, ops[i].rows);
-  *nbuf = std::min(2, (int)f.size());
-  return sizeof(double) * csr_rm_size(r, p);
-}
-
 // Bytes of each of the (at most two) intermediates of an FP64 chain product;
 // *nbuf: how many of them the product uses.
 size_t faust_ws_need_f64(const std::vector<DMatP>& f, char op, int p, int* nbuf) {
@@ -195,18 +182,33 @@ ChainWs faust_ws_grow(DBuf* ws, size_t need, int nbuf, hipStream_t st, DBuf* ctl
   return w;
 }
 
+// The same with room for a form that takes more (want bytes in want_nbuf
+// buffers, 0: none such) where that is to be had without refusing the call:
+// under capture and when memory is short the product keeps to `need`.
+// short_of: the least that could not be had so far, which is not asked for again.
+ChainWs faust_ws_take(DBuf* ws, size_t need, int nbuf, size_t want, int want_nbuf, size_t* short_of, hipStream_t st,
+                      DBuf* ctl) {
+  if (want > 0) {
+    want = std::max(want, need);
+    want_nbuf = std::max(want_nbuf, nbuf);
+    bool room = true;
+    for (int b = 0; b < want_nbuf; ++b) room = room && ws[b].bytes >= want;
+    if (room) return faust_ws_grow(ws, want, want_nbuf, st, ctl);
+    if (want < *short_of && !stream_capturing(st)) {
+      try {
+        return faust_ws_grow(ws, want, want_nbuf, st, ctl);
+      } catch (const Error&) {
+        (void)hipGetLastError();
+        *short_of = want;
+      }
+    }
+  }
+  return faust_ws_grow(ws, need, nbuf, st, ctl);
+}
+
 // Y = op(F) X for an FP64 chain; X, Y col-major with ld = rows; ws holds the
 // intermediates (faust_ws_need_f64 bytes each).
 // ---------------------------------------------------------------- autotune
-// Execution forms of an FP64 CSR chain, all with the same bits: one launch
-// per factor, the staged one-launch chain (wc columns per workgroup), the
-// prefetched one-launch chain (wc columns, pf entries per row ahead), one
-// launch per factor on row-major intermediates.
-struct ChainForm {
-  int kind;  // 0 per factor, 1 staged, 2 prefetched, 3 row-major
-  int wc, pf;
-};
-
 namespace {
 std::mutex g_tune_mu;
 std::map<std::string, ChainForm> g_tune;  // chain signature -> quickest form measured
@@ -249,18 +251,63 @@ static std::string chain_sig(char op, int p, int in_rows, const std::vector<Chai
   return k;
 }
 
-// Y = op(F) X with the FP64 chain.  AUTO mode on an all-CSR chain uses the
-// form measured quickest for this chain signature (measured on its first
-// call outside graph capture: every candidate once untimed, then the minimum
-// of three timings of five back-to-back products, HIP events on the launch
-// stream; the default form stays unless another is at least 3% quicker);
-// otherwise, and when
-// measuring is off or impossible, the prefetched one-launch chain where the
-// shape allows it, the staged one where the planner takes it, else one launch
-// per factor.  `tune` false (allocation-free callers) never measures.
-void faust_multiply_f64(const std::vector<DMatP>& f, char op, const double* X, int p, double* Y, hipStream_t st,
-                        const ChainWs& ws, FaustTimers* tm, int* launches, bool tune) {
+// AUTO mode on an all-CSR chain uses the form measured quickest for this chain
+// signature (measured on its first call outside graph capture: every candidate
+// once untimed, then the minimum of three timings of five back-to-back
+// products, HIP events on the launch stream; the default form stays unless
+// another is at least 3% quicker); otherwise, and when measuring is off or
+// impossible, the prefetched one-launch chain where the shape allows it (8
+// entries ahead unless the rows are long on average and some exceed 8), else
+// row-major intermediates for blocks of columns, else the staged chain where
+// the planner takes it, else one launch per factor.  `tune` false
+// (allocation-free callers) never measures.
+ChainPlan64 chain_plan_f64(const std::vector<DMatP>& f, char op, int p, bool tune, hipStream_t st) {
   FH_CHECK(!f.empty(), "Faust::multiply: empty Faust");
+  ChainPlan64 P;
+  P.need = faust_ws_need_f64(f, op, p, &P.nbuf);
+  double mean_max = 0.0;
+  P.csr = chain_csr_ops(f, op, P.ops, &P.widest, &mean_max);
+  if (!P.csr) return P;
+  P.in_rows = (op == 'N') ? f.back()->n : f.front()->m;
+  const char* e_pf = getenv("FH_CHAIN_PF");
+  const bool plain = mul_mode() == FH_MUL_AUTO && !getenv("FH_CHAIN_FUSED") && !(e_pf && e_pf[0] == '0');
+  const int pwc = csr_chain_pf_plan_f64(P.ops, P.in_rows, p);
+  const int swc = pwc > 0 ? 0 : csr_chain_plan_f64(P.ops, P.in_rows, p);
+  if (pwc > 0)
+    P.def = {2, pwc, (P.widest <= 8 || mean_max <= 4.0) ? 8 : 16};
+  else if (swc > 0)
+    P.def = {1, swc, 0};
+  const bool tunable = plain && autotune_on();
+  if (tunable) {
+    P.key = chain_sig(op, p, P.in_rows, P.ops);
+    std::lock_guard<std::mutex> lk(g_tune_mu);
+    auto it = g_tune.find(P.key);
+    if (it != g_tune.end()) {
+      P.form = it->second;
+      P.known = true;
+    }
+  }
+  P.measure = tunable && !P.known && tune && !stream_capturing(st);
+  // chains that fit the one-launch form keep to that and to one launch per factor
+  if (plain && csr_rm_fits(P.ops, P.in_rows, p) && !csr_chain_pf_fits(P.ops, P.in_rows, p)) {
+    int nnz_max = 0;
+    for (const auto& o : P.ops) nnz_max = std::max(nnz_max, o.nnz);
+    P.rm_rule = (int64_t)nnz_max * p >= RM_TERMS_DEFAULT;
+    if (P.known ? P.form.kind == 3 : P.measure || P.rm_rule) {
+      int r = P.in_rows;  // the last factor's output is Y
+      for (size_t i = 0; i + 1 < P.ops.size(); ++i) r = std::max(r, P.ops[i].rows);
+      P.rm_nbuf = std::min(2, (int)f.size());
+      P.rm_need = sizeof(double) * csr_rm_size(r, p);
+    }
+  }
+  return P;
+}
+
+// Y = op(F) X for an FP64 chain; X, Y col-major with ld = rows; ws holds the
+// intermediates (plan.need bytes each; the row-major form runs where it holds
+// plan.rm_need).
+ChainForm faust_multiply_f64(const std::vector<DMatP>& f, char op, const double* X, int p, double* Y, hipStream_t st,
+                             const ChainPlan64& plan, const ChainWs& ws, FaustTimers* tm, int* launches) {
   const int J = (int)f.size();
   double* const t1 = static_cast<double*>(ws.p[0]);
   double* const t2 = static_cast<double*>(ws.p[1]);
@@ -289,15 +336,14 @@ void faust_multiply_f64(const std::vector<DMatP>& f, char op, const double* X, i
       in_rows = out_rows;
     }
   };
+  if (!plan.csr) {
+    per_factor(tm);
+    if (launches) *launches = J;
+    return {0, 0, 0};
+  }
 
-  // the chain as op'd CSR factors in application order, when it is one
-  std::vector<ChainCsrOp> ops;
-  int widest = 0;
-  double mean_max = 0.0;
-  const bool ok = chain_csr_ops(f, op, ops, &widest, &mean_max);
-  int nnz_max = 0;
-  for (const auto& o : ops) nnz_max = std::max(nnz_max, o.nnz);
-  const int out_rows = ok ? ops.back().rows : 0;
+  const std::vector<ChainCsrOp>& ops = plan.ops;
+  const int out_rows = ops.back().rows;
   auto run = [&](const ChainForm& c, FaustTimers* tmr) {
     if (c.kind == 0) {
       per_factor(tmr);
@@ -327,97 +373,60 @@ void faust_multiply_f64(const std::vector<DMatP>& f, char op, const double* X, i
       csr_chain_pf_run_f64(ops, in_rows0, c.wc, c.pf, X, in_rows0, p, Y, out_rows, 1.0, 0.0, st);
     if (tmr) tmr->end(0, st);
   };
-  auto done = [&](const ChainForm& c) {
-    if (launches) *launches = c.kind == 0 ? J : c.kind == 3 ? J + 1 : 1;
-  };
 
-  if (ok) {
-    // default form: prefetched (8 entries ahead unless the rows are long on
-    // average and some exceed 8), else row-major intermediates for blocks of
-    // columns, else the staged plan, else per factor
-    int rm_nbuf = 0;
-    const size_t rm_need = faust_ws_need_rm_f64(f, op, p, &rm_nbuf);
-    const bool rm_fits = rm_need > 0 && ws.cap >= rm_need && t1 && (rm_nbuf < 2 || t2);
-    const bool one_launch_off = getenv("FH_CHAIN_FUSED") || (getenv("FH_CHAIN_PF") && getenv("FH_CHAIN_PF")[0] == '0');
-    // (chains that fit the one-launch form keep to that and to one launch per factor)
-    const bool rm_auto =
-        rm_fits && mul_mode() == FH_MUL_AUTO && !one_launch_off && !csr_chain_pf_fits(ops, in_rows0, p);
-    ChainForm def{0, 0, 0};
-    const int pwc = csr_chain_pf_plan_f64(ops, in_rows0, p);
-    const int swc = pwc > 0 ? 0 : csr_chain_plan_f64(ops, in_rows0, p);
-    if (pwc > 0)
-      def = {2, pwc, (widest <= 8 || mean_max <= 4.0) ? 8 : 16};
-    else if (rm_auto && (int64_t)nnz_max * p >= RM_TERMS_DEFAULT)
-      def = {3, 0, 0};
-    else if (swc > 0)
-      def = {1, swc, 0};
-    ChainForm use = def;
-    const bool tunable = mul_mode() == FH_MUL_AUTO && autotune_on() && !one_launch_off;
-    if (tunable) {
-      const std::string key = chain_sig(op, p, in_rows0, ops);
-      bool known = false;
-      {
-        std::lock_guard<std::mutex> lk(g_tune_mu);
-        auto it = g_tune.find(key);
-        if (it != g_tune.end()) {
-          use = it->second;
-          known = true;
-          if (use.kind == 3 && !rm_fits) use = def;  // a caller whose workspace is too small for it
-        }
+  const bool rm_fits = plan.rm_need > 0 && ws.cap >= plan.rm_need && t1 && (plan.rm_nbuf < 2 || t2);
+  const ChainForm def = plan.rm_rule && rm_fits ? ChainForm{3, 0, 0} : plan.def;
+  ChainForm use = plan.known && (plan.form.kind != 3 || rm_fits) ? plan.form : def;
+  // a choice made without the row-major form, for want of room, is not kept
+  if (plan.measure && (plan.rm_need == 0 || rm_fits)) {
+    // the default form first: another replaces the quickest so far only
+    // when it is at least 3% quicker, so near-ties keep the default and
+    // the choice does not flip between processes on timing noise
+    std::vector<ChainForm> cand{def};
+    auto add = [&](ChainForm c) {
+      if (c.kind != def.kind || c.wc != def.wc || c.pf != def.pf) cand.push_back(c);
+    };
+    add({0, 0, 0});
+    if (rm_fits) add({3, 0, 0});
+    const int fwc = csr_chain_fit_wc(ops, in_rows0, p);
+    if (fwc > 0) add({1, fwc, 0});
+    if (csr_chain_pf_fits(ops, in_rows0, p))
+      for (int pf : {8, 16}) {
+        if (pf == 16 && plan.widest <= 8) continue;
+        for (int wc : {1, 2, 4})
+          if (wc == 1 || (p + wc - 1) / wc >= 8) add({2, wc, pf});
       }
-      if (!known && tune && !stream_capturing(st)) {
-        // the default form first: another replaces the quickest so far only
-        // when it is at least 3% quicker, so near-ties keep the default and
-        // the choice does not flip between processes on timing noise
-        std::vector<ChainForm> cand{def};
-        auto add = [&](ChainForm c) {
-          if (c.kind != def.kind || c.wc != def.wc || c.pf != def.pf) cand.push_back(c);
-        };
-        add({0, 0, 0});
-        if (rm_auto) add({3, 0, 0});
-        const int fwc = csr_chain_fit_wc(ops, in_rows0, p);
-        if (fwc > 0) add({1, fwc, 0});
-        if (csr_chain_pf_fits(ops, in_rows0, p))
-          for (int pf : {8, 16}) {
-            if (pf == 16 && widest <= 8) continue;
-            for (int wc : {1, 2, 4})
-              if (wc == 1 || (p + wc - 1) / wc >= 8) add({2, wc, pf});
-          }
-        hipEvent_t e0, e1;
-        FH_HIP(hipEventCreate(&e0));
-        FH_HIP(hipEventCreate(&e1));
-        float best_ms = 1e30f;
-        // each timing covers five back-to-back products: the steady state a
-        // caller's loop or graph sees
-        for (const ChainForm& c : cand) {
-          run(c, nullptr);
-          float m = 1e30f;
-          for (int rep = 0; rep < 3; ++rep) {
-            FH_HIP(hipEventRecord(e0, st));
-            for (int r = 0; r < 5; ++r) run(c, nullptr);
-            FH_HIP(hipEventRecord(e1, st));
-            FH_HIP(hipEventSynchronize(e1));
-            float ms = 0.f;
-            FH_HIP(hipEventElapsedTime(&ms, e0, e1));
-            m = std::min(m, ms);
-          }
-          if (m < 0.97f * best_ms) {
-            best_ms = m;
-            use = c;
-          }
-        }
-        (void)hipEventDestroy(e0);
-        (void)hipEventDestroy(e1);
-        std::lock_guard<std::mutex> lk(g_tune_mu);
-        g_tune[key] = use;
+    hipEvent_t e0, e1;
+    FH_HIP(hipEventCreate(&e0));
+    FH_HIP(hipEventCreate(&e1));
+    float best_ms = 1e30f;
+    // each timing covers five back-to-back products: the steady state a
+    // caller's loop or graph sees
+    for (const ChainForm& c : cand) {
+      run(c, nullptr);
+      float m = 1e30f;
+      for (int rep = 0; rep < 3; ++rep) {
+        FH_HIP(hipEventRecord(e0, st));
+        for (int r = 0; r < 5; ++r) run(c, nullptr);
+        FH_HIP(hipEventRecord(e1, st));
+        FH_HIP(hipEventSynchronize(e1));
+        float ms = 0.f;
+        FH_HIP(hipEventElapsedTime(&ms, e0, e1));
+        m = std::min(m, ms);
+      }
+      if (m < 0.97f * best_ms) {
+        best_ms = m;
+        use = c;
       }
     }
-    run(use, tm);
-    done(use);
-    return;
+    (void)hipEventDestroy(e0);
+    (void)hipEventDestroy(e1);
+    std::lock_guard<std::mutex> lk(g_tune_mu);
+    g_tune[plan.key] = use;
   }
-  per_factor(tm);
-  if (launches) *launches = J;
+  run(use, tm);
+  if (launches) *launches = use.kind == 0 ? J : use.kind == 3 ? J + 1 : 1;
+  return use;
 }
 
 void autotune_clear() {
@@ -772,18 +781,38 @@ int fh_faust_multiply(fh_faust_t F, char op, const void* X, int p, void* Y, void
   }
   FH_CHECK(X && Y, "null argument");
   hipStream_t st = (hipStream_t)stream;
-  int nbuf = 0;
   if (F->f.front()->dtype == FH_F64) {
-    size_t need = faust_ws_need_f64(F->f, op, p, &nbuf);
-    int rm_nbuf = 0;
-    need = std::max(need, faust_ws_need_rm_f64(F->f, op, p, &rm_nbuf));
-    const ChainWs ws = faust_ws_grow(F->ws, need, std::max(nbuf, rm_nbuf), st);
-    faust_multiply_f64(F->f, op, (const double*)X, p, (double*)Y, st, ws, &F->timers, &F->last_launches);
+    ChainPlan64 pl = chain_plan_f64(F->f, op, p, true, st);
+    if (F->f.size() == 1 && pl.rm_need > 0) {
+      // a one-factor product uses no workspace but the row-major form's copy
+      // of X: that stays out of captured graphs and belongs to the stream that
+      // had it first, and products on other streams run without it
+      const bool mine = st != hipStreamPerThread && !stream_capturing(st) && (!F->ws_owned || F->ws_stream == st);
+      if (mine) {
+        F->ws_owned = true;
+        F->ws_stream = st;
+      } else {
+        pl.rm_need = 0;
+        pl.measure = false;
+      }
+    }
+    const size_t had[2] = {F->ws[0].bytes, F->ws[1].bytes};
+    const ChainWs ws = faust_ws_take(F->ws, pl.need, pl.nbuf, pl.rm_need, pl.rm_nbuf, &F->ws_short, st);
+    const ChainForm ran =
+        faust_multiply_f64(F->f, op, (const double*)X, p, (double*)Y, st, pl, ws, &F->timers, &F->last_launches);
+    if (pl.measure && pl.rm_need > 0 && ran.kind != 3)
+      // the row-major form was measured and not kept: nor is its room
+      for (int b = 0; b < 2; ++b) {
+        const size_t keep = std::max(had[b], b < pl.nbuf ? pl.need : 0);
+        if (F->ws[b].bytes <= keep) continue;
+        FH_HIP(hipStreamSynchronize(st));
+        F->ws[b].alloc(keep);
+      }
   } else {
     const std::vector<DMatP> f = fp32_chain_factors(F->f, st);
     const bool act_f32 = F->act_dtype == FH_F32;
+    int nbuf = 0, tbuf = 0;
     size_t need = faust_ws_need_mixed(f, op, p, &nbuf, act_f32);
-    int tbuf = 0;
     if (act_f32)
       need = std::max(need, faust_ws_need_f32_tiled(f, op, p, &tbuf));
     else if (f.front()->kind == K_CSR)

@@ -80,6 +80,9 @@ struct FaustTimers {
 struct fh_faust_s {
   std::vector<fh::DMatP> f;
   fh::DBuf ws[2];         // ping-pong activations
+  bool ws_owned = false;  // a one-factor product has used ws[0], on ws_stream
+  hipStream_t ws_stream = nullptr;
+  size_t ws_short = SIZE_MAX;  // bytes of optional workspace that were not to be had
   fh::DBuf ctl;           // control block of the one-launch BSR chain
   int last_launches = 0;  // kernel launches of the last product
   int mul_mode = 0;       // FH_MUL_*
@@ -112,10 +115,36 @@ struct ChainWs {
   size_t cap = 0;  // bytes of each non-null p[]
 };
 size_t faust_ws_need_f64(const std::vector<DMatP>& f, char op, int p, int* nbuf);
-// The same for the form with row-major intermediates (X's copy included);
-// 0 when the chain or its shape does not take it.
-size_t faust_ws_need_rm_f64(const std::vector<DMatP>& f, char op, int p, int* nbuf);
 ChainWs faust_ws_grow(DBuf* ws, size_t need, int nbuf, hipStream_t st, DBuf* ctl = nullptr);
+ChainWs faust_ws_take(DBuf* ws, size_t need, int nbuf, size_t want, int want_nbuf, size_t* short_of, hipStream_t st,
+                      DBuf* ctl = nullptr);
+// Execution forms of an FP64 CSR chain, all with the same bits: one launch
+// per factor, the staged one-launch chain (wc columns per workgroup), the
+// prefetched one-launch chain (wc columns, pf entries per row ahead), one
+// launch per factor on row-major intermediates.
+struct ChainForm {
+  int kind;  // 0 per factor, 1 staged, 2 prefetched, 3 row-major
+  int wc, pf;
+};
+// What an FP64 product is going to do, worked out once: chain_plan_f64 before
+// the workspace is sized, faust_multiply_f64 by it.
+struct ChainPlan64 {
+  size_t need = 0;  // bytes of each of nbuf column-major intermediates
+  int nbuf = 0;
+  // the row-major form's (X's copy included); 0 unless this product runs it,
+  // given the room, or measures it
+  size_t rm_need = 0;
+  int rm_nbuf = 0;
+  bool csr = false;               // every factor is FP64 CSR; what follows is set only then
+  std::vector<ChainCsrOp> ops;    // op'd factors in application order
+  int in_rows = 0, widest = 0;    // widest: the longest op'd row, 1 << 30 when unknown
+  bool rm_rule = false;           // row-major is the unmeasured choice
+  bool measure = false;           // this call times the forms
+  bool known = false;             // they have been timed: form
+  ChainForm def{0, 0, 0}, form{0, 0, 0};  // def: the unmeasured choice among the other forms
+  std::string key;                // what the timing is kept under
+};
+ChainPlan64 chain_plan_f64(const std::vector<DMatP>& f, char op, int p, bool tune, hipStream_t st);
 // Forgets the forms measured by the chain autotuners (FP64 and BSR / FP32 CSR).
 void autotune_clear();
 // Shared by the autotuners: FH_AUTOTUNE=0 turns measuring off; a stream being
@@ -125,8 +154,10 @@ bool autotune_on();
 bool stream_capturing(hipStream_t st);
 bool autotune_get_mode(const std::string& key, int* mode);
 void autotune_put_mode(const std::string& key, int mode);
-void faust_multiply_f64(const std::vector<DMatP>& f, char op, const double* X, int p, double* Y, hipStream_t st,
-                        const ChainWs& ws, FaustTimers* tm = nullptr, int* launches = nullptr, bool tune = true);
+// returns the form it ran in (kind 0 for chains that are not all CSR)
+ChainForm faust_multiply_f64(const std::vector<DMatP>& f, char op, const double* X, int p, double* Y, hipStream_t st,
+                             const ChainPlan64& plan, const ChainWs& ws, FaustTimers* tm = nullptr,
+                             int* launches = nullptr);
 DMatP faust_get_product_f64(const std::vector<DMatP>& f, hipStream_t st);
 double faust_spectral_norm_f64(const std::vector<DMatP>& f, int maxit, double thr, int* flag, hipStream_t st,
                                bool count = true);

@@ -80,17 +80,21 @@ extern "C" int fh_faust_multiply_noalloc(fh_faust_t F, char op, const void* X, i
       }
   int nbuf = 0;
   const bool act_f32 = F->act_dtype == FH_F32;
-  size_t need = f64 ? faust_ws_need_f64(f, op, p, &nbuf) : faust_ws_need_mixed(f, op, p, &nbuf, act_f32);
+  ChainPlan64 pl;
+  size_t need;
   if (f64) {
-    // room for the row-major form too where the array has it; without it the
-    // product runs in the forms that fit
-    int rm_nbuf = 0;
-    const size_t rm = std::max(need, faust_ws_need_rm_f64(f, op, p, &rm_nbuf));
-    rm_nbuf = std::max(rm_nbuf, nbuf);
-    if ((size_t)rm_nbuf * align256(rm) <= kScratchBytes) {
+    pl = chain_plan_f64(f, op, p, false, st);
+    need = pl.need;
+    nbuf = pl.nbuf;
+    // room for the row-major form too where the array has it (without it the
+    // product runs in the forms that fit); a one-factor product uses no scratch
+    const size_t rm = std::max(need, pl.rm_need);
+    if (pl.rm_need > 0 && f.size() > 1 && (size_t)pl.rm_nbuf * align256(rm) <= kScratchBytes) {
       need = rm;
-      nbuf = rm_nbuf;
+      nbuf = pl.rm_nbuf;
     }
+  } else {
+    need = faust_ws_need_mixed(f, op, p, &nbuf, act_f32);
   }
   if (!f64 && (act_f32 || f.front()->kind == K_CSR)) {
     // likewise for the padded layouts of FP32 intermediates
@@ -112,7 +116,7 @@ extern "C" int fh_faust_multiply_noalloc(fh_faust_t F, char op, const void* X, i
   const ChainWs ws{{nbuf > 0 ? base + ctl_bytes : nullptr, nbuf > 1 ? base + ctl_bytes + slot : nullptr},
                    bsr ? reinterpret_cast<int*>(base) : nullptr, need};
   if (f64)
-    faust_multiply_f64(f, op, (const double*)X, p, (double*)Y, st, ws, nullptr, &F->last_launches, false);
+    faust_multiply_f64(f, op, (const double*)X, p, (double*)Y, st, pl, ws, nullptr, &F->last_launches);
   else
     F->last_launches = faust_multiply_mixed(f, op, X, p, Y, st, ws, nullptr, act_f32, false);
   FH_API_END

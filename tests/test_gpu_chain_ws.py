@@ -1,0 +1,136 @@
+"""The workspace of FP64 chain products: the row-major form's room is asked for
+only where the form can run, is never needed for a call to be accepted, and a
+one-factor Faust shares none between streams, captured graphs or with the
+allocation-free entry point."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+import faust_amd
+import oracle
+from faust_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+
+def _launches(F):
+    n = C.c_int()
+    _lib.check(_lib.lib().fh_faust_last_launches(F.h, C.byref(n)))
+    return n.value
+
+
+def _capture(call):
+    """call() in a graph of its own, on a side stream that nothing has run on."""
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(s):
+        g.capture_begin(capture_error_mode="thread_local")
+        try:
+            call()
+        finally:
+            g.capture_end()
+    torch.cuda.current_stream().wait_stream(s)
+    return g
+
+
+def _replays_right(g, facs, op, X, Y):
+    for _ in range(3):
+        X.copy_(torch.randn(X.shape, dtype=X.dtype, device="cuda"))
+        g.replay()
+        torch.cuda.synchronize()
+        want = oracle.chain_multiply(facs, np.asfortranarray(X.cpu().numpy().T), op)
+        assert np.array_equal(Y.cpu().numpy().T, want)
+
+
+@pytest.mark.parametrize("autotune", ["0", "1"])
+@pytest.mark.parametrize("p", [12, 300])  # below and above the rule's line
+def test_one_factor_captured_first(gpu, monkeypatch, p, autotune):
+    monkeypatch.setenv("FH_AUTOTUNE", autotune)
+    rng = np.random.default_rng(p)
+    facs = [faust_amd.rand_csr(3001, 2501, 9, rng)]
+    F, W = faust_amd.Faust(facs), faust_amd.Faust(facs)
+    for G, V, op, n, m in ((F, W, "N", 2501, 3001), (F.T, W.T, "T", 3001, 2501)):
+        X = torch.zeros((p, n), dtype=torch.float64, device="cuda")
+        Y = torch.empty((p, m), dtype=torch.float64, device="cuda")
+        V.matmul_device(X, Y)  # the kernels are loaded, the forms measured; G's handle has no workspace yet
+        g = _capture(lambda: G.matmul_device(X, Y))
+        assert _launches(G) == 1
+        _replays_right(g, facs, op, X, Y)
+
+
+def test_capture_keeps_to_the_room_there_is(gpu, monkeypatch):
+    # a chain warmed up in the form that one launch per factor takes: the row-major one's room is not there
+    monkeypatch.setenv("FH_AUTOTUNE", "0")
+    rng = np.random.default_rng(2)
+    facs = [faust_amd.rand_csr(3001, 3001, 9, rng) for _ in range(2)]
+    F = faust_amd.Faust(facs)
+    X = torch.randn((64, 3001), dtype=torch.float64, device="cuda")
+    Y = torch.empty_like(X)
+    monkeypatch.setenv("FH_CHAIN_FUSED", "0")
+    F.matmul_device(X, Y)
+    assert _launches(F) == 2
+    monkeypatch.delenv("FH_CHAIN_FUSED")
+    g = _capture(lambda: F.matmul_device(X, Y))
+    assert _launches(F) == 2
+    _replays_right(g, facs, "N", X, Y)
+    F.matmul_device(X, Y)  # outside capture there is room
+    assert _launches(F) == 3
+
+
+def test_one_factor_on_two_streams(gpu, monkeypatch):
+    # the copy of X belongs to the first stream; the second runs without it, and they overlap
+    monkeypatch.setenv("FH_AUTOTUNE", "0")
+    rng = np.random.default_rng(4)
+    facs = [faust_amd.rand_csr(20001, 20001, 12, rng)]
+    F = faust_amd.Faust(facs)
+    Xs = [torch.randn((256, 20001), dtype=torch.float64, device="cuda") for _ in range(2)]
+    Ys = [torch.empty_like(X) for X in Xs]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    seen = [set(), set()]
+    for _ in range(8):
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                F.matmul_device(Xs[i], Ys[i])
+                seen[i].add(_launches(F))
+    torch.cuda.synchronize()
+    assert seen == [{2}, {1}]
+    for X, Y in zip(Xs, Ys):
+        assert np.array_equal(Y.cpu().numpy().T, oracle.chain_multiply(facs, np.asfortranarray(X.cpu().numpy().T), "N"))
+
+
+def test_one_factor_noalloc_uses_no_scratch(gpu, monkeypatch):
+    monkeypatch.setenv("FH_AUTOTUNE", "0")
+    rng = np.random.default_rng(6)
+    facs = [faust_amd.rand_csr(3001, 3001, 9, rng)]
+    F = faust_amd.Faust(facs)
+    X = torch.randn((64, 3001), dtype=torch.float64, device="cuda")
+    Y = torch.empty_like(X)
+    _lib.check(gpu.fh_faust_multiply_noalloc(F.h, b"N", C.c_void_p(X.data_ptr()), 64, C.c_void_p(Y.data_ptr()),
+                                             C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    assert _launches(F) == 1
+    assert np.array_equal(Y.cpu().numpy().T, oracle.chain_multiply(facs, np.asfortranarray(X.cpu().numpy().T), "N"))
+
+
+@pytest.mark.parametrize("mode", ["per_factor", "short"])
+def test_no_room_where_the_form_is_not_run(gpu, monkeypatch, mode):
+    # 512 MB of X: a copy of it would show in the device's free memory
+    monkeypatch.setenv("FH_AUTOTUNE", "0")
+    rng = np.random.default_rng(7)
+    n, p = (1 << 14, 1 << 12) if mode == "per_factor" else (1 << 10, 1 << 16)  # short: one-launch sizes
+    facs = [faust_amd.rand_csr(n, n, 2, rng)] * (1 if mode == "per_factor" else 2)
+    F = faust_amd.Faust(facs)
+    if mode == "per_factor":
+        _lib.check(gpu.fh_faust_set_mul_mode(F.h, 1))
+    X = torch.ones((p, n), dtype=torch.float64, device="cuda")
+    Y = torch.empty_like(X)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    F.matmul_device(X, Y)
+    torch.cuda.synchronize()
+    used = free - torch.cuda.mem_get_info()[0]
+    base = 0 if mode == "per_factor" else 8 * n * p  # one column-major intermediate
+    assert used < base + (256 << 20)
