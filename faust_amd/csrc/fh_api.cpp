@@ -812,13 +812,12 @@ int fh_faust_multiply(fh_faust_t F, char op, const void* X, int p, void* Y, void
     const std::vector<DMatP> f = fp32_chain_factors(F->f, st);
     const bool act_f32 = F->act_dtype == FH_F32;
     int nbuf = 0, tbuf = 0;
-    size_t need = faust_ws_need_mixed(f, op, p, &nbuf, act_f32);
-    if (act_f32)
-      need = std::max(need, faust_ws_need_f32_tiled(f, op, p, &tbuf));
-    else if (f.front()->kind == K_CSR)
-      need = std::max(need, faust_ws_need_f32_panels(f, op, p, &tbuf));
-    const ChainWs ws =
-        faust_ws_grow(F->ws, need, nbuf, st, (f.front()->kind == K_BSR && !act_f32) ? &F->ctl : nullptr);
+    const size_t need = faust_ws_need_mixed(f, op, p, &nbuf, act_f32);
+    const size_t padded = act_f32                        ? faust_ws_need_f32_tiled(f, op, p, &tbuf)
+                          : f.front()->kind == K_CSR ? faust_ws_need_f32_panels(f, op, p, &tbuf)
+                                                         : 0;
+    const ChainWs ws = faust_ws_take(F->ws, need, nbuf, padded, tbuf, &F->ws_short, st,
+                                     (f.front()->kind == K_BSR && !act_f32) ? &F->ctl : nullptr);
     F->last_launches = faust_multiply_mixed(f, op, X, p, Y, st, ws, &F->timers, act_f32);
   }
   FH_API_END

@@ -1,4 +1,4 @@
-"""The workspace of FP64 chain products: the row-major form's room is asked for
+"""The workspace of chain products: the FP64 row-major form's room is asked for
 only where the form can run, is never needed for a call to be accepted, and a
 one-factor Faust shares none between streams, captured graphs or with the
 allocation-free entry point."""
@@ -11,6 +11,7 @@ import torch
 import faust_amd
 import oracle
 from faust_amd import _lib
+from faust_amd.bsr import rand_bsr
 
 pytestmark = pytest.mark.gpu
 
@@ -134,3 +135,21 @@ def test_no_room_where_the_form_is_not_run(gpu, monkeypatch, mode):
     used = free - torch.cuda.mem_get_info()[0]
     base = 0 if mode == "per_factor" else 8 * n * p  # one column-major intermediate
     assert used < base + (256 << 20)
+
+
+def test_fp32_capture_keeps_to_the_room_there_is(gpu):
+    # 20 columns one way leave room for 36 the other way in plain columns, not in whole panels of 32
+    rng = np.random.default_rng(9)
+    facs = [rand_bsr(d[0], d[1], 32, 2, rng).astype(np.float32) for d in ((6400, 3200), (3200, 64))]
+    F = faust_amd.Faust(facs, dtype=np.float32, act_dtype=np.float32)
+    F.matmul_device(torch.randn((20, 64), device="cuda"))
+    W = faust_amd.Faust(facs, dtype=np.float32, act_dtype=np.float32)
+    X = torch.randn((36, 6400), device="cuda")
+    Y = torch.empty((36, 64), device="cuda")
+    W.T.matmul_device(X, Y)
+    g = _capture(lambda: F.T.matmul_device(X, Y))
+    for _ in range(3):
+        X.copy_(torch.randn(X.shape, device="cuda"))
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(Y, W.T.matmul_device(X))
