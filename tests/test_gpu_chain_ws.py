@@ -143,13 +143,18 @@ def test_fp32_capture_keeps_to_the_room_there_is(gpu):
     facs = [rand_bsr(d[0], d[1], 32, 2, rng).astype(np.float32) for d in ((6400, 3200), (3200, 64))]
     F = faust_amd.Faust(facs, dtype=np.float32, act_dtype=np.float32)
     F.matmul_device(torch.randn((20, 64), device="cuda"))
-    W = faust_amd.Faust(facs, dtype=np.float32, act_dtype=np.float32)
+    W = faust_amd.Faust(facs, dtype=np.float32, act_dtype=np.float32).T
     X = torch.randn((36, 6400), device="cuda")
     Y = torch.empty((36, 64), device="cuda")
-    W.T.matmul_device(X, Y)
-    g = _capture(lambda: F.T.matmul_device(X, Y))
+    W.matmul_device(X, Y)
+
+    def transposed():  # F.T would be a handle of its own
+        _lib.check(gpu.fh_faust_multiply(F.h, b"T", X.data_ptr(), 36, Y.data_ptr(),
+                                         torch.cuda.current_stream().cuda_stream))
+
+    g = _capture(transposed)
     for _ in range(3):
         X.copy_(torch.randn(X.shape, device="cuda"))
         g.replay()
         torch.cuda.synchronize()
-        assert torch.equal(Y, W.T.matmul_device(X))
+        assert torch.equal(Y, W.matmul_device(X))
