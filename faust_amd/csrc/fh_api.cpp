@@ -451,12 +451,19 @@ DMatP faust_get_product_f64(const std::vector<DMatP>& f, hipStream_t st) {
 }
 
 // count: dense factors whose entries have not been counted are counted now
-// (a wait); without it only the known counts are looked at, and a chain with
-// an all-zero factor gives norm 0 by its first round's product
+// (a wait); without it only the known counts are looked at: a chain with an
+// all-zero factor gives norm 0 by its first round's product, or NaN where that
+// meets infinities, which zero_or_nan looks into
 static bool chain_is_zero(const std::vector<DMatP>& f, bool count, hipStream_t st) {
   for (auto& x : f)
     if ((count || x->nnz >= 0) && nnz_of(*x, st) == 0) return true;
   return false;
+}
+
+// a norm computed without the counts: 0 where NaN came of an all-zero factor
+static double zero_or_nan(const std::vector<DMatP>& f, double lam, hipStream_t st) {
+  if (std::isnan(lam) && chain_is_zero(f, true, st)) return 0.0;
+  return std::fabs(std::sqrt(lam));
 }
 
 // the power-iteration chain of F^H F (or F F^H, the smaller side); false when
@@ -491,8 +498,7 @@ double faust_spectral_norm_f64(const std::vector<DMatP>& f, int maxit, double th
   int n = 0;
   double known;
   if (!spectral_chain(f, ops, n, &known, count, st)) return known;
-  double lam = power_iteration_f64(ops, n, maxit, thr, flag, st);
-  return std::fabs(std::sqrt(lam));
+  return zero_or_nan(f, power_iteration_f64(ops, n, maxit, thr, flag, st), st);
 }
 
 // the 2-norms of two Fausts (PALM's R and L of one factor update), their
@@ -507,12 +513,12 @@ void faust_spectral_norm_pair_f64(const std::vector<DMatP>& f1, const std::vecto
   if (p1 && p2) {
     double l1, l2;
     power_iteration_pair_f64(o1, m1, o2, m2, maxit, thr, &l1, &l2, flag, st);
-    *n1 = std::fabs(std::sqrt(l1));
-    *n2 = std::fabs(std::sqrt(l2));
+    *n1 = zero_or_nan(f1, l1, st);
+    *n2 = zero_or_nan(f2, l2, st);
     return;
   }
-  *n1 = p1 ? std::fabs(std::sqrt(power_iteration_f64(o1, m1, maxit, thr, flag, st))) : k1;
-  *n2 = p2 ? std::fabs(std::sqrt(power_iteration_f64(o2, m2, maxit, thr, flag, st))) : k2;
+  *n1 = p1 ? zero_or_nan(f1, power_iteration_f64(o1, m1, maxit, thr, flag, st), st) : k1;
+  *n2 = p2 ? zero_or_nan(f2, power_iteration_f64(o2, m2, maxit, thr, flag, st), st) : k2;
 }
 
 }  // namespace fh
