@@ -436,15 +436,15 @@ void autotune_clear() {
 }
 
 // Transform::get_product (faust_Transform.hpp:599-626)
-DMatP faust_get_product_f64(const std::vector<DMatP>& f, hipStream_t st) {
+DMatP faust_get_product_f64(const std::vector<DMatP>& f, hipStream_t st, int64_t view_min) {
   FH_CHECK(!f.empty(), "get_product: empty Faust");
   const size_t n = f.size();
   if (n == 1) return dense_of(*f[0], st);
   auto mat = std::make_shared<DMat>();
-  matmul_f64(*f[n - 2], 'N', *f[n - 1], 'N', 1.0, 0.0, *mat, st);
+  matmul_f64(*f[n - 2], 'N', *f[n - 1], 'N', 1.0, 0.0, *mat, st, view_min);
   for (int i = (int)n - 3; i >= 0; --i) {
     auto nm = std::make_shared<DMat>();
-    matmul_f64(*f[i], 'N', *mat, 'N', 1.0, 0.0, *nm, st);
+    matmul_f64(*f[i], 'N', *mat, 'N', 1.0, 0.0, *nm, st, view_min);
     mat = nm;
   }
   return mat;
@@ -866,9 +866,28 @@ int fh_faust_get_product(fh_faust_t F, void* out_dev, void* stream) {
     if (x->dtype != FH_F64 || x->kind == K_BSR)
       throw Error(FH_ERR_UNSUPPORTED, "get_product: FP64 dense / CSR chains only (multiply other chains by the identity)");
   hipStream_t st = (hipStream_t)stream;
+  const auto give = [&](const DMatP& P) {
+    FH_HIP(hipMemcpyAsync(out_dev, P->d.p, sizeof(double) * (size_t)P->m * P->n, hipMemcpyDeviceToDevice, st));
+  };
   DMatP P = faust_get_product_f64(F->f, st);
-  FH_HIP(hipMemcpyAsync(out_dev, P->d.p, sizeof(double) * (size_t)P->m * P->n, hipMemcpyDeviceToDevice, st));
+  give(P);
+  // Operands of 64K .. VIEW_MIN entries are multiplied zeros and all, and a zero
+  // against an infinity makes NaN where the product of the other terms need
+  // not be one: with NaN in the result they are looked at for zeros too.
+  constexpr int64_t VIEW_LOOK = 1 << 16;
+  bool look = false;
+  if (F->f.size() > 1)
+    for (auto& x : F->f)
+      for (const int64_t n : {(int64_t)x->n, (int64_t)P->n}) look = look || (x->m * n >= VIEW_LOOK && x->m * n < VIEW_MIN);
+  double* nan = mail() + MAIL_SUM;
+  *nan = 0.0;
+  if (look) any_nan_f64(P->d.as<double>(), (int64_t)P->m * P->n, nan, st);
   FH_HIP(hipStreamSynchronize(st));
+  if (*nan != 0.0) {
+    P = faust_get_product_f64(F->f, st, VIEW_LOOK);
+    give(P);
+    FH_HIP(hipStreamSynchronize(st));
+  }
   FH_API_END
 }
 

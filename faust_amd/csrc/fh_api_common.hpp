@@ -158,7 +158,7 @@ void autotune_put_mode(const std::string& key, int mode);
 ChainForm faust_multiply_f64(const std::vector<DMatP>& f, char op, const double* X, int p, double* Y, hipStream_t st,
                              const ChainPlan64& plan, const ChainWs& ws, FaustTimers* tm = nullptr,
                              int* launches = nullptr);
-DMatP faust_get_product_f64(const std::vector<DMatP>& f, hipStream_t st);
+DMatP faust_get_product_f64(const std::vector<DMatP>& f, hipStream_t st, int64_t view_min = VIEW_MIN);
 double faust_spectral_norm_f64(const std::vector<DMatP>& f, int maxit, double thr, int* flag, hipStream_t st,
                                bool count = true);
 void faust_spectral_norm_pair_f64(const std::vector<DMatP>& f1, const std::vector<DMatP>& f2, int maxit, double thr,

@@ -223,6 +223,8 @@ void gemm_f64(char opA, char opB, int m, int n, int k, double alpha, const doubl
 // (device memory or a mail slot), and to out2 too when given
 void reduce_dot_f64(const double* x, const double* y, int64_t n, double* out, hipStream_t st, double* out2 = nullptr);
 void reduce_sum_f64(const double* x, int64_t n, double* out, hipStream_t st, double* out2 = nullptr);
+// *out (which the device can write) = 1 where any of the n values is NaN, else left alone
+void any_nan_f64(const double* x, int64_t n, double* out, hipStream_t st);
 void diag_dot_f64(const double* A, const double* S, int m, int n, double* diag, hipStream_t st);
 // dense -> CSR and CSC (drops exact zeros; synchronizes once, for the sizes)
 void dense_to_csr_f64(const double* D, int m, int n, DMat& out, hipStream_t st);
@@ -262,9 +264,12 @@ void power_iteration_pair_f64(const std::vector<ChainOp>& ops1, int n1, const st
 // host-side start vector: srand(0xF4+'u'+57), Random on [-1, 1]
 const std::vector<double>& power_x0(int n);
 
-// generic FP64 product dispatch: out = alpha*op(A)*op(B) + beta*out (dense out)
+// generic FP64 product dispatch: out = alpha*op(A)*op(B) + beta*out (dense out);
+// dense operands of at least view_min entries are multiplied without their
+// zeros where those are many
+constexpr int64_t VIEW_MIN = 1 << 19;
 void matmul_f64(const DMat& A, char opA, const DMat& B, char opB, double alpha, double beta, DMat& out,
-                hipStream_t st);
+                hipStream_t st, int64_t view_min = VIEW_MIN);
 DMatP dense_of(const DMat& A, hipStream_t st);
 int64_t nnz_of(DMat& A, hipStream_t st);
 

@@ -41,13 +41,14 @@ int64_t nnz_of(DMat& A, hipStream_t st) {
 
 // A dense operand whose density is below 1/8 is multiplied through a CSR
 // copy (the densified products of a few butterfly-like factors are such
-// matrices).  Only matrices of at least 512K entries are examined: the count
-// and the conversion wait for the device twice and take 35 to 50 us, a dense
-// product of order 512 takes 14 us and one of order 1024 56 us.
-static const DMat* sparse_view(const DMat& A, hipStream_t st) {
+// matrices).  Only matrices of at least view_min entries are examined, by
+// default 512K: the count and the conversion wait for the device twice and
+// take 35 to 50 us, a dense product of order 512 takes 14 us and one of order
+// 1024 56 us.
+static const DMat* sparse_view(const DMat& A, int64_t view_min, hipStream_t st) {
   if (A.kind != K_DENSE || A.dtype != FH_F64) return &A;
   const int64_t N = (int64_t)A.m * A.n;
-  if (N < (1 << 19)) return &A;
+  if (N < view_min) return &A;
   if (!A.sparsity_checked) {
     A.sparsity_checked = true;
     int64_t nz = nnz_of(const_cast<DMat&>(A), st);
@@ -62,9 +63,9 @@ static const DMat* sparse_view(const DMat& A, hipStream_t st) {
 
 // out = alpha*op(A)*op(B) + beta*out ; out is dense (allocated here when beta == 0)
 void matmul_f64(const DMat& A0, char opA, const DMat& B0, char opB, double alpha, double beta, DMat& out,
-                hipStream_t st) {
-  const DMat& A = *sparse_view(A0, st);
-  const DMat& B = (A.kind == K_CSR) ? B0 : *sparse_view(B0, st);
+                hipStream_t st, int64_t view_min) {
+  const DMat& A = *sparse_view(A0, view_min, st);
+  const DMat& B = (A.kind == K_CSR) ? B0 : *sparse_view(B0, view_min, st);
   const int M = (opA == 'N') ? A.m : A.n;
   const int K = (opA == 'N') ? A.n : A.m;
   const int KB = (opB == 'N') ? B.m : B.n;

@@ -73,6 +73,18 @@ void reduce_sum_f64(const double* x, int64_t n, double* out, hipStream_t st, dou
   reduce_launch(0, x, nullptr, n, out, out2, st);
 }
 
+__global__ __launch_bounds__(256) void k_any_nan(const double* __restrict__ x, int64_t n, double* __restrict__ out) {
+  bool nan = false;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) nan |= x[i] != x[i];
+  if (__any(nan) && (threadIdx.x & 63) == 0) *out = 1.0;  // the same value from every wave that gets here
+}
+
+void any_nan_f64(const double* x, int64_t n, double* out, hipStream_t st) {
+  if (n <= 0) return;
+  hipLaunchKernelGGL(k_any_nan, dim3((unsigned)std::min<int64_t>(1024, (n + 255) / 256)), dim3(256), 0, st, x, n, out);
+  FH_LAUNCH_CHECK();
+}
+
 // diag[i] = sum_k A[k,i]*S[k,i] in ascending k (the diagonal of A^T S): one
 // fma chain per column.  A workgroup stages 16 columns of both matrices in LDS,
 // 128 rows at a time and coalesced (the next 128 in flight meanwhile), and 16
