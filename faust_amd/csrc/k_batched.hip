@@ -1790,9 +1790,12 @@ __global__ __launch_bounds__(256) void k_bload(const BLoadJob* __restrict__ jobs
 
 template <class T>
 void launch_bload(const BLoadJob* jobs, int njobs, hipStream_t st) {
-  if (njobs == 0) return;
-  hipLaunchKernelGGL(k_bload<T>, dim3(64, (unsigned)njobs), dim3(256), 0, st, jobs);
-  FH_LAUNCH_CHECK();
+  // one job per target and default factor, 64K - 1 jobs to a launch (gridDim.y)
+  constexpr int MOST = 65535;
+  for (int j0 = 0; j0 < njobs; j0 += MOST) {
+    hipLaunchKernelGGL(k_bload<T>, dim3(64, (unsigned)std::min(MOST, njobs - j0)), dim3(256), 0, st, jobs + j0);
+    FH_LAUNCH_CHECK();
+  }
 }
 
 template <class S>

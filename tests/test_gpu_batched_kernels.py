@@ -95,3 +95,16 @@ def test_dense_step_sizes(gpu, n):
                           num_its=3)
     # as the neighbouring test of the same comparison: sums in another order, 1e-8
     assert abs(res.lambdas[0] - ref.lam) <= 1e-8 * abs(ref.lam)
+
+
+def test_more_jobs_than_a_grid_dimension(gpu):
+    # 33000 targets of two factors: 66000 targets and default factors to load
+    rng = np.random.default_rng(33)
+    As = [np.full((1, 1), v) for v in rng.standard_normal(33000)]
+    kw = dict(dtype="f64", num_its=1, refine_its=0)
+    got = palm4msa_batched(As, 2, k=[1] * len(As), **kw)
+    ends = np.r_[0:40, 32960:33000]
+    want = palm4msa_batched([As[i] for i in ends], 2, k=[1] * len(ends), **kw)
+    assert np.array_equal(np.asarray(got.lambdas)[ends], want.lambdas)
+    for i, fs in zip(ends, want.factors):
+        assert all(np.array_equal(a, b) for a, b in zip(got.factors[i], fs))
