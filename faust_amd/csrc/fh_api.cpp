@@ -242,12 +242,14 @@ bool stream_capturing(hipStream_t st) {
 }
 
 // What the quickest form depends on: direction, columns, each op'd factor's
-// shape and entries, and the device.
+// shape, entries and ELL slots (the forms read those where every factor has
+// them), and the device.
 static std::string chain_sig(char op, int p, int in_rows, const std::vector<ChainCsrOp>& ops) {
   int dev = 0;
   (void)hipGetDevice(&dev);
   std::string k = std::to_string(dev) + op + ":" + std::to_string(p) + ":" + std::to_string(in_rows);
-  for (const auto& o : ops) k += "," + std::to_string(o.rows) + "/" + std::to_string(o.nnz);
+  for (const auto& o : ops)
+    k += "," + std::to_string(o.rows) + "/" + std::to_string(o.nnz) + "/" + std::to_string(o.ell);
   return k;
 }
 

@@ -6,6 +6,7 @@ import ctypes as C
 
 import numpy as np
 import pytest
+import scipy.sparse as sp
 import torch
 
 import faust_amd
@@ -158,3 +159,31 @@ def test_fp32_capture_keeps_to_the_room_there_is(gpu):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(Y, W.matmul_device(X))
+
+
+def _banded(n, per_row):
+    """per_row entries (in turn) at consecutive columns around the diagonal."""
+    k = np.resize(per_row, n)
+    cols = np.concatenate([(np.arange(c) + min(max(i - c // 2, 0), n - c)) for i, c in enumerate(k)])
+    data = np.random.default_rng(n).standard_normal(len(cols))
+    return sp.csr_matrix((data, cols, np.concatenate([[0], np.cumsum(k)])), shape=(n, n))
+
+
+def test_measured_form_is_of_the_row_widths(gpu, monkeypatch):
+    # equal shapes and entries, rows of 3 (4 ELL slots) and of 1 and 5 (8 slots).  Banded factors gather column-major
+    # X from cache, so the first chain keeps one launch per factor; the second, not measured yet, has the default form
+    n, p = 20000, 64
+    narrow, wide = [_banded(n, [3])] * 2, [_banded(n, [1, 5])] * 2
+    A, B = faust_amd.Faust(narrow), faust_amd.Faust(wide)
+    X = torch.randn((p, n), dtype=torch.float64, device="cuda")
+    Y = torch.empty_like(X)
+    _lib.check(gpu.fh_autotune_clear())
+    monkeypatch.setenv("FH_AUTOTUNE", "0")
+    B.matmul_device(X, Y)
+    assert _launches(B) == 3  # the default, row-major: B's handle has its room
+    monkeypatch.setenv("FH_AUTOTUNE", "1")
+    A.matmul_device(X, Y)
+    assert _launches(A) == 2
+    g = _capture(lambda: B.matmul_device(X, Y))
+    assert _launches(B) == 3
+    _replays_right(g, wide, "N", X, Y)
