@@ -1102,11 +1102,15 @@ static const double* pl_x0() {
 }
 
 // Per-round time estimates (seconds).  The persistent kernel streams every
-// operator through one CU (~100 GB/s), and an entry of a row it does not load
-// ahead (dense, or more than PW_PF) is a dependent load (~90 ns: 10.7 us per
-// operator of a dense 128 x 100 chain, 4.5 us with 32 entries per row); the
-// wide form pays a launch per operator but spreads the rows over the chip,
-// leaving each row's fma chain (about 4 ns per term) as its floor.
+// operator through one CU (~100 GB/s; 30 where rows are longer than it loads
+// ahead, PW_PF entries), and an entry of such a row is a dependent load: dense
+// 90 ns (10.7 us per operator of a 128 x 100 chain), sparse 80 ns while few
+// rows are long and 150 ns when many are and their lines displace each other.
+// The wide form pays a launch per operator but spreads the rows over the chip,
+// leaving each row's fma chain as its floor: 4 ns per term of a dense row,
+// 44 ns of a sparse one (the gather from LDS is in the chain).
+// us per round, persistent / wide, 5 factors of 1024 rows of 2: one row of 128
+// 70 / 78; 64 rows of 64 111 / 81; all rows of 20 163 / 62, of 8 60 / 54.
 // FH_POWER_WIDE=0/1 forces a form.
 static bool use_wide_form(const std::vector<PwOp>& h) {
   if (const char* e = getenv("FH_POWER_WIDE")) {
@@ -1116,10 +1120,17 @@ static bool use_wide_form(const std::vector<PwOp>& h) {
   double single = 3e-6, wide = 1e-6;
   for (const PwOp& o : h) {
     const double entries = o.kind == 1 ? (double)o.nnz : (double)o.rows * o.cols;
-    const double bytes = entries * (o.kind == 1 ? 12.0 : 8.0);
-    const double row = o.kind == 1 ? (o.width >= 0 ? o.width : entries / std::max(o.rows, 1)) : o.cols;
-    single += std::max(bytes / 100e9, row > PW_PF ? row * 90e-9 : 0.0) + 0.4e-6;
-    wide += 4e-6 + row * 4e-9 + bytes / 3e12;
+    const bool sparse = o.kind == 1;
+    const double bytes = entries * (sparse ? 12.0 : 8.0);
+    const double row = sparse ? (o.width >= 0 ? o.width : entries / std::max(o.rows, 1)) : o.cols;
+    if (row > PW_PF) {
+      // (many long rows: 1000 entries beyond two per row)
+      const double load = !sparse ? 90e-9 : entries - 2.0 * o.rows > 1000.0 ? 150e-9 : 80e-9;
+      single += std::max(bytes / (sparse ? 30e9 : 100e9), row * load) + 0.4e-6;
+    } else {
+      single += bytes / 100e9 + 0.4e-6;
+    }
+    wide += 4e-6 + row * (sparse ? 44e-9 : 4e-9) + bytes / 3e12;
   }
   return wide < single;
 }
