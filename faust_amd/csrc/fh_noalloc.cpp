@@ -6,8 +6,9 @@
 // entry points give the same bits.
 //
 // `scratch` is one FH_NOALLOC_SCRATCH_BYTES array per GPU, held from module
-// load to process end; BSR chains keep the control block of the one-launch
-// chain at its start.  In host code its name is only a host-side stand-in
+// load to process end, with the control block of the one-launch BSR chain
+// behind it: that has to be zero when such a chain starts, so no other
+// product's intermediates may lie there.  In host code its name is only a host-side stand-in
 // for the symbol: the device address comes from hipGetSymbolAddress, once per
 // device (with that device current), and only that address is handed to
 // kernels.  Every call on one GPU shares the array; calls that overlap on one
@@ -22,7 +23,8 @@
 namespace {
 
 constexpr size_t kScratchBytes = FH_NOALLOC_SCRATCH_BYTES;
-static __device__ __align__(256) unsigned char scratch[kScratchBytes];
+constexpr size_t kCtlBytes = 64 * 1024;  // at least bsr_chain_ctl_bytes()
+static __device__ __align__(256) unsigned char scratch[kScratchBytes + kCtlBytes];
 
 constexpr int kMaxDevices = 64;
 std::mutex g_mu;
@@ -104,17 +106,19 @@ extern "C" int fh_faust_multiply_noalloc(fh_faust_t F, char op, const void* X, i
     if ((size_t)nbuf * align256(padded) <= kScratchBytes) need = padded;
   }
   const size_t slot = align256(need);
-  // BSR chains also keep the one-launch chain's control block at the start of
-  // the array (zero at load; every chain leaves its counters cleared)
+  // the one-launch BSR chain's control block lies behind the intermediates
+  // (zero at load; every chain leaves its counters cleared); its bytes count
+  // towards what a BSR chain may take
   const bool bsr = f.front()->kind == K_BSR && !act_f32;
   const size_t ctl_bytes = bsr ? align256(bsr_chain_ctl_bytes()) : 0;
+  FH_CHECK(ctl_bytes <= kCtlBytes, "fh_faust_multiply_noalloc: no room for the chain's control block");
   if (ctl_bytes + (size_t)nbuf * slot > kScratchBytes)
     throw Error(FH_ERR_ARG, "fh_faust_multiply_noalloc: this product needs " + std::to_string(nbuf) + " x " +
                                 std::to_string(need) + " bytes of intermediates, more than the " +
                                 std::to_string(kScratchBytes) + "-byte scratch array");
   char* base = (nbuf > 0 || bsr) ? static_cast<char*>(scratch_address()) : nullptr;
-  const ChainWs ws{{nbuf > 0 ? base + ctl_bytes : nullptr, nbuf > 1 ? base + ctl_bytes + slot : nullptr},
-                   bsr ? reinterpret_cast<int*>(base) : nullptr, need};
+  const ChainWs ws{{nbuf > 0 ? base : nullptr, nbuf > 1 ? base + slot : nullptr},
+                   bsr ? reinterpret_cast<int*>(base + kScratchBytes) : nullptr, need};
   if (f64)
     faust_multiply_f64(f, op, (const double*)X, p, (double*)Y, st, pl, ws, nullptr, &F->last_launches);
   else

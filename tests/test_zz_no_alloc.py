@@ -91,3 +91,29 @@ def test_noalloc_refuses_oversized_product(gpu):
     assert b"scratch array" in L.fh_last_error()
     # the same product with 256 columns fits
     _both(L, F, "N", 8192, 8192, 256, torch.float64, 9)
+
+
+@pytest.mark.parametrize("kind", ["fp64", "fp32", "bsr_f32"])
+def test_noalloc_bsr_chain_after_other_products(gpu, monkeypatch, kind):
+    # the one-launch BSR chain's counters start at zero: the intermediates of a product before it, which fill the
+    # array from its start, must not lie on them
+    print(f"noalloc {kind} 2048^2 x3, then a one-launch BSR chain 2048^2 x3", flush=True)
+    rng = np.random.default_rng(8)
+    if kind == "bsr_f32":
+        first = faust_amd.Faust([rand_bsr(2048, 2048, 32, 3, rng).astype(np.float32) for _ in range(3)],
+                                dtype=np.float32, act_dtype=np.float32)
+    else:
+        dt = np.float64 if kind == "fp64" else np.float32
+        first = faust_amd.Faust([_csr(2048, 6, rng, dt) for _ in range(3)], dtype=dt)
+    td = torch.float64 if kind == "fp64" else torch.float32
+    _both(gpu, first, "N", 2048, 2048, 200, td, 9)
+    chain = faust_amd.Faust([rand_bsr(2048, 2048, 32, 4, rng) for _ in range(3)], dtype="bf16")
+    X = torch.randn((96, 2048), device="cuda").to(torch.bfloat16)
+    Y0, Y1 = torch.empty_like(X), torch.empty_like(X)
+    assert _call(gpu.fh_faust_multiply, chain, "N", X, 96, Y0) == _lib.FH_OK, gpu.fh_last_error()
+    monkeypatch.setenv("FH_BSR_CHAIN", "1")
+    monkeypatch.setenv("FH_BSR_CHAIN_CHECK", "1")
+    for _ in range(2):
+        assert _call(gpu.fh_faust_multiply_noalloc, chain, "N", X, 96, Y1) == _lib.FH_OK, gpu.fh_last_error()
+        torch.cuda.synchronize()
+        assert torch.equal(Y0.view(torch.int16), Y1.view(torch.int16))
