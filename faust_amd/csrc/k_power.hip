@@ -1102,15 +1102,18 @@ static const double* pl_x0() {
 }
 
 // Per-round time estimates (seconds).  The persistent kernel streams every
-// operator through one CU (~100 GB/s; 30 where rows are longer than it loads
-// ahead, PW_PF entries), and an entry of such a row is a dependent load: dense
-// 90 ns (10.7 us per operator of a 128 x 100 chain), sparse 80 ns while few
-// rows are long and 150 ns when many are and their lines displace each other.
-// The wide form pays a launch per operator but spreads the rows over the chip,
-// leaving each row's fma chain as its floor: 4 ns per term of a dense row,
-// 44 ns of a sparse one (the gather from LDS is in the chain).
-// us per round, persistent / wide, 5 factors of 1024 rows of 2: one row of 128
-// 70 / 78; 64 rows of 64 111 / 81; all rows of 20 163 / 62, of 8 60 / 54.
+// operator through one CU (~100 GB/s), and an entry of a row longer than it
+// loads ahead (PW_PF entries, or dense) is a dependent load: dense 90 ns (10.7
+// us per operator of a 128 x 100 chain), sparse 75 ns while few rows are long,
+// 120 to 200 ns by the number of rows when many are (more than 1000 entries
+// beyond two per row), whose loads together get 12 GB/s.  The wide form pays a
+// launch per operator but spreads the rows over the chip, leaving each row's
+// fma chain as its floor: 4 ns per term of a dense row, 44 ns of a sparse one
+// (the gather from LDS is in the chain); the rounds queued past the end and the
+// host's waits come to 15%.  Of 160 chains of 1 to 10 factors of 128 to 2000
+// rows all but two ran within 6% of the quicker form (those 13%).  us per
+// round, persistent / wide, 5 factors of 1024 rows of 2: one row of 128 70 / 78; 64
+// rows of 64 111 / 81; all rows of 20 163 / 62, of 8 60 / 54.
 // FH_POWER_WIDE=0/1 forces a form.
 static bool use_wide_form(const std::vector<PwOp>& h) {
   if (const char* e = getenv("FH_POWER_WIDE")) {
@@ -1123,16 +1126,15 @@ static bool use_wide_form(const std::vector<PwOp>& h) {
     const bool sparse = o.kind == 1;
     const double bytes = entries * (sparse ? 12.0 : 8.0);
     const double row = sparse ? (o.width >= 0 ? o.width : entries / std::max(o.rows, 1)) : o.cols;
+    single += bytes / 100e9 + 0.4e-6;
     if (row > PW_PF) {
-      // (many long rows: 1000 entries beyond two per row)
-      const double load = !sparse ? 90e-9 : entries - 2.0 * o.rows > 1000.0 ? 150e-9 : 80e-9;
-      single += std::max(bytes / (sparse ? 30e9 : 100e9), row * load) + 0.4e-6;
-    } else {
-      single += bytes / 100e9 + 0.4e-6;
+      const double more = sparse ? entries - 2.0 * o.rows : 0.0;
+      const double load = !sparse ? 90e-9 : more <= 1000.0 ? 75e-9 : o.rows <= 512 ? 120e-9 : o.rows <= 1024 ? 150e-9 : 200e-9;
+      single += std::max(row * load, more * 12.0 / 12e9);
     }
     wide += 4e-6 + row * (sparse ? 44e-9 : 4e-9) + bytes / 3e12;
   }
-  return wide < single;
+  return 1.15 * wide < single;
 }
 
 static double power_iteration_wide(const std::vector<PwOp>& h, int n, const std::vector<double>& x0, int maxit,
