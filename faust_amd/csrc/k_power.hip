@@ -1172,16 +1172,25 @@ static double power_iteration_wide(const std::vector<PwOp>& h, int n, const std:
     b.in = dst + ((round - 1) & 1);
     b.out = dst + (round & 1);
     const bool last = round > maxit;  // every round ran: the loop test alone
+    // the host looks whether the iteration is over before rounds 5, 13, ...:
+    // their boundary is a launch of its own, so that it is decided by then
+    const bool look = round - 1 == next_check;
+    const bool alone = !fused || last || look;
     b.first = 0;
-    if (!fused || last) {
+    if (alone) {
       hipLaunchKernelGGL(k_pw_step, dim3(1), dim3(PW_THREADS), 0, st, b);
       FH_LAUNCH_CHECK();
       if (last) break;
     }
+    if (look) {
+      FH_HIP(hipStreamSynchronize(st));
+      if (res[3] != 0.0) break;
+      next_check += 8;
+    }
     const double* cur = b.xn_out;
     for (int s = nops - 1; s >= 0; --s) {
       const PwOp& o = h[s];
-      b.first = fused && s == nops - 1;
+      b.first = !alone && s == nops - 1;
       double* out = (s == 0) ? xa_out : (((nops - 1 - s) & 1) ? b1.as<double>() : b0.as<double>());
       if (o.cols > PW_VMAX) {  // x does not fit LDS: read it from global memory
         const dim3 gg((o.rows + PW_WIDE_THREADS - 1) / PW_WIDE_THREADS);
@@ -1208,11 +1217,6 @@ static double power_iteration_wide(const std::vector<PwOp>& h, int n, const std:
       }
       FH_LAUNCH_CHECK();
       cur = out;
-    }
-    if (round == next_check) {
-      FH_HIP(hipStreamSynchronize(st));
-      if (res[3] != 0.0) break;
-      next_check += 8;
     }
   }
   FH_HIP(hipStreamSynchronize(st));
