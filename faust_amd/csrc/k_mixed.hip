@@ -31,6 +31,7 @@
 // columns cycle over the XCDs the same way.  The chain input is transposed
 // once into row-major and the last factor writes column-major through LDS.
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 #include "bsr_frag.hpp"
@@ -612,11 +613,13 @@ __global__ __launch_bounds__(256) void k_bsr_f32(int nbr, int p, const int* __re
 // two 512-byte runs.  Column-major, each of those loads touches 32 cache lines
 // a whole column apart (a power of two for most orders, so few L2 channels)
 // and comes back to them four times.  8192^2, 4 blocks per row, 512 columns:
-// 19.3 -> 17.4 us per launch (rows of 1 to 12 blocks, the transpose: 24 -> 21
-// us with partial rounds loaded as whole ones, not block by block).  A launch
-// reads 50 MB through the fabric (each XCD its 128 columns of X and half the
-// blocks) and has 6.8 us of MFMA, which starts when the loads land.
-constexpr int BF32_CH = 4;  // blocks staged per round
+// 17.8 us per launch column-major, 15.3 tiled.  Lanes past column p read one
+// column, and a row's last round loads the blocks there are: with whole panels
+// and four blocks always, 33 columns took 30.1 us for five factors (27.7 now,
+// 27.2 column-major), rows of two blocks 2.9 us in place of 2.7.  A
+// launch reads 50 MB through the fabric (each XCD its 128 columns of X and half
+// the blocks) and has 6.8 us of MFMA, which starts when the loads land.
+constexpr int BF32_CH = 4;  // blocks staged per round (its last, partial one: as many as there are)
 template <bool IN_TILED, bool OUT_TILED>
 __global__ __launch_bounds__(256) void k_bsr_f32s(int nbr, int p, const int* __restrict__ brp,
                                                   const int* __restrict__ bci, const float* __restrict__ blk,
@@ -627,28 +630,27 @@ __global__ __launch_bounds__(256) void k_bsr_f32s(int nbr, int p, const int* __r
   const int g = blockIdx.x % ngroups, br = blockIdx.x / ngroups;
   if (br >= nbr) return;
   const int h = lane >> 5, r = lane & 31;
-  const int G = (p + 31) >> 5, panel = min(g * 4 + wave, G - 1);  // waves past the last panel repeat it
+  const int G = (p + 31) >> 5, panel = g * 4 + wave;
   const int jc = g * 128 + wave * 32 + r;
   const bool jok = jc < p;
   const int j = jok ? jc : 0;  // columns past p read column 0; their outputs are not stored
+  const int xo = jok ? panel * 256 + lane : 32 * h;  // this lane's first float4 in a block row's tiles
   f32x16 acc = {};
   const int b0 = brp[br], b1 = brp[br + 1];
-  for (int c0 = b0; c0 < b1; c0 += BF32_CH) {
-    const int nb = min(BF32_CH, b1 - c0);
-    // the staging loads and this wave's X operands of the round's blocks are
-    // issued together, before any LDS write or MFMA (a partial round loads its
-    // last block again in place of the missing ones)
-    f32x4 stg[BF32_CH], x[BF32_CH][4];
-    int bc[BF32_CH];
+  // one round of NB blocks: the staging loads and this wave's X operands are
+  // issued together, before any LDS write or MFMA
+  auto round = [&](auto nbc, int c0) {
+    constexpr int NB = decltype(nbc)::value;
+    f32x4 stg[NB], x[NB][4];
+    int bc[NB];
 #pragma unroll
-    for (int q = 0; q < BF32_CH; ++q) {
-      const int b = c0 + min(q, nb - 1);
-      bc[q] = bci[b];
-      stg[q] = reinterpret_cast<const f32x4*>(blk + (size_t)b * 1024)[t];
+    for (int q = 0; q < NB; ++q) {
+      bc[q] = bci[c0 + q];
+      stg[q] = reinterpret_cast<const f32x4*>(blk + (size_t)(c0 + q) * 1024)[t];
     }
 #pragma unroll
-    for (int q = 0; q < BF32_CH; ++q) {
-      const f32x4* xp = IN_TILED ? reinterpret_cast<const f32x4*>(X) + ((size_t)bc[q] * G + panel) * 256 + lane
+    for (int q = 0; q < NB; ++q) {
+      const f32x4* xp = IN_TILED ? reinterpret_cast<const f32x4*>(X) + (size_t)bc[q] * G * 256 + xo
                                  : reinterpret_cast<const f32x4*>(X + (size_t)j * ldx + bc[q] * 32 + h * 16);
 #pragma unroll
       for (int u = 0; u < 4; ++u) x[q][u] = xp[IN_TILED ? 64 * u : u];
@@ -656,11 +658,10 @@ __global__ __launch_bounds__(256) void k_bsr_f32s(int nbr, int p, const int* __r
     __builtin_amdgcn_sched_barrier(0);
     if (c0 > b0) lds_barrier();  // the previous round's blocks are consumed
 #pragma unroll
-    for (int q = 0; q < BF32_CH; ++q) sa[q * 256 + t] = stg[q];
+    for (int q = 0; q < NB; ++q) sa[q * 256 + t] = stg[q];
     lds_barrier();
 #pragma unroll
-    for (int q = 0; q < BF32_CH; ++q) {
-      if (q >= nb) break;
+    for (int q = 0; q < NB; ++q) {
       f32x4 a[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) a[u] = sa[q * 256 + u * 64 + lane];
@@ -668,6 +669,14 @@ __global__ __launch_bounds__(256) void k_bsr_f32s(int nbr, int p, const int* __r
       for (int s4 = 0; s4 < 16; ++s4)
         acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s4 >> 2][s4 & 3], x[q][s4 >> 2][s4 & 3], acc, 0, 0, 0);
     }
+  };
+  int c0 = b0;
+  for (; c0 + BF32_CH <= b1; c0 += BF32_CH) round(std::integral_constant<int, BF32_CH>{}, c0);
+  switch (b1 - c0) {  // the same for the whole workgroup
+    case 3: round(std::integral_constant<int, 3>{}, c0); break;
+    case 2: round(std::integral_constant<int, 2>{}, c0); break;
+    case 1: round(std::integral_constant<int, 1>{}, c0); break;
+    default: break;
   }
   if (!jok) return;
 #pragma unroll
@@ -1166,7 +1175,11 @@ static bool chain_verified(int sync, int* ctl, hipStream_t st) {
 // Bytes of each tiled intermediate of an FP32 BSR chain with FP32 activations
 // (p padded to whole 32-column panels); 0 where the chain keeps column-major
 // ones: a single factor, the per-wave kernel, or so few columns that the
-// padding costs more than the layout gives.
+// padding doubles the intermediates for nothing.  us for five factors of 4
+// blocks per row, column-major / tiled: 2048^2, 8 columns 21.6 / 21.7, 17
+// 22.0 / 21.6, 32 22.6 / 22.0, 128 29.1 / 25.6; 8192^2 22.8 / 22.7, 24.0 / 24.7,
+// 27.2 / 26.6, 41.8 / 38.5; of 2 blocks 8192^2, 17 columns 16.7 / 17.3, 512
+// 60.8 / 53.1.
 constexpr int BF32_TILED_MIN = 17;
 size_t faust_ws_need_f32_tiled(const std::vector<DMatP>& f, char op, int p, int* nbuf) {
   const int J = (int)f.size();
