@@ -73,6 +73,22 @@ DMatP make_csr_from_host(int dtype, int m, int n, int nnz, const int32_t* rp, co
   for (int i = 0; i < m; ++i) M->max_row = std::max(M->max_row, rp[i + 1] - rp[i]);
   M->max_col = 0;
   for (int j = 0; j < n; ++j) M->max_col = std::max(M->max_col, cp[j + 1] - cp[j]);
+  if (dtype == FH_F64) {
+    auto far = [](int nr, const int* ptr, const int* idx) {
+      int64_t n = 0;
+      for (int r = 0; r < nr; ++r) {
+        int q = r > 0 ? ptr[r - 1] : 0;
+        const int qe = r > 0 ? ptr[r] : 0;
+        for (int e = ptr[r]; e < ptr[r + 1]; ++e) {
+          while (q < qe && idx[q] < idx[e] - 16) ++q;
+          n += !(q < qe && idx[q] <= idx[e] + 16);
+        }
+      }
+      return n;
+    };
+    M->far_row = far(m, rp, ci);
+    M->far_col = far(n, cp.data(), ri.data());
+  }
   if (dtype == FH_F32 || dtype == FH_F64) {
     // ELL views for the gather kernels (rows of S, rows of S^T).  FP32: the
     // widest row rounded up to 4, at most 16 slots, a row's slots together (its
@@ -142,11 +158,12 @@ static bool chain_csr_ops(const std::vector<DMatP>& f, char op, std::vector<Chai
     const int rows = tr ? S.n : S.m;
     *mean_max = std::max(*mean_max, (double)S.nnz / std::max(rows, 1));
     const int ew = tr ? S.csr_tell_w : S.csr_ell_w;
+    const int64_t far = tr ? S.far_col : S.far_row;
     ops.push_back({tr ? S.cp.as<int>() : S.rp.as<int>(), tr ? S.ri.as<int>() : S.ci.as<int>(),
                    tr ? S.cv.as<double>() : S.v.as<double>(), rows, (int)S.nnz,
                    ell_on && ew > 0 && ew <= 32 ? ew : 0,
                    tr ? S.csr_tell_ci.as<int>() : S.csr_ell_ci.as<int>(),
-                   tr ? S.csr_tell_v.as<double>() : S.csr_ell_v.as<double>()});
+                   tr ? S.csr_tell_v.as<double>() : S.csr_ell_v.as<double>(), far < 0 ? S.nnz : far});
     r = rows;
   }
   return true;
@@ -242,14 +259,16 @@ bool stream_capturing(hipStream_t st) {
 }
 
 // What the quickest form depends on: direction, columns, each op'd factor's
-// shape, entries and ELL slots (the forms read those where every factor has
-// them), and the device.
+// shape, entries, ELL slots (the forms read those where every factor has them)
+// and share of far entries (in eighths: the gathers of column-major X are as
+// quick as these are few), and the device.
 static std::string chain_sig(char op, int p, int in_rows, const std::vector<ChainCsrOp>& ops) {
   int dev = 0;
   (void)hipGetDevice(&dev);
   std::string k = std::to_string(dev) + op + ":" + std::to_string(p) + ":" + std::to_string(in_rows);
   for (const auto& o : ops)
-    k += "," + std::to_string(o.rows) + "/" + std::to_string(o.nnz) + "/" + std::to_string(o.ell);
+    k += "," + std::to_string(o.rows) + "/" + std::to_string(o.nnz) + "/" + std::to_string(o.ell) + "/" +
+         std::to_string(o.far * 8 / std::max(o.nnz, 1));
   return k;
 }
 
@@ -292,9 +311,9 @@ ChainPlan64 chain_plan_f64(const std::vector<DMatP>& f, char op, int p, bool tun
   P.measure = tunable && !P.known && tune && !stream_capturing(st);
   // chains that fit the one-launch form keep to that and to one launch per factor
   if (plain && csr_rm_fits(P.ops, P.in_rows, p) && !csr_chain_pf_fits(P.ops, P.in_rows, p)) {
-    int nnz_max = 0;
-    for (const auto& o : P.ops) nnz_max = std::max(nnz_max, o.nnz);
-    P.rm_rule = (int64_t)nnz_max * p >= RM_TERMS_DEFAULT;
+    int64_t far = 0;
+    for (const auto& o : P.ops) far = std::max(far, o.far);
+    P.rm_rule = far * p >= (f.size() > 1 ? RM_TERMS_DEFAULT : RM_TERMS_SINGLE);
     if (P.known ? P.form.kind == 3 : P.measure || P.rm_rule) {
       int r = P.in_rows;  // the last factor's output is Y
       for (size_t i = 0; i + 1 < P.ops.size(); ++i) r = std::max(r, P.ops[i].rows);

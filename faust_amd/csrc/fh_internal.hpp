@@ -112,6 +112,9 @@ struct DMat {
   DBuf rp, ci, v;         // CSR
   int64_t nnz = 0;        // CSR: stored entries; dense: -1 until counted
   int max_row = -1, max_col = -1;  // CSR: widest row / column (-1: unknown)
+  // CSR: entries with none within 16 columns (a 128-byte line of FP64) in the
+  // row before (far_col: the transpose's); -1: unknown
+  int64_t far_row = -1, far_col = -1;
   mutable bool has_csc = false;
   mutable DBuf cp, ri, cv; // CSC
   // BSR (32x32 blocks): bdat holds each block in MFMA A-operand order, entry
@@ -184,6 +187,7 @@ struct ChainCsrOp {
   int ell;            // slots per row of the ELL view, 0: none
   const int* eci;     // ELL view: columns (-1: unused slot) and values
   const double* ev;
+  int64_t far;        // entries that share no line of X with the row before (DMat::far_row; all when unknown)
 };
 int csr_chain_plan_f64(const std::vector<ChainCsrOp>& ops, int in_rows, int p);
 void csr_chain_run_f64(const std::vector<ChainCsrOp>& ops, int in_rows, int wc, const double* X, int ldx, int p,
@@ -205,8 +209,19 @@ int csr_chain_fit_wc(const std::vector<ChainCsrOp>& ops, int in_rows, int p);
 // (k_csr_rm_f64): csr_rm_from_col transposes X (column-major, ld = rows) into
 // panels of rows of csr_rm_ld(p) values (csr_rm_size in all), csr_rm_mul applies one op'd factor to such rows
 // (out_col: Y column-major, ld = S.rows).  fits: the shapes it takes.
-constexpr int RM_MIN_COLS = 12;               // columns from which the form is measured
-constexpr int64_t RM_TERMS_DEFAULT = 1 << 20;  // entries x columns of a factor from which it is the unmeasured choice
+// Lines of the dispatch, us column-major / row-major for chains of two factors:
+// - columns from which the form is measured: fewer paid only for the largest
+//   (16000^2, 20 entries per row, 8 columns 22.6 / 15.6; 8000^2 11.4 / 11.3; 4000^2
+//   8.6 / 9.9; 7 entries per row 16000^2 11.7 / 11.5, 8000^2 7.2 / 8.6);
+// - far entries x columns of a factor from which it is the unmeasured choice:
+//   2000^2, 20 per row, 32 columns (1.2 M entries x columns) 8.5 / 10.9, 48 12.3 /
+//   11.0; 8000^2, 7 per row, 16 columns (0.9 M) 10.8 / 9.7, 64 30.0 / 18.2; one
+//   factor, which pays the transpose alone, 8000^2 32 columns (1.8 M) 7.4 / 7.7,
+//   64 14.3 / 9.2.  Entries near those of the row before are found in a line
+//   that is there already: banded 16000^2, 2 per row, 256 columns (7.8 M) 28.9 /
+//   43.8, 4000^2 10.6 / 19.3, and they count for nothing.
+constexpr int RM_MIN_COLS = 12;
+constexpr int64_t RM_TERMS_DEFAULT = 5 << 18, RM_TERMS_SINGLE = 7 << 18;  // chains; one factor
 int csr_rm_ld(int p);
 size_t csr_rm_size(int rows, int p);
 bool csr_rm_fits(const std::vector<ChainCsrOp>& ops, int in_rows, int p);

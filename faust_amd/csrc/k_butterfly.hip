@@ -819,6 +819,7 @@ static BflyLeafJob leaf_job(const double* v, int n, int logs, const int* colmap,
   M.cv.alloc(sizeof(double) * nz);
   M.has_csc = true;
   M.max_row = M.max_col = 2;
+  M.far_row = M.far_col = 0;  // columns r and r ^ stride: beside the row before's, but for one row in a stride
   M.csr_ell_w = M.csr_tell_w = 2;
   M.csr_ell_ci.alloc(sizeof(int) * nz);
   M.csr_ell_v.alloc(sizeof(double) * nz);

@@ -170,20 +170,49 @@ def _banded(n, per_row):
 
 
 def test_measured_form_is_of_the_row_widths(gpu, monkeypatch):
-    # equal shapes and entries, rows of 3 (4 ELL slots) and of 1 and 5 (8 slots).  Banded factors gather column-major
-    # X from cache, so the first chain keeps one launch per factor; the second, not measured yet, has the default form
-    n, p = 20000, 64
-    narrow, wide = [_banded(n, [3])] * 2, [_banded(n, [1, 5])] * 2
+    # equal shapes and entries, rows of 20 (24 ELL slots) and of 15 and 25 (32 slots).  For banded factors the
+    # unmeasured choice is one launch per factor, and the row-major form the quicker one at this size
+    n, p = 4000, 250
+    narrow, wide = [_banded(n, [20])] * 2, [_banded(n, [15, 25])] * 2
     A, B = faust_amd.Faust(narrow), faust_amd.Faust(wide)
-    X = torch.randn((p, n), dtype=torch.float64, device="cuda")
+    X = torch.randn((256, n), dtype=torch.float64, device="cuda")
     Y = torch.empty_like(X)
     _lib.check(gpu.fh_autotune_clear())
-    monkeypatch.setenv("FH_AUTOTUNE", "0")
-    B.matmul_device(X, Y)
-    assert _launches(B) == 3  # the default, row-major: B's handle has its room
     monkeypatch.setenv("FH_AUTOTUNE", "1")
-    A.matmul_device(X, Y)
-    assert _launches(A) == 2
-    g = _capture(lambda: B.matmul_device(X, Y))
-    assert _launches(B) == 3
-    _replays_right(g, wide, "N", X, Y)
+    A.matmul_device(X[:p], Y[:p])
+    B.matmul_device(X, Y)  # B's handle has the form's room, its form for p columns is not measured
+    assert _launches(A) == _launches(B) == 3
+    g = _capture(lambda: B.matmul_device(X[:p], Y[:p]))
+    assert _launches(B) == 2
+    _replays_right(g, wide, "N", X[:p], Y[:p])
+
+
+@pytest.mark.parametrize("op", ["N", "T"])
+def test_unmeasured_form_is_of_the_locality(gpu, monkeypatch, op):
+    # one launch per factor on column-major intermediates where a row's entries lie by those of the row before;
+    # row-major intermediates for uniform ones of the same size
+    monkeypatch.setenv("FH_AUTOTUNE", "0")
+    n, p = 8000, 64
+    for facs, launches in (([_banded(n, [7])] * 2, 2),
+                           ([faust_amd.rand_csr(n, n, 7, np.random.default_rng(i)) for i in range(2)], 3)):
+        F = faust_amd.Faust(facs)
+        G = F if op == "N" else F.T
+        X = torch.randn((p, n), dtype=torch.float64, device="cuda")
+        Y = G.matmul_device(X)
+        assert _launches(G) == launches
+        want = oracle.chain_multiply(facs, np.asfortranarray(X.cpu().numpy().T), op)
+        assert np.array_equal(Y.cpu().numpy().T, want)
+
+
+def test_measured_form_is_of_the_locality(gpu, monkeypatch):
+    # two entries in every row of both chains: banded ones keep one launch per factor, uniform ones are measured anew
+    n, p = 16000, 64
+    monkeypatch.setenv("FH_AUTOTUNE", "1")
+    _lib.check(gpu.fh_autotune_clear())
+    X = torch.randn((p, n), dtype=torch.float64, device="cuda")
+    Y = torch.empty_like(X)
+    for facs, launches in (([_banded(n, [2])] * 2, 2),
+                           ([faust_amd.rand_csr(n, n, 2, np.random.default_rng(i)) for i in range(2)], 3)):
+        F = faust_amd.Faust(facs)
+        F.matmul_device(X, Y)
+        assert _launches(F) == launches
