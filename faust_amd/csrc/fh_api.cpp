@@ -74,17 +74,18 @@ DMatP make_csr_from_host(int dtype, int m, int n, int nnz, const int32_t* rp, co
   M->max_col = 0;
   for (int j = 0; j < n; ++j) M->max_col = std::max(M->max_col, cp[j + 1] - cp[j]);
   if (dtype == FH_F64) {
-    auto far = [](int nr, const int* ptr, const int* idx) {
-      int64_t n = 0;
-      for (int r = 0; r < nr; ++r) {
-        int q = r > 0 ? ptr[r - 1] : 0;
-        const int qe = r > 0 ? ptr[r] : 0;
+    // from some 256 rows (all of them added 20% to the upload of 20 entries per row)
+    auto far = [nnz](int nr, const int* ptr, const int* idx) -> int64_t {
+      int64_t seen = 0, n = 0;
+      for (int r = 1; r < nr; r += std::max(1, nr / 256)) {
+        int q = ptr[r - 1];
         for (int e = ptr[r]; e < ptr[r + 1]; ++e) {
-          while (q < qe && idx[q] < idx[e] - 16) ++q;
-          n += !(q < qe && idx[q] <= idx[e] + 16);
+          while (q < ptr[r] && idx[q] < idx[e] - 16) ++q;
+          n += !(q < ptr[r] && idx[q] <= idx[e] + 16);
         }
+        seen += ptr[r + 1] - ptr[r];
       }
-      return n;
+      return seen > 0 ? n * nnz / seen : nnz;
     };
     M->far_row = far(m, rp, ci);
     M->far_col = far(n, cp.data(), ri.data());
@@ -259,16 +260,21 @@ bool stream_capturing(hipStream_t st) {
 }
 
 // What the quickest form depends on: direction, columns, each op'd factor's
-// shape, entries, ELL slots (the forms read those where every factor has them)
-// and share of far entries (in eighths: the gathers of column-major X are as
-// quick as these are few), and the device.
+// shape, entries and whether half of them lie far from the row before (the
+// gathers of column-major X are quick where they do not), the ELL slots that
+// decide which kernels the forms run (all factors with at most 8, at most 16;
+// finer, matrices that differ by a column's count would each be measured), and
+// the device.
 static std::string chain_sig(char op, int p, int in_rows, const std::vector<ChainCsrOp>& ops) {
   int dev = 0;
   (void)hipGetDevice(&dev);
   std::string k = std::to_string(dev) + op + ":" + std::to_string(p) + ":" + std::to_string(in_rows);
-  for (const auto& o : ops)
-    k += "," + std::to_string(o.rows) + "/" + std::to_string(o.nnz) + "/" + std::to_string(o.ell) + "/" +
-         std::to_string(o.far * 8 / std::max(o.nnz, 1));
+  int slots = 0;
+  for (const auto& o : ops) {
+    k += "," + std::to_string(o.rows) + "/" + std::to_string(o.nnz) + (o.far * 2 >= o.nnz ? "f" : "n");
+    slots = std::max(slots, o.ell > 0 ? o.ell : 99);
+  }
+  k += slots <= 8 ? "/8" : slots <= 16 ? "/16" : "";
   return k;
 }
 

@@ -113,7 +113,7 @@ struct DMat {
   int64_t nnz = 0;        // CSR: stored entries; dense: -1 until counted
   int max_row = -1, max_col = -1;  // CSR: widest row / column (-1: unknown)
   // CSR: entries with none within 16 columns (a 128-byte line of FP64) in the
-  // row before (far_col: the transpose's); -1: unknown
+  // row before (far_col: the transpose's), estimated; -1: unknown
   int64_t far_row = -1, far_col = -1;
   mutable bool has_csc = false;
   mutable DBuf cp, ri, cv; // CSC

@@ -170,10 +170,10 @@ def _banded(n, per_row):
 
 
 def test_measured_form_is_of_the_row_widths(gpu, monkeypatch):
-    # equal shapes and entries, rows of 20 (24 ELL slots) and of 15 and 25 (32 slots).  For banded factors the
+    # equal shapes and entries, rows of 7 (8 ELL slots) and of 3 and 11 (16 slots).  For banded factors the
     # unmeasured choice is one launch per factor, and the row-major form the quicker one at this size
-    n, p = 4000, 250
-    narrow, wide = [_banded(n, [20])] * 2, [_banded(n, [15, 25])] * 2
+    n, p = 8000, 250
+    narrow, wide = [_banded(n, [7])] * 2, [_banded(n, [3, 11])] * 2
     A, B = faust_amd.Faust(narrow), faust_amd.Faust(wide)
     X = torch.randn((256, n), dtype=torch.float64, device="cuda")
     Y = torch.empty_like(X)
