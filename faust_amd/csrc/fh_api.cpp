@@ -73,11 +73,15 @@ DMatP make_csr_from_host(int dtype, int m, int n, int nnz, const int32_t* rp, co
   for (int i = 0; i < m; ++i) M->max_row = std::max(M->max_row, rp[i + 1] - rp[i]);
   M->max_col = 0;
   for (int j = 0; j < n; ++j) M->max_col = std::max(M->max_col, cp[j + 1] - cp[j]);
-  if (dtype == FH_F64) {
-    // from some 256 rows (all of them added 20% to the upload of 20 entries per row)
+  if (dtype == FH_F64 && std::max(m, n) > 1024) {
+    // from rows of some 1000 entries in all, spread as by chance (5 ns an entry:
+    // all of them doubled the upload); chains of smaller factors run in one launch
     auto far = [nnz](int nr, const int* ptr, const int* idx) -> int64_t {
       int64_t seen = 0, n = 0;
-      for (int r = 1; r < nr; r += std::max(1, nr / 256)) {
+      const int rows = nr - 1;
+      const int look = (int)std::min<int64_t>(rows, std::max<int64_t>(8, (int64_t)nr * 1000 / std::max(nnz, 1)));
+      for (int i = 0; i < look; ++i) {
+        const int r = 1 + (int)((uint64_t)i * 2654435761u % (unsigned)rows);
         int q = ptr[r - 1];
         for (int e = ptr[r]; e < ptr[r + 1]; ++e) {
           while (q < ptr[r] && idx[q] < idx[e] - 16) ++q;

@@ -221,7 +221,7 @@ int csr_chain_fit_wc(const std::vector<ChainCsrOp>& ops, int in_rows, int p);
 //   that is there already: banded 16000^2, 2 per row, 256 columns (7.8 M) 28.9 /
 //   43.8, 4000^2 10.6 / 19.3, and they count for nothing.
 constexpr int RM_MIN_COLS = 12;
-constexpr int64_t RM_TERMS_DEFAULT = 5 << 18, RM_TERMS_SINGLE = 7 << 18;  // chains; one factor
+constexpr int64_t RM_TERMS_DEFAULT = 5 << 18, RM_TERMS_SINGLE = 6 << 18;  // chains; one factor
 int csr_rm_ld(int p);
 size_t csr_rm_size(int rows, int p);
 bool csr_rm_fits(const std::vector<ChainCsrOp>& ops, int in_rows, int p);
