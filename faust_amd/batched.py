@@ -34,7 +34,8 @@ def palm4msa_batched(targets, nfacts, k=None, supports=None, init=None, lambda_i
     int) for the sp projector; supports: per target a list of nfacts 0/1 masks
     (prox supp) instead.  init: per target a list of nfacts initial factors.
     target_err: the FP64 relative error to reach (checked every check_every
-    iterations), one for all targets or one per target."""
+    iterations), one for all targets or one per target.  autotune: accepted
+    and without effect (one GEMM tile is the quickest at every size)."""
     L = lib()
     nt = len(targets)
     As = [np.asfortranarray(a, dtype=np.float64) for a in targets]

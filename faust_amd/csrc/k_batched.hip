@@ -49,6 +49,8 @@ __device__ __forceinline__ int xcd_tile(int per) {
   return per > 0 ? (b & 7) * per + (b >> 3) : b;
 }
 
+// VALU tiles: the plain form of the sums that k_bgemm_mfma is tested against.
+// No call takes them by default.
 template <class T, int TILE>
 __global__ __launch_bounds__(256) void k_bgemm(const BGemmJob<T>* __restrict__ jobs, const int3* __restrict__ tiles,
                                                BScal sc, int ntiles, int per) {

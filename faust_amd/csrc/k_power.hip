@@ -434,8 +434,9 @@ __global__ __launch_bounds__(PW_THREADS) void k_power_iteration(const PwJob* __r
 // [q][r] and needs no columns.  Rows of up to four entries are read into
 // registers while the operator before is computed.
 // Measured on the hierarchy of the Hadamard matrix of order 64 (10 iterations
-// per PALM4MSA, 300 launches of one or two chains of 2 to 10 operators): 339
-// -> 97 us per launch, 168 -> 99 ms in all.  Norms of chains of random
+// per PALM4MSA, 300 launches of one or two chains of 2 to 10 operators): mean
+// 339 -> 104 us per launch (medians 52 with one chain, 18 with two: most of
+// those converge early), 168 -> 99 ms in all by this form alone.  Norms of chains of random
 // factors, us per call: 5 factors of 64^2 with 2 entries per row 374 -> 132,
 // 2 of 64^2 with 32 entries 1920 -> 454, a dense 64^2 one 1037 -> 199.
 constexpr int PL_MAX_OPS = 36;             // operators per chain (both chains' descriptors are kernel arguments)
@@ -1376,7 +1377,11 @@ static void power_iteration_persistent(const std::vector<std::vector<PwOp>>& hs_
 
 // the LDS form's job for a chain, when it fits: every operator dense or of
 // known width, at most PL_ROWS rows and columns, all entries in PL_LDS_BYTES;
-// lds receives the bytes
+// lds receives the bytes.  No estimate decides between this form and the wide
+// one: over the dense and sparse chains that fit it took 1/1.8 to 1/4 of the
+// others' best, and lost only with few long rows (dense 4 x 1024: 1681 us per
+// norm against 1457 wide; 128^2 with one row of 128 entries: 568 against 532
+// persistent).
 static bool pl_job(const std::vector<PwOp>& h, int n, PlJob& j, size_t* lds) {
   if (getenv("FH_POWER_WIDE")) return false;  // one of the other forms is asked for
   if (h.empty() || h.size() > (size_t)PL_MAX_OPS || n < 1 || n > PL_ROWS) return false;
