@@ -206,22 +206,25 @@ ChainWs faust_ws_grow(DBuf* ws, size_t need, int nbuf, hipStream_t st, DBuf* ctl
 
 // The same with room for a form that takes more (want bytes in want_nbuf
 // buffers, 0: none such) where that is to be had without refusing the call:
-// under capture and when memory is short the product keeps to `need`.
-// short_of: the least that could not be had so far, which is not asked for again.
-ChainWs faust_ws_take(DBuf* ws, size_t need, int nbuf, size_t want, int want_nbuf, size_t* short_of, hipStream_t st,
+// under capture, when memory is short, and once a captured graph holds the
+// buffers (its replays write them where they are), the product keeps to `need`.
+ChainWs faust_ws_take(DBuf* ws, size_t need, int nbuf, size_t want, int want_nbuf, WsLimits* lim, hipStream_t st,
                       DBuf* ctl) {
+  const bool capturing = (need > 0 || want > 0) && stream_capturing(st);
+  lim->in_graph = lim->in_graph || capturing;
   if (want > 0) {
     want = std::max(want, need);
     want_nbuf = std::max(want_nbuf, nbuf);
-    bool room = true;
+    bool room = true, enough = true;
     for (int b = 0; b < want_nbuf; ++b) room = room && ws[b].bytes >= want;
+    for (int b = 0; b < nbuf; ++b) enough = enough && ws[b].bytes >= need;
     if (room) return faust_ws_grow(ws, want, want_nbuf, st, ctl);
-    if (want < *short_of && !stream_capturing(st)) {
+    if (want < lim->short_of && !capturing && !(lim->in_graph && enough)) {
       try {
         return faust_ws_grow(ws, want, want_nbuf, st, ctl);
       } catch (const Error&) {
         (void)hipGetLastError();
-        *short_of = want;
+        lim->short_of = want;
       }
     }
   }
@@ -834,7 +837,7 @@ int fh_faust_multiply(fh_faust_t F, char op, const void* X, int p, void* Y, void
       }
     }
     const size_t had[2] = {F->ws[0].bytes, F->ws[1].bytes};
-    const ChainWs ws = faust_ws_take(F->ws, pl.need, pl.nbuf, pl.rm_need, pl.rm_nbuf, &F->ws_short, st);
+    const ChainWs ws = faust_ws_take(F->ws, pl.need, pl.nbuf, pl.rm_need, pl.rm_nbuf, &F->ws_lim, st);
     const ChainForm ran =
         faust_multiply_f64(F->f, op, (const double*)X, p, (double*)Y, st, pl, ws, &F->timers, &F->last_launches);
     if (pl.measure && pl.rm_need > 0 && ran.kind != 3)
@@ -853,7 +856,7 @@ int fh_faust_multiply(fh_faust_t F, char op, const void* X, int p, void* Y, void
     const size_t padded = act_f32                        ? faust_ws_need_f32_tiled(f, op, p, &tbuf)
                           : f.front()->kind == K_CSR ? faust_ws_need_f32_panels(f, op, p, &tbuf)
                                                          : 0;
-    const ChainWs ws = faust_ws_take(F->ws, need, nbuf, padded, tbuf, &F->ws_short, st,
+    const ChainWs ws = faust_ws_take(F->ws, need, nbuf, padded, tbuf, &F->ws_lim, st,
                                      (f.front()->kind == K_BSR && !act_f32) ? &F->ctl : nullptr);
     F->last_launches = faust_multiply_mixed(f, op, X, p, Y, st, ws, &F->timers, act_f32);
   }

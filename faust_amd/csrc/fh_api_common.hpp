@@ -71,6 +71,11 @@ struct FaustTimers {
     for (auto e : spare) (void)hipEventDestroy(e);
   }
 };
+// What keeps a handle's workspace from growing for a form that could be done without.
+struct WsLimits {
+  size_t short_of = SIZE_MAX;  // the least that could not be had so far
+  bool in_graph = false;       // a captured graph uses the buffers
+};
 }  // namespace fh
 
 // A Faust keeps its two ping-pong intermediates (Transform::multiply's
@@ -82,7 +87,7 @@ struct fh_faust_s {
   fh::DBuf ws[2];         // ping-pong activations
   bool ws_owned = false;  // a one-factor product has used ws[0], on ws_stream
   hipStream_t ws_stream = nullptr;
-  size_t ws_short = SIZE_MAX;  // bytes of optional workspace that were not to be had
+  fh::WsLimits ws_lim;
   fh::DBuf ctl;           // control block of the one-launch BSR chain
   int last_launches = 0;  // kernel launches of the last product
   int mul_mode = 0;       // FH_MUL_*
@@ -116,7 +121,7 @@ struct ChainWs {
 };
 size_t faust_ws_need_f64(const std::vector<DMatP>& f, char op, int p, int* nbuf);
 ChainWs faust_ws_grow(DBuf* ws, size_t need, int nbuf, hipStream_t st, DBuf* ctl = nullptr);
-ChainWs faust_ws_take(DBuf* ws, size_t need, int nbuf, size_t want, int want_nbuf, size_t* short_of, hipStream_t st,
+ChainWs faust_ws_take(DBuf* ws, size_t need, int nbuf, size_t want, int want_nbuf, WsLimits* lim, hipStream_t st,
                       DBuf* ctl = nullptr);
 // Execution forms of an FP64 CSR chain, all with the same bits: one launch
 // per factor, the staged one-launch chain (wc columns per workgroup), the

@@ -78,7 +78,36 @@ def test_capture_keeps_to_the_room_there_is(gpu, monkeypatch):
     g = _capture(lambda: F.matmul_device(X, Y))
     assert _launches(F) == 2
     _replays_right(g, facs, "N", X, Y)
-    F.matmul_device(X, Y)  # outside capture there is room
+    F.matmul_device(X, Y)  # the graph holds the buffers: they stay where they are
+    assert _launches(F) == 2
+    _replays_right(g, facs, "N", X, Y)
+
+
+@pytest.mark.parametrize("op", ["N", "T"])
+def test_graph_keeps_its_workspace(gpu, monkeypatch, op):
+    # fewer columns than the graph's, whose row-major form takes more room than the graph's intermediate
+    monkeypatch.setenv("FH_AUTOTUNE", "0")
+    rng = np.random.default_rng(3)
+    dims = ((3001, 3001), (3001, 16001)) if op == "N" else ((16001, 3001), (3001, 3001))
+    facs = [faust_amd.rand_csr(m, n, 9, rng) for m, n in dims]
+    F = faust_amd.Faust(facs)
+    X = torch.randn((400, 16001), dtype=torch.float64, device="cuda")
+    Y = torch.empty((400, 3001), dtype=torch.float64, device="cuda")
+
+    def multiply(p):  # F.T would be a handle of its own
+        _lib.check(gpu.fh_faust_multiply(F.h, op.encode(), X.data_ptr(), p, Y.data_ptr(),
+                                         torch.cuda.current_stream().cuda_stream))
+
+    monkeypatch.setenv("FH_CHAIN_FUSED", "0")
+    multiply(100)
+    g = _capture(lambda: multiply(100))
+    monkeypatch.delenv("FH_CHAIN_FUSED")
+    for autotune in ("0", "1"):
+        monkeypatch.setenv("FH_AUTOTUNE", autotune)
+        multiply(64)
+        assert _launches(F) == 2
+        _replays_right(g, facs, op, X[:100], Y[:100])
+    multiply(400)  # more columns need more room anyway
     assert _launches(F) == 3
 
 
@@ -159,6 +188,7 @@ def test_fp32_capture_keeps_to_the_room_there_is(gpu):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(Y, W.matmul_device(X))
+        transposed()  # and the graph's buffers stay where they are
 
 
 def _banded(n, per_row):
